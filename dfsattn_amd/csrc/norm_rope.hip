@@ -34,26 +34,50 @@ namespace {
 
 constexpr int kMaxChunks = 16;  // at most 16 x 512 channels per row
 
+// How the RoPE table is stored.
+enum TableKind {
+  kTableF32 = 0,   // two fp32 arrays (cos, sin)
+  kTableC64 = 1,   // one array of (re, im) fp32 pairs
+  kTableC128 = 2,  // one array of (re, im) float64 pairs, rounded to fp32 as they are read
+};
+
 struct NormRopeParams {
+  // Up to three tensors of one shape (q, k, v of a layer) in one launch.
+  const uint16_t* x[3];
+  uint16_t* out[3];  // may alias x (in place)
+  const void* weight[3];
+  int w_dtype[3];  // weight dtype, -1 = no norm
+  float eps[3];
+  int rope_kind[3];  // 0 none; 1 complex, float64; 2 real, fp32
+  int n;             // tensors
   int64_t x_sb, x_sl, x_sh;  // element strides of x (channel stride 1)
   int64_t o_sb, o_sl, o_sh;  // element strides of out
   int64_t rows;              // B * L
   int L, H, D, C, nch;
-  int dtype;                 // DFS_DTYPE_BF16 / F16
-  int w_dtype;               // weight dtype, -1 = no norm
-  float eps;
-  int per_head;              // 0: norm over all H*D channels (weight [H*D]); 1: per head (weight [D])
-  int rope_kind;             // 0 none; 1 complex, float64; 2 real, fp32
-  int rope_skip;             // kind 1: rows l < rope_skip are not rotated, table row l - rope_skip
-  int rope_rows;             // kind 2: rows l < rope_rows are rotated, table row l
+  int per_head;   // 0: norm over all H*D channels (weight [H*D]); 1: per head (weight [D])
+  int rope_skip;  // kind 1: rows l < rope_skip are not rotated, table row l - rope_skip
+  int rope_rows;  // kind 2: rows l < rope_rows are rotated, table row l
+  int table_kind;     // TableKind (kind 2 tables are kTableF32)
+  const void* cos_t;  // the complex table for kTableC64 / kTableC128
+  const float* sin_t;
 };
 
-__device__ __forceinline__ float to_f32(uint32_t bits, int dtype) {
-  return dtype == DFS_DTYPE_BF16 ? bf16_bits_to_f32(bits) : f16_bits_to_f32(bits);
+template <bool F16>
+__device__ __forceinline__ float to_f32(uint32_t bits) {
+  return F16 ? f16_bits_to_f32(bits) : bf16_bits_to_f32(bits);
 }
 
-__device__ __forceinline__ uint32_t from_f32(float v, int dtype) {
-  return dtype == DFS_DTYPE_BF16 ? f32_to_bf16_bits(v) : f32_to_f16_bits(v);
+// Two values rounded to the storage type, packed (the first in the low half).
+template <bool F16>
+__device__ __forceinline__ uint32_t pack2(float a, float b) {
+  typedef float f32x2_t __attribute__((ext_vector_type(2)));
+  if constexpr (F16) {
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t){a, b}, h2));
+  } else {
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t){a, b}, b2));
+  }
 }
 
 __device__ __forceinline__ float wave_sum(float v) {
@@ -68,41 +92,62 @@ __device__ __forceinline__ float wave_sum(float v) {
 // the row: 10 for 5,120 channels). The weights and the RoPE table row are
 // fetched together with x, before the reduction, so no second memory round
 // trip sits between the reduction and the stores.
-template <int NCH>
-__global__ void __launch_bounds__(256) norm_rope_kernel(const uint16_t* x, uint16_t* out,  // may alias (in place)
-                                                        const void* __restrict__ weight,
-                                                        const float* __restrict__ cos_t,
-                                                        const float* __restrict__ sin_t, NormRopeParams p) {
+//
+// F16: the storage type; W16: the weights have that type too (else fp32 or the
+// other 16-bit type, converted at run time). Workgroup b takes tensor b % n
+// and the four rows of b / n, so the three tensors' workgroups of a row group
+// run together and read its table row from the cache.
+template <int NCH, bool F16, bool W16>
+__global__ void __launch_bounds__(256) norm_rope_kernel(NormRopeParams p) {
   const int lane = threadIdx.x & 63;
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  const int t = p.n == 1 ? 0 : static_cast<int>(blockIdx.x % 3u);
+  const int64_t row = static_cast<int64_t>(p.n == 1 ? blockIdx.x : blockIdx.x / 3u) * 4 + (threadIdx.x >> 6);
   if (row >= p.rows) return;
   const int64_t b = row / p.L;
   const int l = static_cast<int>(row - b * p.L);
-  const uint16_t* xr = x + b * p.x_sb + static_cast<int64_t>(l) * p.x_sl;
-  uint16_t* orow = out + b * p.o_sb + static_cast<int64_t>(l) * p.o_sl;
-  const bool norm = p.w_dtype >= 0;
+  const uint16_t* xr = p.x[t] + b * p.x_sb + static_cast<int64_t>(l) * p.x_sl;
+  uint16_t* orow = p.out[t] + b * p.o_sb + static_cast<int64_t>(l) * p.o_sl;
+  const int w_dtype = p.w_dtype[t];
+  const bool norm = w_dtype >= 0;
+  const void* weight = p.weight[t];
   // kind 1: complex pairs, table [L - skip][D/2]; kind 2: real, table [rows][D]
-  const bool rope1 = p.rope_kind == 1 && l >= p.rope_skip;
-  const bool rope2 = p.rope_kind == 2 && l < p.rope_rows;
+  const bool rope1 = p.rope_kind[t] == 1 && l >= p.rope_skip;
+  const bool rope2 = p.rope_kind[t] == 2 && l < p.rope_rows;
   const int64_t trow = rope1 ? static_cast<int64_t>(l - p.rope_skip) * (p.D >> 1) : static_cast<int64_t>(l) * p.D;
   // 512 % D == 0 (D = 64, 128, ...): every chunk of a lane has the same
   // channel d, so one slice of the table row serves all of them
   const bool same_d = (512 % p.D) == 0;
 
   uint4 v[NCH];
-  uint4 wv[NCH];  // bf16/f16 weights
+  uint4 wv[NCH];  // weights of the storage type
   float cs[8] = {}, sn[8] = {};
   auto load_table = [&](int d) {
     if (rope1) {
-      const float4 c4 = *reinterpret_cast<const float4*>(cos_t + trow + (d >> 1));
-      const float4 s4 = *reinterpret_cast<const float4*>(sin_t + trow + (d >> 1));
-      cs[0] = c4.x; cs[1] = c4.y; cs[2] = c4.z; cs[3] = c4.w;
-      sn[0] = s4.x; sn[1] = s4.y; sn[2] = s4.z; sn[3] = s4.w;
+      if (p.table_kind == kTableF32) {
+        const float4 c4 = *reinterpret_cast<const float4*>(static_cast<const float*>(p.cos_t) + trow + (d >> 1));
+        const float4 s4 = *reinterpret_cast<const float4*>(p.sin_t + trow + (d >> 1));
+        cs[0] = c4.x; cs[1] = c4.y; cs[2] = c4.z; cs[3] = c4.w;
+        sn[0] = s4.x; sn[1] = s4.y; sn[2] = s4.z; sn[3] = s4.w;
+      } else if (p.table_kind == kTableC64) {
+        const float4* z = reinterpret_cast<const float4*>(static_cast<const float*>(p.cos_t) + 2 * (trow + (d >> 1)));
+        const float4 z0 = z[0], z1 = z[1];
+        cs[0] = z0.x; sn[0] = z0.y; cs[1] = z0.z; sn[1] = z0.w;
+        cs[2] = z1.x; sn[2] = z1.y; cs[3] = z1.z; sn[3] = z1.w;
+      } else {
+        const double2* z = static_cast<const double2*>(p.cos_t) + trow + (d >> 1);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const double2 zi = z[i];
+          cs[i] = static_cast<float>(zi.x);
+          sn[i] = static_cast<float>(zi.y);
+        }
+      }
     } else if (rope2) {
-      const float4 c0 = *reinterpret_cast<const float4*>(cos_t + trow + d);
-      const float4 c1 = *reinterpret_cast<const float4*>(cos_t + trow + d + 4);
-      const float4 s0 = *reinterpret_cast<const float4*>(sin_t + trow + d);
-      const float4 s1 = *reinterpret_cast<const float4*>(sin_t + trow + d + 4);
+      const float* ct = static_cast<const float*>(p.cos_t);
+      const float4 c0 = *reinterpret_cast<const float4*>(ct + trow + d);
+      const float4 c1 = *reinterpret_cast<const float4*>(ct + trow + d + 4);
+      const float4 s0 = *reinterpret_cast<const float4*>(p.sin_t + trow + d);
+      const float4 s1 = *reinterpret_cast<const float4*>(p.sin_t + trow + d + 4);
       cs[0] = c0.x; cs[1] = c0.y; cs[2] = c0.z; cs[3] = c0.w; cs[4] = c1.x; cs[5] = c1.y; cs[6] = c1.z; cs[7] = c1.w;
       sn[0] = s0.x; sn[1] = s0.y; sn[2] = s0.z; sn[3] = s0.w; sn[4] = s1.x; sn[5] = s1.y; sn[6] = s1.z; sn[7] = s1.w;
     }
@@ -113,8 +158,8 @@ __global__ void __launch_bounds__(256) norm_rope_kernel(const uint16_t* x, uint1
     const int e = j * 512 + lane * 8;
     if (e < p.C) {
       const int h = e / p.D, d = e - h * p.D;
-      v[j] = *reinterpret_cast<const uint4*>(xr + h * p.x_sh + d);
-      if (norm && p.w_dtype != DFS_DTYPE_F32)
+      v[j] = load_stream(reinterpret_cast<const uint4*>(xr + h * p.x_sh + d));
+      if (W16 && norm)
         wv[j] = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(weight) + (p.per_head ? d : e));
     }
   }
@@ -124,6 +169,7 @@ __global__ void __launch_bounds__(256) norm_rope_kernel(const uint16_t* x, uint1
 #pragma unroll
   for (int j = 0; j < NCH; ++j) rstd[j] = 1.f;
   if (norm) {
+    const float eps = p.eps[t];
     if (!p.per_head) {
       float ss = 0.f;
 #pragma unroll
@@ -131,12 +177,12 @@ __global__ void __launch_bounds__(256) norm_rope_kernel(const uint16_t* x, uint1
         if (j * 512 + lane * 8 < p.C) {
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
-            const float f = to_f32(u16_at(v[j], i), p.dtype);
+            const float f = to_f32<F16>(u16_at(v[j], i));
             ss += f * f;
           }
         }
       }
-      const float r = 1.0f / sqrtf(wave_sum(ss) / static_cast<float>(p.C) + p.eps);
+      const float r = 1.0f / sqrtf(wave_sum(ss) / static_cast<float>(p.C) + eps);
 #pragma unroll
       for (int j = 0; j < NCH; ++j) rstd[j] = r;
     } else {
@@ -146,14 +192,14 @@ __global__ void __launch_bounds__(256) norm_rope_kernel(const uint16_t* x, uint1
         if (j * 512 + lane * 8 < p.C) {
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
-            const float f = to_f32(u16_at(v[j], i), p.dtype);
+            const float f = to_f32<F16>(u16_at(v[j], i));
             ss += f * f;
           }
         }
         // the D/8 lanes of a head (aligned groups, as 512 % D == 0): a xor
         // butterfly leaves the same bits in all of them
         for (int off = p.D >> 4; off >= 1; off >>= 1) ss += __shfl_xor(ss, off, 64);
-        rstd[j] = 1.0f / sqrtf(ss / static_cast<float>(p.D) + p.eps);
+        rstd[j] = 1.0f / sqrtf(ss / static_cast<float>(p.D) + eps);
       }
     }
   }
@@ -163,25 +209,39 @@ __global__ void __launch_bounds__(256) norm_rope_kernel(const uint16_t* x, uint1
     const int e = j * 512 + lane * 8;
     if (e >= p.C) continue;
     const int h = e / p.D, d = e - h * p.D;
+    uint4* const dst = reinterpret_cast<uint4*>(orow + h * p.o_sh + d);
+    if (!norm && !rope1 && !rope2) {
+      store_stream(dst, v[j]);  // head split alone
+      continue;
+    }
+    uint32_t packed[4];
     float y[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) y[i] = to_f32(u16_at(v[j], i), p.dtype);
+    for (int i = 0; i < 8; ++i) y[i] = to_f32<F16>(u16_at(v[j], i));
     if (norm) {
       float w[8];
-      if (p.w_dtype == DFS_DTYPE_F32) {
+      if constexpr (W16) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) w[i] = to_f32<F16>(u16_at(wv[j], i));
+      } else if (w_dtype == DFS_DTYPE_F32) {
         const float* wp = static_cast<const float*>(weight) + (p.per_head ? d : e);
         const float4 w0 = *reinterpret_cast<const float4*>(wp);
         const float4 w1 = *reinterpret_cast<const float4*>(wp + 4);
         w[0] = w0.x; w[1] = w0.y; w[2] = w0.z; w[3] = w0.w;
         w[4] = w1.x; w[5] = w1.y; w[6] = w1.z; w[7] = w1.w;
       } else {
+        const uint4 wx = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(weight) + (p.per_head ? d : e));
 #pragma unroll
-        for (int i = 0; i < 8; ++i) w[i] = to_f32(u16_at(wv[j], i), p.w_dtype);
+        for (int i = 0; i < 8; ++i)
+          w[i] = w_dtype == DFS_DTYPE_BF16 ? bf16_bits_to_f32(u16_at(wx, i)) : f16_bits_to_f32(u16_at(wx, i));
       }
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float xh = y[i] * rstd[j];  // two roundings, as x_hat = x * rstd; y = x_hat * w
-        y[i] = to_f32(from_f32(xh * w[i], p.dtype), p.dtype);
+      for (int i = 0; i < 8; i += 2) {
+        // two roundings, as x_hat = x * rstd; y = x_hat * w
+        const float a = y[i] * rstd[j], c = y[i + 1] * rstd[j];
+        packed[i / 2] = pack2<F16>(a * w[i], c * w[i + 1]);
+        y[i] = to_f32<F16>(packed[i / 2] & 0xffffu);
+        y[i + 1] = to_f32<F16>(packed[i / 2] >> 16);
       }
     }
     if (!same_d) load_table(d);
@@ -193,8 +253,7 @@ __global__ void __launch_bounds__(256) norm_rope_kernel(const uint16_t* x, uint1
         // only the sums round
         const double re = xe * static_cast<double>(cs[i]) - xo * static_cast<double>(sn[i]);
         const double im = xo * static_cast<double>(cs[i]) + xe * static_cast<double>(sn[i]);
-        y[2 * i] = static_cast<float>(re);
-        y[2 * i + 1] = static_cast<float>(im);
+        packed[i] = pack2<F16>(static_cast<float>(re), static_cast<float>(im));
       }
     } else if (rope2) {
 #pragma clang fp contract(off)
@@ -202,28 +261,22 @@ __global__ void __launch_bounds__(256) norm_rope_kernel(const uint16_t* x, uint1
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float xe = y[2 * i], xo = y[2 * i + 1];
-        y[2 * i] = xe * cs[2 * i] + (-xo) * sn[2 * i];
-        y[2 * i + 1] = xo * cs[2 * i + 1] + xe * sn[2 * i + 1];
+        packed[i] = pack2<F16>(xe * cs[2 * i] + (-xo) * sn[2 * i], xo * cs[2 * i + 1] + xe * sn[2 * i + 1]);
       }
     }
-    uint32_t packed[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      packed[i] = from_f32(y[2 * i], p.dtype) | (from_f32(y[2 * i + 1], p.dtype) << 16);
-    *reinterpret_cast<uint4*>(orow + h * p.o_sh + d) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
+    store_stream(dst, make_uint4(packed[0], packed[1], packed[2], packed[3]));
   }
 }
 
-// Checks shared by both entry points, then the launch. per_head selects the
-// norm group (a head of D channels, weight [D]) and the RoPE form (real
-// tables [rope_rows][D] for rows l < rope_rows); otherwise the group is the
-// whole row (weight [H*D]) and the RoPE complex (tables [L - rope_skip][D/2]
-// for rows l >= rope_skip).
-int launch_norm_rope(const char* name, const void* x, const int64_t* xs3, void* out, const int64_t* os3,
-                     int64_t batch, int64_t seq_len, int64_t heads, int64_t head_dim, int dtype, const void* weight,
-                     int weight_dtype, float eps, const float* cos_table, const float* sin_table, int per_head,
-                     int64_t rope_param, hipStream_t st) {
-  DFS_REQUIRE(x != nullptr && out != nullptr, "%s: x and out must be non-NULL", name);
+// Checks of the layout and the tables shared by the entry points, then the
+// launch. per_head selects the norm group (a head of D channels, weight [D])
+// and the RoPE form (real tables [rope_rows][D] for rows l < rope_rows);
+// otherwise the group is the whole row (weight [H*D]) and the RoPE complex
+// (tables [L - rope_skip][D/2] for rows l >= rope_skip). p arrives with its
+// tensors, weights, eps, tables and strides filled in.
+int launch_norm_rope(const char* name, NormRopeParams& p, int64_t batch, int64_t seq_len, int64_t heads,
+                     int64_t head_dim, int dtype, int per_head, int64_t rope_param, const bool* rope,
+                     hipStream_t st) {
   DFS_REQUIRE(batch > 0 && seq_len > 0 && heads > 0, "%s: batch, seq_len and heads must be positive", name);
   DFS_REQUIRE(head_dim > 0 && head_dim % 8 == 0, "%s: head_dim %lld must be a positive multiple of 8", name,
               (long long)head_dim);
@@ -232,54 +285,61 @@ int launch_norm_rope(const char* name, const void* x, const int64_t* xs3, void* 
   const int64_t C = heads * head_dim;
   DFS_REQUIRE(C <= 512 * kMaxChunks, "%s: heads*head_dim = %lld exceeds %d", name, (long long)C, 512 * kMaxChunks);
   DFS_REQUIRE(dtype == DFS_DTYPE_BF16 || dtype == DFS_DTYPE_F16, "%s: dtype must be bf16 or f16", name);
-  DFS_REQUIRE(weight == nullptr || weight_dtype == DFS_DTYPE_BF16 || weight_dtype == DFS_DTYPE_F16 ||
-                  weight_dtype == DFS_DTYPE_F32,
-              "%s: weight dtype code %d is not supported", name, weight_dtype);
-  DFS_REQUIRE(weight == nullptr || eps >= 0.f, "%s: eps must be non-negative", name);
-  DFS_REQUIRE((cos_table == nullptr) == (sin_table == nullptr), "%s: pass both cos and sin tables or neither", name);
   if (per_head)
     DFS_REQUIRE(rope_param >= 0 && rope_param <= seq_len, "%s: rope_rows %lld must lie in [0, seq_len]", name,
                 (long long)rope_param);
   else
     DFS_REQUIRE(rope_param >= 0 && rope_param < seq_len, "%s: rope_skip %lld must lie in [0, seq_len)", name,
                 (long long)rope_param);
-  for (int i = 0; i < 3; ++i)
-    DFS_REQUIRE(xs3[i] >= 0 && xs3[i] % 8 == 0 && os3[i] >= 0 && os3[i] % 8 == 0,
-                "%s: strides must be non-negative multiples of 8 elements (16-byte rows)", name);
-  DFS_REQUIRE((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out)) % 16 == 0,
-              "%s: x and out must be 16-byte aligned", name);
-  DFS_REQUIRE(weight == nullptr || reinterpret_cast<uintptr_t>(weight) % 16 == 0, "%s: weight must be 16-byte aligned",
-              name);
-  DFS_REQUIRE(cos_table == nullptr ||
-                  (reinterpret_cast<uintptr_t>(cos_table) | reinterpret_cast<uintptr_t>(sin_table)) % 16 == 0,
+  const int64_t strides[6] = {p.x_sb, p.x_sl, p.x_sh, p.o_sb, p.o_sl, p.o_sh};
+  for (int64_t sd : strides)
+    DFS_REQUIRE(sd >= 0 && sd % 8 == 0, "%s: strides must be non-negative multiples of 8 elements (16-byte rows)",
+                name);
+  bool w16 = true;
+  for (int i = 0; i < p.n; ++i) {
+    DFS_REQUIRE(p.x[i] != nullptr && p.out[i] != nullptr, "%s: x and out must be non-NULL", name);
+    DFS_REQUIRE((reinterpret_cast<uintptr_t>(p.x[i]) | reinterpret_cast<uintptr_t>(p.out[i])) % 16 == 0,
+                "%s: x and out must be 16-byte aligned", name);
+    if (p.weight[i] != nullptr) {
+      const int wd = p.w_dtype[i];
+      DFS_REQUIRE(wd == DFS_DTYPE_BF16 || wd == DFS_DTYPE_F16 || wd == DFS_DTYPE_F32,
+                  "%s: weight dtype code %d is not supported", name, wd);
+      DFS_REQUIRE(p.eps[i] >= 0.f, "%s: eps must be non-negative", name);
+      DFS_REQUIRE(reinterpret_cast<uintptr_t>(p.weight[i]) % 16 == 0, "%s: weight must be 16-byte aligned", name);
+      w16 = w16 && wd == dtype;
+    } else {
+      p.w_dtype[i] = -1;
+    }
+    p.rope_kind[i] = p.cos_t == nullptr || !rope[i] ? 0 : (per_head ? 2 : 1);
+  }
+  DFS_REQUIRE(p.cos_t == nullptr ||
+                  (reinterpret_cast<uintptr_t>(p.cos_t) | reinterpret_cast<uintptr_t>(p.sin_t)) % 16 == 0,
               "%s: cos and sin tables must be 16-byte aligned", name);
   DFS_REQUIRE(seq_len < (int64_t(1) << 31), "%s: seq_len too large", name);
-  NormRopeParams p;
-  p.x_sb = xs3[0]; p.x_sl = xs3[1]; p.x_sh = xs3[2];
-  p.o_sb = os3[0]; p.o_sl = os3[1]; p.o_sh = os3[2];
   p.rows = batch * seq_len;
   p.L = static_cast<int>(seq_len);
   p.H = static_cast<int>(heads);
   p.D = static_cast<int>(head_dim);
   p.C = static_cast<int>(C);
   p.nch = static_cast<int>((C + 511) / 512);
-  p.dtype = dtype;
-  p.w_dtype = weight ? weight_dtype : -1;
-  p.eps = eps;
   p.per_head = per_head;
-  p.rope_kind = cos_table == nullptr ? 0 : (per_head ? 2 : 1);
   p.rope_skip = per_head ? 0 : static_cast<int>(rope_param);
   p.rope_rows = per_head ? static_cast<int>(rope_param) : 0;
-  const int64_t blocks = (p.rows + 3) / 4;
+  const int64_t blocks = (p.rows + 3) / 4 * p.n;
   DFS_REQUIRE(blocks < (int64_t(1) << 31), "%s: too many rows", name);
   const dim3 grid(static_cast<unsigned>(blocks)), block(256);
-  const uint16_t* xp = static_cast<const uint16_t*>(x);
-  uint16_t* op = static_cast<uint16_t*>(out);
+  const bool f16 = dtype == DFS_DTYPE_F16;
   switch ((p.nch + 1) / 2) {  // smallest even chunk count that covers the row
-#define DFS_NORM_ROPE_CASE(HALF)                                                                        \
-  case HALF:                                                                                           \
-    hipLaunchKernelGGL(norm_rope_kernel<2 * HALF>, grid, block, 0, st, xp, op, weight, cos_table, sin_table, \
-                       p);                                                                             \
+#define DFS_NORM_ROPE_CASE(HALF)                                                             \
+  case HALF:                                                                                \
+    if (f16 && w16)                                                                         \
+      hipLaunchKernelGGL((norm_rope_kernel<2 * HALF, true, true>), grid, block, 0, st, p);  \
+    else if (f16)                                                                           \
+      hipLaunchKernelGGL((norm_rope_kernel<2 * HALF, true, false>), grid, block, 0, st, p); \
+    else if (w16)                                                                           \
+      hipLaunchKernelGGL((norm_rope_kernel<2 * HALF, false, true>), grid, block, 0, st, p); \
+    else                                                                                    \
+      hipLaunchKernelGGL((norm_rope_kernel<2 * HALF, false, false>), grid, block, 0, st, p); \
     break;
     DFS_NORM_ROPE_CASE(1)
     DFS_NORM_ROPE_CASE(2)
@@ -297,6 +357,28 @@ int launch_norm_rope(const char* name, const void* x, const int64_t* xs3, void* 
   return check_launch(name);
 }
 
+// One tensor with fp32 tables (the two single-tensor entry points).
+int norm_rope_one(const char* name, const void* x, const int64_t* xs3, void* out, const int64_t* os3, int64_t batch,
+                  int64_t seq_len, int64_t heads, int64_t head_dim, int dtype, const void* weight, int weight_dtype,
+                  float eps, const float* cos_table, const float* sin_table, int per_head, int64_t rope_param,
+                  hipStream_t st) {
+  DFS_REQUIRE((cos_table == nullptr) == (sin_table == nullptr), "%s: pass both cos and sin tables or neither", name);
+  NormRopeParams p{};
+  p.n = 1;
+  p.x[0] = static_cast<const uint16_t*>(x);
+  p.out[0] = static_cast<uint16_t*>(out);
+  p.weight[0] = weight;
+  p.w_dtype[0] = weight_dtype;
+  p.eps[0] = eps;
+  p.x_sb = xs3[0]; p.x_sl = xs3[1]; p.x_sh = xs3[2];
+  p.o_sb = os3[0]; p.o_sl = os3[1]; p.o_sh = os3[2];
+  p.table_kind = kTableF32;
+  p.cos_t = cos_table;
+  p.sin_t = sin_table;
+  const bool rope[1] = {true};
+  return launch_norm_rope(name, p, batch, seq_len, heads, head_dim, dtype, per_head, rope_param, rope, st);
+}
+
 }  // namespace
 }  // namespace dfs
 
@@ -306,9 +388,9 @@ extern "C" int dfs_norm_rope(const void* x, int64_t x_sb, int64_t x_sl, int64_t 
                              const float* cos_table, const float* sin_table, int64_t rope_skip,
                              dfs_stream_t stream) {
   const int64_t xs3[3] = {x_sb, x_sl, x_sh}, os3[3] = {o_sb, o_sl, o_sh};
-  return dfs::launch_norm_rope("norm_rope", x, xs3, out, os3, batch, seq_len, heads, head_dim, dtype, weight,
-                               weight_dtype, eps, cos_table, sin_table, 0, rope_skip,
-                               reinterpret_cast<hipStream_t>(stream));
+  return dfs::norm_rope_one("norm_rope", x, xs3, out, os3, batch, seq_len, heads, head_dim, dtype, weight,
+                            weight_dtype, eps, cos_table, sin_table, 0, rope_skip,
+                            reinterpret_cast<hipStream_t>(stream));
 }
 
 extern "C" int dfs_head_norm_rope(const void* x, int64_t x_sb, int64_t x_sl, int64_t x_sh, void* out,
@@ -317,7 +399,46 @@ extern "C" int dfs_head_norm_rope(const void* x, int64_t x_sb, int64_t x_sl, int
                                   float eps, const float* cos_table, const float* sin_table, int64_t rope_rows,
                                   dfs_stream_t stream) {
   const int64_t xs3[3] = {x_sb, x_sl, x_sh}, os3[3] = {o_sb, o_sl, o_sh};
-  return dfs::launch_norm_rope("head_norm_rope", x, xs3, out, os3, batch, seq_len, heads, head_dim, dtype, weight,
-                               weight_dtype, eps, cos_table, sin_table, 1, rope_rows,
-                               reinterpret_cast<hipStream_t>(stream));
+  return dfs::norm_rope_one("head_norm_rope", x, xs3, out, os3, batch, seq_len, heads, head_dim, dtype, weight,
+                            weight_dtype, eps, cos_table, sin_table, 1, rope_rows,
+                            reinterpret_cast<hipStream_t>(stream));
+}
+
+extern "C" int dfs_qkv_heads(const void* q, const void* k, const void* v, int64_t x_sb, int64_t x_sl, int64_t x_sh,
+                             void* q_out, void* k_out, void* v_out, int64_t o_sb, int64_t o_sl, int64_t o_sh,
+                             int64_t batch, int64_t seq_len, int64_t heads, int64_t head_dim, int dtype,
+                             const void* q_weight, int q_weight_dtype, float q_eps, const void* k_weight,
+                             int k_weight_dtype, float k_eps, int per_head, int table_kind, const void* cos_table,
+                             const void* sin_table, int64_t rope_param, dfs_stream_t stream) {
+  using namespace dfs;
+  const char* name = "qkv_heads";
+  DFS_REQUIRE(table_kind >= kTableF32 && table_kind <= kTableC128, "%s: table_kind=%d (supported: 0, 1, 2)", name,
+              table_kind);
+  DFS_REQUIRE(!per_head || table_kind == kTableF32, "%s: the per-head form takes fp32 tables", name);
+  if (table_kind == kTableF32)
+    DFS_REQUIRE((cos_table == nullptr) == (sin_table == nullptr), "%s: pass both cos and sin tables or neither", name);
+  else
+    DFS_REQUIRE(cos_table != nullptr && sin_table == nullptr, "%s: a complex table is passed as cos_table alone", name);
+  NormRopeParams p{};
+  p.n = 3;
+  const void* xs[3] = {q, k, v};
+  void* os[3] = {q_out, k_out, v_out};
+  for (int i = 0; i < 3; ++i) {
+    p.x[i] = static_cast<const uint16_t*>(xs[i]);
+    p.out[i] = static_cast<uint16_t*>(os[i]);
+  }
+  p.weight[0] = q_weight;
+  p.weight[1] = k_weight;
+  p.w_dtype[0] = q_weight_dtype;
+  p.w_dtype[1] = k_weight_dtype;
+  p.eps[0] = q_eps;
+  p.eps[1] = k_eps;
+  p.x_sb = x_sb; p.x_sl = x_sl; p.x_sh = x_sh;
+  p.o_sb = o_sb; p.o_sl = o_sl; p.o_sh = o_sh;
+  p.table_kind = table_kind;
+  p.cos_t = cos_table;
+  p.sin_t = static_cast<const float*>(sin_table);
+  const bool rope[3] = {true, true, false};  // v is split into heads as it is
+  return launch_norm_rope(name, p, batch, seq_len, heads, head_dim, dtype, per_head, rope_param, rope,
+                          reinterpret_cast<hipStream_t>(stream));
 }

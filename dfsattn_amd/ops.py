@@ -472,6 +472,67 @@ def head_norm_rope_heads(x: torch.Tensor, heads: int, weight: Optional[torch.Ten
     return _split_heads(head_norm_rope, x, heads, weight, eps, cos, sin, rope_rows)
 
 
+def qkv_heads_fusable(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
+    """Whether qkv_heads takes these projections in one launch: one shape,
+    dtype, device and stride set, channel stride 1 and 16-byte rows (a
+    cross-attention's shorter k and v go one tensor at a time)."""
+    same = all(t.shape == q.shape and t.dtype == q.dtype and t.device == q.device and t.stride() == q.stride()
+               for t in (k, v))
+    return same and q.dim() == 3 and q.stride(2) == 1 and all(
+        t.data_ptr() % 16 == 0 and t.stride(0) % 8 == 0 and t.stride(1) % 8 == 0 for t in (q, k, v))
+
+
+def _norm_weight(w: Optional[torch.Tensor], length: int, name: str) -> int:
+    if w is None:
+        return 0
+    if w.dim() != 1 or w.numel() != length or not w.is_contiguous():
+        raise ValueError(f"qkv_heads: {name} must be a contiguous [{length}] vector")
+    if w.dtype not in DTYPE_CODE:
+        raise ValueError(f"qkv_heads: {name} dtype {w.dtype} is not supported")
+    return DTYPE_CODE[w.dtype]
+
+
+def qkv_heads(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, heads: int, q_weight: Optional[torch.Tensor],
+              q_eps: float, k_weight: Optional[torch.Tensor], k_eps: float, table=None,
+              rope_rows: Optional[int] = None):
+    """norm_rope_heads (or, with ``rope_rows``, head_norm_rope_heads) of q and
+    k and the head split of v in one launch, for projections that
+    ``qkv_heads_fusable`` accepts: [B, L, H*D] each -> three new [B, H, L, D]
+    tensors. ``table``: complex [L, D/2] frequencies, or (cos, sin) fp32
+    tables of the single-tensor functions, or None."""
+    if not qkv_heads_fusable(q, k, v):
+        raise ValueError("qkv_heads: q, k and v must share shape, dtype, device and strides (16-byte rows)")
+    if q.shape[-1] % heads:
+        raise ValueError(f"expected [B, L, H*D] with H = {heads}, got {tuple(q.shape)}")
+    if q.dtype not in (torch.bfloat16, torch.float16):
+        raise ValueError(f"qkv_heads: q, k and v must be bf16 or f16, got {q.dtype}")
+    B, L, C = q.shape
+    D = C // heads
+    per_head = rope_rows is not None
+    kind, cos, sin, shape = 0, None, None, None
+    if isinstance(table, torch.Tensor):
+        kind = {torch.complex64: 1, torch.complex128: 2}.get(table.dtype, 0)
+        if kind == 0 or per_head:
+            raise ValueError("qkv_heads: a table tensor is complex and belongs to the all-heads form")
+        cos, shape = table, (L, D // 2)
+    elif table is not None:
+        (cos, sin), shape = table, ((rope_rows, D) if per_head else (L, D // 2))
+        if cos.dtype != torch.float32 or sin.dtype != torch.float32:
+            raise ValueError("qkv_heads: cos and sin must be float32")
+    _require_device(q, k, v, q_weight, k_weight, cos, sin)
+    for t in (cos, sin):
+        if t is not None and (tuple(t.shape) != shape or not t.is_contiguous() or t.is_conj()):
+            raise ValueError(f"qkv_heads: tables must be contiguous {shape}, got {tuple(t.shape)}")
+    width = D if per_head else C
+    wq, wk = _norm_weight(q_weight, width, "q_weight"), _norm_weight(k_weight, width, "k_weight")
+    outs = [torch.empty((B, heads, L, D), dtype=q.dtype, device=q.device) for _ in range(3)]
+    _lib.call("dfs_qkv_heads", _ptr(q), _ptr(k), _ptr(v), q.stride(0), q.stride(1), D, *(_ptr(o) for o in outs),
+              heads * L * D, D, L * D, B, L, heads, D, DTYPE_CODE[q.dtype], _ptr(q_weight), wq, float(q_eps),
+              _ptr(k_weight), wk, float(k_eps), int(per_head), kind, _ptr(cos), _ptr(sin),
+              int(rope_rows) if per_head else 0, _stream(q))
+    return tuple(outs)
+
+
 def _vec(t: Optional[torch.Tensor], channels: int, name: str) -> Optional[torch.Tensor]:
     if t is None:
         return None

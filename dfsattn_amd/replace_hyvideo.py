@@ -53,7 +53,7 @@ def fused_qkv_heads_per_head(attn, query: torch.Tensor, key: torch.Tensor, value
     the first rope_rows tokens of q and k (the text after them is not
     rotated), where the reference runs its RMSNorm and RoPE kernels
     (replace_hyvideo.py:252-268)."""
-    from .ops import head_norm_rope_heads
+    from .ops import head_norm_rope_heads, qkv_heads, qkv_heads_fusable
     from .replace_wan import _norm_args
 
     heads = attn.heads
@@ -64,6 +64,8 @@ def fused_qkv_heads_per_head(attn, query: torch.Tensor, key: torch.Tensor, value
                     for t in image_rotary_emb)
     wq, eq = _norm_args(attn.norm_q, d, query)
     wk, ek = _norm_args(attn.norm_k, d, key)
+    if qkv_heads_fusable(query, key, value):  # one launch for the three tensors
+        return qkv_heads(query, key, value, heads, wq, eq, wk, ek, None if cos is None else (cos, sin), rope_rows)
     q = head_norm_rope_heads(query, heads, wq, eq, cos, sin, rope_rows)
     k = head_norm_rope_heads(key, heads, wk, ek, cos, sin, rope_rows)
     v = head_norm_rope_heads(value, heads)

@@ -44,6 +44,14 @@ def rope_tables(rotary_emb: torch.Tensor):
     return f.real.to(torch.float32).contiguous(), f.imag.to(torch.float32).contiguous()
 
 
+def rope_table_readable(table: torch.Tensor) -> bool:
+    """Whether the fused kernel can read the complex table in place: plain
+    contiguous complex64/128 entries (no lazy conjugate or negation) on 16
+    bytes; other forms go through rope_tables' copies."""
+    return (table.dtype in (torch.complex64, torch.complex128) and table.is_contiguous()
+            and not table.is_conj() and not table.is_neg() and table.data_ptr() % 16 == 0)
+
+
 def rms_norm_like(norm, channels: int) -> bool:
     """True for None or an RMSNorm-style module (eps, optional [channels]
     scale, no bias) that the fused kernels can apply."""
@@ -72,15 +80,24 @@ def fused_qkv_heads(attn, query: torch.Tensor, key: torch.Tensor, value: torch.T
                     rotary_emb: Optional[torch.Tensor]):
     """[B, L, H*D] projections -> [B, H, L, D] q, k, v: RMSNorm over all heads
     (attn.norm_q / norm_k) and complex RoPE on q and k, and the head split, in
-    the library's fused kernel (one pass per tensor)."""
-    from .ops import norm_rope_heads
+    the library's fused kernel (one pass per tensor, the three tensors of a
+    self-attention in one launch)."""
+    from .ops import norm_rope_heads, qkv_heads, qkv_heads_fusable
 
     heads = attn.heads
+    wq, eq = _norm_args(attn.norm_q, query.shape[-1], query)
+    wk, ek = _norm_args(attn.norm_k, key.shape[-1], key)
+    if qkv_heads_fusable(query, key, value):
+        # self-attention: one launch, the complex table read as it is
+        table = None
+        if rotary_emb is not None:
+            table = rotary_emb.reshape(-1, rotary_emb.shape[-1])
+            if not rope_table_readable(table):
+                table = rope_tables(rotary_emb)
+        return qkv_heads(query, key, value, heads, wq, eq, wk, ek, table)
     cos = sin = None
     if rotary_emb is not None:
         cos, sin = rope_tables(rotary_emb)
-    wq, eq = _norm_args(attn.norm_q, query.shape[-1], query)
-    wk, ek = _norm_args(attn.norm_k, key.shape[-1], key)
     q = norm_rope_heads(query, heads, wq, eq, cos, sin)
     k = norm_rope_heads(key, heads, wk, ek, cos, sin)
     v = norm_rope_heads(value, heads)

@@ -348,6 +348,29 @@ int dfs_head_norm_rope(const void* x, int64_t x_sb, int64_t x_sl, int64_t x_sh,
                        dfs_stream_t stream);
 
 /*
+ * q, k and v of one layer in one launch: dfs_norm_rope (per_head 0) or
+ * dfs_head_norm_rope (per_head 1) of q and of k with their own weights
+ * (NULL: no norm), and the head split alone of v. The three tensors share
+ * shape and strides, and so do the three outputs.
+ *   table_kind 0: cos_table / sin_table are fp32 arrays as for the single
+ *     tensors (both NULL: no RoPE);
+ *   table_kind 1 or 2 (per_head 0): cos_table is the complex table
+ *     [L - rope_skip][D/2] itself, fp32 or float64 (re, im) pairs, sin_table
+ *     NULL; float64 entries are rounded to fp32 as they are read, which is the
+ *     conversion made at replace_wan.py:193-198.
+ * rope_param: rope_skip (per_head 0) or rope_rows (per_head 1).
+ */
+int dfs_qkv_heads(const void* q, const void* k, const void* v, int64_t x_sb,
+                  int64_t x_sl, int64_t x_sh, void* q_out, void* k_out,
+                  void* v_out, int64_t o_sb, int64_t o_sl, int64_t o_sh,
+                  int64_t batch, int64_t seq_len, int64_t heads,
+                  int64_t head_dim, int dtype, const void* q_weight,
+                  int q_weight_dtype, float q_eps, const void* k_weight,
+                  int k_weight_dtype, float k_eps, int per_head,
+                  int table_kind, const void* cos_table, const void* sin_table,
+                  int64_t rope_param, dfs_stream_t stream);
+
+/*
  * DiT block elementwise steps around the attention (the Wan transformer
  * block of diffusers that the reference's Wan driver loads,
  * wan21_t2v_inference.py:102-103; not part of the reference's own code).

@@ -117,6 +117,47 @@ def test_head_norm_rope_matches_oracle(dev, B, L, H, D, dtype, wdt, rope, rows):
     assert bool(((got.float() - r).abs() <= 2.0 ** -mant * (pair + r.abs()) + 1e-6).all())
 
 
+QKV_CASES = [
+    # B, L, H, D, dtype, (q, k) weight dtypes, table (None, "f32", "c64", "c128"; "real": per head), video rows
+    (1, 301, 40, 128, torch.bfloat16, (torch.bfloat16, torch.bfloat16), "c128", 301),  # 4 rows per group: a ragged end
+    (1, 1, 2, 64, torch.float16, (torch.float16, torch.float16), "c64", 1),  # one token
+    (2, 77, 3, 96, torch.bfloat16, (torch.bfloat16, torch.float32), "c128", 77),  # 512 % D != 0, mixed weights
+    (1, 50, 64, 128, torch.float16, (torch.bfloat16, torch.bfloat16), "f32", 50),  # widest row, other 16-bit weights
+    (1, 66, 5, 64, torch.bfloat16, (None, torch.bfloat16), None, 66),  # k normed alone, no RoPE
+    (2, 130, 24, 128, torch.bfloat16, (torch.bfloat16, torch.bfloat16), "real", 99),  # text rows after 99
+    (1, 35, 3, 64, torch.float16, (torch.float32, None), "real", 35),
+]
+
+
+@pytest.mark.parametrize("B,L,H,D,dtype,wdt,table,rows", QKV_CASES)
+def test_qkv_heads_matches_single_tensors(dev, B, L, H, D, dtype, wdt, table, rows):
+    """q, k and v in one launch (complex tables read in place) against one
+    launch per tensor with fp32 tables: the same arithmetic, so the same bits."""
+    from dfsattn_amd import ops
+    print(f"qkv_heads B={B} L={L} H={H} D={D} {dtype} w={wdt} table={table} rows={rows}", flush=True)
+    g = torch.Generator().manual_seed(L * H + D + 2)
+    x = [(torch.randn(B, L, H * D, generator=g) * 3).to(dev, dtype) for _ in range(3)]
+    per_head = table == "real"
+    w = [None if t is None else (torch.rand(D if per_head else H * D, generator=g) + 0.5).to(dev, t) for t in wdt]
+    cos = sin = tab = None
+    if per_head:
+        ang = (torch.rand(rows, D // 2, generator=g, dtype=torch.float64) * 50).repeat_interleave(2, dim=-1)
+        cos, sin = torch.cos(ang).float().to(dev), torch.sin(ang).float().to(dev)
+        tab = (cos, sin)
+    elif table is not None:
+        ang = torch.rand(L, D // 2, generator=g, dtype=torch.float64) * 50
+        z = torch.polar(torch.ones_like(ang), ang).to(dev)
+        z = z.to(torch.complex64) if table == "c64" else z
+        cos, sin = z.real.float().contiguous(), z.imag.float().contiguous()
+        tab = (cos, sin) if table == "f32" else z
+    got = ops.qkv_heads(*x, H, w[0], 1e-6, w[1], 1e-5, tab, rows if per_head else None)
+    for t, weight, eps, out in zip(x[:2], w, (1e-6, 1e-5), got):
+        ref = (ops.head_norm_rope_heads(t, H, weight, eps, cos, sin, rows) if per_head
+               else ops.norm_rope_heads(t, H, weight, eps, cos, sin))
+        assert torch.equal(out, ref)
+    assert torch.equal(got[2], x[2].unflatten(2, (H, D)).transpose(1, 2))
+
+
 @torch.no_grad()
 def test_hunyuan_fused_qkv_matches_torch_path(dev):
     """The Hunyuan processor's fused per-head norm + RoPE against its torch
