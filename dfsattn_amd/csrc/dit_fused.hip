@@ -15,18 +15,34 @@ namespace {
 
 constexpr int kMaxChunks = 16;  // at most 16 x 512 channels per row
 
-__device__ __forceinline__ float to_f32(uint32_t bits, int dtype) {
-  return dtype == DFS_DTYPE_BF16 ? bf16_bits_to_f32(bits) : f16_bits_to_f32(bits);
+template <bool F16>
+__device__ __forceinline__ float to_f32(uint32_t bits) {
+  return F16 ? f16_bits_to_f32(bits) : bf16_bits_to_f32(bits);
 }
 
-__device__ __forceinline__ uint32_t from_f32(float v, int dtype) {
-  return dtype == DFS_DTYPE_BF16 ? f32_to_bf16_bits(v) : f32_to_f16_bits(v);
+template <bool F16>
+__device__ __forceinline__ uint32_t from_f32(float v) {
+  return F16 ? f32_to_f16_bits(v) : f32_to_bf16_bits(v);
 }
 
+template <int CTRL>
+__device__ __forceinline__ float dpp_plus(float v) {
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+
+// Sum over the wave, the same bits in every lane: each step adds a value and
+// its mirror (or the other half's), so both sides form the same sum. Register
+// moves throughout; through LDS (__shfl_xor) the two reductions of a row were
+// the longest part of its chain.
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
+  v = dpp_plus<0xB1>(v);   // quad_perm [1, 0, 3, 2]
+  v = dpp_plus<0x4E>(v);   // quad_perm [2, 3, 0, 1]
+  v = dpp_plus<0x141>(v);  // row_half_mirror: the other four lanes of eight
+  v = dpp_plus<0x140>(v);  // row_mirror: the other eight of sixteen
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
 __device__ __forceinline__ void load8(const float* p, float* v) {
@@ -36,41 +52,58 @@ __device__ __forceinline__ void load8(const float* p, float* v) {
   v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
 }
 
-// One wave per row of C channels (16-byte chunks, 512 channels per wave
-// step, the row held in registers for the two-pass mean and variance).
-template <int NCH>
-__global__ void __launch_bounds__(256) adaln_kernel(const uint16_t* __restrict__ x, int64_t rows, int C, int dtype,
+// One wave per RPW rows of C channels (16-byte chunks, 512 channels per wave
+// step, the rows held in registers for the two-pass mean and variance).
+// HBM-bound (one read and one write of x; a device copy of the same bytes
+// takes 125 us at 32,760 x 5,120). The fp32 vectors come from L2 for every
+// wave, 4 bytes a channel and vector beside a row's own 2, so large calls give
+// a wave two rows per fetch: 140 us against 158 with one row and 211 with the
+// types chosen at run time and the reductions through LDS. A workgroup per row
+// with the vectors kept in registers took 208 us (two barriers per row).
+template <int NCH, bool F16, int RPW>
+__global__ void __launch_bounds__(256) adaln_kernel(const uint16_t* __restrict__ x, int64_t rows, int C,
                                                     const float* __restrict__ weight, const float* __restrict__ bias,
                                                     const float* __restrict__ scale, const float* __restrict__ shift,
                                                     float eps, uint16_t* __restrict__ out) {
   const int lane = threadIdx.x & 63;
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  const int64_t row = (static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6)) * RPW;
   if (row >= rows) return;
+  const int n = rows - row < RPW ? 1 : RPW;  // rows of this wave; a missing second row repeats the first
   const uint16_t* xr = x + row * C;
-  uint4 v[NCH];
-  float sum = 0.f;
+  uint4 v[RPW][NCH];
 #pragma unroll
-  for (int j = 0; j < NCH; ++j) {
-    const int e = j * 512 + lane * 8;
-    if (e < C) {
-      v[j] = *reinterpret_cast<const uint4*>(xr + e);
+  for (int q = 0; q < RPW; ++q)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) sum += to_f32(u16_at(v[j], i), dtype);
+    for (int j = 0; j < NCH; ++j) {
+      const int e = j * 512 + lane * 8;
+      v[q][j] = make_uint4(0, 0, 0, 0);
+      if (e < C) v[q][j] = load_stream(reinterpret_cast<const uint4*>(xr + (q < n ? q : 0) * static_cast<int64_t>(C) + e));
     }
+  float mean[RPW], rstd[RPW];
+#pragma unroll
+  for (int q = 0; q < RPW; ++q) {
+    float sum = 0.f;
+#pragma unroll
+    for (int j = 0; j < NCH; ++j)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) sum += to_f32<F16>(u16_at(v[q][j], i));  // zeros past the row's end
+    mean[q] = wave_sum(sum) / static_cast<float>(C);
   }
-  const float mean = wave_sum(sum) / static_cast<float>(C);
-  float sq = 0.f;
 #pragma unroll
-  for (int j = 0; j < NCH; ++j) {
-    if (j * 512 + lane * 8 < C) {
+  for (int q = 0; q < RPW; ++q) {
+    float sq = 0.f;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float d = to_f32(u16_at(v[j], i), dtype) - mean;
-        sq += d * d;
+    for (int j = 0; j < NCH; ++j) {
+      if (j * 512 + lane * 8 < C) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const float d = to_f32<F16>(u16_at(v[q][j], i)) - mean[q];
+          sq += d * d;
+        }
       }
     }
+    rstd[q] = 1.0f / sqrtf(wave_sum(sq) / static_cast<float>(C) + eps);
   }
-  const float rstd = 1.0f / sqrtf(wave_sum(sq) / static_cast<float>(C) + eps);
 #pragma unroll
   for (int j = 0; j < NCH; ++j) {
     const int e = j * 512 + lane * 8;
@@ -80,37 +113,74 @@ __global__ void __launch_bounds__(256) adaln_kernel(const uint16_t* __restrict__
     if (bias) load8(bias + e, b);
     if (scale) load8(scale + e, sc);
     if (shift) load8(shift + e, sh);
-    uint32_t packed[4];
 #pragma unroll
-    for (int i = 0; i < 8; i += 2) {
-      float y2[2];
+    for (int q = 0; q < RPW; ++q) {
+      if (q >= n) continue;
+      uint32_t packed[4];
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
+      for (int i = 0; i < 8; i += 2) {
+        float y2[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
 #pragma clang fp contract(off)
-        float y = (to_f32(u16_at(v[j], i + t), dtype) - mean) * rstd;
-        if (weight) y = y * w[i + t];
-        if (bias) y = y + b[i + t];
-        if (scale) y = y * (1.0f + sc[i + t]);
-        if (shift) y = y + sh[i + t];
-        y2[t] = y;
+          float y = (to_f32<F16>(u16_at(v[q][j], i + t)) - mean[q]) * rstd[q];
+          if (weight) y = y * w[i + t];
+          if (bias) y = y + b[i + t];
+          if (scale) y = y * (1.0f + sc[i + t]);
+          if (shift) y = y + sh[i + t];
+          y2[t] = y;
+        }
+        packed[i / 2] = from_f32<F16>(y2[0]) | (from_f32<F16>(y2[1]) << 16);
       }
-      packed[i / 2] = from_f32(y2[0], dtype) | (from_f32(y2[1], dtype) << 16);
+      store_stream(reinterpret_cast<uint4*>(out + (row + q) * C + e),
+                   make_uint4(packed[0], packed[1], packed[2], packed[3]));
     }
-    *reinterpret_cast<uint4*>(out + row * C + e) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
   }
 }
 
-// out = float(x) + float(y) * gate[c], eight channels per thread.
+struct AdalnArgs {
+  const uint16_t* x;
+  int64_t rows;
+  int C;
+  const float *weight, *bias, *scale, *shift;
+  float eps;
+  uint16_t* out;
+};
+
+template <int NCH, int RPW>
+void launch_adaln_as(const AdalnArgs& a, bool f16, hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>((a.rows + 4 * RPW - 1) / (4 * RPW)));
+  if (f16)
+    adaln_kernel<NCH, true, RPW><<<grid, 256, 0, s>>>(a.x, a.rows, a.C, a.weight, a.bias, a.scale, a.shift, a.eps, a.out);
+  else
+    adaln_kernel<NCH, false, RPW><<<grid, 256, 0, s>>>(a.x, a.rows, a.C, a.weight, a.bias, a.scale, a.shift, a.eps, a.out);
+}
+
+// Two rows per wave from 8,192 rows on, where the halved wave count still
+// gives each of the 1,024 SIMDs four waves, and while two rows fit the
+// registers (20 chunks of 16 bytes: 218 VGPRs at 5,120 channels).
+template <int NCH>
+void launch_adaln(const AdalnArgs& a, bool f16, hipStream_t s) {
+  if constexpr (NCH <= 10) {
+    if (a.rows >= 8192) return launch_adaln_as<NCH, 2>(a, f16, s);
+  }
+  launch_adaln_as<NCH, 1>(a, f16, s);
+}
+
+// out = float(x) + float(y) * gate[c], eight channels per thread. HBM-bound:
+// streaming accesses and one conversion per type reach 6.4 TB/s (158 us at
+// 32,760 x 5,120; 174 us with ordinary accesses and run-time types).
 // x and out may alias (each thread reads its eight elements before writing them).
+template <bool F16>
 __global__ void __launch_bounds__(256) gated_residual_kernel(const uint16_t* x, const uint16_t* __restrict__ y,
                                                              const float* __restrict__ gate, int64_t n8, int C,
-                                                             int dtype, uint16_t* out) {
+                                                             uint16_t* out) {
   const int64_t i8 = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i8 >= n8) return;
   const int64_t e = i8 * 8;
+  const uint4 xv = load_stream(reinterpret_cast<const uint4*>(x + e));
+  const uint4 yv = load_stream(reinterpret_cast<const uint4*>(y + e));
   const int c = static_cast<int>(e % C);
-  const uint4 xv = *reinterpret_cast<const uint4*>(x + e);
-  const uint4 yv = *reinterpret_cast<const uint4*>(y + e);
   float g[8];
   load8(gate + c, g);
   uint32_t packed[4];
@@ -120,11 +190,11 @@ __global__ void __launch_bounds__(256) gated_residual_kernel(const uint16_t* x, 
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
 #pragma clang fp contract(off)
-      r[t] = to_f32(u16_at(xv, i + t), dtype) + to_f32(u16_at(yv, i + t), dtype) * g[i + t];
+      r[t] = to_f32<F16>(u16_at(xv, i + t)) + to_f32<F16>(u16_at(yv, i + t)) * g[i + t];
     }
-    packed[i / 2] = from_f32(r[0], dtype) | (from_f32(r[1], dtype) << 16);
+    packed[i / 2] = from_f32<F16>(r[0]) | (from_f32<F16>(r[1]) << 16);
   }
-  *reinterpret_cast<uint4*>(out + e) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
+  store_stream(reinterpret_cast<uint4*>(out + e), make_uint4(packed[0], packed[1], packed[2], packed[3]));
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -145,29 +215,21 @@ extern "C" int dfs_adaln_modulate(const void* x, int64_t rows, int64_t channels,
   DFS_REQUIRE(eps >= 0.f, "%s: eps must be non-negative", name);
   const void* ptrs[6] = {x, out, weight, bias, scale, shift};
   for (const void* q : ptrs) DFS_REQUIRE(q == nullptr || aligned16(q), "%s: operands must be 16-byte aligned", name);
-  const int64_t blocks = (rows + 3) / 4;
-  DFS_REQUIRE(blocks < (int64_t(1) << 31), "%s: too many rows", name);
+  DFS_REQUIRE((rows + 3) / 4 < (int64_t(1) << 31), "%s: too many rows", name);
   const int nch = static_cast<int>((channels + 511) / 512);
-  const dim3 grid(static_cast<unsigned>(blocks)), block(256);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const uint16_t* xp = static_cast<const uint16_t*>(x);
-  uint16_t* op = static_cast<uint16_t*>(out);
-  const int C = static_cast<int>(channels);
+  const AdalnArgs a{static_cast<const uint16_t*>(x), rows, static_cast<int>(channels), weight, bias, scale, shift, eps,
+                    static_cast<uint16_t*>(out)};
+  const bool f16 = dtype == DFS_DTYPE_F16;
   switch ((nch + 1) / 2) {  // smallest even chunk count that covers the row
-#define DFS_ADALN_CASE(HALF)                                                                                  \
-  case HALF:                                                                                                  \
-    hipLaunchKernelGGL(adaln_kernel<2 * HALF>, grid, block, 0, st, xp, rows, C, dtype, weight, bias, scale, shift, \
-                       eps, op);                                                                              \
-    break;
-    DFS_ADALN_CASE(1)
-    DFS_ADALN_CASE(2)
-    DFS_ADALN_CASE(3)
-    DFS_ADALN_CASE(4)
-    DFS_ADALN_CASE(5)
-    DFS_ADALN_CASE(6)
-    DFS_ADALN_CASE(7)
-    DFS_ADALN_CASE(8)
-#undef DFS_ADALN_CASE
+    case 1: launch_adaln<2>(a, f16, st); break;
+    case 2: launch_adaln<4>(a, f16, st); break;
+    case 3: launch_adaln<6>(a, f16, st); break;
+    case 4: launch_adaln<8>(a, f16, st); break;
+    case 5: launch_adaln<10>(a, f16, st); break;
+    case 6: launch_adaln<12>(a, f16, st); break;
+    case 7: launch_adaln<14>(a, f16, st); break;
+    case 8: launch_adaln<16>(a, f16, st); break;
     default:
       set_error("%s: internal chunk count %d", name, nch);
       return 1;
@@ -189,9 +251,13 @@ extern "C" int dfs_gated_residual(const void* x, const void* y, const float* gat
   const int64_t n8 = rows * channels / 8;
   const int64_t blocks = (n8 + 255) / 256;
   DFS_REQUIRE(blocks < (int64_t(1) << 31), "%s: too many elements", name);
-  hipLaunchKernelGGL(gated_residual_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0,
-                     reinterpret_cast<hipStream_t>(stream), static_cast<const uint16_t*>(x),
-                     static_cast<const uint16_t*>(y), gate, n8, static_cast<int>(channels), dtype,
-                     static_cast<uint16_t*>(out));
+  const dim3 grid(static_cast<unsigned>(blocks)), block(256);
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const uint16_t *xp = static_cast<const uint16_t*>(x), *yp = static_cast<const uint16_t*>(y);
+  uint16_t* op = static_cast<uint16_t*>(out);
+  if (dtype == DFS_DTYPE_F16)
+    gated_residual_kernel<true><<<grid, block, 0, st>>>(xp, yp, gate, n8, static_cast<int>(channels), op);
+  else
+    gated_residual_kernel<false><<<grid, block, 0, st>>>(xp, yp, gate, n8, static_cast<int>(channels), op);
   return check_launch(name);
 }

@@ -320,6 +320,31 @@ def test_adaln_modulate_matches_torch(dev, rows, C, mode):
     torch.testing.assert_close(got.float(), ref.float(), rtol=2.0 ** -7, atol=1e-5)
 
 
+@pytest.mark.parametrize("dtype,rows,C", [
+    (torch.bfloat16, 8191, 520), (torch.bfloat16, 8192, 520), (torch.float16, 8193, 64),  # one | two rows per wave
+    (torch.bfloat16, 8197, 5120),  # a lone last row in the widest two-row form
+    (torch.float16, 8195, 5128), (torch.float16, 1, 8192),  # wider rows stay at one per wave
+])
+def test_adaln_rows_per_wave(dev, dtype, rows, C):
+    """The two-rows-per-wave form of large calls and the sizes around it
+    against torch's LayerNorm in fp32 on the same device."""
+    import torch.nn.functional as F
+    from dfsattn_amd import ops
+    print(f"adaln {dtype} rows={rows} C={C}", flush=True)
+    g = torch.Generator().manual_seed(rows + C)
+    x = (torch.randn(1, rows, C, generator=g) * 3 + 0.5).to(dev, dtype)
+    sc, sh = torch.randn(C, generator=g).to(dev) * 0.2, torch.randn(C, generator=g).to(dev)
+    got = ops.adaln_modulate(x, 1e-6, scale=sc, shift=sh)
+    ref = (F.layer_norm(x.float(), (C,), eps=1e-6) * (1 + sc) + sh).to(dtype)
+    assert got.shape == x.shape and got.dtype == dtype
+    # statistics summed in another order: a few ulp of fp32 in y, i.e. mostly
+    # the same 16-bit value, otherwise one unit in its last place; where shift
+    # cancels the product the fp32 error (2^-22 of terms below 16) remains
+    assert float((got == ref).float().mean()) > 0.99
+    ulp = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)
+    torch.testing.assert_close(got.float(), ref.float(), rtol=ulp, atol=1e-5)
+
+
 def test_gated_residual_bit_exact(dev):
     from dfsattn_amd import ops
     g = torch.Generator().manual_seed(31)
