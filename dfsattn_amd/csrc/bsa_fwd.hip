@@ -11,23 +11,15 @@
 // tiles are copied straight from global memory into LDS with 16-byte buffer
 // loads.
 //
-// Two schedules:
-//  * split (default): one workgroup = one (head, 128-row query block), four
-//    waves of 32 query rows walking the row's kept key blocks; two
-//    workgroups per CU, single K and V buffers, the K copy of the next block
-//    overlapping softmax and PV, the V copy overlapping the next QK^T; the
-//    other workgroup on the CU fills the gaps. With f16 operands the row's
-//    reference maximum comes from its first block and later blocks skip the
-//    maximum (a block is redone only if its P overflows f16); the LDS operand
-//    reads run four MFMAs ahead, and the QK phase runs at raised wave
-//    priority. A row visits its key blocks in order of distance from its own
-//    block, so neighbouring query blocks fetch shared key blocks together.
-//  * ping-pong (DFSATTN_AMD_BSA_KERNEL=pp, f16 operands): one eight-wave
-//    workgroup per CU for two adjacent query blocks, the two four-wave groups
-//    alternating MFMA and softmax phases half a cycle apart (described at the
-//    kernel). It overlaps VALU with MFMA work but concentrates the LDS operand
-//    reads of a CU into its MFMA phases; at the 75.6k-token shape it runs
-//    10-15% slower than split.
+// Schedule: one workgroup = one (head, 128-row query block), four waves of 32
+// query rows walking the row's kept key blocks; two workgroups per CU, single
+// K and V buffers, the K copy of the next block overlapping softmax and PV,
+// the V copy overlapping the next QK^T; the other workgroup on the CU fills
+// the gaps. The row's reference maximum comes from its first block and later
+// blocks skip the maximum (a block is redone only if its P leaves its range);
+// the LDS operand reads run four MFMAs ahead, and the QK phase runs at raised
+// wave priority. A row visits its key blocks in order of distance from its own
+// block, so neighbouring query blocks fetch shared key blocks together.
 //
 // LDS rows are 256 bytes; 16-byte chunk c of row r is stored at chunk
 // c ^ (r % 16) so the 32 rows read by one MFMA operand fetch hit distinct
@@ -159,28 +151,6 @@ __device__ __forceinline__ void load_q(const uint16_t* __restrict__ q, const Bsa
     qf[s] = __builtin_bit_cast(typename QkOp::vec, src ? src[2 * s + hl] : make_uint4(0, 0, 0, 0));
 }
 
-// S^T (128 keys x this wave's 32 queries) = K Q^T from an LDS K tile; the
-// operands of the next 32-key chunk are fetched while this chunk's MFMAs run.
-template <int D, typename QkOp>
-__device__ __forceinline__ void qk_tile(const uint16_t* k_tile, const typename QkOp::vec* qf, int l32, int hl,
-                                        f32x16* s, const f32x16& init = f32x16{}) {
-  constexpr int CPR = D / 8, DS = D / 16;
-  uint4 a[2][DS];
-#pragma unroll
-  for (int ds = 0; ds < DS; ++ds) a[0][ds] = lds_chunk<CPR>(k_tile, l32, ds * 2 + hl);
-#pragma unroll
-  for (int kc = 0; kc < 4; ++kc) {
-    if (kc + 1 < 4) {
-#pragma unroll
-      for (int ds = 0; ds < DS; ++ds) a[(kc + 1) & 1][ds] = lds_chunk<CPR>(k_tile, (kc + 1) * 32 + l32, ds * 2 + hl);
-    }
-    s[kc] = init;
-#pragma unroll
-    for (int ds = 0; ds < DS; ++ds)
-      s[kc] = QkOp::run(__builtin_bit_cast(typename QkOp::vec, a[kc & 1][ds]), qf[ds], s[kc]);
-  }
-}
-
 // Keys >= valid of the block get -inf (only the last block can be partial).
 __device__ __forceinline__ void mask_tail(f32x16* s, int valid, int hl) {
 #pragma unroll
@@ -188,58 +158,6 @@ __device__ __forceinline__ void mask_tail(f32x16* s, int valid, int hl) {
 #pragma unroll
     for (int r = 0; r < 16; ++r)
       if (kc * 32 + (r >> 2) * 8 + hl * 4 + (r & 3) >= valid) s[kc][r] = -INFINITY;
-}
-
-// Online-softmax bookkeeping of one block: returns the new running maximum
-// (log2 domain) and rescales O and l by exp2(m_old - m_new). With LAZY the
-// rescale is skipped when no row's maximum moved (alpha == 1 exactly).
-template <int DCH, bool LAZY>
-__device__ __forceinline__ float softmax_max(const f32x16* s, float scale_log2, float& m, float& lsum,
-                                             f32x16* o) {
-  float mx = -INFINITY;
-#pragma unroll
-  for (int kc = 0; kc < 4; ++kc)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[kc][r]);
-  const float mnew = fmaxf(m, xhalf_max(mx) * scale_log2);
-  if (!LAZY || __any(mnew > m)) {
-    const float alpha = exp2_fast(m - mnew);
-    lsum *= alpha;
-#pragma unroll
-    for (int i = 0; i < DCH; ++i)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) o[i][r] *= alpha;
-  }
-  m = mnew;
-  return mnew;
-}
-
-// O^T += V^T P^T, 16 keys per step. P = exp2(S * scale * log2e - m) is formed
-// step by step so its VALU work runs under the previous step's MFMAs; it is
-// rounded to the PV operand type and the row sum accumulates the rounded
-// values (numerator and denominator of O = P V / sum(P) see the same P).
-template <int D, typename PvOp>
-__device__ __forceinline__ void pv_tile(const uint16_t* v_tile, const f32x16* s, float scale_log2, float mnew,
-                                        float& lsum, f32x16* o, int l32, int hl) {
-  constexpr int DCH = D / 32;
-#pragma unroll
-  for (int ks = 0; ks < 8; ++ks) {
-    const f32x16& src = s[ks >> 1];
-    const int r0 = (ks & 1) * 8;
-    typename PvOp::pair pr[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      pr[j] = PvOp::pack(exp2_fast(fmaf(src[r0 + 2 * j], scale_log2, -mnew)),
-                         exp2_fast(fmaf(src[r0 + 2 * j + 1], scale_log2, -mnew)));
-      lsum = PvOp::sum2(pr[j], lsum);
-    }
-    const typename PvOp::vec pf = __builtin_bit_cast(typename PvOp::vec, pr);
-#pragma unroll
-    for (int dc = 0; dc < DCH; ++dc) {
-      const uint4 a = lds_chunk<16>(v_tile, dc * 32 + l32, ks * 2 + hl);
-      o[dc] = PvOp::run(__builtin_bit_cast(typename PvOp::vec, a), pf, o[dc]);
-    }
-  }
 }
 
 // f16 Q fragments with c = scale * log2(e) folded in (q * c rounded to f16),
@@ -285,17 +203,18 @@ __device__ __forceinline__ void load_q_scaled(const uint16_t* __restrict__ q, co
     for (int i = 0; i < 8; ++i) qf[s][i] = static_cast<_Float16>(x[s][i] * inv);
 }
 
-// Lazy online softmax on S' = S c - m, where the running reference m enters
+// Lazy online softmax on S' = S - m, where the running reference m enters
 // through the QK MFMA's C input (negm holds -m in every element, times qinv
-// = 2^-r for a row whose Q fragments carry 2^-r). On a row's
-// first block m becomes the block maximum; later, m moves only when some row
-// of the wave sees a block maximum above m + kLazyTau, and O and l are
-// rescaled then. The result is the same softmax: numerator and denominator
-// share the reference. (With f16 P the split kernel calls this only for a
-// row's first block and for a block whose P overflowed f16.)
+// = 2^-r for a row whose Q fragments carry 2^-r). S' and m are in units of
+// 1 / c in the log2 domain: c = 1 for f16 Q (prescaled), scale * log2(e) for
+// bf16 Q (whose bits are kept). On a row's first block m becomes the block
+// maximum; later, m moves only when some row of the wave sees a block maximum
+// above m + kLazyTau, and O and l are rescaled then. The result is the same
+// softmax: numerator and denominator share the reference. The kernel calls
+// this only for a row's first block and for a block whose P left its range.
 constexpr float kLazyTau = 8.0f;
 template <int DCH>
-__device__ __forceinline__ void softmax_lazy(f32x16* s, bool first, float& m, float& lsum, f32x16* o,
+__device__ __forceinline__ void softmax_lazy(f32x16* s, float c, bool first, float& m, float& lsum, f32x16* o,
                                              f32x16& negm, float qinv = 1.f) {
   float mx = -INFINITY;
 #pragma unroll
@@ -303,7 +222,7 @@ __device__ __forceinline__ void softmax_lazy(f32x16* s, bool first, float& m, fl
 #pragma unroll
     for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[kc][r]);
   const float bm = xhalf_max(mx);
-  if (first || __any(bm > kLazyTau)) {
+  if (first || __any(bm * c > kLazyTau)) {
     float shift = first ? bm : fmaxf(bm, 0.f);
     if (!(shift > -INFINITY)) shift = 0.f;  // a row with every key masked keeps m
 #pragma unroll
@@ -311,7 +230,7 @@ __device__ __forceinline__ void softmax_lazy(f32x16* s, bool first, float& m, fl
 #pragma unroll
       for (int r = 0; r < 16; ++r) s[kc][r] -= shift;
     if (!first) {
-      const float alpha = exp2_fast(-shift);
+      const float alpha = exp2_fast(-shift * c);
       lsum *= alpha;
 #pragma unroll
       for (int i = 0; i < DCH; ++i)
@@ -324,35 +243,10 @@ __device__ __forceinline__ void softmax_lazy(f32x16* s, bool first, float& m, fl
   }
 }
 
-// O^T += V^T P^T with P = exp2(S') (S' already in log2 units relative to m).
-template <int D, typename PvOp>
-__device__ __forceinline__ void pv_tile_log2(const uint16_t* v_tile, const f32x16* s, float& lsum, f32x16* o,
-                                             int l32, int hl) {
-  constexpr int DCH = D / 32;
-#pragma unroll
-  for (int ks = 0; ks < 8; ++ks) {
-    const f32x16& src = s[ks >> 1];
-    const int r0 = (ks & 1) * 8;
-    typename PvOp::pair pr[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      pr[j] = PvOp::pack(exp2_fast(src[r0 + 2 * j]), exp2_fast(src[r0 + 2 * j + 1]));
-      lsum = PvOp::sum2(pr[j], lsum);
-    }
-    const typename PvOp::vec pf = __builtin_bit_cast(typename PvOp::vec, pr);
-#pragma unroll
-    for (int dc = 0; dc < DCH; ++dc) {
-      const uint4 a = lds_chunk<16>(v_tile, dc * 32 + l32, ks * 2 + hl);
-      o[dc] = PvOp::run(__builtin_bit_cast(typename PvOp::vec, a), pf, o[dc]);
-    }
-  }
-}
-
 // Scheduling of an MFMA phase: the LDS operand reads run kAhead MFMAs ahead
 // of their MFMAs, so each read's latency is covered by the MFMAs before its
-// use (in the ping-pong schedule the other wave on the SIMD is doing VALU
-// work and cannot fill MFMA gaps; in the split schedule the two waves of a
-// SIMD come from independent workgroups and often read at the same time).
+// use (the two waves of a SIMD come from independent workgroups and often
+// read at the same time).
 // Pinned with scheduling-group barriers:
 // kAhead reads, then alternately one MFMA and one read, then the last MFMAs.
 constexpr int kAhead = 4;
@@ -369,22 +263,23 @@ __device__ __forceinline__ void pin_read_ahead_schedule() {
 }
 
 // O^T += V^T P^T from an LDS V^T tile and P held in registers.
-template <int D>
-__device__ __forceinline__ void pv_tile_regs(const uint16_t* v_tile, const f16x8* pf, f32x16* o, int l32, int hl) {
+template <int D, typename PvOp>
+__device__ __forceinline__ void pv_tile_regs(const uint16_t* v_tile, const typename PvOp::vec* pf, f32x16* o, int l32,
+                                             int hl) {
   constexpr int DCH = D / 32, N = 8 * DCH;
   uint4 a[N];
 #pragma unroll
   for (int i = 0; i < N; ++i) a[i] = lds_chunk<16>(v_tile, (i % DCH) * 32 + l32, (i / DCH) * 2 + hl);
 #pragma unroll
   for (int i = 0; i < N; ++i)
-    o[i % DCH] = MfmaOp<true>::run(__builtin_bit_cast(f16x8, a[i]), pf[i / DCH], o[i % DCH]);
+    o[i % DCH] = PvOp::run(__builtin_bit_cast(typename PvOp::vec, a[i]), pf[i / DCH], o[i % DCH]);
   pin_read_ahead_schedule<N>();
 }
 
 // S^T = init + K Q^T from an LDS K tile, with the read-ahead schedule above.
-template <int D>
-__device__ __forceinline__ void qk_tile_ahead(const uint16_t* k_tile, const f16x8* qf, int l32, int hl, f32x16* s,
-                                              const f32x16& init = f32x16{}) {
+template <int D, typename QkOp>
+__device__ __forceinline__ void qk_tile_ahead(const uint16_t* k_tile, const typename QkOp::vec* qf, int l32, int hl,
+                                              f32x16* s, const f32x16& init) {
   constexpr int CPR = D / 8, DS = D / 16, N = 4 * DS;
   uint4 a[N];
 #pragma unroll
@@ -393,25 +288,28 @@ __device__ __forceinline__ void qk_tile_ahead(const uint16_t* k_tile, const f16x
   for (int kc = 0; kc < 4; ++kc) s[kc] = init;
 #pragma unroll
   for (int i = 0; i < N; ++i)
-    s[i / DS] = MfmaOp<true>::run(__builtin_bit_cast(f16x8, a[i]), qf[i % DS], s[i / DS]);
+    s[i / DS] = QkOp::run(__builtin_bit_cast(typename QkOp::vec, a[i]), qf[i % DS], s[i / DS]);
   pin_read_ahead_schedule<N>();
 }
 
-// P = exp2(S') of a whole block as f16 PV operands; lblk receives this lane's
-// share of the block's row sum (of the rounded values).
-__device__ __forceinline__ void make_p(const f32x16* s, f16x8* pf, float& lblk) {
+// P = exp2(c S') of a whole block as PV operands; lblk receives this lane's
+// share of the block's row sum (of the rounded values). LOG2: S' arrives in
+// log2 units (c = 1).
+template <typename PvOp, bool LOG2>
+__device__ __forceinline__ void make_p(const f32x16* s, float c, typename PvOp::vec* pf, float& lblk) {
   lblk = 0.f;
 #pragma unroll
   for (int ks = 0; ks < 8; ++ks) {
     const f32x16& src = s[ks >> 1];
     const int r0 = (ks & 1) * 8;
-    f16x2 pr[4];
+    typename PvOp::pair pr[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      pr[j] = MfmaOp<true>::pack(exp2_fast(src[r0 + 2 * j]), exp2_fast(src[r0 + 2 * j + 1]));
-      lblk = MfmaOp<true>::sum2(pr[j], lblk);
+      const float x0 = src[r0 + 2 * j], x1 = src[r0 + 2 * j + 1];
+      pr[j] = PvOp::pack(exp2_fast(LOG2 ? x0 : x0 * c), exp2_fast(LOG2 ? x1 : x1 * c));
+      lblk = PvOp::sum2(pr[j], lblk);
     }
-    pf[ks] = __builtin_bit_cast(f16x8, pr);
+    pf[ks] = __builtin_bit_cast(typename PvOp::vec, pr);
   }
 }
 
@@ -552,9 +450,10 @@ __device__ __forceinline__ void bsa_split_block(const uint16_t* __restrict__ q, 
   f32x16 o[DCH];
 #pragma unroll
   for (int i = 0; i < DCH; ++i) o[i] = f32x16{};
-  // f16 Q/K: S arrives in log2 units relative to m (lazy softmax); bf16 Q/K:
-  // S is scaled in the exponent and m is the exact running maximum.
-  float m = QK_F16 ? 0.f : -INFINITY, lsum = 0.f;
+  // Lazy softmax: S arrives relative to m, in log2 units with f16 Q/K (Q
+  // prescaled) and in units of q.k with bf16 Q/K (scaled in the exponent).
+  const float c = QK_F16 ? 1.f : p.scale_log2;
+  float m = 0.f, lsum = 0.f;
 
   if (beg < end) {
     const uint32_t head_bytes = static_cast<uint32_t>(p.R) * D * 2;
@@ -572,7 +471,7 @@ __device__ __forceinline__ void bsa_split_block(const uint16_t* __restrict__ q, 
     else
       load_q<D, QkOp>(q, p, h, qrow, hl, qf);
     const float qinv = 1.f / row_scale;
-    f32x16 negm = f32x16{};  // -m (times 2^-r) in every element (f16 Q/K)
+    f32x16 negm = f32x16{};  // -m (times 2^-r) in every element
     // Column list of this row into LDS (read back with uniform ds_reads), and
     // Q fragments forced complete here so no wait for them lands in the loop.
     const int n = distance_order_cols<256>(Kb, col_idx, qb, beg, end - beg, cols,
@@ -598,21 +497,18 @@ __device__ __forceinline__ void bsa_split_block(const uint16_t* __restrict__ q, 
       wait_vmcnt<V_LOADS>();  // this wave's K copies have landed
       block_barrier();        // ... and everybody else's
       f32x16 s[4];
-      if constexpr (QK_F16) {
-        // Raised wave priority for the QK MFMAs: when both waves of a SIMD
-        // reach their MFMA phases together, this one runs ahead and the two
-        // drift into alternating MFMA and softmax phases (measured 1.6%).
-        __builtin_amdgcn_s_setprio(1);
-        qk_tile_ahead<D>(k_lds, qf, l32, hl, s, negm);
-        __builtin_amdgcn_s_setprio(0);
-        if constexpr (SCALED) {  // rows whose q c' exceeds the f16 range carry 2^-r
+      // Raised wave priority for the QK MFMAs: when both waves of a SIMD
+      // reach their MFMA phases together, this one runs ahead and the two
+      // drift into alternating MFMA and softmax phases (measured 1.6%).
+      __builtin_amdgcn_s_setprio(1);
+      qk_tile_ahead<D, QkOp>(k_lds, qf, l32, hl, s, negm);
+      __builtin_amdgcn_s_setprio(0);
+      if constexpr (SCALED) {  // rows whose q c' exceeds the f16 range carry 2^-r
 #pragma unroll
-          for (int kc = 0; kc < 4; ++kc)
+        for (int kc = 0; kc < 4; ++kc)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) s[kc][r] *= row_scale;
-        }
-      } else
-        qk_tile<D, QkOp>(k_lds, qf, l32, hl, s);
+          for (int r = 0; r < 16; ++r) s[kc][r] *= row_scale;
+      }
       block_barrier();  // K tile fully consumed
       kcopy.template issue<K_LOADS>(krs, kb_next * TILE_BYTES, k_base, ws);
       if ((Lk & 127) != 0 && kb == (Lk >> 7)) {  // the keys' last block is partial
@@ -620,35 +516,24 @@ __device__ __forceinline__ void bsa_split_block(const uint16_t* __restrict__ q, 
         asm volatile("" : "+s"(valid));  // compares stay in this (rare) branch
         mask_tail(s, valid, hl);
       }
-      if constexpr (QK_F16 && PV_F16) {
-        // The row reference m is set from the first block's maximum. Later
-        // blocks skip the maximum: P = exp2(S - m) is formed directly and
-        // accepted unless it overflows f16 (some S - m >= 16, which turns
-        // the block's row sum inf); only then is the block redone with a
-        // moved reference. P <= 2^16 keeps f16's 11-bit precision.
-        if (t == 0) softmax_lazy<DCH>(s, true, m, lsum, o, negm, qinv);
-        f16x8 pf[8];
-        float lblk;
-        make_p(s, pf, lblk);
-        if (t > 0 && __any(!(lblk < INFINITY))) {
-          softmax_lazy<DCH>(s, false, m, lsum, o, negm, qinv);
-          make_p(s, pf, lblk);
-        }
-        lsum += lblk;
-        wait_vmcnt<K_LOADS>();  // V copies landed (the next K may be in flight)
-        block_barrier();
-        pv_tile_regs<D>(v_lds, pf, o, l32, hl);
-      } else if constexpr (QK_F16) {
-        softmax_lazy<DCH>(s, t == 0, m, lsum, o, negm, qinv);
-        wait_vmcnt<K_LOADS>();
-        block_barrier();
-        pv_tile_log2<D, PvOp>(v_lds, s, lsum, o, l32, hl);
-      } else {
-        const float mnew = softmax_max<DCH, true>(s, p.scale_log2, m, lsum, o);
-        wait_vmcnt<K_LOADS>();
-        block_barrier();
-        pv_tile<D, PvOp>(v_lds, s, p.scale_log2, mnew, lsum, o, l32, hl);
+      // The row reference m is set from the first block's maximum. Later
+      // blocks skip the maximum: P = exp2(S - m) is formed directly and
+      // accepted unless it leaves its range (f16: some S - m >= 16 overflows,
+      // which turns the block's row sum inf; bf16: a sum above 2^16 moves the
+      // reference too, so that O keeps its fp32 range); only then is the
+      // block redone with a moved reference. P keeps its full precision.
+      if (t == 0) softmax_lazy<DCH>(s, c, true, m, lsum, o, negm, qinv);
+      typename PvOp::vec pf[8];
+      float lblk;
+      make_p<PvOp, QK_F16>(s, c, pf, lblk);
+      if (t > 0 && __any(!(lblk < (PV_F16 ? INFINITY : 65536.f)))) {
+        softmax_lazy<DCH>(s, c, false, m, lsum, o, negm, qinv);
+        make_p<PvOp, QK_F16>(s, c, pf, lblk);
       }
+      lsum += lblk;
+      wait_vmcnt<K_LOADS>();  // V copies landed (the next K may be in flight)
+      block_barrier();
+      pv_tile_regs<D, PvOp>(v_lds, pf, o, l32, hl);
       block_barrier();  // V tile fully consumed
       vcopy.template issue<V_LOADS>(vrs, kb_next * TILE_BYTES, v_base, ws);
       kb = kb_next;
@@ -656,7 +541,7 @@ __device__ __forceinline__ void bsa_split_block(const uint16_t* __restrict__ q, 
     wait_vmcnt_0();  // the trailing copies have landed before the workgroup's LDS is released
   }
   store_out<D>(p, VARLEN ? min(max(p.cu_q[1], 0), p.L) : p.L, p.exps ? p.exps[2 * p.H + h] : 0, out, out_perm,
-               lse, o, m, lsum, h, qrow, hl);
+               lse, o, m * c, lsum, h, qrow, hl);
 }
 
 template <int D, bool QK_F16, bool PV_F16, bool VARLEN, bool SCALED>

@@ -525,6 +525,28 @@ def test_bsa_fwd_rising_and_negative_logits(dev, scale):
         (float((out - ref).abs().max()), mean_rel(out, ref))
 
 
+@pytest.mark.parametrize("d,length,scale,v_size", [(128, 1200, None, 1.0), (64, 641, None, 1e30), (128, 385, 0.6, 1.0)])
+def test_bsa_fwd_bf16_operands_moving_reference(dev, d, length, scale, v_size):
+    """bf16 operands, whose scores stay in units of q.k: block maxima that
+    rise by far more than the 2^16 bound on a block's sums, so the reference
+    moves and blocks are redone; V near the top of the bf16 range."""
+    heads = 2
+    g = torch.Generator().manual_seed(27)
+    q, k, v = (torch.randn((1, heads, length, d), generator=g) for _ in range(3))
+    nb = math.ceil(length / 128)
+    k = k * torch.linspace(0.2, 4.0, nb).repeat_interleave(128)[:length][None, None, :, None]
+    q[:, 1], k[:, 1] = -q[:, 1].abs(), k[:, 1].abs()  # head 1: large negative logits
+    q, k, v = q.to(torch.bfloat16), k.to(torch.bfloat16), (v * v_size).to(torch.bfloat16)
+    mask = torch.rand((heads, nb, nb), generator=g) < 0.6
+    mask[:, torch.arange(nb), torch.arange(nb)] = True
+    out = _run_bsa(dev, q, k, v, mask, torch.bfloat16, torch.float32, scale=scale)
+    ref = orc.masked_attention(q, k, v, mask, scale=scale)
+    assert torch.isfinite(out).all()
+    # P is rounded to bf16 (2^-9 each): the class tolerance of the shape test
+    assert mean_rel(out, ref) <= 3e-3, mean_rel(out, ref)
+    assert float((out - ref).abs().max()) <= 2e-2 * v_size
+
+
 def test_wrappers_reject_bad_index_operands(dev):
     """Index operands must be contiguous int32 on the operands' device, and
     CSR offsets must cover every (head, query block) row: checked on the host
