@@ -60,6 +60,16 @@ struct BsaParams {
   const uint16_t* q_src;
   const int32_t* q_rows;
   int q_src_f16;
+  // Element strides of out between heads and between rows.
+  int64_t o_sh, o_sl;
+  // Order and split of the work (see wg_work): query blocks from long_row on
+  // are started first, each by long_parts workgroups; of an XCD's other query
+  // blocks the first full_rows are one workgroup each and the rest parts.
+  int long_row, long_parts, full_rows, parts;
+  // Partial results of split query blocks: O [slot][128][D] and (m, l)
+  // [slot][128][2], fp32, m in log2 units.
+  float* part_o;
+  float* part_ml;
 };
 
 // Start of the D-element Q row of execution row qrow of head h: q_perm's row,
@@ -124,31 +134,84 @@ __device__ __forceinline__ float xhalf_sum(float v) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// (head, query block) of this workgroup; false for a padding slot.
-// Hardware deals workgroup b to XCD b % 8 and each XCD runs its workgroups in
-// increasing b. The i-th workgroup of XCD x takes head h = i / S and query
-// block ((x + h) % 8) * S + i % S (S = ceil(Qb / 8)), so all eight XCDs sweep
-// the same head together: one head's K/V (38.7 MB at 75.6k tokens) stays
-// resident in the shared last-level cache while each XCD's L2 serves
-// neighbouring query blocks. The range an XCD takes rotates with the head,
-// so rows of unequal length (HunyuanVideo's dense text rows at the end of
-// every head) spread over all XCDs instead of one.
-__device__ __forceinline__ bool wg_coords(const BsaParams& p, int& h, int& qb) {
-  const int b = blockIdx.x, xcd = b & 7, i = b >> 3;
-  const int S = (p.Qb + 7) >> 3;
+// Work of one workgroup: a query block of a head, or part `piece` of the
+// `pieces` its column list is cut into, whose result goes to partial slot
+// `slot`.
+struct Work {
+  int h, qb, piece, pieces, slot;
+};
+
+// Split query blocks come in two lists: the long ones (8 * ceil(heads *
+// blocks / 8), when long_parts > 1), then the tails of the XCDs' lists.
+__host__ __device__ inline int long_per_head(const BsaParams& p) { return p.Qb - p.long_row; }
+__host__ __device__ inline int long_per_xcd(const BsaParams& p) { return (p.H * long_per_head(p) + 7) >> 3; }
+__host__ __device__ inline int blocks_per_xcd(const BsaParams& p) { return (p.long_row + 7) >> 3; }  // of one head
+__host__ __device__ inline int split_long(const BsaParams& p) { return p.long_parts > 1 ? 8 * long_per_xcd(p) : 0; }
+__host__ __device__ inline int split_tail(const BsaParams& p) {
+  return p.parts > 1 ? 8 * (blocks_per_xcd(p) * p.H - p.full_rows) : 0;
+}
+// Query block i of XCD x's list of ordinary blocks; false for a padding slot.
+__device__ __forceinline__ bool ordinary_block(const BsaParams& p, int x, int i, int& h, int& qb) {
+  const int S = blocks_per_xcd(p);
   h = i / S;
-  qb = ((xcd + h) & 7) * S + (i - h * S);
-  return qb < p.Qb;
+  qb = ((x + h) & 7) * S + (i - h * S);
+  return qb < p.long_row;
+}
+__device__ __forceinline__ bool long_block(const BsaParams& p, int g, int& h, int& qb) {
+  const int n = long_per_head(p);
+  h = g / n;
+  qb = p.long_row + (g - h * n);
+  return h < p.H;
 }
 
-template <int D, typename QkOp>
-__device__ __forceinline__ void load_q(const uint16_t* __restrict__ q, const BsaParams& p, int h, int qrow,
-                                       int hl, typename QkOp::vec* qf) {
-  bool f16;  // the bf16-operand path takes bf16 rows only (q_perm or a bf16 q_src)
+// Work of this workgroup; false for a padding slot. Hardware deals workgroup
+// b to XCD b % 8 and each XCD runs its workgroups in increasing b.
+//  * Ordinary query blocks: the i-th of XCD x takes head h = i / S and query
+//    block ((x + h) % 8) * S + i % S (S = ceil(blocks / 8)), so all eight XCDs
+//    sweep the same head together: one head's K/V (38.7 MB at 75.6k tokens)
+//    stays resident in the shared last-level cache while each XCD's L2 serves
+//    neighbouring query blocks. The range an XCD takes rotates with the head.
+//  * Long query blocks (HunyuanVideo's text rows keep every key block, three
+//    times the others at sparsity 0.3) go first: started in their place at the
+//    end of their head, the last head's ran on alone after everything else.
+//  * Where the workgroups would not fill the chip's slots evenly, the last
+//    blocks of every XCD's list (all of them for small problems) are cut into
+//    parts along their columns and bsa_combine_kernel adds the parts up.
+__device__ __forceinline__ bool wg_work(const BsaParams& p, Work& wk) {
+  const int x = blockIdx.x & 7;
+  int j = blockIdx.x >> 3;
+  const int n_long = long_per_xcd(p) * p.long_parts;
+  if (j < n_long) {
+    const int g = j / p.long_parts;
+    wk.piece = j - g * p.long_parts;
+    wk.pieces = p.long_parts;
+    wk.slot = (g * 8 + x) * p.long_parts + wk.piece;
+    return long_block(p, g * 8 + x, wk.h, wk.qb);
+  }
+  j -= n_long;
+  int i = j;
+  wk.piece = 0;
+  wk.pieces = 1;
+  wk.slot = 0;
+  if (j >= p.full_rows && p.parts > 1) {
+    const int t = (j - p.full_rows) / p.parts;
+    wk.piece = j - p.full_rows - t * p.parts;
+    wk.pieces = p.parts;
+    wk.slot = split_long(p) * p.long_parts + (t * 8 + x) * p.parts + wk.piece;
+    i = p.full_rows + t;
+  }
+  return ordinary_block(p, x, i, wk.h, wk.qb);
+}
+
+// This lane's share of a Q row as it lies in memory (16-byte chunk 2 s + hl
+// of every 32); f16 tells its type. Issued before the column list is built:
+// the permutation read and the row read then run under it.
+template <int D>
+__device__ __forceinline__ void load_q_raw(const uint16_t* __restrict__ q, const BsaParams& p, int h, int qrow, int hl,
+                                           uint4* raw, bool& f16) {
   const uint4* src = reinterpret_cast<const uint4*>(q_row_ptr<D>(q, p, h, qrow, f16));
 #pragma unroll
-  for (int s = 0; s < D / 16; ++s)
-    qf[s] = __builtin_bit_cast(typename QkOp::vec, src ? src[2 * s + hl] : make_uint4(0, 0, 0, 0));
+  for (int s = 0; s < D / 16; ++s) raw[s] = src ? src[2 * s + hl] : make_uint4(0, 0, 0, 0);
 }
 
 // Keys >= valid of the block get -inf (only the last block can be partial).
@@ -170,21 +233,18 @@ __device__ __forceinline__ void mask_tail(f32x16* s, int valid, int hl) {
 // a scale where |q c| < 2^15 always holds (f16 q_perm values, or Q source
 // values of a head inside the f16 range, times c < 0.5).
 template <int D, bool SCALED>
-__device__ __forceinline__ void load_q_scaled(const uint16_t* __restrict__ q, const BsaParams& p, int h, int qrow,
-                                              int hl, f16x8* qf, float& row_scale) {
+__device__ __forceinline__ void scale_q(const uint4* raw, bool f16, const BsaParams& p, int h, f16x8* qf,
+                                        float& row_scale) {
   float c = p.scale_log2;
   // q_perm holds q 2^-eq; a Q source is read unscaled
   if (SCALED && p.exps) c = ldexpf(c, (p.q_src ? 0 : p.exps[h]) + p.exps[p.H + h]);
-  bool f16;
-  const uint4* src = reinterpret_cast<const uint4*>(q_row_ptr<D>(q, p, h, qrow, f16));
   float x[D / 16][8];
   float mx = 0.f;
 #pragma unroll
   for (int s = 0; s < D / 16; ++s) {
-    const uint4 raw = src ? src[2 * s + hl] : make_uint4(0, 0, 0, 0);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      x[s][i] = (f16 ? f16_bits_to_f32(u16_at(raw, i)) : bf16_bits_to_f32(u16_at(raw, i))) * c;
+      x[s][i] = (f16 ? f16_bits_to_f32(u16_at(raw[s], i)) : bf16_bits_to_f32(u16_at(raw[s], i))) * c;
       if (SCALED) mx = fmaxf(mx, fabsf(x[s][i]));
     }
   }
@@ -325,7 +385,7 @@ __device__ __forceinline__ void store_out(const BsaParams& p, int Lq, int ev, vo
   const float inv = ltot > 0.f ? ldexpf(1.0f / ltot, ev) : 0.f;  // v_t holds v 2^-ev
   if (qrow >= Lq) return;
   const int orow = out_perm ? out_perm[qrow] : qrow;
-  const int64_t obase = (static_cast<int64_t>(h) * p.Lo + orow) * D;
+  const int64_t obase = h * p.o_sh + orow * p.o_sl;
 #pragma unroll
   for (int dc = 0; dc < DCH; ++dc)
 #pragma unroll
@@ -349,6 +409,22 @@ __device__ __forceinline__ void store_out(const BsaParams& p, int Lq, int ev, vo
     lse[static_cast<int64_t>(h) * p.Lo + qrow] = ltot > 0.f ? (m + log2f(ltot)) * 0.69314718055994531f : -INFINITY;
 }
 
+// This wave's 32 rows of a part: O, m (log2 units) and l as they are.
+template <int D>
+__device__ __forceinline__ void store_part(const BsaParams& p, int slot, const f32x16* o, float m, float lsum, int w,
+                                           int l32, int hl) {
+  const float ltot = xhalf_sum(lsum);
+  const int64_t row = static_cast<int64_t>(slot) * 128 + w * 32 + l32;
+  float* dst = p.part_o + row * D;
+#pragma unroll
+  for (int dc = 0; dc < D / 32; ++dc)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<float4*>(dst + dc * 32 + g * 8 + hl * 4) =
+          make_float4(o[dc][g * 4 + 0], o[dc][g * 4 + 1], o[dc][g * 4 + 2], o[dc][g * 4 + 3]);
+  if (hl == 0) *reinterpret_cast<float2*>(p.part_ml + row * 2) = make_float2(m, ltot);
+}
+
 // Column list of one CSR row into LDS, ordered by distance |c - qb| from the
 // row's own block (c = qb first, then qb - 1, qb + 1, qb - 2, ...). The
 // workgroups resident on an XCD at one time run neighbouring Hilbert query
@@ -356,7 +432,7 @@ __device__ __forceinline__ void store_out(const BsaParams& p, int Lq, int ev, vo
 // the same key blocks at about the same time (2% fewer L2 misses than
 // ascending order with the partner row's shared columns first, 0.4-1.2%
 // faster). Columns live in a bitmap at bit 2|c - qb| + (c > qb), compacted in
-// bit order. Columns >= Kb (the keys' blocks) are dropped. bm: W words of
+// bit order. Columns >= Kb (the keys' blocks) are dropped. bm: 2 W + 1 words of
 // LDS scratch, W = (2 Kb + 31) / 32. Every thread of the NT-thread workgroup
 // calls this; it returns the number of columns written to cols.
 template <int NT>
@@ -373,6 +449,9 @@ __device__ int distance_order_cols(int Kb, const int32_t* __restrict__ col_idx, 
     }
   }
   block_barrier();
+  // First column position of each word into pre[] (one wave scans), then every
+  // thread places its own columns.
+  uint32_t* const pre = bm + W;
   if (w == 0) {
     const int per = (W + 63) >> 6;
     const int w0 = lane * per;
@@ -384,21 +463,23 @@ __device__ int distance_order_cols(int Kb, const int32_t* __restrict__ col_idx, 
       const int y = __shfl_up(incl, off, 64);
       if (lane >= off) incl += y;
     }
-    int pos = incl - cnt;
-    const int total = __shfl(incl, 63, 64);
+    uint32_t pos = static_cast<uint32_t>(incl - cnt);
     for (int j = 0; j < per && w0 + j < W; ++j) {
-      uint32_t x = bm[w0 + j];
-      while (x) {
-        const int b = (w0 + j) * 32 + __ffs(x) - 1;
-        cols[pos++] = (b & 1) ? qb + (b >> 1) : qb - (b >> 1);
-        x &= x - 1;
-      }
+      pre[w0 + j] = pos;
+      pos += __popc(bm[w0 + j]);
     }
-    if (lane == 63) bm[0] = static_cast<uint32_t>(total);  // this row's count
+    if (lane == 63) pre[W] = static_cast<uint32_t>(incl);  // this row's count
   }
   block_barrier();
-  const int count = static_cast<int>(bm[0]);
-  block_barrier();  // bm[0] read by everybody before any later LDS write
+  for (int i = tid; i < n; i += NT) {
+    const int c = col_idx[beg + i];
+    if (static_cast<unsigned>(c) < static_cast<unsigned>(Kb)) {
+      const int b = 2 * (c >= qb ? c - qb : qb - c) + (c > qb ? 1 : 0);
+      cols[pre[b >> 5] + __popc(bm[b >> 5] & ((1u << (b & 31)) - 1u))] = c;
+    }
+  }
+  const int count = static_cast<int>(pre[W]);
+  block_barrier();
   return count;
 }
 
@@ -425,8 +506,9 @@ __device__ __forceinline__ void bsa_split_block(const uint16_t* __restrict__ q, 
                                                 const int32_t* __restrict__ row_ptr,
                                                 const int32_t* __restrict__ col_idx, void* __restrict__ out,
                                                 const int32_t* __restrict__ out_perm, float* __restrict__ lse,
-                                                const BsaParams& p, int h, int qb, uint16_t* k_lds,
+                                                const BsaParams& p, const Work& wk, uint16_t* k_lds,
                                                 uint16_t* v_lds, int32_t* cols) {
+  const int h = wk.h, qb = wk.qb;
   constexpr int DCH = D / 32;
   constexpr int K_LOADS = D / 16;  // buffer loads per thread for a K tile
   constexpr int V_LOADS = D / 16;  // ... for a V^T tile (D rows x 256 bytes)
@@ -466,30 +548,40 @@ __device__ __forceinline__ void bsa_split_block(const uint16_t* __restrict__ q, 
     const TileCopy<256> vcopy(ws, lane);
     typename QkOp::vec qf[D / 16];
     float row_scale = 1.f;  // 2^r of a row whose Q fragments carry 2^-r (SCALED)
-    if constexpr (QK_F16)
-      load_q_scaled<D, SCALED>(q, p, h, qrow, hl, qf, row_scale);
-    else
-      load_q<D, QkOp>(q, p, h, qrow, hl, qf);
-    const float qinv = 1.f / row_scale;
-    f32x16 negm = f32x16{};  // -m (times 2^-r) in every element
-    // Column list of this row into LDS (read back with uniform ds_reads), and
-    // Q fragments forced complete here so no wait for them lands in the loop.
-    const int n = distance_order_cols<256>(Kb, col_idx, qb, beg, end - beg, cols,
-                                           reinterpret_cast<uint32_t*>(cols + p.Kb), tid, w, lane);
-#pragma unroll
-    for (int s = 0; s < D / 16; ++s) asm volatile("" ::"v"(qf[s]));
-    block_barrier();
+    bool q_f16;  // the bf16-operand path takes bf16 rows only (q_perm or a bf16 q_src)
+    uint4 q_raw[D / 16];
+    load_q_raw<D>(q, p, h, qrow, hl, q_raw, q_f16);
+    // Column list of this row into LDS (read back with uniform ds_reads).
+    const int total = __builtin_amdgcn_readfirstlane(
+        distance_order_cols<256>(Kb, col_idx, qb, beg, end - beg, cols, reinterpret_cast<uint32_t*>(cols + p.Kb), tid,
+                                 w, lane));
+    // This workgroup's part of the list (all of it for an unsplit block).
+    const int t0 = SCALED ? 0 : total * wk.piece / wk.pieces;
+    const int n = SCALED ? total : total * (wk.piece + 1) / wk.pieces;
     auto col_at = [&](int t) -> int { return __builtin_amdgcn_readfirstlane(cols[t]); };
-    // n == 0: every kept column lies past this sequence's keys (a shorter
-    // key segment), so cols holds nothing to copy; the row stays empty.
-    // n is the same for every wave (read from LDS after a barrier).
-    int kb = n > 0 ? col_at(0) : 0;
-    if (n > 0) {
+    // n == t0: nothing to do for this part, or every kept column lies past
+    // this sequence's keys (a shorter key segment), so cols holds nothing to
+    // copy; the row stays empty. n is the same for every wave (read from LDS
+    // after a barrier).
+    int kb = n > t0 ? col_at(t0) : 0;
+    if (n > t0) {
       kcopy.template issue<K_LOADS>(krs, kb * TILE_BYTES, k_base, ws);
       vcopy.template issue<V_LOADS>(vrs, kb * TILE_BYTES, v_base, ws);
     }
 
-    for (int t = 0; t < n; ++t) {
+    // Q fragments, made under the first copies and forced complete here so no
+    // wait for them lands in the loop.
+    if constexpr (QK_F16)
+      scale_q<D, SCALED>(q_raw, q_f16, p, h, qf, row_scale);
+    else
+#pragma unroll
+      for (int s = 0; s < D / 16; ++s) qf[s] = __builtin_bit_cast(typename QkOp::vec, q_raw[s]);
+    const float qinv = 1.f / row_scale;
+    f32x16 negm = f32x16{};  // -m (times 2^-r) in every element
+#pragma unroll
+    for (int s = 0; s < D / 16; ++s) asm volatile("" ::"v"(qf[s]));
+
+    for (int t = t0; t < n; ++t) {
       // After the last block the copies reload the current block into the
       // buffers it has just left (in range; nobody reads them again), so every
       // iteration issues the same loads and the vmcnt waits stay fixed.
@@ -522,11 +614,11 @@ __device__ __forceinline__ void bsa_split_block(const uint16_t* __restrict__ q, 
       // which turns the block's row sum inf; bf16: a sum above 2^16 moves the
       // reference too, so that O keeps its fp32 range); only then is the
       // block redone with a moved reference. P keeps its full precision.
-      if (t == 0) softmax_lazy<DCH>(s, c, true, m, lsum, o, negm, qinv);
+      if (t == t0) softmax_lazy<DCH>(s, c, true, m, lsum, o, negm, qinv);
       typename PvOp::vec pf[8];
       float lblk;
       make_p<PvOp, QK_F16>(s, c, pf, lblk);
-      if (t > 0 && __any(!(lblk < (PV_F16 ? INFINITY : 65536.f)))) {
+      if (t > t0 && __any(!(lblk < (PV_F16 ? INFINITY : 65536.f)))) {
         softmax_lazy<DCH>(s, c, false, m, lsum, o, negm, qinv);
         make_p<PvOp, QK_F16>(s, c, pf, lblk);
       }
@@ -540,6 +632,10 @@ __device__ __forceinline__ void bsa_split_block(const uint16_t* __restrict__ q, 
     }
     wait_vmcnt_0();  // the trailing copies have landed before the workgroup's LDS is released
   }
+  if (!SCALED && wk.pieces > 1) {
+    store_part<D>(p, wk.slot, o, m * c, lsum, w, l32, hl);
+    return;
+  }
   store_out<D>(p, VARLEN ? min(max(p.cu_q[1], 0), p.L) : p.L, p.exps ? p.exps[2 * p.H + h] : 0, out, out_perm,
                lse, o, m * c, lsum, h, qrow, hl);
 }
@@ -550,12 +646,12 @@ __global__ void __launch_bounds__(256, 2) bsa_fwd_split_kernel(BSA_KERNEL_ARGS) 
   __shared__ __attribute__((aligned(16))) uint16_t v_lds[D * 128];
   extern __shared__ int32_t cols[];  // kept key blocks of this row (dynamic)
   if constexpr (!SCALED) {
-    // Common instance: one workgroup per (head, query block), XCD-aware.
-    int h, qb;
-    if (!wg_coords(p_in, h, qb)) return;
-    if (QK_F16 && head_scaled(p_in, h)) return;  // the scaled instance's head
-    bsa_split_block<D, QK_F16, PV_F16, VARLEN, false>(q, k, vt, row_ptr, col_idx, out, out_perm, lse, p_in, h, qb,
-                                                      k_lds, v_lds, cols);
+    // Common instance: a query block of a head, or a part of one, XCD-aware.
+    Work wk;
+    if (!wg_work(p_in, wk)) return;
+    if (QK_F16 && head_scaled(p_in, wk.h)) return;  // the scaled instance's head
+    bsa_split_block<D, QK_F16, PV_F16, VARLEN, false>(q, k, vt, row_ptr, col_idx, out, out_perm, lse, p_in, wk, k_lds,
+                                                      v_lds, cols);
   } else {
     // Scaled instance: a small grid (x: workgroups per head, y: head) whose
     // workgroups walk the query blocks of the heads that carry exponents and
@@ -564,10 +660,80 @@ __global__ void __launch_bounds__(256, 2) bsa_fwd_split_kernel(BSA_KERNEL_ARGS) 
     if (!head_scaled(p_in, h)) return;
     for (int qb = blockIdx.x; qb < p_in.Qb; qb += gridDim.x) {
       block_barrier();  // the previous block's LDS reads are done
-      bsa_split_block<D, QK_F16, PV_F16, VARLEN, true>(q, k, vt, row_ptr, col_idx, out, out_perm, lse, p_in, h, qb,
-                                                       k_lds, v_lds, cols);
+      bsa_split_block<D, QK_F16, PV_F16, VARLEN, true>(q, k, vt, row_ptr, col_idx, out, out_perm, lse, p_in,
+                                                       Work{h, qb, 0, 1, 0}, k_lds, v_lds, cols);
     }
   }
+}
+
+// Adds up the parts of the split query blocks: O = sum_p 2^(m_p - M) O_p over
+// the same sum of l_p, M the largest m_p, then the scaling, rounding and
+// unpermute of store_out. One workgroup per 32 query rows, eight threads a
+// row. Reads each part once (64 KB of O per part and block at D = 128).
+template <int D, bool VARLEN>
+__global__ void __launch_bounds__(256) bsa_combine_kernel(void* __restrict__ out, const int32_t* __restrict__ out_perm,
+                                                          float* __restrict__ lse, int qk_f16, BsaParams p) {
+  constexpr int DPT = D / 8;  // head dims per thread
+  const int r = blockIdx.x >> 2;  // split query block
+  const int n_long = split_long(p);
+  int h, qb, parts, slot;
+  if (r < n_long) {
+    if (!long_block(p, r, h, qb)) return;
+    parts = p.long_parts;
+    slot = r * parts;
+  } else {
+    const int t = r - n_long;
+    if (!ordinary_block(p, t & 7, p.full_rows + (t >> 3), h, qb)) return;
+    parts = p.parts;
+    slot = n_long * p.long_parts + t * parts;
+  }
+  if (qk_f16 && head_scaled(p, h)) return;  // written whole by the scaled instance
+  const int Lq = VARLEN ? min(max(p.cu_q[1], 0), p.L) : p.L;
+  const int in_block = (blockIdx.x & 3) * 32 + (threadIdx.x >> 3);
+  const int qrow = qb * 128 + in_block;
+  if (qrow >= Lq) return;
+  const int d0 = (threadIdx.x & 7) * DPT;
+  const int64_t row0 = static_cast<int64_t>(slot) * 128 + in_block;
+  float M = -INFINITY;
+  for (int i = 0; i < parts; ++i) {
+    const float2 ml = *reinterpret_cast<const float2*>(p.part_ml + (row0 + i * 128) * 2);
+    if (ml.y > 0.f) M = fmaxf(M, ml.x);
+  }
+  float acc[DPT] = {}, l = 0.f;
+  for (int i = 0; i < parts; ++i) {
+    const float2 ml = *reinterpret_cast<const float2*>(p.part_ml + (row0 + i * 128) * 2);
+    if (!(ml.y > 0.f)) continue;  // a part without keys
+    const float f = exp2_fast(ml.x - M);
+    l += ml.y * f;
+    const float4* src = reinterpret_cast<const float4*>(p.part_o + (row0 + i * 128) * D + d0);
+#pragma unroll
+    for (int j = 0; j < DPT / 4; ++j) {
+      const float4 v = src[j];
+      acc[4 * j + 0] += v.x * f;
+      acc[4 * j + 1] += v.y * f;
+      acc[4 * j + 2] += v.z * f;
+      acc[4 * j + 3] += v.w * f;
+    }
+  }
+  const float inv = l > 0.f ? ldexpf(1.0f / l, p.exps ? p.exps[2 * p.H + h] : 0) : 0.f;
+  const int orow = out_perm ? out_perm[qrow] : qrow;
+  const int64_t obase = h * p.o_sh + orow * p.o_sl + d0;
+#pragma unroll
+  for (int j = 0; j < DPT; j += 4) {
+    const float v0 = acc[j] * inv, v1 = acc[j + 1] * inv, v2 = acc[j + 2] * inv, v3 = acc[j + 3] * inv;
+    if (p.out_kind == DFS_DTYPE_F32)
+      *reinterpret_cast<float4*>(static_cast<float*>(out) + obase + j) = make_float4(v0, v1, v2, v3);
+    else if (p.out_kind == DFS_DTYPE_BF16)
+      *reinterpret_cast<uint2*>(static_cast<uint16_t*>(out) + obase + j) =
+          make_uint2(f32_to_bf16_bits(v0) | (f32_to_bf16_bits(v1) << 16),
+                     f32_to_bf16_bits(v2) | (f32_to_bf16_bits(v3) << 16));
+    else
+      *reinterpret_cast<uint2*>(static_cast<uint16_t*>(out) + obase + j) =
+          make_uint2(f32_to_f16_bits(v0) | (f32_to_f16_bits(v1) << 16),
+                     f32_to_f16_bits(v2) | (f32_to_f16_bits(v3) << 16));
+  }
+  if (lse && d0 == 0)
+    lse[static_cast<int64_t>(h) * p.Lo + qrow] = l > 0.f ? (M + log2f(l)) * 0.69314718055994531f : -INFINITY;
 }
 
 struct BsaArgs {
@@ -589,6 +755,7 @@ struct SegParams {
   const uint16_t* q_src;  // optional Q source (as in BsaParams)
   const int32_t* q_rows;
   int q_src_f16;
+  int64_t o_sh, o_sl;  // element strides of out
 };
 
 __device__ __forceinline__ float operand_at(const uint16_t* base, int64_t i, bool f16) {
@@ -755,7 +922,7 @@ __global__ void __launch_bounds__(256) bsa_segment_kernel(const uint16_t* __rest
       if (r >= cq2) l[i] = 0.f;
       const float inv = l[i] > 0.f ? sv / l[i] : 0.f;
       const int orow = out_perm ? out_perm[r] : r;
-      const int64_t ob = (static_cast<int64_t>(h) * p.Lo + orow) * D + lane * DPL;
+      const int64_t ob = h * p.o_sh + orow * p.o_sl + lane * DPL;
 #pragma unroll
       for (int j = 0; j < DPL; ++j) {
         const float v = o[i][j] * inv;
@@ -775,11 +942,15 @@ __global__ void __launch_bounds__(256) bsa_segment_kernel(const uint16_t* __rest
 template <int D, bool QK_F16, bool PV_F16, bool VARLEN>
 void launch_split_as(const BsaArgs& a, const BsaParams& p, hipStream_t s) {
   const size_t smem = static_cast<size_t>(p.Kb) * sizeof(int32_t) +
-                      static_cast<size_t>((2 * p.Kb + 31) / 32) * sizeof(uint32_t);
+                      static_cast<size_t>(2 * ((2 * p.Kb + 31) / 32) + 1) * sizeof(uint32_t);
   if (!p.scale_all) {
-    const int S = (p.Qb + 7) / 8;
-    bsa_fwd_split_kernel<D, QK_F16, PV_F16, VARLEN, false><<<dim3(static_cast<unsigned>(8 * S * p.H)), 256, smem, s>>>(
+    const int per_xcd = long_per_xcd(p) * p.long_parts + p.full_rows + (blocks_per_xcd(p) * p.H - p.full_rows) * p.parts;
+    bsa_fwd_split_kernel<D, QK_F16, PV_F16, VARLEN, false><<<dim3(static_cast<unsigned>(8 * per_xcd)), 256, smem, s>>>(
         a.q, a.k, a.vt, a.row_ptr, a.col_idx, a.out, a.out_perm, a.lse, p);
+    const int split = split_long(p) + split_tail(p);
+    if (split > 0)
+      bsa_combine_kernel<D, VARLEN><<<dim3(static_cast<unsigned>(4 * split)), 256, 0, s>>>(a.out, a.out_perm, a.lse,
+                                                                                          QK_F16 ? 1 : 0, p);
   }
   if constexpr (QK_F16) {
     // Heads with exponents (only when some bf16 input exceeds the f16 range)
@@ -812,15 +983,18 @@ void launch_bsa(const BsaArgs& a, const BsaParams& p, bool qk_f16, bool pv_f16, 
 }  // namespace
 }  // namespace dfs
 
-extern "C" int dfs_bsa_fwd(const void* q_perm, const void* k_perm, const void* v_t,
+namespace dfs {
+namespace {
+
+int bsa_fwd_impl(const char* name, const void* q_perm, const void* k_perm, const void* v_t,
                            const int32_t* row_ptr, const int32_t* col_idx, int64_t heads,
                            int64_t seq_len, int64_t head_dim, int dtype, int pv_dtype, float scale,
                            void* out, int out_dtype, const int32_t* out_perm, float* lse,
                            const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int64_t n_seq,
                            const int32_t* exps, const void* q_src, const int32_t* q_rows, int q_src_dtype,
+                           int64_t out_head_stride, int64_t out_row_stride, int64_t long_row, int64_t long_parts,
+                           int64_t full_rows, int64_t parts, void* workspace, int64_t workspace_bytes,
                            dfs_stream_t stream) {
-  using namespace dfs;
-  const char* name = "dfs_bsa_fwd";
   DFS_REQUIRE((q_perm || q_src) && k_perm && v_t && row_ptr && col_idx && out, "%s: NULL operand", name);
   DFS_REQUIRE(!q_src || q_rows, "%s: q_src needs q_rows", name);
   DFS_REQUIRE(!q_src || q_src_dtype == DFS_DTYPE_BF16 || q_src_dtype == DFS_DTYPE_F16,
@@ -868,6 +1042,34 @@ extern "C" int dfs_bsa_fwd(const void* q_perm, const void* k_perm, const void* v
   p.q_src = static_cast<const uint16_t*>(q_src);
   p.q_rows = q_rows;
   p.q_src_f16 = q_src_dtype == DFS_DTYPE_F16 ? 1 : 0;
+  DFS_REQUIRE(out_head_stride > 0 && out_row_stride >= head_dim && out_head_stride % 4 == 0 && out_row_stride % 4 == 0,
+              "%s: out strides %lld, %lld must be multiples of 4 elements that hold a row", name,
+              (long long)out_head_stride, (long long)out_row_stride);
+  p.o_sh = out_head_stride;
+  p.o_sl = out_row_stride;
+  DFS_REQUIRE(long_row >= 0 && long_row <= qb, "%s: long_row=%lld outside [0, %lld]", name, (long long)long_row,
+              (long long)qb);
+  const int64_t per_xcd = heads * ((long_row + 7) / 8);
+  DFS_REQUIRE(parts >= 1 && parts <= 64 && long_parts >= 1 && long_parts <= 64, "%s: parts=%lld, %lld outside [1, 64]",
+              name, (long long)parts, (long long)long_parts);
+  DFS_REQUIRE(full_rows >= 0 && full_rows <= per_xcd, "%s: full_rows=%lld outside [0, %lld]", name,
+              (long long)full_rows, (long long)per_xcd);
+  p.long_row = static_cast<int>(long_row);
+  p.long_parts = static_cast<int>(long_parts);
+  p.full_rows = static_cast<int>(parts > 1 ? full_rows : per_xcd);
+  p.parts = static_cast<int>(parts);
+  if (p.scale_all) {  // every head runs unsplit in the scaled instance
+    p.long_parts = p.parts = 1;
+    p.full_rows = static_cast<int>(per_xcd);
+  }
+  const int64_t slots = static_cast<int64_t>(split_long(p)) * p.long_parts + static_cast<int64_t>(split_tail(p)) * p.parts;
+  DFS_REQUIRE(slots < (int64_t(1) << 24), "%s: too many parts", name);
+  const int64_t need = slots * 128 * (head_dim + 2) * static_cast<int64_t>(sizeof(float));
+  DFS_REQUIRE(slots == 0 || (workspace && workspace_bytes >= need), "%s: workspace of %lld bytes, %lld needed", name,
+              (long long)(workspace ? workspace_bytes : 0), (long long)need);
+  DFS_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 15u) == 0, "%s: workspace must be 16-byte aligned", name);
+  p.part_o = static_cast<float*>(workspace);
+  p.part_ml = p.part_o + slots * 128 * head_dim;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const bool qk_f16 = dtype == DFS_DTYPE_F16, pv_f16 = pv_dtype == DFS_DTYPE_F16;
   if (head_dim == 128)
@@ -892,6 +1094,8 @@ extern "C" int dfs_bsa_fwd(const void* q_perm, const void* k_perm, const void* v
     sp.q_src = p.q_src;
     sp.q_rows = q_rows;
     sp.q_src_f16 = p.q_src_f16;
+    sp.o_sh = p.o_sh;
+    sp.o_sl = p.o_sl;
     // Enough waves for a few hundred rows per head; each wave strides over
     // the rows after segment 0.
     const dim3 grid(16, static_cast<unsigned>(heads));
@@ -901,4 +1105,53 @@ extern "C" int dfs_bsa_fwd(const void* q_perm, const void* k_perm, const void* v
       bsa_segment_kernel<64><<<grid, 256, 0, s>>>(a.q, a.k, a.vt, row_ptr, col_idx, out, out_perm, lse, sp);
   }
   return check_launch(name);
+}
+
+}  // namespace
+}  // namespace dfs
+
+extern "C" int64_t dfs_bsa_fwd_workspace_size(int64_t heads, int64_t seq_len, int64_t head_dim, int64_t long_row,
+                                              int64_t long_parts, int64_t full_rows, int64_t parts) {
+  using namespace dfs;
+  const int64_t qb = (seq_len + kBlock - 1) / kBlock;
+  if (heads <= 0 || seq_len <= 0 || head_dim <= 0 || long_row < 0 || long_row > qb || long_parts < 1 || parts < 1 ||
+      full_rows < 0 || heads * qb >= (int64_t(1) << 31))
+    return -1;
+  BsaParams p{};
+  p.H = static_cast<int>(heads);
+  p.Qb = static_cast<int>(qb);
+  p.long_row = static_cast<int>(long_row);
+  p.long_parts = static_cast<int>(long_parts);
+  p.parts = static_cast<int>(parts);
+  const int64_t per_xcd = static_cast<int64_t>(blocks_per_xcd(p)) * heads;
+  p.full_rows = static_cast<int>(full_rows < per_xcd ? full_rows : per_xcd);
+  const int64_t slots = split_long(p) * long_parts + split_tail(p) * parts;
+  return slots * 128 * (head_dim + 2) * static_cast<int64_t>(sizeof(float));
+}
+
+extern "C" int dfs_bsa_fwd(const void* q_perm, const void* k_perm, const void* v_t,
+                           const int32_t* row_ptr, const int32_t* col_idx, int64_t heads,
+                           int64_t seq_len, int64_t head_dim, int dtype, int pv_dtype, float scale,
+                           void* out, int out_dtype, const int32_t* out_perm, float* lse,
+                           const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int64_t n_seq,
+                           const int32_t* exps, const void* q_src, const int32_t* q_rows, int q_src_dtype,
+                           dfs_stream_t stream) {
+  return dfs::bsa_fwd_impl("dfs_bsa_fwd", q_perm, k_perm, v_t, row_ptr, col_idx, heads, seq_len, head_dim, dtype,
+                           pv_dtype, scale, out, out_dtype, out_perm, lse, cu_seqlens_q, cu_seqlens_k, n_seq, exps,
+                           q_src, q_rows, q_src_dtype, seq_len * head_dim, head_dim,
+                           (seq_len + dfs::kBlock - 1) / dfs::kBlock, 1, 0, 1, nullptr, 0, stream);
+}
+
+extern "C" int dfs_bsa_fwd_parts(const void* q_perm, const void* k_perm, const void* v_t, const int32_t* row_ptr,
+                                 const int32_t* col_idx, int64_t heads, int64_t seq_len, int64_t head_dim, int dtype,
+                                 int pv_dtype, float scale, void* out, int out_dtype, const int32_t* out_perm,
+                                 float* lse, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int64_t n_seq,
+                                 const int32_t* exps, const void* q_src, const int32_t* q_rows, int q_src_dtype,
+                                 int64_t out_head_stride, int64_t out_row_stride, int64_t long_row,
+                                 int64_t long_parts, int64_t full_rows, int64_t parts, void* workspace,
+                                 int64_t workspace_bytes, dfs_stream_t stream) {
+  return dfs::bsa_fwd_impl("dfs_bsa_fwd_parts", q_perm, k_perm, v_t, row_ptr, col_idx, heads, seq_len, head_dim, dtype,
+                           pv_dtype, scale, out, out_dtype, out_perm, lse, cu_seqlens_q, cu_seqlens_k, n_seq, exps,
+                           q_src, q_rows, q_src_dtype, out_head_stride, out_row_stride, long_row, long_parts,
+                           full_rows, parts, workspace, workspace_bytes, stream);
 }

@@ -7,9 +7,10 @@ numbers; nothing here touches a device.
 """
 from __future__ import annotations
 
+import functools
 import math
 from dataclasses import dataclass
-from typing import Optional
+from typing import Optional, Tuple
 
 import numpy as np
 
@@ -187,3 +188,44 @@ def csr_flops(row_ptr: np.ndarray, col_idx: np.ndarray, heads: int, seq_len: int
     np.cumsum(sizes[col], out=cum[1:])
     key_tok = (cum[row_ptr[1:]] - cum[row_ptr[:-1]]).reshape(heads, nblk)
     return int(4 * head_dim * (key_tok * sizes[None, :]).sum())
+
+
+XCDS = 8
+XCD_SLOTS = 64  # attention workgroups an XCD holds: 32 CUs, two each
+
+
+@functools.lru_cache(maxsize=1024)
+def attention_plan(heads: int, q_blocks: int, long_row: int, kept: int, kept_long: int) -> Tuple[int, int, int]:
+    """(long_parts, full_rows, parts) of an attention call (see
+    dfs_bsa_fwd_parts): how its query blocks are cut into workgroups along
+    their column lists. ``kept`` / ``kept_long``: columns of a query block
+    before / from ``long_row`` on.
+
+    A workgroup alone on a CU takes 1.75 us per key block, two together 3.65:
+    beyond one workgroup per CU cutting gains nothing by itself (power sets
+    the pace), and every part costs the write and read of 64 KB and the
+    combining launch (about 6 us). So query blocks are cut
+      * in problems of at most 16 blocks per XCD, into as many parts as keep
+        one workgroup per CU and four key blocks per part (one head of 7,872
+        tokens, all blocks kept: 116 -> 52 us with 4 parts, 70 with 2; 2,290
+        tokens: 40 -> 27 us);
+      * at the tail of one or two full rounds, when at most half a round is
+        left over and the lists are long (20 heads of 4,000 tokens, 1.25
+        rounds, 32 columns: 201 -> 185 us; at 12 columns 87 -> 88, at 5
+        rounds within noise);
+      * where they are long and few rounds hide them (2 heads of 30,250
+        tokens, 3 text blocks per head keeping 237 columns against 60: 515 ->
+        248 us; with 44 rounds, as at 119,056 tokens and 24 heads, starting
+        them first is enough)."""
+    per_xcd = heads * -(-long_row // XCDS)
+    full_rows, parts = 0, 1
+    if 0 < per_xcd <= 16:
+        parts = max(1, min(XCD_SLOTS // 2 // per_xcd, kept // 4, 8))
+    elif XCD_SLOTS < per_xcd < 3 * XCD_SLOTS:
+        tail = per_xcd % XCD_SLOTS
+        if 0 < tail <= XCD_SLOTS // 2 and kept >= 16:
+            full_rows, parts = per_xcd - tail, min(XCD_SLOTS // tail, kept // 5, 4)
+    long_parts = 1
+    if long_row < q_blocks and kept > 0 and kept_long * 4 * XCD_SLOTS > kept * max(per_xcd, XCD_SLOTS // 2):
+        long_parts = max(1, min(-(-kept_long // kept), 8, kept_long // 4))
+    return long_parts, full_rows if parts > 1 else 0, parts

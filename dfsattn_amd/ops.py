@@ -14,7 +14,7 @@ from typing import Dict, Optional, Sequence, Tuple
 import torch
 
 from . import _lib
-from .layout import ScoringLayout, TopkPolicy
+from .layout import ScoringLayout, TopkPolicy, attention_plan
 
 DTYPE_CODE = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
 
@@ -330,11 +330,23 @@ def bsa_fwd(prep: Prepared, row_ptr: torch.Tensor, col_idx: torch.Tensor, scale:
         raise ValueError("out must be a contiguous [1, H, L, D] tensor of out_dtype")
     lse = torch.empty((prep.heads, L), dtype=torch.float32, device=out.device) if want_lse else None
     scale = 1.0 / math.sqrt(prep.head_dim) if scale is None else float(scale)
-    _lib.call("dfs_bsa_fwd", _ptr(prep.q_perm), _ptr(prep.k_perm), _ptr(prep.v_t), _ptr(row_ptr),
+    lay = prep.layout
+    # Text query blocks keep every key block and are several times longer.
+    long_row = lay.video_len // lay.block if lay.text_len > 0 else lay.q_blocks
+    kept_long = lay.k_blocks
+    kept = max(0, col_idx.numel() // prep.heads - (lay.q_blocks - long_row) * kept_long) // max(long_row, 1)
+    long_parts, full_rows, parts = attention_plan(prep.heads, lay.q_blocks, long_row, kept, kept_long)
+    ws_bytes = 0
+    if long_parts > 1 or parts > 1:
+        ws_bytes = int(_lib.lib().dfs_bsa_fwd_workspace_size(prep.heads, L, prep.head_dim, long_row, long_parts,
+                                                             full_rows, parts))
+    ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=prep.device) if ws_bytes else None
+    _lib.call("dfs_bsa_fwd_parts", _ptr(prep.q_perm), _ptr(prep.k_perm), _ptr(prep.v_t), _ptr(row_ptr),
               _ptr(col_idx), prep.heads, L, prep.head_dim, DTYPE_CODE[prep.operand_dtype],
               DTYPE_CODE[prep.operand_dtype], scale, _ptr(out), DTYPE_CODE[out_dtype], _ptr(out_perm),
               _ptr(lse), _ptr(cu_seqlens_q), _ptr(cu_seqlens_k), n_seq, _ptr(prep.exps), _ptr(prep.q_src),
-              _ptr(prep.q_rows), DTYPE_CODE[prep.dtype], _stream(prep.k_perm))
+              _ptr(prep.q_rows), DTYPE_CODE[prep.dtype], L * prep.head_dim, prep.head_dim, long_row, long_parts,
+              full_rows, parts, _ptr(ws), ws_bytes, _stream(prep.k_perm))
     return (out, lse) if want_lse else out
 
 

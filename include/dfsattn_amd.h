@@ -278,6 +278,42 @@ int dfs_bsa_fwd(const void* q_perm, const void* k_perm, const void* v_t,
                 int64_t n_seq, const int32_t* exps, const void* q_src,
                 const int32_t* q_rows, int q_src_dtype, dfs_stream_t stream);
 
+/*
+ * dfs_bsa_fwd with the output's strides, the order of its work and the split
+ * of its query blocks over workgroups chosen by the caller (dfs_bsa_fwd is
+ * this call with a contiguous [H][L][D] output, long_row = ceil(L / 128),
+ * full_rows 0 and one part each):
+ *   out_head_stride, out_row_stride  elements between heads and between rows
+ *     of out (multiples of 4; [L][H][D] storage has strides D and H * D);
+ *   long_row    query blocks long_row.. of every head keep more columns than
+ *     the others (text rows): they are started first, each cut along its
+ *     column list into long_parts workgroups;
+ *   full_rows, parts  of the S * heads (S = ceil(long_row / 8)) other query
+ *     blocks each XCD runs in order, those from full_rows on are cut into
+ *     `parts` workgroups each;
+ *   workspace   dfs_bsa_fwd_workspace_size bytes of device memory (16-byte
+ *     aligned, may be NULL when nothing is cut): fp32 partial results, added
+ *     up by a second kernel. Parts and long_parts lie in [1, 64].
+ * The split changes the order of the fp32 sums only. Heads that need the
+ * range exponents (exps) run uncut.
+ */
+int64_t dfs_bsa_fwd_workspace_size(int64_t heads, int64_t seq_len,
+                                   int64_t head_dim, int64_t long_row,
+                                   int64_t long_parts, int64_t full_rows,
+                                   int64_t parts);
+int dfs_bsa_fwd_parts(const void* q_perm, const void* k_perm, const void* v_t,
+                      const int32_t* row_ptr, const int32_t* col_idx,
+                      int64_t heads, int64_t seq_len, int64_t head_dim,
+                      int dtype, int pv_dtype, float scale, void* out,
+                      int out_dtype, const int32_t* out_perm, float* lse,
+                      const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                      int64_t n_seq, const int32_t* exps, const void* q_src,
+                      const int32_t* q_rows, int q_src_dtype,
+                      int64_t out_head_stride, int64_t out_row_stride,
+                      int64_t long_row, int64_t long_parts, int64_t full_rows,
+                      int64_t parts, void* workspace, int64_t workspace_bytes,
+                      dfs_stream_t stream);
+
 /* uint8/bool block mask [H][Qb][Kb] -> per-row counts int32 [H*Qb].
  * Part of the bool-mask interface of block_sparse_attn_func
  * (base_blockmask, attention_wan.py:359). */

@@ -547,6 +547,55 @@ def test_bsa_fwd_bf16_operands_moving_reference(dev, d, length, scale, v_size):
     assert float((out - ref).abs().max()) <= 2e-2 * v_size
 
 
+@pytest.mark.parametrize("d,heads,video,text,cut,dtype,out_dtype,plan", [
+    (128, 3, 1300, 0, None, torch.bfloat16, torch.float32, (1, 0, 3)),   # every block in 3 parts, a ragged last one
+    (64, 2, 2000, 0, None, torch.float16, torch.bfloat16, (1, 3, 2)),    # the tail of each XCD's list
+    (128, 2, 1024, 200, None, torch.bfloat16, torch.bfloat16, (4, 0, 1)),  # long rows in parts, the rest whole
+    (128, 1, 1152, 150, 1200, torch.bfloat16, torch.float32, (8, 1, 5)),   # both, with a second sequence
+    (64, 3, 300, 0, None, torch.bfloat16, torch.float32, (1, 0, 64)),    # more parts than columns: empty parts
+    (128, 2, 1000, 0, 700, torch.bfloat16, torch.float16, (1, 0, 4)),    # whole query blocks past the first sequence
+])
+def test_bsa_fwd_parts_match_unsplit(dev, monkeypatch, d, heads, video, text, cut, dtype, out_dtype, plan):
+    """Query blocks cut into parts against the same call uncut: the sums run
+    in another order (and P is rounded against another reference), nothing
+    else changes. Head 0 holds a value beyond f16, so its blocks run whole in
+    the scaled instance beside the cut ones."""
+    print(f"parts d={d} heads={heads} video={video} text={text} cut={cut} plan={plan}", flush=True)
+    L = video + text
+    g = torch.Generator().manual_seed(L + d)
+    q, k, v = (torch.randn((1, heads, L, d), generator=g).to(dtype) for _ in range(3))
+    if dtype == torch.bfloat16:
+        q[0, 0, 5, 3] = 1.0e5
+        k[0, 0, 5, 3] = 0.0
+    layout = ScoringLayout(L, video, 16)
+    perm = torch.randperm(L, generator=g).to(torch.int32)
+    mask = torch.rand((heads, layout.q_blocks, layout.k_blocks), generator=g) < 0.5
+    mask[:, 0] = False  # empty rows
+    mask[:, video // 128:] = True
+    mask[:, 1] = False
+    mask[:, 1, -1] = True  # one column: most parts empty
+    prep = ops.prepare_qkv(*(x.to(dev) for x in (q, k, v)), perm.to(dev), layout, pool=False, q_operand=False)
+    row_ptr, col_idx = ops.mask_to_csr(mask.to(dev))
+    cu = None if cut is None else torch.tensor([0, cut, L], dtype=torch.int32, device=dev)
+    got = {}
+    for name, pl in (("whole", (1, 0, 1)), ("parts", plan)):
+        monkeypatch.setattr(ops, "attention_plan", lambda *a: pl)
+        got[name] = ops.bsa_fwd(prep, row_ptr, col_idx, out_dtype=out_dtype, out_perm=perm.to(dev), want_lse=True,
+                                cu_seqlens_q=cu, cu_seqlens_k=cu)
+    (o0, l0), (o1, l1) = ((o.float().cpu(), l.cpu()) for o, l in (got["whole"], got["parts"]))
+    assert torch.equal(torch.isinf(l0), torch.isinf(l1))
+    fin = torch.isfinite(l0)
+    # l sums f16-rounded P (2^-11 each, against another power-of-two-free
+    # reference per part): relative 2^-11 at most, so lse within 2^-11 absolute
+    assert float((l0 - l1)[fin].abs().max()) <= 2.0 ** -11 + 2e-6 * float(l0[fin].abs().max())
+    if dtype == torch.bfloat16:
+        assert torch.equal(o0[0, 0], o1[0, 0])  # the scaled head is never cut
+    rel = float((o0 - o1).norm() / o0.norm())
+    ulp = {torch.float32: 0.0, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[out_dtype]
+    assert rel <= 2.0 ** -11 + ulp, rel  # P's rounding, averaged over the keys, and the output's
+    assert float((o0 - o1).abs().max()) <= 1e-2
+
+
 def test_wrappers_reject_bad_index_operands(dev):
     """Index operands must be contiguous int32 on the operands' device, and
     CSR offsets must cover every (head, query block) row: checked on the host

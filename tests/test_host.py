@@ -241,3 +241,65 @@ def test_noalloc_wrapper_runs_under_the_tensors_device(monkeypatch):
     row_ptr = torch.from_numpy(pol.row_ptr(2))
     ops.block_score_topk_noalloc(prep, pol, row_ptr)
     assert events == [("enter", target), ("call", "dfs_block_score_topk_noalloc", 16, 16), ("exit", target)]
+
+
+@pytest.mark.parametrize("heads,length,text,kept", [
+    (1, 100, 0, 1), (1, 7872, 0, 62), (2, 1024, 0, 2), (9, 9000, 0, 20), (40, 75600, 0, 177), (24, 119056, 256, 279),
+    (2, 30250, 250, 60), (8, 6200, 200, 14), (16, 5000, 0, 12), (3, 200, 100, 0), (1, 5, 4, 1)])
+def test_attention_plan_covers_every_block_once(heads, length, text, kept):
+    """The workgroup -> (head, query block, part) map of dfs_bsa_fwd_parts,
+    restated here, visits every part of every query block exactly once under
+    the plan, partial slots are distinct and lie inside the workspace, and
+    the combining kernel's map finds the same blocks."""
+    from dfsattn_amd.layout import attention_plan
+    Qb = -(-length // 128)
+    long_row = (length - text) // 128 if text else Qb
+    lp, full, parts = attention_plan(heads, Qb, long_row, kept, Qb)
+    assert 1 <= lp <= 64 and 1 <= parts <= 64 and 0 <= full <= heads * -(-long_row // 8)
+    S, n_long = -(-long_row // 8), Qb - long_row
+    long_x = -(-heads * n_long // 8)
+    full_k = full if parts > 1 else S * heads
+    split_long = 8 * long_x if lp > 1 else 0
+    split_tail = 8 * (S * heads - full_k) if parts > 1 else 0
+    size = _lib.lib().dfs_bsa_fwd_workspace_size(heads, length, 128, long_row, lp, full, parts)
+    slots = split_long * lp + split_tail * parts
+    assert size == slots * 128 * 130 * 4
+    per = long_x * lp + full_k + (S * heads - full_k) * parts
+    seen, used = {}, {}
+
+    def ordinary(x, i):
+        h, qb = i // S, ((x + i // S) & 7) * S + i % S
+        return (h, qb) if qb < long_row else None
+
+    for b in range(8 * per):
+        x, j = b & 7, b >> 3
+        if j < long_x * lp:
+            g = (j // lp) * 8 + x
+            blk = (g // n_long, long_row + g % n_long) if g < heads * n_long else None
+            piece, pieces, slot = j % lp, lp, g * lp + j % lp
+        else:
+            j -= long_x * lp
+            if parts > 1 and j >= full_k:
+                t, piece = divmod(j - full_k, parts)
+                blk, pieces = ordinary(x, full_k + t), parts
+                slot = split_long * lp + (t * 8 + x) * parts + piece
+            else:
+                blk, piece, pieces, slot = ordinary(x, j), 0, 1, None
+        if blk is None:
+            continue
+        seen.setdefault(blk, []).append((piece, pieces))
+        if pieces > 1:
+            assert 0 <= slot < slots and slot not in used
+            used[slot] = (blk, piece)
+    assert set(seen) == {(h, qb) for h in range(heads) for qb in range(Qb)}
+    for got in seen.values():
+        assert sorted(got) == [(i, got[0][1]) for i in range(got[0][1])]
+    for r in range(split_long + split_tail):  # the combining kernel's blocks
+        if r < split_long:
+            blk = (r // n_long, long_row + r % n_long) if r < heads * n_long else None
+            base, n = r * lp, lp
+        else:
+            t = r - split_long
+            blk, base, n = ordinary(t & 7, full_k + (t >> 3)), split_long * lp + t * parts, parts
+        if blk is not None:
+            assert [used[base + i] for i in range(n)] == [(blk, i) for i in range(n)]
