@@ -26,6 +26,7 @@ SIGNATURES = {
     "dfs_prepare_qkv": [_p, _p, _p, _p, _i64, _i64, _i64, _i32, _i64, _i64, _i64, _i32,
                         _p, _p, _p, _p, _p, _p, _p, _p, _p],
     "dfs_block_score_topk_workspace_size": [_i64, _i64, _i64, _i64, _i64],
+    "dfs_block_score_topk_split_size": [_i64, _i64, _i64, _i64, _i64],
     "dfs_block_score_topk": [_p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
                              _i64, _i64, _i64, _p, _p, _p, _p, _p, _i64, _p],
     "dfs_block_score_topk_noalloc": [_p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
@@ -50,7 +51,7 @@ SIGNATURES = {
     "dfs_gated_residual": [_p, _p, _p, _i64, _i64, _i32, _p, _p],
 }
 _RESTYPES = {"dfs_last_error": ctypes.c_char_p, "dfs_block_score_topk_workspace_size": ctypes.c_int64,
-             "dfs_bsa_fwd_workspace_size": ctypes.c_int64}
+             "dfs_block_score_topk_split_size": ctypes.c_int64, "dfs_bsa_fwd_workspace_size": ctypes.c_int64}
 ABI_VERSION = 5
 
 _lock = threading.Lock()

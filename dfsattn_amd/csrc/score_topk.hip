@@ -159,6 +159,11 @@ struct ScoreParams {
   uint8_t* mask_out;
   float* tile_sums;  // one pass: [H][workgroup][tile_cols][tiles of the workgroup] unnormalised block sums
   int tile_cols;     // key blocks of all 32-tile chunks (Kb rounded up to a chunk)
+  // Split form: the key chunks are divided over `splits` workgroups of `cps`
+  // (even) chunks; tile_mz [H][workgroup][splits][tiles of the workgroup][2]
+  // holds each one's reference m and sum z.
+  float2* tile_mz;
+  int splits, cps;
   Policy pol;
   int q_tiles, k_tiles;
   float scale_log2;
@@ -388,7 +393,11 @@ __device__ __forceinline__ void head_major_xcd(int& h, int& wgx) {
 // GB (global block sums): the block sums go straight to scores_out (which
 // the caller provides) instead of LDS, so a workgroup needs only its key
 // chunks and the top-k histograms in LDS and four workgroups fit on a CU.
-template <int D, int TPB, bool GB, bool ONE_PASS = false>
+//
+// SPLIT (one pass only): blockIdx.z takes a share of the key chunks and leaves
+// its sums, m and z in the workspace; select_rows_kernel combines the shares
+// and selects, a wave per row.
+template <int D, int TPB, bool GB, bool ONE_PASS = false, bool SPLIT = false>
 __global__ void __launch_bounds__(256, 2) score_topk_wide_kernel(ScoreParams p) {
   constexpr int CPR = D / 8;             // 16-byte chunks per pooled row
   constexpr int QBW = 32 / TPB;          // query blocks per wave
@@ -429,6 +438,8 @@ __global__ void __launch_bounds__(256, 2) score_topk_wide_kernel(ScoreParams p) 
     for (int ds = 0; ds < D / 16; ++ds) asm volatile("" ::"v"(qh[ds]), "v"(ql[ds]));
     const bool wave_scores = qbw < score_rows;
     const int nchunks = (p.k_tiles + ROWS - 1) / ROWS;
+    const int c0 = SPLIT ? static_cast<int>(blockIdx.z) * p.cps : 0;  // even: chunk c uses buffer c & 1
+    const int c1 = SPLIT ? min(c0 + p.cps, nchunks) : nchunks;
     const uint32_t head_bytes = static_cast<uint32_t>(p.k_tiles) * D * 2;
     const auto hrs = make_rsrc(p.k_hi + static_cast<int64_t>(h) * p.k_tiles * CPR, head_bytes);
     const auto lrs = make_rsrc(p.k_lo + static_cast<int64_t>(h) * p.k_tiles * CPR, head_bytes);
@@ -494,7 +505,7 @@ __global__ void __launch_bounds__(256, 2) score_topk_wide_kernel(ScoreParams p) 
       return acc;
     };
 
-    issue(0, B0);
+    issue(c0, B0);
     if constexpr (ONE_PASS) {
       // One pass: exp2(s - m) against a reference m shared by the two lane
       // halves of a query tile (the first chunk's maximum; moved only when a
@@ -522,7 +533,7 @@ __global__ void __launch_bounds__(256, 2) score_topk_wide_kernel(ScoreParams p) 
 #pragma unroll
         for (int j = 0; j < NST; ++j) U(st_col(c, j)) = pend[j];
       };
-      for_steps(0, nchunks, [&](int c, auto buf) {
+      for_steps(c0, c1, [&](int c, auto buf) {
         wait_vmcnt_0();
         block_barrier();
         issue(c + 1, std::integral_constant<int, 1 - decltype(buf)::value>{});
@@ -531,7 +542,7 @@ __global__ void __launch_bounds__(256, 2) score_topk_wide_kernel(ScoreParams p) 
         // The previous chunk's sums go out after this chunk's operand reads:
         // issued before them, the stores made the compiler wait for part of
         // the next chunk's copy ahead of the reads in every other step.
-        if (c > 0) flush(c - 1);
+        if (c > c0) flush(c - 1);
         const int lim = (c + 1) * ROWS <= p.k_tiles ? ROWS : p.k_tiles - c * ROWS;  // valid key tiles
         auto joint_max = [&]() {
           float cm = -INFINITY;
@@ -566,7 +577,7 @@ __global__ void __launch_bounds__(256, 2) score_topk_wide_kernel(ScoreParams p) 
             const float f = exp2_fast(m - mn);
             z *= f;
             __threadfence_block();  // this lane's earlier row stores are visible to its loads
-            for (int j = hl; j < c * BPC; j += 2) U(j) *= f;
+            for (int j = c0 * BPC + hl; j < c * BPC; j += 2) U(j) *= f;
             m = mn;
           }
           sum = sums(m);
@@ -583,8 +594,15 @@ __global__ void __launch_bounds__(256, 2) score_topk_wide_kernel(ScoreParams p) 
           for (int j = 0; j < NST; ++j) pend[j] = u[j];  // group j, half hl: key block 2j + hl
         }
       });
-      if (wave_scores && nchunks > 0) flush(nchunks - 1);
+      if (wave_scores && c1 > c0) flush(c1 - 1);
       wait_vmcnt_0();  // the trailing (empty) copies and the last sums have retired
+      if constexpr (SPLIT) {
+        const float Z = xhalf_sum(z);  // same reference in both halves
+        if (wave_scores && hl == 0)
+          p.tile_mz[((static_cast<int64_t>(h) * gridDim.x + wgx) * p.splits + blockIdx.z) * WG_TILES + w * 32 + l32] =
+              make_float2(m, Z);
+        return;
+      }
       if (wave_scores) {
         const float Z = xhalf_sum(z);  // same reference in both halves
         if (hl == 0) inv_z[w * 32 + l32] = Z > 0.f ? 1.0f / Z : 0.f;
@@ -705,6 +723,7 @@ __global__ void __launch_bounds__(256, 2) score_topk_wide_kernel(ScoreParams p) 
     }
   }
 
+  if constexpr (SPLIT) return;
   if constexpr (ONE_PASS) {
     // Block sums of a row: the sum over its TPB query tiles of (workspace
     // sum) / Z. They are formed for a group of the wave's rows at a time in
@@ -788,6 +807,138 @@ __global__ void __launch_bounds__(256, 2) score_topk_wide_kernel(ScoreParams p) 
                             mrow, hist + w * 256 * SEL_SUB, lane);
     }
   }
+}
+
+// select_row for at most 64 R candidates, whose order keys the lanes hold
+// (key[r]: column 64 r + lane, 0 past n_cand): the k-th largest key is found
+// bit by bit with ballots, without LDS atomics or histograms. The bits stop
+// early once exactly k_pick keys reach the prefix.
+template <int R>
+__device__ __forceinline__ void select_row_regs(const uint32_t* key, int n_cand, int k_pick, int dense_col, int kb,
+                                                int32_t* cols, uint8_t* mask_row, int lane) {
+  uint32_t prefix = 0;
+  bool exact = false;  // the keys >= prefix are the k_pick largest
+  for (int bit = 31; bit >= 0 && !exact; --bit) {
+    const uint32_t cand = prefix | (1u << bit);
+    int cnt = 0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) cnt += __popcll(__ballot(64 * r + lane < n_cand && key[r] >= cand));
+    if (cnt >= k_pick) prefix = cand;
+    exact = cnt == k_pick;
+  }
+  int remaining = k_pick;  // of the keys equal to the k-th, lowest column first
+  if (!exact) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) remaining -= __popcll(__ballot(64 * r + lane < n_cand && key[r] > prefix));
+  }
+  const uint64_t below = lanes_below(lane);
+  int out = 0, ties = 0;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int j = 64 * r + lane;
+    const bool valid = j < n_cand;
+    const bool eq = !exact && valid && key[r] == prefix;
+    const uint64_t eqb = __ballot(eq);
+    const bool take = valid && (exact ? key[r] >= prefix
+                                      : key[r] > prefix || (eq && ties + __popcll(eqb & below) < remaining));
+    const uint64_t tb = __ballot(take);
+    if (take) cols[out + __popcll(tb & below)] = j;
+    if (mask_row && valid) mask_row[j] = take ? 1 : 0;
+    out += __popcll(tb);
+    ties += __popcll(eqb);
+  }
+  if (mask_row)
+    for (int j = n_cand + lane; j < dense_col; j += kWave) mask_row[j] = 0;
+  for (int j = dense_col + lane; j < kb; j += kWave) {
+    cols[out + (j - dense_col)] = j;
+    if (mask_row) mask_row[j] = 1;
+  }
+}
+
+constexpr int kMaxSplits = 8;  // shares of the key chunks (8 splits x 8 tiles: one lane each)
+
+// Second kernel of the split form: one wave per query block. The shares of
+// its TPB tiles are weighted by 2^(m - M) / Z (M the largest reference, Z the
+// joined sum), summed into the row's block sums and selected from. Four
+// consecutive rows per workgroup, so the 128-byte workspace lines they share
+// are fetched together. Latency-bound: the wide kernel's own epilogue selects
+// up to eight rows per wave one after the other, which took most of the time
+// of a call with few workgroups.
+template <int TPB>
+__global__ void __launch_bounds__(256) select_rows_kernel(ScoreParams p, int nx) {
+  constexpr int QBW = 32 / TPB, G = 4 * QBW, WG_TILES = G * TPB;
+  extern __shared__ __attribute__((aligned(16))) float smem[];  // [4][Kb] block sums
+  __shared__ float wt[4][kMaxSplits * TPB];                     // tile weights per split
+  __shared__ uint32_t hist[4][256];
+  const Policy& pol = p.pol;
+  const int h = blockIdx.y, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int qb = blockIdx.x * 4 + w;
+  if (qb >= pol.Qb) return;
+  const int64_t row = static_cast<int64_t>(h) * pol.Qb + qb;
+  int32_t* cols = p.col_idx + p.row_ptr[row];
+  uint8_t* mrow = p.mask_out ? p.mask_out + row * pol.Kb : nullptr;
+  const int score_rows = p.scores_out ? pol.scored_rows : min(pol.scored_rows, pol.dense_row);
+  float* const sums = smem + w * pol.Kb;
+  const bool small = pol.n_cand <= 256;  // keys fit four registers per lane
+  uint32_t key[4] = {};
+  if (qb < score_rows) {
+    const int wg = qb / G, t0 = (qb - wg * G) * TPB;  // the row's tiles in its workgroup's workspace
+    const int64_t base = static_cast<int64_t>(h) * nx + wg;
+    const int t = lane % TPB, s = lane / TPB;
+    float2 mz = make_float2(-INFINITY, 0.f);
+    if (s < p.splits) mz = p.tile_mz[(base * p.splits + s) * WG_TILES + t0 + t];
+    float M = mz.x;
+#pragma unroll
+    for (int off = TPB; off < 64; off <<= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
+    const float f = mz.x > -INFINITY ? exp2_fast(mz.x - M) : 0.f;
+    float Z = mz.y * f;
+#pragma unroll
+    for (int off = TPB; off < 64; off <<= 1) Z += __shfl_xor(Z, off, 64);
+    if (s < p.splits) wt[w][s * TPB + t] = Z > 0.f ? f / Z : 0.f;
+    lds_sync_wave();
+    const float* src = p.tile_sums + base * p.tile_cols * WG_TILES + t0;
+    float* out = p.scores_out ? p.scores_out + (static_cast<int64_t>(h) * pol.scored_rows + qb) * pol.Kb : nullptr;
+    const int bps = p.cps * (32 / TPB);  // key blocks per split
+    auto block_sum = [&](int kb) {
+      const float4* u = reinterpret_cast<const float4*>(src + static_cast<int64_t>(kb) * WG_TILES);
+      const float* g = &wt[w][(kb / bps) * TPB];
+      float v = 0.f;
+#pragma unroll
+      for (int i = 0; i < TPB / 4; ++i) {
+        const float4 a = u[i];
+        v += (a.x * g[4 * i] + a.y * g[4 * i + 1]) + (a.z * g[4 * i + 2] + a.w * g[4 * i + 3]);
+      }
+      return v;
+    };
+    if (small) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int kb = 64 * r + lane;
+        if (kb < pol.Kb) {
+          const float v = block_sum(kb);
+          if (kb < pol.n_cand) key[r] = order_key(v);
+          if (out) out[kb] = v;
+        }
+      }
+      if (out)
+        for (int kb = 256 + lane; kb < pol.Kb; kb += 64) out[kb] = block_sum(kb);
+    } else {
+      for (int kb = lane; kb < pol.Kb; kb += 64) {
+        const float v = block_sum(kb);
+        sums[kb] = v;
+        if (out) out[kb] = v;
+      }
+      lds_sync_wave();
+    }
+  }
+  if (qb >= pol.dense_row || qb >= pol.scored_rows)
+    dense_row(pol.Kb, cols, mrow, lane);
+  else if (pol.n_cand <= 64)
+    select_row_regs<1>(key, pol.n_cand, pol.k_pick, pol.dense_col, pol.Kb, cols, mrow, lane);
+  else if (small)
+    select_row_regs<4>(key, pol.n_cand, pol.k_pick, pol.dense_col, pol.Kb, cols, mrow, lane);
+  else
+    select_row(sums, pol.n_cand, pol.k_pick, pol.dense_col, pol.Kb, cols, mrow, hist[w], lane);
 }
 
 // Block sums of one 32 x 32 chunk of tile probabilities for TPBK key tiles
@@ -1029,6 +1180,31 @@ bool valid_tile(int64_t t) { return t >= 4 && t <= kBlock && kBlock % t == 0; }
 // pass with a workspace); every other pair runs score_topk_tiles_kernel.
 bool tuned_tiles(int64_t q_tile, int64_t k_tile) { return q_tile == k_tile && (q_tile == 16 || q_tile == 32); }
 
+// Split form of the one-pass scorer for `wgs` workgroups and nchunks key
+// chunks; splits 0: the workgroups select for themselves. Up to 768
+// workgroups (three per CU, what the registers allow) the chip has room, and a
+// workgroup's rows selected one after the other are most of its time: the
+// rows then get a wave each in a second kernel, and the key chunks (at least
+// two a share) are divided until the 768 are reached. Scoring and selection,
+// workgroups: 12: 35 -> 11 us; 80: 28 -> 15; 168: 47 -> 32; 185: 166 -> 110;
+// 300: 93 -> 76; 400: 78 -> 69; 640: 101 -> 96. Above, the second kernel's
+// read of the workspace costs more than it saves (1,480: 666 -> 702).
+struct ScoreSplit {
+  int splits, cps;
+};
+ScoreSplit score_split(int64_t wgs, int nchunks) {
+  constexpr int64_t kSlots = 768;
+  if (wgs > kSlots) return {0, 0};
+  const int64_t want = kSlots / wgs < kMaxSplits ? kSlots / wgs : kMaxSplits;
+  int cps = static_cast<int>((nchunks + want - 1) / want);
+  cps += cps & 1;  // shares start on the first of the two LDS buffers
+  return {(nchunks + cps - 1) / cps, cps};
+}
+// Bytes of the split form's m and z behind the per-tile sums.
+int64_t split_bytes(int64_t wgs) {
+  return wgs <= 768 ? wgs * kMaxSplits * 128 * 2 * static_cast<int64_t>(sizeof(float)) : 0;
+}
+
 int score_topk_impl(const char* name, const uint16_t* q_pool_hi, const uint16_t* q_pool_lo,
                     const uint16_t* k_pool_hi, const uint16_t* k_pool_lo, int64_t heads, int64_t head_dim,
                     int64_t q_tile_size, int64_t k_tile_size, int64_t q_blocks, int64_t k_blocks,
@@ -1116,6 +1292,31 @@ int score_topk_impl(const char* name, const uint16_t* q_pool_hi, const uint16_t*
     p.tile_sums = static_cast<float*>(workspace);
     p.tile_cols = static_cast<int>((k_blocks * tpb + 31) / 32 * (32 / tpb));
     dim3 grid(static_cast<unsigned>((q_blocks + Gw - 1) / Gw), static_cast<unsigned>(heads));
+    const int nchunks = (p.k_tiles + 31) / 32;
+    const int64_t wgs = static_cast<int64_t>(grid.x) * heads;
+    const ScoreSplit sp = score_split(wgs, nchunks);
+    if (sp.splits > 0 && workspace_bytes >= need + split_bytes(wgs)) {
+      p.splits = sp.splits;
+      p.cps = sp.cps;
+      p.tile_mz = reinterpret_cast<float2*>(static_cast<char*>(workspace) + need);
+      grid.z = static_cast<unsigned>(sp.splits);
+      if (head_dim == 128 && tpb == 8)
+        score_topk_wide_kernel<128, 8, true, true, true><<<grid, 256, smem_gb, s>>>(p);
+      else if (head_dim == 128)
+        score_topk_wide_kernel<128, 4, true, true, true><<<grid, 256, smem_gb, s>>>(p);
+      else if (tpb == 8)
+        score_topk_wide_kernel<64, 8, true, true, true><<<grid, 256, smem_gb, s>>>(p);
+      else
+        score_topk_wide_kernel<64, 4, true, true, true><<<grid, 256, smem_gb, s>>>(p);
+      const dim3 rows(static_cast<unsigned>((q_blocks + 3) / 4), static_cast<unsigned>(heads));
+      const size_t smem_rows = static_cast<size_t>(4) * k_blocks * sizeof(float);
+      const int nx = static_cast<int>(grid.x);
+      if (tpb == 8)
+        select_rows_kernel<8><<<rows, 256, smem_rows, s>>>(p, nx);
+      else
+        select_rows_kernel<4><<<rows, 256, smem_rows, s>>>(p, nx);
+      return check_launch(name);
+    }
     if (head_dim == 128 && tpb == 8)
       score_topk_wide_kernel<128, 8, true, true><<<grid, 256, smem_gb, s>>>(p);
     else if (head_dim == 128)
@@ -1177,6 +1378,14 @@ int64_t dfs_block_score_topk_workspace_size(int64_t heads, int64_t q_tile_size, 
   const int64_t rows = (q_blocks + Gw - 1) / Gw * Gw * tpb;        // tile rows of every workgroup
   const int64_t cols = (k_blocks * tpb + 31) / 32 * (32 / tpb);  // key blocks of every 32-tile chunk
   return heads * rows * cols * static_cast<int64_t>(sizeof(float));
+}
+
+int64_t dfs_block_score_topk_split_size(int64_t heads, int64_t q_tile_size, int64_t k_tile_size, int64_t q_blocks,
+                                        int64_t k_blocks) {
+  const int64_t n = dfs_block_score_topk_workspace_size(heads, q_tile_size, k_tile_size, q_blocks, k_blocks);
+  if (n <= 0) return n;
+  const int64_t Gw = 4 * (32 / (dfs::kBlock / q_tile_size));
+  return n + dfs::split_bytes(heads * ((q_blocks + Gw - 1) / Gw));
 }
 
 int dfs_block_score_topk(const uint16_t* q_pool_hi, const uint16_t* q_pool_lo,

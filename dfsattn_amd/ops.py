@@ -196,11 +196,14 @@ def _policy_args(policy: TopkPolicy):
             policy.dense_col, policy.dense_row)
 
 
-def score_workspace_bytes(heads: int, q_tile: int, k_tile: int, q_blocks: int, k_blocks: int) -> int:
-    """Bytes of the one-pass scoring workspace (per-tile partial block sums);
-    0 when these tile sizes have no one-pass form (the scorer then runs its
-    two passes)."""
-    n = int(_lib.lib().dfs_block_score_topk_workspace_size(heads, q_tile, k_tile, q_blocks, k_blocks))
+def score_workspace_bytes(heads: int, q_tile: int, k_tile: int, q_blocks: int, k_blocks: int,
+                          split: bool = False) -> int:
+    """Bytes of the one-pass scoring workspace (per-tile partial block sums;
+    with ``split`` also what the split form of small problems needs); 0 when
+    these tile sizes have no one-pass form (the scorer then runs its two
+    passes)."""
+    size = _lib.lib().dfs_block_score_topk_split_size if split else _lib.lib().dfs_block_score_topk_workspace_size
+    n = int(size(heads, q_tile, k_tile, q_blocks, k_blocks))
     if n < 0:
         raise ValueError(f"no scoring workspace for heads={heads} tiles={q_tile}/{k_tile} "
                          f"blocks={q_blocks}x{k_blocks}")
@@ -208,12 +211,14 @@ def score_workspace_bytes(heads: int, q_tile: int, k_tile: int, q_blocks: int, k
 
 
 def block_score_topk(prep: Prepared, policy: TopkPolicy, row_ptr: torch.Tensor,
-                     want_scores: bool = False, want_mask: bool = False, one_pass: bool = True):
+                     want_scores: bool = False, want_mask: bool = False, one_pass: bool = True,
+                     split: bool = True):
     """Scores + top-k: returns (col_idx int32 [nnz], scores fp32 [H,Vb,Kb] or
     None, mask uint8 [H,Qb,Kb] or None). With ``one_pass`` a workspace of
     per-tile partial sums lets the kernel score every tile pair once instead
     of twice (normaliser pass, then block-sum pass), and the score matrix is
-    written only when asked for. The two-pass form (and rows wider than the
+    written only when asked for; ``split`` lets small problems divide the keys
+    over more workgroups and select in a second kernel. The two-pass form (and rows wider than the
     one-pass form's 16 * head_dim columns) always gets the score matrix,
     where it keeps its block sums rather than in LDS (more workgroups per
     CU)."""
@@ -229,7 +234,7 @@ def block_score_topk(prep: Prepared, policy: TopkPolicy, row_ptr: torch.Tensor,
     q_tile, k_tile = prep.layout.q_tile, prep.layout.k_tile
     ws_bytes = 0
     if one_pass and policy.k_blocks <= 16 * prep.head_dim:
-        ws_bytes = score_workspace_bytes(prep.heads, q_tile, k_tile, policy.q_blocks, policy.k_blocks)
+        ws_bytes = score_workspace_bytes(prep.heads, q_tile, k_tile, policy.q_blocks, policy.k_blocks, split=split)
     one_pass_rows = ws_bytes > 0
     scores = (torch.empty((prep.heads, policy.scored_rows, policy.k_blocks), dtype=torch.float32, device=dev)
               if want_scores or not one_pass_rows else None)

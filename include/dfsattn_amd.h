@@ -181,6 +181,16 @@ int dfs_block_score_topk(const uint16_t* q_pool_hi, const uint16_t* q_pool_lo,
 int64_t dfs_block_score_topk_workspace_size(int64_t heads, int64_t q_tile_size,
                                             int64_t k_tile_size, int64_t q_blocks,
                                             int64_t k_blocks);
+/*
+ * Bytes that also let dfs_block_score_topk use its split form where that is
+ * the faster one (few workgroups: the key chunks are divided over more of
+ * them and a second kernel selects, one wave per row); equal to the above for
+ * larger problems. A workspace of at least the above but less than this keeps
+ * the one-kernel form.
+ */
+int64_t dfs_block_score_topk_split_size(int64_t heads, int64_t q_tile_size,
+                                        int64_t k_tile_size, int64_t q_blocks,
+                                        int64_t k_blocks);
 
 /*
  * dfs_block_score_topk that allocates nothing and takes no caller scratch:

@@ -359,6 +359,45 @@ def test_block_score_topk_all_tied_keeps_lowest_columns(dev, heads, length, text
         assert torch.equal(mask.cpu().bool(), want), one_pass
 
 
+@pytest.mark.parametrize("d,tile,heads,video,text,q_size", [
+    (128, 16, 2, 64 * 128, 0, 1.0),      # 64 columns: one register of keys
+    (64, 16, 1, 64 * 128 + 5, 0, 1.0),   # 65 columns: four registers
+    (128, 32, 3, 256 * 128, 0, 1.0),     # 256 columns, 8 rows per wave of the unsplit form
+    (64, 32, 1, 257 * 128 - 3, 0, 1.0),  # 257 columns: radix selection
+    (128, 16, 8, 2000, 100, 1.0),        # dense text rows and columns
+    (128, 16, 1, 100, 0, 1.0),           # one block, one chunk
+    (64, 16, 2, 3000, 0, 0.0),           # every score tied
+    (128, 16, 2, 6000, 0, 40.0),         # logits far apart: shares with references far apart
+])
+def test_block_score_topk_split_matches_unsplit(dev, d, tile, heads, video, text, q_size):
+    """Small problems divide the key chunks over workgroups and select in a
+    second kernel: scores against the one-kernel form within fp32 rounding of
+    sums in another order, and the selection of each form's own scores."""
+    print(f"split d={d} tile={tile} heads={heads} video={video} text={text}", flush=True)
+    L = video + text
+    g = torch.Generator().manual_seed(L + tile)
+    field = torch.randn((1, heads, -(-L // 96), d), generator=g).repeat_interleave(96, dim=2)[:, :, :L]
+    q, k = (field + 0.5 * torch.randn((1, heads, L, d), generator=g) for _ in range(2))
+    q, k = (q * q_size).to(torch.bfloat16).to(dev), k.to(torch.bfloat16).to(dev)
+    layout = ScoringLayout(L, video, tile)
+    pol = hunyuan_policy(layout, 0.5) if text else wan_policy(layout, 0.3)
+    row_ptr = torch.from_numpy(pol.row_ptr(heads)).to(dev)
+    prep = ops.prepare_qkv(q, k, q, torch.arange(L, dtype=torch.int32, device=dev), layout)
+    res = {}
+    for split in (False, True):
+        cols, scores, mask = ops.block_score_topk(prep, pol, row_ptr, want_scores=True, want_mask=True, split=split)
+        only, _, _ = ops.block_score_topk(prep, pol, row_ptr, split=split)
+        assert torch.equal(cols, only)  # asking for scores changes nothing
+        sel = (orc.mask_from_scores_hunyuan(scores.cpu(), 0.5, L, video) if text
+               else orc.mask_from_scores_wan(scores.cpu(), 0.3))
+        assert torch.equal(mask.bool().cpu(), sel)
+        back = ops.csr_to_mask(row_ptr, cols, heads, pol.q_blocks, pol.k_blocks)
+        assert torch.equal(back, mask.bool())
+        res[split] = scores.cpu()
+    # sums of at most 2^8 terms per tile and of the shares in another order
+    assert torch.allclose(res[True], res[False], rtol=1e-5, atol=1e-10)
+
+
 @pytest.mark.parametrize("direction", ["rising", "falling"])
 @pytest.mark.parametrize("tile,one_pass", [(16, True), (32, True), (16, False), (32, False)])
 def test_block_scores_with_far_apart_logits(dev, direction, tile, one_pass):
