@@ -38,6 +38,8 @@ SIGNATURES = {
     "dfs_bsa_fwd_workspace_size": [_i64, _i64, _i64, _i64, _i64, _i64, _i64],
     "dfs_bsa_fwd_parts": [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i32, _i32, _f32, _p, _i32, _p, _p, _p, _p, _i64, _p,
                           _p, _p, _i32, _i64, _i64, _i64, _i64, _i64, _i64, _p, _i64, _p],
+    "dfs_call_workspace_size": [_p],
+    "dfs_call": [_p, _i32, _p],
     "dfs_mask_row_counts": [_p, _i64, _i64, _p, _p],
     "dfs_mask_to_csr": [_p, _i64, _i64, _p, _p, _p],
     "dfs_csr_to_mask": [_p, _p, _i64, _i64, _p, _p],
@@ -50,8 +52,22 @@ SIGNATURES = {
     "dfs_adaln_modulate": [_p, _i64, _i64, _i32, _p, _p, _p, _p, _f32, _p, _p],
     "dfs_gated_residual": [_p, _p, _p, _i64, _i64, _i32, _p, _p],
 }
+
+class CallArgs(ctypes.Structure):
+    """dfs_call_args, field by field."""
+
+    _fields_ = [(n, _i64) for n in (
+        "heads", "seq_len", "head_dim", "video_len", "q_tile", "k_tile", "dtype", "operand_dtype", "out_dtype",
+        "select", "q_blocks", "k_blocks", "scored_rows", "n_cand", "k_pick", "dense_col", "dense_row", "long_row",
+        "long_parts", "full_rows", "parts", "out_head_stride", "out_row_stride", "n_seq", "workspace_bytes")] + [
+        ("scale", ctypes.c_double)] + [(n, _p) for n in (
+            "q", "k", "v", "perm", "row_ptr", "col_idx", "out", "out_perm", "cu_seqlens_q", "cu_seqlens_k",
+            "workspace")]
+
+
 _RESTYPES = {"dfs_last_error": ctypes.c_char_p, "dfs_block_score_topk_workspace_size": ctypes.c_int64,
-             "dfs_block_score_topk_split_size": ctypes.c_int64, "dfs_bsa_fwd_workspace_size": ctypes.c_int64}
+             "dfs_block_score_topk_split_size": ctypes.c_int64, "dfs_bsa_fwd_workspace_size": ctypes.c_int64,
+             "dfs_call_workspace_size": ctypes.c_int64}
 ABI_VERSION = 5
 
 _lock = threading.Lock()

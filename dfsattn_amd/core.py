@@ -14,7 +14,7 @@ import numpy as np
 import torch
 
 from . import ops
-from .layout import ScoringLayout, TopkPolicy
+from .layout import ScoringLayout, TopkPolicy, scoring_layout
 
 SUPPORTED_EXECUTION = "native"
 
@@ -76,11 +76,6 @@ class DfsCore:
     # get_cache_info counts these per entry, as the reference does (:664-670).
     _entry_fields: Tuple[str, ...] = ("block_mask", "block_indices", "flex_block_mask")
 
-    def _prepare(self, q, k, v, perm, layout, pool: bool) -> "ops.Prepared":
-        # No permuted Q: the attention kernel gathers Q rows from the input.
-        return ops.prepare_qkv(q, k, v, perm, layout, operand_dtype=operand_dtype_for(q.dtype, self.operand_dtype),
-                               pool=pool, q_operand=False)
-
     # --- permutation -----------------------------------------------------
     def _device_permutation(self, seq_len: int, device: torch.device) -> torch.Tensor:
         """int32 execution permutation on ``device`` (video order, then the
@@ -105,8 +100,8 @@ class DfsCore:
     def _layout(self, seq_len: int) -> ScoringLayout:
         """Scoring layout with the instance's query and key tile sizes (each
         must divide the block, attention_wan.py:227-228)."""
-        return ScoringLayout(seq_len, self._video_len(seq_len), self.q_tile_size, self.block_size,
-                             k_tile=self.k_tile_size)
+        return scoring_layout(seq_len, self._video_len(seq_len), self.q_tile_size, self.block_size,
+                              self.k_tile_size)
 
     # --- checks ---------------------------------------------------------------
     def _check_call(self, q, k, v, attn_mask, causal, drop_rate, batch_size):
@@ -159,27 +154,6 @@ class DfsCore:
         return flat.to(torch.int32).contiguous()
 
     # --- selection and execution --------------------------------------------
-    def _select(self, prep: ops.Prepared, layout: ScoringLayout, sparse_ratio: float,
-                want_scores: bool = False) -> MaskEntry:
-        policy = self._policy(layout, sparse_ratio)
-        row_ptr = row_ptr_for(policy, prep.heads, prep.device)
-        col_idx, scores, _ = ops.block_score_topk(prep, policy, row_ptr, want_scores=want_scores)
-        entry = MaskEntry(row_ptr=row_ptr, col_idx=col_idx, policy=policy, heads=prep.heads,
-                          **{field: None for field in self._entry_fields})
-        if want_scores:
-            dict.__setitem__(entry, "block_scores", scores)
-        return entry
-
-    def _execute(self, prep: ops.Prepared, entry: MaskEntry, perm: torch.Tensor,
-                 cu_q: Optional[torch.Tensor] = None, cu_k: Optional[torch.Tensor] = None) -> torch.Tensor:
-        """block_sparse_attn_func of the selected mask (attention_wan.py:335-391,
-        attention_hyvideo.py:1026-1087). With cu_seqlens [0, a, L] the
-        second sequence's rows attend its own keys under the mask indexed from
-        its start, as the external kernel does for the repeated mask; the split
-        is read on the device."""
-        return ops.bsa_fwd(prep, entry["row_ptr"], entry["col_idx"], scale=None, out_dtype=prep.dtype,
-                           out_perm=perm, cu_seqlens_q=cu_q, cu_seqlens_k=cu_k)
-
     @staticmethod
     def _tile_counts(entry: MaskEntry) -> np.ndarray:
         pol: TopkPolicy = entry["policy"]
@@ -221,26 +195,43 @@ class DfsCore:
         entry = self._cache_entry(key, layout)
         recompute = entry is None or self.cache_flag
         rec = cls.timing_recorder
-        t_perm = rec.start(device)
-        prep = self._prepare(q, k, v, perm, layout, pool=recompute)
-        rec.stop(t_perm, phase="qkv_permute", step_idx=self.step_idx, layer_idx=self.layer_idx, device=device)
         if recompute:
-            t_topk = rec.start(device)
-            with torch.no_grad():
-                entry = self._select(prep, layout, self.sparse_ratio)
-            rec.stop(t_topk, phase="topk_mask", step_idx=self.step_idx, layer_idx=self.layer_idx, device=device)
+            policy = self._policy(layout, self.sparse_ratio)
+            row_ptr, col_idx = row_ptr_for(policy, q.shape[1], device), None
+        else:
+            policy, row_ptr, col_idx = entry["policy"], entry["row_ptr"], entry["col_idx"]
+        call = ops.Call(q, k, v, perm, layout, policy, row_ptr, col_idx,
+                        operand_dtype=operand_dtype_for(q.dtype, self.operand_dtype), out_perm=perm,
+                        cu_seqlens_q=cu_q, cu_seqlens_k=cu_k)
+        if recompute:
+            entry = MaskEntry(row_ptr=row_ptr, col_idx=call.col_idx, policy=policy, heads=q.shape[1],
+                              **{field: None for field in self._entry_fields})
+        if not rec.enabled:
+            call.run()
+        else:
+            at = dict(step_idx=self.step_idx, layer_idx=self.layer_idx, device=device)
+            mark = rec.start(device)
+            call.run(ops.PREPARE)
+            rec.stop(mark, phase="qkv_permute", **at)
+            if recompute:
+                mark = rec.start(device)
+                call.run(ops.SELECT)
+                rec.stop(mark, phase="topk_mask", **at)
+            mark = rec.start(device)
+            call.run(ops.ATTEND)
+            rec.stop(mark, phase="attention_execution", **at)
+        if recompute:
             if self.cache_flag:
                 self._store(key, entry)
             self._maybe_export(entry)
         if cls.record_density:
             self._record_density(entry, seq_len)
-        t_att = rec.start(device)
-        out = self._execute(prep, entry, perm, cu_q, cu_k)
-        rec.stop(t_att, phase="attention_execution", step_idx=self.step_idx, layer_idx=self.layer_idx, device=device)
-        return out
+        return call.out
 
     def _store(self, key, entry: MaskEntry) -> None:
-        type(self)._cached_metadata[key] = entry.clone()
+        # The columns were written for this entry alone and nothing writes them
+        # again, so the cache holds them without a copy.
+        type(self)._cached_metadata[key] = MaskEntry(entry)
 
     def _maybe_export(self, entry: MaskEntry) -> None:
         cls = type(self)

@@ -103,7 +103,11 @@ struct PrepParams {
   uint4* q_lo;
   uint4* k_hi;  // [H][k_tiles][D] bf16
   uint4* k_lo;
-  int32_t* flags;  // optional [3][H] overflow flags (Q, K, V)
+  int32_t* flags;  // optional [3][H] overflow flags (Q, K, V), zeroed by the caller
+  // Or one word per wave, each written once (nothing to zero): Q and K
+  // [2][H][nqk], then V [H][nv]. prep_fixup_kernel joins them.
+  int32_t* wave_flags;
+  int nqk, nv;
   int L;         // tokens
   int Lv;        // video tokens (== L for Wan)
   int R;         // execution rows per head, ceil(L/128)*128
@@ -172,7 +176,11 @@ __device__ __forceinline__ void prep_qk_tiles(const PrepParams& p, int bx, int n
 
   const int tile = is_k ? p.tile_k : p.tile_q;
   const int t = bx * 4 + wave;
-  if (t * tile >= p.R) return;  // past the scoring layout (R tokens) of this tensor
+  int32_t* const word = p.wave_flags ? p.wave_flags + ((is_k ? H : 0) + h) * static_cast<int64_t>(p.nqk) + t : nullptr;
+  if (t * tile >= p.R) {  // past the scoring layout (R tokens) of this tensor
+    if (word && lane == 0) *word = 0;
+    return;
+  }
   const int c = lane % CPR;
   const int g = lane / CPR;
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -202,6 +210,10 @@ __device__ __forceinline__ void prep_qk_tiles(const PrepParams& p, int bx, int n
     }
   }
   if (p.flags && overflow) atomicOr(&p.flags[(is_k ? 1 : 0) * H + h], 1);
+  if (word) {
+    const int any = __any(overflow);
+    if (lane == 0) *word = any;
+  }
   const int n_tiles = is_k ? p.k_tiles : p.q_tiles;
   if (!p.pool || t >= n_tiles) return;
 #pragma unroll
@@ -297,6 +309,12 @@ __device__ __forceinline__ void prep_v_block(const PrepParams& p, int kb, int h,
     if (half == 0) __syncthreads();  // every staged chunk is read before the second half overwrites it
   }
   if (p.flags && overflow) atomicOr(&p.flags[2 * H + h], 1);
+  if (p.wave_flags && active) {
+    const int any = __any(overflow);
+    constexpr int NW = NT / kWave;
+    if ((tid & 63) == 0)
+      p.wave_flags[2 * H * static_cast<int64_t>(p.nqk) + h * static_cast<int64_t>(p.nv) + kb * NW + (tid >> 6)] = any;
+  }
 }
 
 // Q and K: one wave per (tensor, head, scoring tile), four tiles per
@@ -313,6 +331,22 @@ __global__ void __launch_bounds__(16 * (D / 8)) prep_v_kernel(PrepParams p) {
   prep_v_block<D>(p, blockIdx.x, blockIdx.y, gridDim.y, threadIdx.x, stage);
 }
 
+// Q, K and V of a small problem in one launch (grid: x, heads, 3): the second
+// kernel's start-up and the gap before it are most of its time there.
+template <int D>
+__global__ void __launch_bounds__(256) prep_qkv_kernel(PrepParams p, int nbx_qk) {
+  constexpr int NT = 16 * (D / 8), PER = 256 / NT;  // V blocks per workgroup
+  __shared__ uint4 stage[PER * (D / 2 * (kBlock / 8))];
+  if (blockIdx.z < 2) {
+    if (static_cast<int>(blockIdx.x) < nbx_qk)
+      prep_qk_tiles<D>(p, blockIdx.x, nbx_qk, blockIdx.y, gridDim.y, blockIdx.z == 1);
+    return;
+  }
+  const int sub = threadIdx.x / NT;
+  prep_v_block<D>(p, blockIdx.x * PER + sub, blockIdx.y, gridDim.y, threadIdx.x - sub * NT,
+                  stage + sub * (D / 2 * (kBlock / 8)));
+}
+
 // bf16 -> f16 of eight packed values times sc (a power of two).
 __device__ __forceinline__ uint4 bf16x8_to_f16x8_scaled(const uint4& v, float sc) {
   uint32_t e[8];
@@ -323,7 +357,7 @@ __device__ __forceinline__ uint4 bf16x8_to_f16x8_scaled(const uint4& v, float sc
 
 // One workgroup per (head, tensor) of a call whose bf16 inputs were rounded
 // to f16 operands. When the prepare kernel flagged the head (a finite value
-// beyond the f16 range), the head's operand is rewritten from the inputs as
+// beyond the f16 range, in the head's word or in any of its waves'), the head's operand is rewritten from the inputs as
 // x * 2^-e, with e >= 1 the smallest exponent that brings the head's largest
 // finite |x| below 2^15, and exps[tensor][h] = e; otherwise exps[tensor][h] =
 // 0. The flag is cleared. Powers of two are exact, so the attention kernel
@@ -333,7 +367,18 @@ __global__ void __launch_bounds__(1024) prep_fixup_kernel(PrepParams p, int32_t*
   constexpr int CPR = D / 8;
   const int h = blockIdx.x, t = blockIdx.y, H = gridDim.x;
   const int slot = t * H + h;
-  if (flags[slot] == 0) {
+  int flagged;
+  if (p.wave_flags) {
+    const int n = t < 2 ? p.nqk : p.nv;
+    const int32_t* words = p.wave_flags + (t < 2 ? slot * static_cast<int64_t>(p.nqk)
+                                                 : 2 * H * static_cast<int64_t>(p.nqk) + h * static_cast<int64_t>(p.nv));
+    int any = 0;
+    for (int i = threadIdx.x; i < n; i += blockDim.x) any |= words[i];
+    flagged = __syncthreads_or(any);
+  } else {
+    flagged = flags[slot];
+  }
+  if (flagged == 0) {
     if (threadIdx.x == 0) exps[slot] = 0;
     return;
   }
@@ -394,36 +439,25 @@ __global__ void __launch_bounds__(1024) prep_fixup_kernel(PrepParams p, int32_t*
   }
   if (threadIdx.x == 0) {
     exps[slot] = e;
-    flags[slot] = 0;
+    if (flags) flags[slot] = 0;
   }
 }
 
+// Waves of the Q/K part and of the V part of a head that write a flag word.
+void wave_flag_counts(int64_t kb, int64_t head_dim, int64_t q_tile, int64_t k_tile, int* nqk, int* nv) {
+  const int64_t max_tiles = kb * kBlock / (q_tile < k_tile ? q_tile : k_tile);
+  *nqk = static_cast<int>((max_tiles + 3) / 4 * 4);
+  *nv = static_cast<int>(kb * (head_dim / 32));  // 16 * D / 8 threads
+}
+
 }  // namespace
-}  // namespace dfs
 
-extern "C" {
-
-int dfs_permute_gather(const void* src, const int32_t* perm, void* dst, int64_t heads,
-                       int64_t src_rows, int64_t n_perm, int64_t dst_rows, int64_t row_bytes,
-                       dfs_stream_t stream) {
-  return dfs::permute_rows(false, src, perm, dst, heads, src_rows, n_perm, dst_rows, row_bytes,
-                           reinterpret_cast<hipStream_t>(stream));
-}
-
-int dfs_permute_scatter(const void* src, const int32_t* perm, void* dst, int64_t heads,
-                        int64_t src_rows, int64_t n_perm, int64_t dst_rows, int64_t row_bytes,
-                        dfs_stream_t stream) {
-  return dfs::permute_rows(true, src, perm, dst, heads, src_rows, n_perm, dst_rows, row_bytes,
-                           reinterpret_cast<hipStream_t>(stream));
-}
-
-int dfs_prepare_qkv(const void* q, const void* k, const void* v, const int32_t* perm,
+int prepare_qkv_impl(const void* q, const void* k, const void* v, const int32_t* perm,
                     int64_t heads, int64_t seq_len, int64_t head_dim, int dtype,
                     int64_t video_len, int64_t q_tile_size, int64_t k_tile_size, int operand_dtype, void* q_perm,
                     void* k_perm, void* v_t, uint16_t* q_pool_hi, uint16_t* q_pool_lo,
-                    uint16_t* k_pool_hi, uint16_t* k_pool_lo, int32_t* overflow,
+                    uint16_t* k_pool_hi, uint16_t* k_pool_lo, int32_t* overflow, int32_t* wave_flags,
                     dfs_stream_t stream) {
-  using namespace dfs;
   DFS_REQUIRE(q && k && v && perm && k_perm && v_t, "dfs_prepare_qkv: NULL operand");
   DFS_REQUIRE(head_dim == 64 || head_dim == 128, "dfs_prepare_qkv: head_dim=%lld (supported: 64, 128)",
               (long long)head_dim);
@@ -467,6 +501,8 @@ int dfs_prepare_qkv(const void* q, const void* k, const void* v, const int32_t* 
   p.k_hi = reinterpret_cast<uint4*>(k_pool_hi);
   p.k_lo = reinterpret_cast<uint4*>(k_pool_lo);
   p.flags = overflow;
+  p.wave_flags = wave_flags;
+  wave_flag_counts(kb, head_dim, q_tile_size, k_tile_size, &p.nqk, &p.nv);
   p.L = static_cast<int>(seq_len);
   p.Lv = static_cast<int>(video_len);
   p.R = static_cast<int>(kb * kBlock);
@@ -484,6 +520,17 @@ int dfs_prepare_qkv(const void* q, const void* k, const void* v, const int32_t* 
   const int64_t max_tiles = kb * kBlock / (q_tile_size < k_tile_size ? q_tile_size : k_tile_size);
   dim3 gqk(static_cast<unsigned>((max_tiles + 3) / 4), static_cast<unsigned>(heads), 2);
   dim3 gv(static_cast<unsigned>(kb), static_cast<unsigned>(heads));
+  // One launch below 2,048 workgroups (eight per CU), where it saves a
+  // kernel's start-up; larger calls run 0-2% faster as two.
+  const int64_t per = head_dim == 128 ? 1 : 2, nbv = (kb + per - 1) / per;
+  if (heads * (2 * static_cast<int64_t>(gqk.x) + nbv) < 2048) {
+    const dim3 g(gqk.x > nbv ? gqk.x : static_cast<unsigned>(nbv), static_cast<unsigned>(heads), 3);
+    if (head_dim == 128)
+      prep_qkv_kernel<128><<<g, 256, 0, s>>>(p, static_cast<int>(gqk.x));
+    else
+      prep_qkv_kernel<64><<<g, 256, 0, s>>>(p, static_cast<int>(gqk.x));
+    return check_launch("dfs_prepare_qkv");
+  }
   if (head_dim == 128) {
     prep_qk_kernel<128><<<gqk, 256, 0, s>>>(p);
     prep_v_kernel<128><<<gv, 16 * 16, 0, s>>>(p);
@@ -494,11 +541,17 @@ int dfs_prepare_qkv(const void* q, const void* k, const void* v, const int32_t* 
   return check_launch("dfs_prepare_qkv");
 }
 
-int dfs_prepare_fixup(const void* q, const void* k, const void* v, const int32_t* perm, int64_t heads,
+int64_t prepare_flag_words(int64_t heads, int64_t seq_len, int64_t head_dim, int64_t q_tile, int64_t k_tile) {
+  int nqk, nv;
+  wave_flag_counts((seq_len + kBlock - 1) / kBlock, head_dim, q_tile, k_tile, &nqk, &nv);
+  return heads * (2 * static_cast<int64_t>(nqk) + nv);
+}
+
+int prepare_fixup_impl(const void* q, const void* k, const void* v, const int32_t* perm, int64_t heads,
                       int64_t seq_len, int64_t head_dim, void* q_perm, void* k_perm, void* v_t,
-                      int32_t* overflow, int32_t* exps, dfs_stream_t stream) {
-  using namespace dfs;
-  DFS_REQUIRE(q && k && v && perm && k_perm && v_t && overflow && exps, "dfs_prepare_fixup: NULL operand");
+                      int32_t* overflow, int32_t* wave_flags, int64_t q_tile_size, int64_t k_tile_size,
+                      int32_t* exps, dfs_stream_t stream) {
+  DFS_REQUIRE(q && k && v && perm && k_perm && v_t && (overflow || wave_flags) && exps, "dfs_prepare_fixup: NULL operand");
   DFS_REQUIRE(head_dim == 64 || head_dim == 128, "dfs_prepare_fixup: head_dim=%lld (supported: 64, 128)",
               (long long)head_dim);
   DFS_REQUIRE(heads > 0 && heads < 65536, "dfs_prepare_fixup: heads=%lld out of range", (long long)heads);
@@ -516,6 +569,8 @@ int dfs_prepare_fixup(const void* q, const void* k, const void* v, const int32_t
   p.v_t = static_cast<uint4*>(v_t);
   p.L = static_cast<int>(seq_len);
   p.R = static_cast<int>(kb * kBlock);
+  p.wave_flags = wave_flags;
+  if (wave_flags) wave_flag_counts(kb, head_dim, q_tile_size, k_tile_size, &p.nqk, &p.nv);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const dim3 grid(static_cast<unsigned>(heads), 3);
   if (head_dim == 128)
@@ -523,6 +578,42 @@ int dfs_prepare_fixup(const void* q, const void* k, const void* v, const int32_t
   else
     prep_fixup_kernel<64><<<grid, 1024, 0, s>>>(p, overflow, exps);
   return check_launch("dfs_prepare_fixup");
+}
+
+}  // namespace dfs
+
+extern "C" {
+
+int dfs_permute_gather(const void* src, const int32_t* perm, void* dst, int64_t heads,
+                       int64_t src_rows, int64_t n_perm, int64_t dst_rows, int64_t row_bytes,
+                       dfs_stream_t stream) {
+  return dfs::permute_rows(false, src, perm, dst, heads, src_rows, n_perm, dst_rows, row_bytes,
+                           reinterpret_cast<hipStream_t>(stream));
+}
+
+int dfs_permute_scatter(const void* src, const int32_t* perm, void* dst, int64_t heads,
+                        int64_t src_rows, int64_t n_perm, int64_t dst_rows, int64_t row_bytes,
+                        dfs_stream_t stream) {
+  return dfs::permute_rows(true, src, perm, dst, heads, src_rows, n_perm, dst_rows, row_bytes,
+                           reinterpret_cast<hipStream_t>(stream));
+}
+
+int dfs_prepare_qkv(const void* q, const void* k, const void* v, const int32_t* perm,
+                    int64_t heads, int64_t seq_len, int64_t head_dim, int dtype,
+                    int64_t video_len, int64_t q_tile_size, int64_t k_tile_size, int operand_dtype, void* q_perm,
+                    void* k_perm, void* v_t, uint16_t* q_pool_hi, uint16_t* q_pool_lo,
+                    uint16_t* k_pool_hi, uint16_t* k_pool_lo, int32_t* overflow,
+                    dfs_stream_t stream) {
+  return dfs::prepare_qkv_impl(q, k, v, perm, heads, seq_len, head_dim, dtype, video_len, q_tile_size, k_tile_size,
+                               operand_dtype, q_perm, k_perm, v_t, q_pool_hi, q_pool_lo, k_pool_hi, k_pool_lo,
+                               overflow, nullptr, stream);
+}
+
+int dfs_prepare_fixup(const void* q, const void* k, const void* v, const int32_t* perm, int64_t heads,
+                      int64_t seq_len, int64_t head_dim, void* q_perm, void* k_perm, void* v_t,
+                      int32_t* overflow, int32_t* exps, dfs_stream_t stream) {
+  return dfs::prepare_fixup_impl(q, k, v, perm, heads, seq_len, head_dim, q_perm, k_perm, v_t, overflow, nullptr, 0, 0,
+                                 exps, stream);
 }
 
 }  // extern "C"

@@ -25,7 +25,7 @@ import torch
 import torch.nn.functional as F
 
 from . import ops
-from .layout import ScoringLayout, dense_policy
+from .layout import dense_policy, scoring_layout
 
 _DENSE_CSR: Dict[Tuple[torch.device, int, int], Tuple[torch.Tensor, torch.Tensor]] = {}
 
@@ -34,7 +34,7 @@ def _dense_csr(device: torch.device, heads: int, seq_len: int) -> Tuple[torch.Te
     """Device CSR keeping every key block of every row, cached per shape."""
     key = (device, heads, seq_len)
     if key not in _DENSE_CSR:
-        layout = ScoringLayout(seq_len, seq_len, 16)
+        layout = scoring_layout(seq_len, seq_len, 16, 128, 16)
         pol = dense_policy(layout)
         row_ptr = torch.from_numpy(pol.row_ptr(heads)).to(device)
         col_idx = torch.arange(pol.k_blocks, dtype=torch.int32, device=device).repeat(heads * pol.q_blocks)
@@ -60,11 +60,12 @@ def dense_attention_native(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     cu_seqlens (2 or 3 entries) split it into sequences as the varlen
     kernel does, without a host read."""
     _, heads, length, _ = q.shape
-    layout = ScoringLayout(length, length, 16)
-    prep = ops.prepare_qkv(q, k, v, _identity(q.device, length), layout, operand_dtype=operand_dtype, pool=False,
-                           q_operand=False)
+    layout = scoring_layout(length, length, 16, 128, 16)
     row_ptr, col_idx = _dense_csr(q.device, heads, length)
-    return ops.bsa_fwd(prep, row_ptr, col_idx, cu_seqlens_q=cu_seqlens_q, cu_seqlens_k=cu_seqlens_k)
+    call = ops.Call(q, k, v, _identity(q.device, length), layout, dense_policy(layout), row_ptr, col_idx,
+                    operand_dtype=operand_dtype, cu_seqlens_q=cu_seqlens_q, cu_seqlens_k=cu_seqlens_k)
+    call.run()
+    return call.out
 
 
 def _sdpa(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -134,6 +135,8 @@ def _flash(q, k, v, cu_seqlens_q, cu_seqlens_kv, batch_size, operand_dtype=None)
             ck = whole_k if ck is None else ck
         if cq is not None and cq.numel() != ck.numel():
             raise ValueError("cu_seqlens_q and cu_seqlens_kv describe different segment counts")
+        if native and b == 1 and q.is_contiguous():
+            return dense_attention_native(q, k, v, cq, ck, operand_dtype)
         if native:
             out = torch.empty_like(q)
             for bi in range(b):

@@ -120,7 +120,14 @@ class TopkPolicy:
         return ptr.astype(np.int32)
 
     def nnz(self, heads: int) -> int:
-        return int(self.row_counts().sum()) * heads
+        kept = self.k_pick + (self.k_blocks - self.dense_col)
+        return (self.dense_row * kept + (self.q_blocks - self.dense_row) * self.k_blocks) * heads
+
+
+@functools.lru_cache(maxsize=1024)
+def scoring_layout(seq_len: int, video_len: int, tile: int, block: int, k_tile: int) -> ScoringLayout:
+    """ScoringLayout of these sizes (checked once per set of sizes)."""
+    return ScoringLayout(seq_len, video_len, tile, block, k_tile=k_tile)
 
 
 def topk_count(sparse_ratio: float, k_blocks: int) -> int:
@@ -129,6 +136,7 @@ def topk_count(sparse_ratio: float, k_blocks: int) -> int:
     return max(1, int(sparse_ratio * k_blocks))
 
 
+@functools.lru_cache(maxsize=1024)
 def wan_policy(layout: ScoringLayout, sparse_ratio: float) -> TopkPolicy:
     """attention_wan.py:248-253: every row keeps its top-k columns."""
     kb = layout.k_blocks
@@ -138,6 +146,7 @@ def wan_policy(layout: ScoringLayout, sparse_ratio: float) -> TopkPolicy:
     return TopkPolicy(layout.q_blocks, kb, layout.q_blocks, kb, k, kb, layout.q_blocks)
 
 
+@functools.lru_cache(maxsize=1024)
 def hunyuan_policy(layout: ScoringLayout, sparse_ratio: float) -> TopkPolicy:
     """attention_hyvideo.py:424-501 (top-k selector): the columns from
     video_len // 128 on are kept in every video row, the video budget is
@@ -160,6 +169,7 @@ def hunyuan_policy(layout: ScoringLayout, sparse_ratio: float) -> TopkPolicy:
     return TopkPolicy(layout.q_blocks, kb, layout.video_blocks, kb, k, kb, dense_row)
 
 
+@functools.lru_cache(maxsize=1024)
 def dense_policy(layout: ScoringLayout) -> TopkPolicy:
     """Every block kept (dense attention through the block-sparse kernel)."""
     return TopkPolicy(layout.q_blocks, layout.k_blocks, layout.q_blocks, 0, 0, 0, 0)
@@ -229,3 +239,12 @@ def attention_plan(heads: int, q_blocks: int, long_row: int, kept: int, kept_lon
     if long_row < q_blocks and kept > 0 and kept_long * 4 * XCD_SLOTS > kept * max(per_xcd, XCD_SLOTS // 2):
         long_parts = max(1, min(-(-kept_long // kept), 8, kept_long // 4))
     return long_parts, full_rows if parts > 1 else 0, parts
+
+
+def query_plan(layout: ScoringLayout, heads: int, nnz: int) -> Tuple[int, int, int, int]:
+    """(long_row, long_parts, full_rows, parts) of a call whose mask keeps
+    ``nnz`` blocks: attention_plan with the text query blocks, which keep
+    every key block, as the long ones."""
+    long_row = layout.video_len // layout.block if layout.text_len > 0 else layout.q_blocks
+    kept = max(0, nnz // heads - (layout.q_blocks - long_row) * layout.k_blocks) // max(long_row, 1)
+    return (long_row, *attention_plan(heads, layout.q_blocks, long_row, kept, layout.k_blocks))

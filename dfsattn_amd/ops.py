@@ -7,6 +7,7 @@ there is deliberately no CPU path here.
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 from dataclasses import dataclass
 from typing import Dict, Optional, Sequence, Tuple
@@ -14,7 +15,7 @@ from typing import Dict, Optional, Sequence, Tuple
 import torch
 
 from . import _lib
-from .layout import ScoringLayout, TopkPolicy, attention_plan
+from .layout import ScoringLayout, TopkPolicy, query_plan
 
 DTYPE_CODE = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
 
@@ -335,12 +336,7 @@ def bsa_fwd(prep: Prepared, row_ptr: torch.Tensor, col_idx: torch.Tensor, scale:
         raise ValueError("out must be a contiguous [1, H, L, D] tensor of out_dtype")
     lse = torch.empty((prep.heads, L), dtype=torch.float32, device=out.device) if want_lse else None
     scale = 1.0 / math.sqrt(prep.head_dim) if scale is None else float(scale)
-    lay = prep.layout
-    # Text query blocks keep every key block and are several times longer.
-    long_row = lay.video_len // lay.block if lay.text_len > 0 else lay.q_blocks
-    kept_long = lay.k_blocks
-    kept = max(0, col_idx.numel() // prep.heads - (lay.q_blocks - long_row) * kept_long) // max(long_row, 1)
-    long_parts, full_rows, parts = attention_plan(prep.heads, lay.q_blocks, long_row, kept, kept_long)
+    long_row, long_parts, full_rows, parts = query_plan(prep.layout, prep.heads, col_idx.numel())
     ws_bytes = 0
     if long_parts > 1 or parts > 1:
         ws_bytes = int(_lib.lib().dfs_bsa_fwd_workspace_size(prep.heads, L, prep.head_dim, long_row, long_parts,
@@ -353,6 +349,84 @@ def bsa_fwd(prep: Prepared, row_ptr: torch.Tensor, col_idx: torch.Tensor, scale:
               _ptr(prep.q_rows), DTYPE_CODE[prep.dtype], L * prep.head_dim, prep.head_dim, long_row, long_parts,
               full_rows, parts, _ptr(ws), ws_bytes, _stream(prep.k_perm))
     return (out, lse) if want_lse else out
+
+
+@functools.lru_cache(maxsize=1024)
+def _call_template(layout: ScoringLayout, policy: TopkPolicy, heads: int, dim: int, dtype: torch.dtype,
+                   operand_dtype: torch.dtype, select: bool) -> Tuple[bytes, int, int]:
+    """(dfs_call_args bytes without pointers, workspace bytes, kept blocks)
+    of a call: host arithmetic on its sizes only."""
+    nnz = policy.nnz(heads)
+    a = _lib.CallArgs()
+    a.heads, a.seq_len, a.head_dim, a.video_len = heads, layout.seq_len, dim, layout.video_len
+    a.q_tile, a.k_tile = layout.q_tile, layout.k_tile
+    a.dtype, a.operand_dtype, a.out_dtype = DTYPE_CODE[dtype], DTYPE_CODE[operand_dtype], DTYPE_CODE[dtype]
+    a.select = int(select)
+    (a.q_blocks, a.k_blocks, a.scored_rows, a.n_cand, a.k_pick, a.dense_col, a.dense_row) = _policy_args(policy)
+    a.long_row, a.long_parts, a.full_rows, a.parts = query_plan(layout, heads, nnz)
+    a.n_seq, a.scale = 1, 1.0 / math.sqrt(dim)
+    size = int(_lib.lib().dfs_call_workspace_size(ctypes.byref(a)))
+    if size < 0:
+        raise _lib.DfsKernelError(_lib.lib().dfs_last_error().decode(errors="replace"))
+    a.workspace_bytes = size
+    return bytes(a), size, nnz
+
+
+PREPARE, SELECT, ATTEND = 1, 2, 4  # DFS_CALL_* phases
+
+
+class Call:
+    """One DFS call of [1, H, L, D] inputs on the current stream: the operand
+    preparation, the mask selection (``col_idx`` None: a new mask, kept in
+    ``self.col_idx``) and the attention, enqueued by ``run`` with every
+    intermediate in one workspace. The same kernels as prepare_qkv,
+    block_score_topk and bsa_fwd, the output in the inputs' dtype."""
+
+    __slots__ = ("args", "out", "col_idx", "refs", "stream")
+
+    def __init__(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, perm: torch.Tensor, layout: ScoringLayout,
+                 policy: TopkPolicy, row_ptr: torch.Tensor, col_idx: Optional[torch.Tensor],
+                 operand_dtype: Optional[torch.dtype] = None, out_perm: Optional[torch.Tensor] = None,
+                 cu_seqlens_q: Optional[torch.Tensor] = None, cu_seqlens_k: Optional[torch.Tensor] = None):
+        dev, dtype = q.device, q.dtype
+        heads, length, dim = _heads_rows(q)
+        if dtype not in (torch.bfloat16, torch.float16):
+            raise RuntimeError("DFS native attention only supports fp16 and bf16 inputs")
+        if k.shape != q.shape or v.shape != q.shape or k.dtype != dtype or v.dtype != dtype:
+            raise ValueError("q, k and v must share shape and dtype")
+        _require_device(q, k, v, perm, row_ptr, col_idx, cu_seqlens_q, cu_seqlens_k)
+        _require_int32(perm=perm, row_ptr=row_ptr, col_idx=col_idx, out_perm=out_perm)
+        if length != layout.seq_len or perm.numel() != length:
+            raise ValueError(f"layout of {layout.seq_len} tokens and permutation of {perm.numel()} for {length} tokens")
+        operand_dtype = operand_dtype or torch.float16
+        if operand_dtype not in (torch.bfloat16, torch.float16):
+            raise ValueError(f"operand_dtype must be bf16 or f16, got {operand_dtype}")
+        if row_ptr.numel() != heads * layout.q_blocks + 1:
+            raise ValueError(f"row_ptr has {row_ptr.numel()} entries for {heads} x {layout.q_blocks} rows")
+        if (cu_seqlens_q is None) != (cu_seqlens_k is None):
+            raise ValueError("pass both cu_seqlens_q and cu_seqlens_k or neither")
+        template, size, nnz = _call_template(layout, policy, heads, dim, dtype, operand_dtype, col_idx is None)
+        a = _lib.CallArgs.from_buffer_copy(template)
+        if cu_seqlens_q is not None:
+            a.n_seq = _check_cu(cu_seqlens_q, "cu_seqlens_q", dev)
+            if _check_cu(cu_seqlens_k, "cu_seqlens_k", dev) != a.n_seq:
+                raise ValueError("cu_seqlens_q and cu_seqlens_k describe different sequence counts")
+            a.cu_seqlens_q, a.cu_seqlens_k = cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr()
+        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+        if col_idx is None:
+            col_idx = torch.empty(nnz, dtype=torch.int32, device=dev)
+        ws = torch.empty(size, dtype=torch.uint8, device=dev)
+        out = torch.empty((1, heads, length, dim), dtype=dtype, device=dev)
+        a.out_head_stride, a.out_row_stride = length * dim, dim
+        a.q, a.k, a.v, a.perm, a.row_ptr = q.data_ptr(), k.data_ptr(), v.data_ptr(), perm.data_ptr(), row_ptr.data_ptr()
+        a.col_idx, a.out, a.workspace = col_idx.data_ptr(), out.data_ptr(), ws.data_ptr()
+        if out_perm is not None:
+            a.out_perm = out_perm.data_ptr()
+        self.args, self.out, self.col_idx, self.stream = a, out, col_idx, _stream(q)
+        self.refs = (q, k, v, perm, row_ptr, cu_seqlens_q, cu_seqlens_k, ws)
+
+    def run(self, phases: int = PREPARE | SELECT | ATTEND) -> None:
+        _lib.call("dfs_call", ctypes.byref(self.args), phases, self.stream)
 
 
 _CU_CACHE: Dict[Tuple[Tuple[int, ...], str], torch.Tensor] = {}

@@ -324,6 +324,38 @@ int dfs_bsa_fwd_parts(const void* q_perm, const void* k_perm, const void* v_t,
                       int64_t parts, void* workspace, int64_t workspace_bytes,
                       dfs_stream_t stream);
 
+/*
+ * One whole call: dfs_prepare_qkv (without a permuted Q) with its fixup,
+ * dfs_block_score_topk and dfs_bsa_fwd_parts on `stream`, in that order, every
+ * intermediate in one caller workspace of dfs_call_workspace_size bytes
+ * (16-byte aligned). Fields are the arguments of those entry points under the
+ * same names; q, k, v are [H][L][D], row_ptr / col_idx the CSR mask, written by
+ * the call when `select` is set (the policy fields apply then) and read
+ * otherwise. `phases` is a sum of DFS_CALL_*; phases of one call may be
+ * enqueued one after the other with the same arguments and workspace.
+ * Replaces the body of the reference's forward (attention_wan.py:394-547).
+ */
+enum { DFS_CALL_PREPARE = 1, DFS_CALL_SELECT = 2, DFS_CALL_ATTEND = 4 };
+typedef struct dfs_call_args {
+  int64_t heads, seq_len, head_dim, video_len, q_tile, k_tile;
+  int64_t dtype, operand_dtype, out_dtype;
+  int64_t select;
+  int64_t q_blocks, k_blocks, scored_rows, n_cand, k_pick, dense_col, dense_row;
+  int64_t long_row, long_parts, full_rows, parts;
+  int64_t out_head_stride, out_row_stride;
+  int64_t n_seq, workspace_bytes;
+  double scale;
+  const void *q, *k, *v;
+  const int32_t *perm, *row_ptr;
+  int32_t* col_idx;
+  void* out;
+  const int32_t *out_perm, *cu_seqlens_q, *cu_seqlens_k;
+  void* workspace;
+} dfs_call_args;
+int64_t dfs_call_workspace_size(const dfs_call_args* args);
+int dfs_call(const dfs_call_args* args, int phases, dfs_stream_t stream);
+
+
 /* uint8/bool block mask [H][Qb][Kb] -> per-row counts int32 [H*Qb].
  * Part of the bool-mask interface of block_sparse_attn_func
  * (base_blockmask, attention_wan.py:359). */

@@ -618,7 +618,7 @@ def test_bsa_fwd_parts_match_unsplit(dev, monkeypatch, d, heads, video, text, cu
     cu = None if cut is None else torch.tensor([0, cut, L], dtype=torch.int32, device=dev)
     got = {}
     for name, pl in (("whole", (1, 0, 1)), ("parts", plan)):
-        monkeypatch.setattr(ops, "attention_plan", lambda *a: pl)
+        monkeypatch.setattr(ops, "query_plan", lambda lay, *a: (lay.video_len // 128 if lay.text_len else lay.q_blocks, *pl))
         got[name] = ops.bsa_fwd(prep, row_ptr, col_idx, out_dtype=out_dtype, out_perm=perm.to(dev), want_lse=True,
                                 cu_seqlens_q=cu, cu_seqlens_k=cu)
     (o0, l0), (o1, l1) = ((o.float().cpu(), l.cpu()) for o, l in (got["whole"], got["parts"]))
@@ -633,6 +633,47 @@ def test_bsa_fwd_parts_match_unsplit(dev, monkeypatch, d, heads, video, text, cu
     ulp = {torch.float32: 0.0, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[out_dtype]
     assert rel <= 2.0 ** -11 + ulp, rel  # P's rounding, averaged over the keys, and the output's
     assert float((o0 - o1).abs().max()) <= 1e-2
+
+
+@pytest.mark.parametrize("d,heads,video,text,tile,dtype,operand,big", [
+    (128, 2, 1000, 0, 16, torch.bfloat16, None, ("k", 999)),   # one launch for q, k and v; flag in the last wave
+    (64, 3, 1153, 0, 32, torch.bfloat16, None, ("v", 1152)),   # two V blocks per workgroup, an odd block count
+    (128, 1, 900, 124, 16, torch.bfloat16, None, ("q", 0)),    # text; only Q beyond f16
+    (128, 40, 3000, 0, 16, torch.bfloat16, None, ("v", 0)),    # above the one-launch limit
+    (64, 2, 500, 0, 16, torch.float16, None, None),            # nothing to flag
+    (128, 2, 700, 0, 16, torch.bfloat16, torch.bfloat16, ("v", 5)),  # bf16 operands: no flags
+    (128, 2, 700, 0, 64, torch.bfloat16, None, None),          # tiles of the generic scorer (score matrix)
+])
+def test_whole_call_matches_single_entry_points(dev, d, heads, video, text, tile, dtype, operand, big):
+    """dfs_call (all phases at once, then one by one, and with a given mask)
+    against prepare_qkv, block_score_topk and bsa_fwd: the same kernels on the
+    same values, so the same columns and bits."""
+    print(f"call d={d} heads={heads} video={video} text={text} tile={tile} {dtype} {operand} {big}", flush=True)
+    L = video + text
+    g = torch.Generator().manual_seed(L)
+    x = {n: torch.randn((1, heads, L, d), generator=g).to(dtype) for n in "qkv"}
+    if big:
+        x[big[0]][0, heads - 1, big[1], d - 1] = 1.0e6
+    q, k, v = (x[n].to(dev) for n in "qkv")
+    layout = ScoringLayout(L, video, tile)
+    pol = hunyuan_policy(layout, 0.5) if text else wan_policy(layout, 0.3)
+    row_ptr = torch.from_numpy(pol.row_ptr(heads)).to(dev)
+    perm = torch.randperm(video, generator=g)
+    perm = torch.cat([perm, torch.arange(video, L)]).to(torch.int32).to(dev)
+    prep = ops.prepare_qkv(q, k, v, perm, layout, operand_dtype=operand, q_operand=False)
+    cols, _, _ = ops.block_score_topk(prep, pol, row_ptr)
+    ref = ops.bsa_fwd(prep, row_ptr, cols, out_perm=perm)
+    kw = dict(operand_dtype=operand, out_perm=perm)
+    call = ops.Call(q, k, v, perm, layout, pol, row_ptr, None, **kw)
+    call.run()
+    steps = ops.Call(q, k, v, perm, layout, pol, row_ptr, None, **kw)
+    for phase in (ops.PREPARE, ops.SELECT, ops.ATTEND):
+        steps.run(phase)
+    given = ops.Call(q, k, v, perm, layout, pol, row_ptr, cols, **kw)
+    given.run()
+    assert torch.equal(call.col_idx, cols) and torch.equal(steps.col_idx, cols)
+    for c in (call, steps, given):
+        assert torch.equal(c.out, ref)
 
 
 def test_wrappers_reject_bad_index_operands(dev):

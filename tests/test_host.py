@@ -303,3 +303,32 @@ def test_attention_plan_covers_every_block_once(heads, length, text, kept):
             blk, base, n = ordinary(t & 7, full_k + (t >> 3)), split_long * lp + t * parts, parts
         if blk is not None:
             assert [used[base + i] for i in range(n)] == [(blk, i) for i in range(n)]
+
+
+def test_call_checks_its_arguments_without_launching():
+    """dfs_call refuses sizes, phases and workspaces it cannot run before it
+    touches a device."""
+    from dfsattn_amd.ops import _call_template
+    layout = ScoringLayout(1000, 1000, 16)
+    template, size, nnz = _call_template(layout, wan_policy(layout, 0.3), 2, 128, torch.bfloat16, torch.float16, True)
+    assert nnz == wan_policy(layout, 0.3).nnz(2) and size > 2 * 2 * 1024 * 128 * 2
+    ref = lambda a: ctypes.byref(a)  # noqa: E731
+
+    def args(**kw):
+        a = _lib.CallArgs.from_buffer_copy(template)
+        a.q = a.k = a.v = a.perm = a.row_ptr = a.col_idx = a.out = a.workspace = 256
+        for name, value in kw.items():
+            setattr(a, name, value)
+        return a
+
+    for bad, text in ((dict(workspace_bytes=size - 1), "workspace"), (dict(workspace=None), "workspace"),
+                      (dict(workspace=264), "workspace"), (dict(head_dim=96), "head_dim=96"),
+                      (dict(q_tile=24), "q_tile=24"), (dict(video_len=1001), "video_len=1001"),
+                      (dict(k_blocks=9), "policy"), (dict(parts=0), "parts=0"), (dict(long_row=9), "long_row=9")):
+        with pytest.raises(_lib.DfsKernelError, match=text):
+            _lib.call("dfs_call", ref(args(**bad)), 7, None)
+    with pytest.raises(_lib.DfsKernelError, match="phases=8"):
+        _lib.call("dfs_call", ref(args()), 8, None)
+    with pytest.raises(_lib.DfsKernelError, match="NULL"):
+        _lib.call("dfs_call", None, 7, None)
+    assert _lib.lib().dfs_call_workspace_size(ref(args(head_dim=96))) == -1
