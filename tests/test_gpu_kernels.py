@@ -638,7 +638,7 @@ def test_bsa_fwd_parts_match_unsplit(dev, monkeypatch, d, heads, video, text, cu
 @pytest.mark.parametrize("d,heads,video,text,tile,dtype,operand,big", [
     (128, 2, 1000, 0, 16, torch.bfloat16, None, ("k", 999)),   # one launch for q, k and v; flag in the last wave
     (64, 3, 1153, 0, 32, torch.bfloat16, None, ("v", 1152)),   # two V blocks per workgroup, an odd block count
-    (128, 1, 900, 124, 16, torch.bfloat16, None, ("q", 0)),    # text; only Q beyond f16
+    (128, 1, 900, 125, 16, torch.bfloat16, None, ("q", 0)),    # text; only Q beyond f16
     (128, 40, 3000, 0, 16, torch.bfloat16, None, ("v", 0)),    # above the one-launch limit
     (64, 2, 500, 0, 16, torch.float16, None, None),            # nothing to flag
     (128, 2, 700, 0, 16, torch.bfloat16, torch.bfloat16, ("v", 5)),  # bf16 operands: no flags
