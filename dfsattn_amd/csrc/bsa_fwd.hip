@@ -746,7 +746,7 @@ struct BsaArgs {
 
 struct SegParams {
   int H, L, R, csr_qb, Lo;
-  int qk_f16, pv_f16, out_kind;
+  int out_kind;
   float scale_log2;
   const int32_t* cu_q;  // [n_seq + 1] (device)
   const int32_t* cu_k;
@@ -762,22 +762,48 @@ __device__ __forceinline__ float operand_at(const uint16_t* base, int64_t i, boo
   return f16 ? f16_bits_to_f32(base[i]) : bf16_bits_to_f32(base[i]);
 }
 
-// The rows of a call after segment 0 of cu_seqlens, in fp32. A wave takes
-// RG = 4 consecutive rows of one query block (they share the block's mask
-// row) and walks their kept key blocks 64 keys at a time: one key per lane
-// for the scores of the four rows (each K row read once), an exact running
-// maximum per row and window, then P V with each lane owning D / 64 head
-// dims of the four rows and reading the window's 64 V^T slots of its dims
-// once. For n_seq == 2 the rows [cq1, cq2) attend keys [ck1, ck2) under the
-// same block mask indexed from each segment's own start (query block
-// (r - cq1) / 128 selects the CSR row, key block j covers keys ck1 + 128 j
-// ..), as the reference's varlen kernel treats the second sequence of its
-// batch (attention_hyvideo.py:1054-1082, the mask repeated per sequence at
-// :359). Rows outside every query segment are zero (lse -inf). Windows are
-// aligned to 64 keys so that a window's V^T slots are one contiguous run of
-// a physical 128-key block; keys of a window outside the column's range are
-// masked. Sized for short padding segments (a few hundred tokens).
-template <int D>
+// Maximum and sum over the wave through register moves, the same bits in
+// every lane (each step joins a lane with its mirror).
+template <int CTRL>
+__device__ __forceinline__ float dpp_mov(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float wave_max(float v) {
+  v = fmaxf(v, dpp_mov<0xB1>(v));   // quad_perm [1, 0, 3, 2]
+  v = fmaxf(v, dpp_mov<0x4E>(v));   // quad_perm [2, 3, 0, 1]
+  v = fmaxf(v, dpp_mov<0x141>(v));  // row_half_mirror
+  v = fmaxf(v, dpp_mov<0x140>(v));  // row_mirror
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return xhalf_max(fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1])));
+}
+__device__ __forceinline__ float wave_sum(float v) {
+  v += dpp_mov<0xB1>(v);
+  v += dpp_mov<0x4E>(v);
+  v += dpp_mov<0x141>(v);
+  v += dpp_mov<0x140>(v);
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return xhalf_sum(__uint_as_float(a[0]) + __uint_as_float(a[1]));
+}
+
+// The rows of a call after segment 0 of cu_seqlens, in fp32. A workgroup takes
+// four consecutive rows of one query block, a wave each, and walks their kept
+// key blocks 64 keys at a time: the window's K rows and V^T slots go through
+// LDS (chunk-swizzled, read by the four waves), one key per lane for the
+// scores, an exact running maximum, then P V with each lane owning head dims
+// lane and lane + 64. For n_seq == 2 the rows [cq1, cq2) attend keys
+// [ck1, ck2) under the same block mask indexed from each segment's own start
+// (query block (r - cq1) / 128 selects the CSR row, key block j covers keys
+// ck1 + 128 j ..), as the reference's varlen kernel treats the second sequence
+// of its batch (attention_hyvideo.py:1054-1082, the mask repeated per sequence
+// at :359). Rows outside every query segment are zero (lse -inf). Windows are
+// aligned to 64 keys so that a window's V^T slots are one contiguous run of a
+// physical 128-key block; keys of a window outside the column's range are
+// masked. Sized for short padding segments (a few hundred tokens), where a
+// row's chain counts: 15 us for 32 padding rows of 24 heads and 33 for 138.
+// Read from global memory, one key or head dim per lane, each load touched 64
+// cache lines: 78 us for the 138 with a row per wave, 100 with four (61 for
+// the 32).
+template <int D, bool QK_F16, bool PV_F16>
 __global__ void __launch_bounds__(256) bsa_segment_kernel(const uint16_t* __restrict__ q,
                                                           const uint16_t* __restrict__ k,
                                                           const uint16_t* __restrict__ vt,
@@ -785,20 +811,20 @@ __global__ void __launch_bounds__(256) bsa_segment_kernel(const uint16_t* __rest
                                                           const int32_t* __restrict__ col_idx,
                                                           void* __restrict__ out, const int32_t* __restrict__ out_perm,
                                                           float* __restrict__ lse, SegParams p) {
-  constexpr int RG = 4;        // rows per wave
-  constexpr int DPL = D / 64;  // head dims per lane in P V
-  constexpr int CPR = D / 8;   // 16-byte chunks of a K row
-  __shared__ float qs[4][RG][D];   // the rows' q (times the scale), per wave
-  __shared__ float ps[4][RG][64];  // the window's P in V^T slot order, per wave
+  constexpr int DPL = D / 64;           // head dims per lane in P V
+  constexpr int CPR = D / 8;            // 16-byte chunks of a K row
+  constexpr int LOADS = 64 * CPR / 256;  // chunks of a K (or V^T) window per thread
+  __shared__ u32x4_t kw[64 * CPR];  // chunk c of key r at r * CPR + (c ^ (r % CPR))
+  __shared__ u32x4_t vw[D * 8];     // chunk c of head dim d at d * 8 + (c ^ (d / 2 % 8))
+  __shared__ __attribute__((aligned(16))) float qs[4][D];   // the row's q (times the scale), per wave
+  __shared__ __attribute__((aligned(16))) float ps[4][64];  // the window's P in V^T slot order, per wave
   const int h = blockIdx.y;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int wave = blockIdx.x * 4 + w, n_waves = gridDim.x * 4;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int cq1 = min(max(p.cu_q[1], 0), p.L);
   const int cq2 = p.n_seq == 2 ? min(max(p.cu_q[2], cq1), p.L) : cq1;
   const int ck1 = p.n_seq == 2 ? min(max(p.cu_k[1], 0), p.L) : 0;
   const int ck2 = p.n_seq == 2 ? min(max(p.cu_k[2], ck1), p.L) : 0;
   const int seg_kb = (ck2 - ck1 + 127) >> 7;
-  const bool qk16 = p.qk_f16 != 0, pv16 = p.pv_f16 != 0;
   float sq = p.scale_log2, sv = 1.f;
   if (p.exps) {
     sq = ldexpf(sq, (p.q_src ? 0 : p.exps[h]) + p.exps[p.H + h]);  // a Q source is read unscaled
@@ -808,31 +834,25 @@ __global__ void __launch_bounds__(256) bsa_segment_kernel(const uint16_t* __rest
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_wave_barrier();
   };
-  auto half_to_f32 = [](uint32_t bits, bool f16) { return f16 ? f16_bits_to_f32(bits) : bf16_bits_to_f32(bits); };
   const int64_t hq = static_cast<int64_t>(h) * p.R * D;
-  const uint4* krows = reinterpret_cast<const uint4*>(k + hq);
+  const u32x4_t* krows = reinterpret_cast<const u32x4_t*>(k + hq);
+  const u32x4_t* vblocks = reinterpret_cast<const u32x4_t*>(vt + hq);
   // Element j of execution row r's query (r < L).
   auto q_at = [&](int r, int j) -> float {
     if (p.q_src)
       return operand_at(p.q_src, (static_cast<int64_t>(h) * p.L + p.q_rows[r]) * D + j, p.q_src_f16 != 0);
-    return operand_at(q, hq + static_cast<int64_t>(r) * D + j, qk16);
+    return operand_at(q, hq + static_cast<int64_t>(r) * D + j, QK_F16);
   };
 
-  for (int r0 = cq1 + RG * wave; r0 < p.L; r0 += RG * n_waves) {
-    float o[RG][DPL], m[RG], l[RG];
+  // Groups of four rows from cq1 on: 4 divides 128, so a group's rows share
+  // query block (r0 - cq1) / 128, its columns and its windows.
+  for (int r0 = cq1 + 4 * static_cast<int>(blockIdx.x); r0 < p.L; r0 += 4 * static_cast<int>(gridDim.x)) {
+    const int r = r0 + w;
+    const bool live = r < cq2;  // a row of the second sequence
+    float o[DPL] = {}, m = -INFINITY, l = 0.f;
+    if (r0 < cq2 && seg_kb > 0) {
 #pragma unroll
-    for (int i = 0; i < RG; ++i) {
-      m[i] = -INFINITY;
-      l[i] = 0.f;
-#pragma unroll
-      for (int j = 0; j < DPL; ++j) o[i][j] = 0.f;
-    }
-    if (r0 < cq2 && seg_kb > 0) {  // RG divides 128: the group's rows share query block (r0 - cq1) / 128
-#pragma unroll
-      for (int i = 0; i < RG; ++i)
-        for (int j = lane; j < D; j += 64)
-          qs[w][i][j] = r0 + i < cq2 ? q_at(r0 + i, j) * sq : 0.f;
-      wave_sync();
+      for (int j = 0; j < DPL; ++j) qs[w][j * 64 + lane] = live ? q_at(r, j * 64 + lane) * sq : 0.f;
       const int64_t crow = static_cast<int64_t>(h) * p.csr_qb + ((r0 - cq1) >> 7);
       const int beg = row_ptr[crow], end = row_ptr[crow + 1];
       for (int idx = beg; idx < end; ++idx) {  // columns ascend: stop at the segment's last block
@@ -840,102 +860,84 @@ __global__ void __launch_bounds__(256) bsa_segment_kernel(const uint16_t* __rest
         if (cb >= seg_kb) break;
         if (cb < 0) continue;
         const int k0 = ck1 + cb * 128, k1 = min(k0 + 128, ck2);
-        for (int w0 = k0 & ~63; w0 < k1; w0 += 64) {
+        for (int w0 = k0 & ~63; w0 < k1; w0 += 64) {  // w0 + 64 <= R: whole windows lie in the operands
+          u32x4_t kr[LOADS], vr[LOADS];  // plain vectors: uint4 copies across the barrier went through scratch
+#pragma unroll
+          for (int i = 0; i < LOADS; ++i) {
+            const int e = i * 256 + tid;
+            kr[i] = krows[static_cast<int64_t>(w0) * CPR + e];
+            // V^T block w0 / 128: 16 chunks per head dim, this window's 8
+            vr[i] = vblocks[(static_cast<int64_t>(w0 >> 7) * D + (e >> 3)) * 16 + ((w0 >> 3) & 8) + (e & 7)];
+          }
+          __syncthreads();  // the previous window has been read
+#pragma unroll
+          for (int i = 0; i < LOADS; ++i) {
+            const int e = i * 256 + tid, kr_row = e / CPR, d = e >> 3;
+            kw[kr_row * CPR + ((e % CPR) ^ (kr_row % CPR))] = kr[i];
+            vw[d * 8 + ((e & 7) ^ ((d >> 1) & 7))] = vr[i];
+          }
+          __syncthreads();
           const int key = w0 + lane;
           const bool valid = key >= k0 && key < k1;
-          // the window's V^T slots of this lane's dims, loaded with the K row
-          const int64_t vb = (static_cast<int64_t>(h) * (p.R / 128) + (w0 >> 7)) * D * 128 + (w0 & 127);
-          uint4 vv[DPL][8];
-#pragma unroll
-          for (int j = 0; j < DPL; ++j)
-#pragma unroll
-            for (int c = 0; c < 8; ++c)
-              vv[j][c] = reinterpret_cast<const uint4*>(vt + vb + static_cast<int64_t>(lane * DPL + j) * 128)[c];
-          float s[RG];
-#pragma unroll
-          for (int i = 0; i < RG; ++i) s[i] = 0.f;
-          if (valid) {
-            const uint4* kr = krows + static_cast<int64_t>(key) * CPR;
+          float s4[4] = {};  // four chains of the dot product
 #pragma unroll 2
-            for (int c = 0; c < CPR; ++c) {
-              asm volatile("" ::: "memory");  // q stays in LDS (read per chunk), not hoisted into registers
-              const uint4 kv = kr[c];
+          for (int c = 0; c < CPR; ++c) {
+            const uint4 kv = __builtin_bit_cast(uint4, kw[lane * CPR + (c ^ (lane % CPR))]);
+            const float4 qa = *reinterpret_cast<const float4*>(&qs[w][c * 8]);
+            const float4 qb = *reinterpret_cast<const float4*>(&qs[w][c * 8 + 4]);
+            const float qe[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
 #pragma unroll
-              for (int e = 0; e < 8; ++e) {
-                const float kf = half_to_f32(u16_at(kv, e), qk16);
-#pragma unroll
-                for (int i = 0; i < RG; ++i) s[i] += qs[w][i][c * 8 + e] * kf;
-              }
-            }
+            for (int e = 0; e < 8; ++e)
+              s4[e & 3] += qe[e] * (QK_F16 ? f16_bits_to_f32(u16_at(kv, e)) : bf16_bits_to_f32(u16_at(kv, e)));
           }
+          const float si = valid ? (s4[0] + s4[1]) + (s4[2] + s4[3]) : -INFINITY;
+          const float mnew = fmaxf(m, wave_max(si));  // finite: the window holds key max(w0, k0) < k1
+          const float alpha = exp2_fast(m - mnew);
+          const float pk = valid ? exp2_fast(si - mnew) : 0.f;
+          l = l * alpha + wave_sum(pk);
+#pragma unroll
+          for (int j = 0; j < DPL; ++j) o[j] *= alpha;
+          m = mnew;
           // slot of window key `lane` in its 16-key group: swap23 (an involution)
-          const int slot = (lane & ~15) | (lane & 3) | ((lane & 4) << 1) | ((lane & 8) >> 1);
-#pragma unroll
-          for (int i = 0; i < RG; ++i) {
-            const float si = valid ? s[i] : -INFINITY;
-            float mx = si;
-#pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-            const float mnew = fmaxf(m[i], mx);  // finite: the window holds key max(w0, k0) < k1
-            const float alpha = exp2_fast(m[i] - mnew);
-            const float pk = valid ? exp2_fast(si - mnew) : 0.f;
-            float psum = pk;
-#pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) psum += __shfl_xor(psum, off, 64);
-            l[i] = l[i] * alpha + psum;
-#pragma unroll
-            for (int j = 0; j < DPL; ++j) o[i][j] *= alpha;
-            m[i] = mnew;
-            ps[w][i][slot] = pk;
-          }
+          ps[w][(lane & ~15) | (lane & 3) | ((lane & 4) << 1) | ((lane & 8) >> 1)] = pk;
           wave_sync();
-#pragma unroll 1
+#pragma unroll 2
           for (int c = 0; c < 8; ++c) {
-            asm volatile("" ::: "memory");  // P of 8 slots read per step, not all at once
-            float pc[RG][8];
-#pragma unroll
-            for (int i = 0; i < RG; ++i)
-#pragma unroll
-              for (int e = 0; e < 8; ++e) pc[i][e] = ps[w][i][c * 8 + e];
+            const float4 pa = *reinterpret_cast<const float4*>(&ps[w][c * 8]);
+            const float4 pb = *reinterpret_cast<const float4*>(&ps[w][c * 8 + 4]);
+            const float pe[8] = {pa.x, pa.y, pa.z, pa.w, pb.x, pb.y, pb.z, pb.w};
 #pragma unroll
             for (int j = 0; j < DPL; ++j) {
-              const uint4 vc = c == 0 ? vv[j][0] : c == 1 ? vv[j][1] : c == 2 ? vv[j][2] : c == 3 ? vv[j][3]
-                             : c == 4 ? vv[j][4] : c == 5 ? vv[j][5] : c == 6 ? vv[j][6] : vv[j][7];
+              const int d = j * 64 + lane;
+              const uint4 vc = __builtin_bit_cast(uint4, vw[d * 8 + (c ^ ((d >> 1) & 7))]);
 #pragma unroll
-              for (int e = 0; e < 8; ++e) {
-                const float vf = half_to_f32(u16_at(vc, e), pv16);
-#pragma unroll
-                for (int i = 0; i < RG; ++i) o[i][j] += pc[i][e] * vf;
-              }
+              for (int e = 0; e < 8; ++e)
+                o[j] += pe[e] * (PV_F16 ? f16_bits_to_f32(u16_at(vc, e)) : bf16_bits_to_f32(u16_at(vc, e)));
             }
           }
           wave_sync();  // ps is read before the next window overwrites it
         }
       }
+      wave_sync();  // qs is read before the next row overwrites it
     }
+    if (r >= p.L) continue;
+    if (!live) l = 0.f;  // scored with q = 0: the row belongs to no sequence (zero, lse -inf)
+    const float inv = l > 0.f ? sv / l : 0.f;
+    const int orow = out_perm ? out_perm[r] : r;
+    const int64_t ob = h * p.o_sh + orow * p.o_sl;
 #pragma unroll
-    for (int i = 0; i < RG; ++i) {
-      const int r = r0 + i;
-      if (r >= p.L) break;
-      // A group may straddle the second sequence's end: its rows past cq2
-      // were scored with q = 0 and belong to no sequence (zero, lse -inf).
-      if (r >= cq2) l[i] = 0.f;
-      const float inv = l[i] > 0.f ? sv / l[i] : 0.f;
-      const int orow = out_perm ? out_perm[r] : r;
-      const int64_t ob = h * p.o_sh + orow * p.o_sl + lane * DPL;
-#pragma unroll
-      for (int j = 0; j < DPL; ++j) {
-        const float v = o[i][j] * inv;
-        if (p.out_kind == DFS_DTYPE_F32)
-          static_cast<float*>(out)[ob + j] = v;
-        else if (p.out_kind == DFS_DTYPE_BF16)
-          static_cast<uint16_t*>(out)[ob + j] = static_cast<uint16_t>(f32_to_bf16_bits(v));
-        else
-          static_cast<uint16_t*>(out)[ob + j] = static_cast<uint16_t>(f32_to_f16_bits(v));
-      }
-      if (lse && lane == 0)
-        lse[static_cast<int64_t>(h) * p.Lo + r] = l[i] > 0.f ? (m[i] + log2f(l[i])) * 0.69314718055994531f : -INFINITY;
+    for (int j = 0; j < DPL; ++j) {
+      const float v = o[j] * inv;
+      const int64_t at = ob + j * 64 + lane;
+      if (p.out_kind == DFS_DTYPE_F32)
+        static_cast<float*>(out)[at] = v;
+      else if (p.out_kind == DFS_DTYPE_BF16)
+        static_cast<uint16_t*>(out)[at] = static_cast<uint16_t>(f32_to_bf16_bits(v));
+      else
+        static_cast<uint16_t*>(out)[at] = static_cast<uint16_t>(f32_to_f16_bits(v));
     }
+    if (lse && lane == 0)
+      lse[static_cast<int64_t>(h) * p.Lo + r] = l > 0.f ? (m + log2f(l)) * 0.69314718055994531f : -INFINITY;
   }
 }
 
@@ -1083,8 +1085,6 @@ int bsa_fwd_impl(const char* name, const void* q_perm, const void* k_perm, const
     sp.R = p.R;
     sp.csr_qb = p.csr_qb;
     sp.Lo = p.Lo;
-    sp.qk_f16 = qk_f16;
-    sp.pv_f16 = pv_f16;
     sp.out_kind = out_dtype;
     sp.scale_log2 = p.scale_log2;
     sp.cu_q = cu_seqlens_q;
@@ -1096,13 +1096,18 @@ int bsa_fwd_impl(const char* name, const void* q_perm, const void* k_perm, const
     sp.q_src_f16 = p.q_src_f16;
     sp.o_sh = p.o_sh;
     sp.o_sl = p.o_sl;
-    // Enough waves for a few hundred rows per head; each wave strides over
-    // the rows after segment 0.
-    const dim3 grid(16, static_cast<unsigned>(heads));
+    // Four rows per workgroup for a few hundred rows per head; a workgroup
+    // strides over the rows after segment 0.
+    const dim3 grid(64, static_cast<unsigned>(heads));
+    auto seg = [&](auto kernel) {
+      kernel<<<grid, 256, 0, s>>>(a.q, a.k, a.vt, row_ptr, col_idx, out, out_perm, lse, sp);
+    };
     if (head_dim == 128)
-      bsa_segment_kernel<128><<<grid, 256, 0, s>>>(a.q, a.k, a.vt, row_ptr, col_idx, out, out_perm, lse, sp);
+      qk_f16 ? seg(bsa_segment_kernel<128, true, true>)
+             : pv_f16 ? seg(bsa_segment_kernel<128, false, true>) : seg(bsa_segment_kernel<128, false, false>);
     else
-      bsa_segment_kernel<64><<<grid, 256, 0, s>>>(a.q, a.k, a.vt, row_ptr, col_idx, out, out_perm, lse, sp);
+      qk_f16 ? seg(bsa_segment_kernel<64, true, true>)
+             : pv_f16 ? seg(bsa_segment_kernel<64, false, true>) : seg(bsa_segment_kernel<64, false, false>);
   }
   return check_launch(name);
 }
