@@ -119,6 +119,7 @@ struct PrepParams {
   int in_f16;    // q/k/v are f16 (else bf16)
   int convert;   // bf16 inputs, f16 operands: q_perm, k_perm and v_t get converted values
   int pool;      // write pooled tiles
+  int first;     // 1: K alone (no pooling and no Q operand: nothing of Q is needed)
 };
 
 // bf16 -> f16 of eight packed values; *overflow is set when a finite value
@@ -318,10 +319,10 @@ __device__ __forceinline__ void prep_v_block(const PrepParams& p, int kb, int h,
 }
 
 // Q and K: one wave per (tensor, head, scoring tile), four tiles per
-// workgroup (grid: tiles / 4, heads, 2).
+// workgroup (grid: tiles / 4, heads, 2; K alone with p.first, heads, 1).
 template <int D>
 __global__ void __launch_bounds__(256) prep_qk_kernel(PrepParams p) {
-  prep_qk_tiles<D>(p, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y, blockIdx.z == 1);
+  prep_qk_tiles<D>(p, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y, blockIdx.z + p.first == 1);
 }
 
 // V: one workgroup per (128-token block, head).
@@ -337,9 +338,10 @@ template <int D>
 __global__ void __launch_bounds__(256) prep_qkv_kernel(PrepParams p, int nbx_qk) {
   constexpr int NT = 16 * (D / 8), PER = 256 / NT;  // V blocks per workgroup
   __shared__ uint4 stage[PER * (D / 2 * (kBlock / 8))];
-  if (blockIdx.z < 2) {
+  const int z = blockIdx.z + p.first;
+  if (z < 2) {
     if (static_cast<int>(blockIdx.x) < nbx_qk)
-      prep_qk_tiles<D>(p, blockIdx.x, nbx_qk, blockIdx.y, gridDim.y, blockIdx.z == 1);
+      prep_qk_tiles<D>(p, blockIdx.x, nbx_qk, blockIdx.y, gridDim.y, z == 1);
     return;
   }
   const int sub = threadIdx.x / NT;
@@ -368,7 +370,9 @@ __global__ void __launch_bounds__(1024) prep_fixup_kernel(PrepParams p, int32_t*
   const int h = blockIdx.x, t = blockIdx.y, H = gridDim.x;
   const int slot = t * H + h;
   int flagged;
-  if (p.wave_flags) {
+  if (p.first && t == 0) {
+    flagged = 0;  // Q was not read: the attention kernel marks its head where a row leaves the range
+  } else if (p.wave_flags) {
     const int n = t < 2 ? p.nqk : p.nv;
     const int32_t* words = p.wave_flags + (t < 2 ? slot * static_cast<int64_t>(p.nqk)
                                                  : 2 * H * static_cast<int64_t>(p.nqk) + h * static_cast<int64_t>(p.nv));
@@ -456,7 +460,7 @@ int prepare_qkv_impl(const void* q, const void* k, const void* v, const int32_t*
                     int64_t heads, int64_t seq_len, int64_t head_dim, int dtype,
                     int64_t video_len, int64_t q_tile_size, int64_t k_tile_size, int operand_dtype, void* q_perm,
                     void* k_perm, void* v_t, uint16_t* q_pool_hi, uint16_t* q_pool_lo,
-                    uint16_t* k_pool_hi, uint16_t* k_pool_lo, int32_t* overflow, int32_t* wave_flags,
+                    uint16_t* k_pool_hi, uint16_t* k_pool_lo, int32_t* overflow, int32_t* wave_flags, bool skip_q,
                     dfs_stream_t stream) {
   DFS_REQUIRE(q && k && v && perm && k_perm && v_t, "dfs_prepare_qkv: NULL operand");
   DFS_REQUIRE(head_dim == 64 || head_dim == 128, "dfs_prepare_qkv: head_dim=%lld (supported: 64, 128)",
@@ -514,17 +518,18 @@ int prepare_qkv_impl(const void* q, const void* k, const void* v, const int32_t*
   p.in_f16 = dtype == DFS_DTYPE_F16;
   p.convert = (dtype == DFS_DTYPE_BF16 && operand_dtype == DFS_DTYPE_F16);
   p.pool = pool ? 1 : 0;
+  p.first = skip_q && !pool && q_perm == nullptr ? 1 : 0;
 
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   // Enough four-wave blocks for the smaller of the two tiles (more tiles).
   const int64_t max_tiles = kb * kBlock / (q_tile_size < k_tile_size ? q_tile_size : k_tile_size);
-  dim3 gqk(static_cast<unsigned>((max_tiles + 3) / 4), static_cast<unsigned>(heads), 2);
+  dim3 gqk(static_cast<unsigned>((max_tiles + 3) / 4), static_cast<unsigned>(heads), p.first ? 1 : 2);
   dim3 gv(static_cast<unsigned>(kb), static_cast<unsigned>(heads));
   // One launch below 2,048 workgroups (eight per CU), where it saves a
   // kernel's start-up; larger calls run 0-2% faster as two.
   const int64_t per = head_dim == 128 ? 1 : 2, nbv = (kb + per - 1) / per;
-  if (heads * (2 * static_cast<int64_t>(gqk.x) + nbv) < 2048) {
-    const dim3 g(gqk.x > nbv ? gqk.x : static_cast<unsigned>(nbv), static_cast<unsigned>(heads), 3);
+  if (heads * (static_cast<int64_t>(gqk.z) * gqk.x + nbv) < 2048) {
+    const dim3 g(gqk.x > nbv ? gqk.x : static_cast<unsigned>(nbv), static_cast<unsigned>(heads), gqk.z + 1);
     if (head_dim == 128)
       prep_qkv_kernel<128><<<g, 256, 0, s>>>(p, static_cast<int>(gqk.x));
     else
@@ -550,7 +555,7 @@ int64_t prepare_flag_words(int64_t heads, int64_t seq_len, int64_t head_dim, int
 int prepare_fixup_impl(const void* q, const void* k, const void* v, const int32_t* perm, int64_t heads,
                       int64_t seq_len, int64_t head_dim, void* q_perm, void* k_perm, void* v_t,
                       int32_t* overflow, int32_t* wave_flags, int64_t q_tile_size, int64_t k_tile_size,
-                      int32_t* exps, dfs_stream_t stream) {
+                      bool skip_q, int32_t* exps, dfs_stream_t stream) {
   DFS_REQUIRE(q && k && v && perm && k_perm && v_t && (overflow || wave_flags) && exps, "dfs_prepare_fixup: NULL operand");
   DFS_REQUIRE(head_dim == 64 || head_dim == 128, "dfs_prepare_fixup: head_dim=%lld (supported: 64, 128)",
               (long long)head_dim);
@@ -570,6 +575,7 @@ int prepare_fixup_impl(const void* q, const void* k, const void* v, const int32_
   p.L = static_cast<int>(seq_len);
   p.R = static_cast<int>(kb * kBlock);
   p.wave_flags = wave_flags;
+  p.first = skip_q ? 1 : 0;
   if (wave_flags) wave_flag_counts(kb, head_dim, q_tile_size, k_tile_size, &p.nqk, &p.nv);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const dim3 grid(static_cast<unsigned>(heads), 3);
@@ -606,14 +612,14 @@ int dfs_prepare_qkv(const void* q, const void* k, const void* v, const int32_t* 
                     dfs_stream_t stream) {
   return dfs::prepare_qkv_impl(q, k, v, perm, heads, seq_len, head_dim, dtype, video_len, q_tile_size, k_tile_size,
                                operand_dtype, q_perm, k_perm, v_t, q_pool_hi, q_pool_lo, k_pool_hi, k_pool_lo,
-                               overflow, nullptr, stream);
+                               overflow, nullptr, false, stream);
 }
 
 int dfs_prepare_fixup(const void* q, const void* k, const void* v, const int32_t* perm, int64_t heads,
                       int64_t seq_len, int64_t head_dim, void* q_perm, void* k_perm, void* v_t,
                       int32_t* overflow, int32_t* exps, dfs_stream_t stream) {
   return dfs::prepare_fixup_impl(q, k, v, perm, heads, seq_len, head_dim, q_perm, k_perm, v_t, overflow, nullptr, 0, 0,
-                                 exps, stream);
+                                 false, exps, stream);
 }
 
 }  // extern "C"

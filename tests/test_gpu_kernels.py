@@ -640,6 +640,8 @@ def test_bsa_fwd_parts_match_unsplit(dev, monkeypatch, d, heads, video, text, cu
     (64, 3, 1153, 0, 32, torch.bfloat16, None, ("v", 1152)),   # two V blocks per workgroup, an odd block count
     (128, 1, 900, 125, 16, torch.bfloat16, None, ("q", 0)),    # text; only Q beyond f16
     (128, 40, 3000, 0, 16, torch.bfloat16, None, ("v", 0)),    # above the one-launch limit
+    (64, 2, 4000, 0, 16, torch.bfloat16, None, ("q", 3999)),   # a given mask: the attention marks the head itself
+    (128, 3, 600, 0, 16, torch.bfloat16, None, ("q", 130, 1.0e5)),  # beyond f16, but not times the scale
     (64, 2, 500, 0, 16, torch.float16, None, None),            # nothing to flag
     (128, 2, 700, 0, 16, torch.bfloat16, torch.bfloat16, ("v", 5)),  # bf16 operands: no flags
     (128, 2, 700, 0, 64, torch.bfloat16, None, None),          # tiles of the generic scorer (score matrix)
@@ -653,7 +655,7 @@ def test_whole_call_matches_single_entry_points(dev, d, heads, video, text, tile
     g = torch.Generator().manual_seed(L)
     x = {n: torch.randn((1, heads, L, d), generator=g).to(dtype) for n in "qkv"}
     if big:
-        x[big[0]][0, heads - 1, big[1], d - 1] = 1.0e6
+        x[big[0]][0, heads - 1, big[1], d - 1] = big[2] if len(big) > 2 else 1.0e6
     q, k, v = (x[n].to(dev) for n in "qkv")
     layout = ScoringLayout(L, video, tile)
     pol = hunyuan_policy(layout, 0.5) if text else wan_policy(layout, 0.3)
