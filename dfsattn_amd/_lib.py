@@ -59,7 +59,8 @@ class CallArgs(ctypes.Structure):
     _fields_ = [(n, _i64) for n in (
         "heads", "seq_len", "head_dim", "video_len", "q_tile", "k_tile", "dtype", "operand_dtype", "out_dtype",
         "select", "q_blocks", "k_blocks", "scored_rows", "n_cand", "k_pick", "dense_col", "dense_row", "long_row",
-        "long_parts", "full_rows", "parts", "out_head_stride", "out_row_stride", "n_seq", "workspace_bytes")] + [
+        "long_parts", "full_rows", "parts", "q_head_stride", "q_row_stride", "k_head_stride", "k_row_stride",
+        "v_head_stride", "v_row_stride", "out_head_stride", "out_row_stride", "n_seq", "workspace_bytes")] + [
         ("scale", ctypes.c_double)] + [(n, _p) for n in (
             "q", "k", "v", "perm", "row_ptr", "col_idx", "out", "out_perm", "cu_seqlens_q", "cu_seqlens_k",
             "workspace")]

@@ -59,6 +59,7 @@ struct BsaParams {
   // values are read unscaled.
   const uint16_t* q_src;
   const int32_t* q_rows;
+  int64_t q_sh, q_sl;  // element strides of q_src between heads and between rows
   int q_src_f16;
   // Optional, = exps when nobody has looked at Q's range yet: the common
   // instance sets word h when a row of its Q leaves the f16 range, and the
@@ -85,7 +86,7 @@ __device__ __forceinline__ const uint16_t* q_row_ptr(const uint16_t* __restrict_
   if (p.q_src) {
     f16 = p.q_src_f16 != 0;
     if (qrow >= p.L) return nullptr;
-    return p.q_src + (static_cast<int64_t>(h) * p.L + p.q_rows[qrow]) * D;
+    return p.q_src + h * p.q_sh + p.q_rows[qrow] * p.q_sl;
   }
   f16 = true;
   return q + (static_cast<int64_t>(h) * p.R + qrow) * D;
@@ -769,6 +770,7 @@ struct SegParams {
   const int32_t* exps;  // optional [3][H]
   const uint16_t* q_src;  // optional Q source (as in BsaParams)
   const int32_t* q_rows;
+  int64_t q_sh, q_sl;  // element strides of q_src
   int q_src_f16;
   int64_t o_sh, o_sl;  // element strides of out
 };
@@ -855,7 +857,7 @@ __global__ void __launch_bounds__(256) bsa_segment_kernel(const uint16_t* __rest
   // Element j of execution row r's query (r < L).
   auto q_at = [&](int r, int j) -> float {
     if (p.q_src)
-      return operand_at(p.q_src, (static_cast<int64_t>(h) * p.L + p.q_rows[r]) * D + j, p.q_src_f16 != 0);
+      return operand_at(p.q_src, h * p.q_sh + p.q_rows[r] * p.q_sl + j, p.q_src_f16 != 0);
     return operand_at(q, hq + static_cast<int64_t>(r) * D + j, QK_F16);
   };
 
@@ -1010,7 +1012,7 @@ int bsa_fwd_impl(const char* name, const void* q_perm, const void* k_perm, const
                            const int32_t* exps, const void* q_src, const int32_t* q_rows, int q_src_dtype,
                            int64_t out_head_stride, int64_t out_row_stride, int64_t long_row, int64_t long_parts,
                            int64_t full_rows, int64_t parts, void* workspace, int64_t workspace_bytes,
-                           int32_t* q_marks, dfs_stream_t stream) {
+                           int32_t* q_marks, const int64_t* q_strides, dfs_stream_t stream) {
   DFS_REQUIRE((q_perm || q_src) && k_perm && v_t && row_ptr && col_idx && out, "%s: NULL operand", name);
   DFS_REQUIRE(!q_src || q_rows, "%s: q_src needs q_rows", name);
   DFS_REQUIRE(!q_src || q_src_dtype == DFS_DTYPE_BF16 || q_src_dtype == DFS_DTYPE_F16,
@@ -1056,6 +1058,11 @@ int bsa_fwd_impl(const char* name, const void* q_perm, const void* k_perm, const
   p.cu_k = cu_seqlens_k;
   p.exps = exps;
   p.q_marks = q_marks;
+  p.q_sh = q_strides ? q_strides[0] : seq_len * head_dim;
+  p.q_sl = q_strides ? q_strides[1] : head_dim;
+  DFS_REQUIRE(p.q_sh >= 0 && p.q_sl >= 0 && p.q_sh % 8 == 0 && p.q_sl % 8 == 0,
+              "%s: q strides %lld, %lld must be non-negative multiples of 8 elements", name, (long long)p.q_sh,
+              (long long)p.q_sl);
   p.q_src = static_cast<const uint16_t*>(q_src);
   p.q_rows = q_rows;
   p.q_src_f16 = q_src_dtype == DFS_DTYPE_F16 ? 1 : 0;
@@ -1108,6 +1115,8 @@ int bsa_fwd_impl(const char* name, const void* q_perm, const void* k_perm, const
     sp.exps = exps;
     sp.q_src = p.q_src;
     sp.q_rows = q_rows;
+    sp.q_sh = p.q_sh;
+    sp.q_sl = p.q_sl;
     sp.q_src_f16 = p.q_src_f16;
     sp.o_sh = p.o_sh;
     sp.o_sl = p.o_sl;
@@ -1158,7 +1167,7 @@ extern "C" int dfs_bsa_fwd(const void* q_perm, const void* k_perm, const void* v
   return dfs::bsa_fwd_impl("dfs_bsa_fwd", q_perm, k_perm, v_t, row_ptr, col_idx, heads, seq_len, head_dim, dtype,
                            pv_dtype, scale, out, out_dtype, out_perm, lse, cu_seqlens_q, cu_seqlens_k, n_seq, exps,
                            q_src, q_rows, q_src_dtype, seq_len * head_dim, head_dim,
-                           (seq_len + dfs::kBlock - 1) / dfs::kBlock, 1, 0, 1, nullptr, 0, nullptr, stream);
+                           (seq_len + dfs::kBlock - 1) / dfs::kBlock, 1, 0, 1, nullptr, 0, nullptr, nullptr, stream);
 }
 
 extern "C" int dfs_bsa_fwd_parts(const void* q_perm, const void* k_perm, const void* v_t, const int32_t* row_ptr,
@@ -1172,5 +1181,5 @@ extern "C" int dfs_bsa_fwd_parts(const void* q_perm, const void* k_perm, const v
   return dfs::bsa_fwd_impl("dfs_bsa_fwd_parts", q_perm, k_perm, v_t, row_ptr, col_idx, heads, seq_len, head_dim, dtype,
                            pv_dtype, scale, out, out_dtype, out_perm, lse, cu_seqlens_q, cu_seqlens_k, n_seq, exps,
                            q_src, q_rows, q_src_dtype, out_head_stride, out_row_stride, long_row, long_parts,
-                           full_rows, parts, workspace, workspace_bytes, nullptr, stream);
+                           full_rows, parts, workspace, workspace_bytes, nullptr, nullptr, stream);
 }

@@ -14,12 +14,12 @@ int prepare_qkv_impl(const void* q, const void* k, const void* v, const int32_t*
                      int64_t head_dim, int dtype, int64_t video_len, int64_t q_tile_size, int64_t k_tile_size,
                      int operand_dtype, void* q_perm, void* k_perm, void* v_t, uint16_t* q_pool_hi,
                      uint16_t* q_pool_lo, uint16_t* k_pool_hi, uint16_t* k_pool_lo, int32_t* overflow,
-                     int32_t* wave_flags, bool skip_q, dfs_stream_t stream);
+                     int32_t* wave_flags, bool skip_q, const int64_t* strides, dfs_stream_t stream);
 int64_t prepare_flag_words(int64_t heads, int64_t seq_len, int64_t head_dim, int64_t q_tile, int64_t k_tile);
 int prepare_fixup_impl(const void* q, const void* k, const void* v, const int32_t* perm, int64_t heads,
                        int64_t seq_len, int64_t head_dim, void* q_perm, void* k_perm, void* v_t, int32_t* overflow,
                        int32_t* wave_flags, int64_t q_tile_size, int64_t k_tile_size, bool skip_q, int32_t* exps,
-                       dfs_stream_t stream);
+                       const int64_t* strides, dfs_stream_t stream);
 
 // bsa_fwd.hip
 int bsa_fwd_impl(const char* name, const void* q_perm, const void* k_perm, const void* v_t, const int32_t* row_ptr,
@@ -28,7 +28,8 @@ int bsa_fwd_impl(const char* name, const void* q_perm, const void* k_perm, const
                  const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int64_t n_seq, const int32_t* exps,
                  const void* q_src, const int32_t* q_rows, int q_src_dtype, int64_t out_head_stride,
                  int64_t out_row_stride, int64_t long_row, int64_t long_parts, int64_t full_rows, int64_t parts,
-                 void* workspace, int64_t workspace_bytes, int32_t* q_marks, dfs_stream_t stream);
+                 void* workspace, int64_t workspace_bytes, int32_t* q_marks, const int64_t* q_strides,
+                 dfs_stream_t stream);
 
 namespace {
 
@@ -126,16 +127,18 @@ extern "C" int dfs_call(const dfs_call_args* a, int phases, dfs_stream_t stream)
   // A call that reuses its mask reads Q in the attention kernel alone, which
   // then also finds the heads whose Q leaves the f16 range.
   const bool skip_q = !a->select;
+  const int64_t strides[6] = {a->q_head_stride, a->q_row_stride, a->k_head_stride,
+                              a->k_row_stride,  a->v_head_stride, a->v_row_stride};
   if (phases & DFS_CALL_PREPARE) {
     int32_t* const flags = rounds ? reinterpret_cast<int32_t*>(ws + r.flags) : nullptr;
     if (int rc = prepare_qkv_impl(a->q, a->k, a->v, a->perm, a->heads, a->seq_len, a->head_dim,
                                   static_cast<int>(a->dtype), a->video_len, a->q_tile, a->k_tile,
                                   static_cast<int>(a->operand_dtype), nullptr, k_perm, v_t, pool[0], pool[1], pool[2],
-                                  pool[3], nullptr, flags, skip_q, stream))
+                                  pool[3], nullptr, flags, skip_q, strides, stream))
       return rc;
     if (rounds)
       if (int rc = prepare_fixup_impl(a->q, a->k, a->v, a->perm, a->heads, a->seq_len, a->head_dim, nullptr, k_perm,
-                                      v_t, nullptr, flags, a->q_tile, a->k_tile, skip_q, exps, stream))
+                                      v_t, nullptr, flags, a->q_tile, a->k_tile, skip_q, exps, strides, stream))
         return rc;
   }
   if ((phases & DFS_CALL_SELECT) && a->select) {
@@ -154,6 +157,6 @@ extern "C" int dfs_call(const dfs_call_args* a, int phases, dfs_stream_t stream)
                         static_cast<float>(a->scale), a->out, static_cast<int>(a->out_dtype), a->out_perm, nullptr,
                         a->cu_seqlens_q, a->cu_seqlens_k, a->n_seq, exps, a->q, a->perm, static_cast<int>(a->dtype),
                         a->out_head_stride, a->out_row_stride, a->long_row, a->long_parts, a->full_rows, a->parts,
-                        r.part_bytes ? ws + r.shared : nullptr, r.part_bytes, skip_q ? exps : nullptr, stream);
+                        r.part_bytes ? ws + r.shared : nullptr, r.part_bytes, skip_q ? exps : nullptr, strides, stream);
   return 0;
 }

@@ -100,8 +100,9 @@ __device__ __forceinline__ float wave_sum(float v) {
 template <int NCH, bool F16, bool W16>
 __global__ void __launch_bounds__(256) norm_rope_kernel(NormRopeParams p) {
   const int lane = threadIdx.x & 63;
-  const int t = p.n == 1 ? 0 : static_cast<int>(blockIdx.x % 3u);
-  const int64_t row = static_cast<int64_t>(p.n == 1 ? blockIdx.x : blockIdx.x / 3u) * 4 + (threadIdx.x >> 6);
+  const unsigned group = p.n == 3 ? blockIdx.x / 3u : p.n == 2 ? blockIdx.x >> 1 : blockIdx.x;
+  const int t = static_cast<int>(blockIdx.x - group * static_cast<unsigned>(p.n));
+  const int64_t row = static_cast<int64_t>(group) * 4 + (threadIdx.x >> 6);
   if (row >= p.rows) return;
   const int64_t b = row / p.L;
   const int l = static_cast<int>(row - b * p.L);
@@ -419,8 +420,9 @@ extern "C" int dfs_qkv_heads(const void* q, const void* k, const void* v, int64_
     DFS_REQUIRE((cos_table == nullptr) == (sin_table == nullptr), "%s: pass both cos and sin tables or neither", name);
   else
     DFS_REQUIRE(cos_table != nullptr && sin_table == nullptr, "%s: a complex table is passed as cos_table alone", name);
+  DFS_REQUIRE((v == nullptr) == (v_out == nullptr), "%s: pass both v and v_out or neither", name);
   NormRopeParams p{};
-  p.n = 3;
+  p.n = v ? 3 : 2;
   const void* xs[3] = {q, k, v};
   void* os[3] = {q_out, k_out, v_out};
   for (int i = 0; i < 3; ++i) {

@@ -92,9 +92,10 @@ int permute_rows(bool scatter, const void* src, const int32_t* perm, void* dst,
 }
 
 struct PrepParams {
-  const uint4* q;  // [H][L][D] as 16-byte chunks
+  const uint4* q;  // H x L rows of D elements, as 16-byte chunks
   const uint4* k;
   const uint4* v;
+  int64_t sh[3], sl[3];  // chunks between heads and between rows of q, k, v
   const int32_t* perm;
   uint4* q_perm;  // [H][R][D]
   uint4* k_perm;
@@ -162,7 +163,8 @@ __device__ __forceinline__ void prep_qk_tiles(const PrepParams& p, int bx, int n
   constexpr int RPP = kWave / CPR;  // rows covered per pass
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  const uint4* src = (is_k ? p.k : p.q) + static_cast<int64_t>(h) * p.L * CPR;
+  const int64_t sl = p.sl[is_k ? 1 : 0];
+  const uint4* src = (is_k ? p.k : p.q) + h * p.sh[is_k ? 1 : 0];
   // Without q_perm the attention kernel gathers its Q rows from the input
   // itself: Q is then only pooled and range-flagged here.
   const bool store = is_k || p.q_perm != nullptr;
@@ -200,7 +202,7 @@ __device__ __forceinline__ void prep_qk_tiles(const PrepParams& p, int bx, int n
     }
 #pragma unroll
     for (int b = 0; b < BATCH; ++b)
-      val[b] = ss[b] >= 0 && ss[b] < p.L ? load_stream(src + static_cast<int64_t>(ss[b]) * CPR + c)
+      val[b] = ss[b] >= 0 && ss[b] < p.L ? load_stream(src + ss[b] * sl + c)
                                          : make_uint4(0, 0, 0, 0);
 #pragma unroll
     for (int b = 0; b < BATCH; ++b) {
@@ -265,7 +267,7 @@ __device__ __forceinline__ void prep_v_block(const PrepParams& p, int kb, int h,
   const bool active = kb < p.R / kBlock;
   const int dg = tid % CPR;   // 8 head dims: dg*8 .. dg*8+7
   const int kg = tid / CPR;   // 8 physical token slots: kg*8 .. kg*8+7
-  const uint4* src = p.v + static_cast<int64_t>(h) * p.L * CPR;
+  const uint4* src = p.v + h * p.sh[2];
   uint4 rows[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
@@ -274,7 +276,7 @@ __device__ __forceinline__ void prep_v_block(const PrepParams& p, int kb, int h,
     rows[i] = make_uint4(0, 0, 0, 0);
     if (active && tok < p.L) {
       const int s = p.perm[tok];
-      if (s >= 0 && s < p.L) rows[i] = load_stream(src + static_cast<int64_t>(s) * CPR + dg);
+      if (s >= 0 && s < p.L) rows[i] = load_stream(src + s * p.sl[2] + dg);
     }
   }
   bool overflow = false;
@@ -386,11 +388,12 @@ __global__ void __launch_bounds__(1024) prep_fixup_kernel(PrepParams p, int32_t*
     if (threadIdx.x == 0) exps[slot] = 0;
     return;
   }
-  const uint4* src = (t == 0 ? p.q : t == 1 ? p.k : p.v) + static_cast<int64_t>(h) * p.L * CPR;
+  const uint4* src = (t == 0 ? p.q : t == 1 ? p.k : p.v) + h * p.sh[t];
+  const int64_t sl = p.sl[t];
   const int n = p.L * CPR;
   float mx = 0.f;
   for (int i = threadIdx.x; i < n; i += blockDim.x) {
-    const uint4 v = src[i];
+    const uint4 v = src[(i / CPR) * sl + i % CPR];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const float f = fabsf(bf16_bits_to_f32(u16_at(v, e)));
@@ -414,7 +417,7 @@ __global__ void __launch_bounds__(1024) prep_fixup_kernel(PrepParams p, int32_t*
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
       const int x = i / CPR, c = i - x * CPR;
       const int s = p.perm[x];
-      const uint4 val = (s >= 0 && s < p.L) ? src[static_cast<int64_t>(s) * CPR + c] : make_uint4(0, 0, 0, 0);
+      const uint4 val = (s >= 0 && s < p.L) ? src[s * sl + c] : make_uint4(0, 0, 0, 0);
       dst[static_cast<int64_t>(x) * CPR + c] = bf16x8_to_f16x8_scaled(val, sc);
     }
   } else {
@@ -433,7 +436,7 @@ __global__ void __launch_bounds__(1024) prep_fixup_kernel(PrepParams p, int32_t*
         float f = 0.f;
         if (tok < p.L) {
           const int s = p.perm[tok];
-          if (s >= 0 && s < p.L) f = bf16_bits_to_f32(vs[static_cast<int64_t>(s) * D + d]);
+          if (s >= 0 && s < p.L) f = bf16_bits_to_f32(vs[s * sl * 8 + d]);
         }
         bits[j] = f32_to_f16_bits(f * sc);
       }
@@ -454,6 +457,22 @@ void wave_flag_counts(int64_t kb, int64_t head_dim, int64_t q_tile, int64_t k_ti
   *nv = static_cast<int>(kb * (head_dim / 32));  // 16 * D / 8 threads
 }
 
+// Chunk strides of q, k, v from element strides {q head, q row, k head, ...}
+// (NULL: contiguous [H][L][D]). Rows are read in 16-byte chunks.
+int set_strides(const char* name, PrepParams& p, const int64_t* strides, int64_t seq_len, int64_t head_dim) {
+  for (int t = 0; t < 3; ++t) {
+    const int64_t sh = strides ? strides[2 * t] : seq_len * head_dim, sl = strides ? strides[2 * t + 1] : head_dim;
+    DFS_REQUIRE(sh >= 0 && sl >= 0 && sh % 8 == 0 && sl % 8 == 0,
+                "%s: strides %lld, %lld must be non-negative multiples of 8 elements", name, (long long)sh,
+                (long long)sl);
+    p.sh[t] = sh / 8;
+    p.sl[t] = sl / 8;
+  }
+  const uintptr_t at = reinterpret_cast<uintptr_t>(p.q) | reinterpret_cast<uintptr_t>(p.k) | reinterpret_cast<uintptr_t>(p.v);
+  DFS_REQUIRE(!strides || at % 16 == 0, "%s: strided q, k and v must be 16-byte aligned", name);
+  return 0;
+}
+
 }  // namespace
 
 int prepare_qkv_impl(const void* q, const void* k, const void* v, const int32_t* perm,
@@ -461,7 +480,7 @@ int prepare_qkv_impl(const void* q, const void* k, const void* v, const int32_t*
                     int64_t video_len, int64_t q_tile_size, int64_t k_tile_size, int operand_dtype, void* q_perm,
                     void* k_perm, void* v_t, uint16_t* q_pool_hi, uint16_t* q_pool_lo,
                     uint16_t* k_pool_hi, uint16_t* k_pool_lo, int32_t* overflow, int32_t* wave_flags, bool skip_q,
-                    dfs_stream_t stream) {
+                    const int64_t* strides, dfs_stream_t stream) {
   DFS_REQUIRE(q && k && v && perm && k_perm && v_t, "dfs_prepare_qkv: NULL operand");
   DFS_REQUIRE(head_dim == 64 || head_dim == 128, "dfs_prepare_qkv: head_dim=%lld (supported: 64, 128)",
               (long long)head_dim);
@@ -496,6 +515,7 @@ int prepare_qkv_impl(const void* q, const void* k, const void* v, const int32_t*
   p.q = static_cast<const uint4*>(q);
   p.k = static_cast<const uint4*>(k);
   p.v = static_cast<const uint4*>(v);
+  if (set_strides("dfs_prepare_qkv", p, strides, seq_len, head_dim)) return 1;
   p.perm = perm;
   p.q_perm = static_cast<uint4*>(q_perm);
   p.k_perm = static_cast<uint4*>(k_perm);
@@ -555,7 +575,7 @@ int64_t prepare_flag_words(int64_t heads, int64_t seq_len, int64_t head_dim, int
 int prepare_fixup_impl(const void* q, const void* k, const void* v, const int32_t* perm, int64_t heads,
                       int64_t seq_len, int64_t head_dim, void* q_perm, void* k_perm, void* v_t,
                       int32_t* overflow, int32_t* wave_flags, int64_t q_tile_size, int64_t k_tile_size,
-                      bool skip_q, int32_t* exps, dfs_stream_t stream) {
+                      bool skip_q, int32_t* exps, const int64_t* strides, dfs_stream_t stream) {
   DFS_REQUIRE(q && k && v && perm && k_perm && v_t && (overflow || wave_flags) && exps, "dfs_prepare_fixup: NULL operand");
   DFS_REQUIRE(head_dim == 64 || head_dim == 128, "dfs_prepare_fixup: head_dim=%lld (supported: 64, 128)",
               (long long)head_dim);
@@ -568,6 +588,7 @@ int prepare_fixup_impl(const void* q, const void* k, const void* v, const int32_
   p.q = static_cast<const uint4*>(q);
   p.k = static_cast<const uint4*>(k);
   p.v = static_cast<const uint4*>(v);
+  if (set_strides("dfs_prepare_fixup", p, strides, seq_len, head_dim)) return 1;
   p.perm = perm;
   p.q_perm = static_cast<uint4*>(q_perm);
   p.k_perm = static_cast<uint4*>(k_perm);
@@ -612,14 +633,14 @@ int dfs_prepare_qkv(const void* q, const void* k, const void* v, const int32_t* 
                     dfs_stream_t stream) {
   return dfs::prepare_qkv_impl(q, k, v, perm, heads, seq_len, head_dim, dtype, video_len, q_tile_size, k_tile_size,
                                operand_dtype, q_perm, k_perm, v_t, q_pool_hi, q_pool_lo, k_pool_hi, k_pool_lo,
-                               overflow, nullptr, false, stream);
+                               overflow, nullptr, false, nullptr, stream);
 }
 
 int dfs_prepare_fixup(const void* q, const void* k, const void* v, const int32_t* perm, int64_t heads,
                       int64_t seq_len, int64_t head_dim, void* q_perm, void* k_perm, void* v_t,
                       int32_t* overflow, int32_t* exps, dfs_stream_t stream) {
   return dfs::prepare_fixup_impl(q, k, v, perm, heads, seq_len, head_dim, q_perm, k_perm, v_t, overflow, nullptr, 0, 0,
-                                 false, exps, stream);
+                                 false, exps, nullptr, stream);
 }
 
 }  // extern "C"

@@ -135,7 +135,7 @@ def _flash(q, k, v, cu_seqlens_q, cu_seqlens_kv, batch_size, operand_dtype=None)
             ck = whole_k if ck is None else ck
         if cq is not None and cq.numel() != ck.numel():
             raise ValueError("cu_seqlens_q and cu_seqlens_kv describe different segment counts")
-        if native and b == 1 and q.is_contiguous():
+        if native and b == 1 and (q.is_contiguous() or q.transpose(1, 2).is_contiguous()):
             return dense_attention_native(q, k, v, cq, ck, operand_dtype)
         if native:
             out = torch.empty_like(q)

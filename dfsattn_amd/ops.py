@@ -372,6 +372,16 @@ def _call_template(layout: ScoringLayout, policy: TopkPolicy, heads: int, dim: i
     return bytes(a), size, nnz
 
 
+def _rows_in_place(x: torch.Tensor) -> Tuple[torch.Tensor, int, int]:
+    """(x or a contiguous copy, head stride, row stride): the kernels read
+    rows of D contiguous elements wherever they lie on 16-byte boundaries."""
+    sh, sl, sd = x.stride()[-3:]
+    if sd != 1 or sh % 8 or sl % 8 or x.data_ptr() % 16:
+        x = x.contiguous()
+        sh, sl = x.stride()[-3:-1]
+    return x, sh, sl
+
+
 PREPARE, SELECT, ATTEND = 1, 2, 4  # DFS_CALL_* phases
 
 
@@ -412,12 +422,19 @@ class Call:
             if _check_cu(cu_seqlens_k, "cu_seqlens_k", dev) != a.n_seq:
                 raise ValueError("cu_seqlens_q and cu_seqlens_k describe different sequence counts")
             a.cu_seqlens_q, a.cu_seqlens_k = cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr()
-        q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+        (q, a.q_head_stride, a.q_row_stride), (k, a.k_head_stride, a.k_row_stride), \
+            (v, a.v_head_stride, a.v_row_stride) = _rows_in_place(q), _rows_in_place(k), _rows_in_place(v)
         if col_idx is None:
             col_idx = torch.empty(nnz, dtype=torch.int32, device=dev)
         ws = torch.empty(size, dtype=torch.uint8, device=dev)
-        out = torch.empty((1, heads, length, dim), dtype=dtype, device=dev)
-        a.out_head_stride, a.out_row_stride = length * dim, dim
+        if a.q_head_stride == dim and a.q_row_stride == heads * dim and heads > 1:
+            # q is a view of [L, H, D] storage: so is the output, and its
+            # heads join into [L, H * D] without a copy
+            out = torch.empty((1, length, heads, dim), dtype=dtype, device=dev).permute(0, 2, 1, 3)
+            a.out_head_stride, a.out_row_stride = dim, heads * dim
+        else:
+            out = torch.empty((1, heads, length, dim), dtype=dtype, device=dev)
+            a.out_head_stride, a.out_row_stride = length * dim, dim
         a.q, a.k, a.v, a.perm, a.row_ptr = q.data_ptr(), k.data_ptr(), v.data_ptr(), perm.data_ptr(), row_ptr.data_ptr()
         a.col_idx, a.out, a.workspace = col_idx.data_ptr(), out.data_ptr(), ws.data_ptr()
         if out_perm is not None:
@@ -585,11 +602,13 @@ def _norm_weight(w: Optional[torch.Tensor], length: int, name: str) -> int:
 
 def qkv_heads(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, heads: int, q_weight: Optional[torch.Tensor],
               q_eps: float, k_weight: Optional[torch.Tensor], k_eps: float, table=None,
-              rope_rows: Optional[int] = None):
+              rope_rows: Optional[int] = None, token_major: bool = False):
     """norm_rope_heads (or, with ``rope_rows``, head_norm_rope_heads) of q and
     k and the head split of v in one launch, for projections that
     ``qkv_heads_fusable`` accepts: [B, L, H*D] each -> three new [B, H, L, D]
-    tensors. ``table``: complex [L, D/2] frequencies, or (cos, sin) fp32
+    tensors. With ``token_major`` q and k stay in [B, L, H, D] storage and v
+    is not touched: all three are returned as [B, H, L, D] views, which the
+    attention calls read in place. ``table``: complex [L, D/2] frequencies, or (cos, sin) fp32
     tables of the single-tensor functions, or None."""
     if not qkv_heads_fusable(q, k, v):
         raise ValueError("qkv_heads: q, k and v must share shape, dtype, device and strides (16-byte rows)")
@@ -616,11 +635,16 @@ def qkv_heads(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, heads: int, q_w
             raise ValueError(f"qkv_heads: tables must be contiguous {shape}, got {tuple(t.shape)}")
     width = D if per_head else C
     wq, wk = _norm_weight(q_weight, width, "q_weight"), _norm_weight(k_weight, width, "k_weight")
-    outs = [torch.empty((B, heads, L, D), dtype=q.dtype, device=q.device) for _ in range(3)]
-    _lib.call("dfs_qkv_heads", _ptr(q), _ptr(k), _ptr(v), q.stride(0), q.stride(1), D, *(_ptr(o) for o in outs),
-              heads * L * D, D, L * D, B, L, heads, D, DTYPE_CODE[q.dtype], _ptr(q_weight), wq, float(q_eps),
-              _ptr(k_weight), wk, float(k_eps), int(per_head), kind, _ptr(cos), _ptr(sin),
-              int(rope_rows) if per_head else 0, _stream(q))
+    if token_major:
+        outs = [torch.empty((B, L, heads, D), dtype=q.dtype, device=q.device).permute(0, 2, 1, 3) for _ in range(2)]
+        outs.append(v.unflatten(2, (heads, D)).transpose(1, 2))
+    else:
+        outs = [torch.empty((B, heads, L, D), dtype=q.dtype, device=q.device) for _ in range(3)]
+    ob, oh, ol = outs[0].stride()[:3]
+    _lib.call("dfs_qkv_heads", _ptr(q), _ptr(k), None if token_major else _ptr(v), q.stride(0), q.stride(1), D,
+              _ptr(outs[0]), _ptr(outs[1]), None if token_major else _ptr(outs[2]), ob, ol, oh, B, L, heads, D,
+              DTYPE_CODE[q.dtype], _ptr(q_weight), wq, float(q_eps), _ptr(k_weight), wk, float(k_eps), int(per_head),
+              kind, _ptr(cos), _ptr(sin), int(rope_rows) if per_head else 0, _stream(q))
     return tuple(outs)
 
 

@@ -47,7 +47,7 @@ def apply_rotary_emb(x: torch.Tensor, freqs_cis: Tuple[torch.Tensor, torch.Tenso
 
 
 def fused_qkv_heads_per_head(attn, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
-                             image_rotary_emb, rope_rows: int):
+                             image_rotary_emb, rope_rows: int, token_major: bool = False):
     """[B, L, H*D] projections -> [B, H, L, D] q, k, v in the library's fused
     kernel: per-head RMSNorm (attn.norm_q / norm_k over D) and real RoPE of
     the first rope_rows tokens of q and k (the text after them is not
@@ -65,7 +65,8 @@ def fused_qkv_heads_per_head(attn, query: torch.Tensor, key: torch.Tensor, value
     wq, eq = _norm_args(attn.norm_q, d, query)
     wk, ek = _norm_args(attn.norm_k, d, key)
     if qkv_heads_fusable(query, key, value):  # one launch for the three tensors
-        return qkv_heads(query, key, value, heads, wq, eq, wk, ek, None if cos is None else (cos, sin), rope_rows)
+        return qkv_heads(query, key, value, heads, wq, eq, wk, ek, None if cos is None else (cos, sin), rope_rows,
+                         token_major)
     q = head_norm_rope_heads(query, heads, wq, eq, cos, sin, rope_rows)
     k = head_norm_rope_heads(key, heads, wk, ek, cos, sin, rope_rows)
     v = head_norm_rope_heads(value, heads)
@@ -235,7 +236,11 @@ class HunyuanVideo_DFSAttn_Processor2_0:
             # fused per-head QK-RMSNorm + RoPE + head split on the GPU, where
             # the reference runs its fast kernels (replace_hyvideo.py:252-268)
             rope_rows = query.shape[1] - (encoder_hidden_states.shape[1] if single_stream else 0)
-            query, key, value = fused_qkv_heads_per_head(attn, query, key, value, image_rotary_emb, rope_rows)
+            # (views of the projections' token order where the library's attention
+            # alone reads them; text projections joined below need a copy)
+            query, key, value = fused_qkv_heads_per_head(
+                attn, query, key, value, image_rotary_emb, rope_rows,
+                token_major=self.mode == "dfs" and attn.add_q_proj is None)
         else:
             query, key, value = self._torch_qkv_heads(attn, query, key, value, image_rotary_emb,
                                                       encoder_hidden_states if single_stream else None)

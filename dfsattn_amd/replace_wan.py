@@ -77,11 +77,13 @@ def _norm_args(norm, channels: int, x: torch.Tensor):
 
 
 def fused_qkv_heads(attn, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
-                    rotary_emb: Optional[torch.Tensor]):
+                    rotary_emb: Optional[torch.Tensor], token_major: bool = False):
     """[B, L, H*D] projections -> [B, H, L, D] q, k, v: RMSNorm over all heads
     (attn.norm_q / norm_k) and complex RoPE on q and k, and the head split, in
     the library's fused kernel (one pass per tensor, the three tensors of a
-    self-attention in one launch)."""
+    self-attention in one launch). ``token_major``: views of [B, L, H, D]
+    storage instead of new head-major tensors where that launch applies (the
+    library's attention reads them in place)."""
     from .ops import norm_rope_heads, qkv_heads, qkv_heads_fusable
 
     heads = attn.heads
@@ -94,7 +96,7 @@ def fused_qkv_heads(attn, query: torch.Tensor, key: torch.Tensor, value: torch.T
             table = rotary_emb.reshape(-1, rotary_emb.shape[-1])
             if not rope_table_readable(table):
                 table = rope_tables(rotary_emb)
-        return qkv_heads(query, key, value, heads, wq, eq, wk, ek, table)
+        return qkv_heads(query, key, value, heads, wq, eq, wk, ek, table, token_major=token_major)
     cos = sin = None
     if rotary_emb is not None:
         cos, sin = rope_tables(rotary_emb)
@@ -176,7 +178,10 @@ class Wan_DFSAttn_Processor2_0:
                 and rms_norm_like(attn.norm_k, key.shape[-1])):
             # fused QK-RMSNorm + RoPE + head split on the GPU, where the
             # reference runs its RMSNorm and RoPE kernels (replace_wan.py:159-205)
-            query, key, value = fused_qkv_heads(attn, query, key, value, rotary_emb)
+            # (views of the projections' token order where the library's
+            # attention alone reads them; it takes any row strides)
+            query, key, value = fused_qkv_heads(attn, query, key, value, rotary_emb,
+                                                token_major=encoder_hidden_states_img is None)
         else:
             if attn.norm_q is not None:
                 query = attn.norm_q(query)

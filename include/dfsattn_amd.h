@@ -329,7 +329,9 @@ int dfs_bsa_fwd_parts(const void* q_perm, const void* k_perm, const void* v_t,
  * dfs_block_score_topk and dfs_bsa_fwd_parts on `stream`, in that order, every
  * intermediate in one caller workspace of dfs_call_workspace_size bytes
  * (16-byte aligned). Fields are the arguments of those entry points under the
- * same names; q, k, v are [H][L][D], row_ptr / col_idx the CSR mask, written by
+ * same names; q, k, v are H x L rows of D elements at the given element
+ * strides (multiples of 8; [H][L][D] or [L][H][D] storage alike) on 16-byte
+ * aligned bases, row_ptr / col_idx the CSR mask, col_idx written by
  * the call when `select` is set (the policy fields apply then) and read
  * otherwise. `phases` is a sum of DFS_CALL_*; phases of one call may be
  * enqueued one after the other with the same arguments and workspace.
@@ -342,7 +344,8 @@ typedef struct dfs_call_args {
   int64_t select;
   int64_t q_blocks, k_blocks, scored_rows, n_cand, k_pick, dense_col, dense_row;
   int64_t long_row, long_parts, full_rows, parts;
-  int64_t out_head_stride, out_row_stride;
+  int64_t q_head_stride, q_row_stride, k_head_stride, k_row_stride;
+  int64_t v_head_stride, v_row_stride, out_head_stride, out_row_stride;
   int64_t n_seq, workspace_bytes;
   double scale;
   const void *q, *k, *v;
@@ -428,8 +431,8 @@ int dfs_head_norm_rope(const void* x, int64_t x_sb, int64_t x_sl, int64_t x_sh,
 /*
  * q, k and v of one layer in one launch: dfs_norm_rope (per_head 0) or
  * dfs_head_norm_rope (per_head 1) of q and of k with their own weights
- * (NULL: no norm), and the head split alone of v. The three tensors share
- * shape and strides, and so do the three outputs.
+ * (NULL: no norm), and the head split alone of v (v and v_out NULL: q and k
+ * only). The tensors share shape and strides, and so do the outputs.
  *   table_kind 0: cos_table / sin_table are fp32 arrays as for the single
  *     tensors (both NULL: no RoPE);
  *   table_kind 1 or 2 (per_head 0): cos_table is the complex table

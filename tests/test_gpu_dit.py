@@ -156,6 +156,10 @@ def test_qkv_heads_matches_single_tensors(dev, B, L, H, D, dtype, wdt, table, ro
                else ops.norm_rope_heads(t, H, weight, eps, cos, sin))
         assert torch.equal(out, ref)
     assert torch.equal(got[2], x[2].unflatten(2, (H, D)).transpose(1, 2))
+    views = ops.qkv_heads(*x, H, w[0], 1e-6, w[1], 1e-5, tab, rows if per_head else None, token_major=True)
+    for a, b in zip(views, got):
+        assert a.shape == b.shape and a.transpose(1, 2).is_contiguous() and torch.equal(a, b)
+    assert views[2].data_ptr() == x[2].data_ptr()  # v stays where it is
 
 
 @torch.no_grad()

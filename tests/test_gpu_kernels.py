@@ -678,6 +678,50 @@ def test_whole_call_matches_single_entry_points(dev, d, heads, video, text, tile
         assert torch.equal(c.out, ref)
 
 
+@pytest.mark.parametrize("d,heads,L,cut,layouts,big", [
+    (128, 3, 1000, None, ("token", "token", "token"), None),
+    (64, 2, 700, None, ("head", "slice", "token"), None),
+    (128, 2, 900, 800, ("token", "head", "slice"), "v"),   # a second sequence; V beyond f16 rewritten by the fix-up
+    (128, 2, 520, None, ("slice", "token", "head"), "k"),
+    (64, 1, 300, None, ("token", "odd", "token"), "q"),    # one head; rows off 16 bytes are copied
+])
+@pytest.mark.parametrize("given", [False, True])
+def test_call_reads_strided_inputs(dev, d, heads, L, cut, layouts, big, given):
+    """q, k and v as views of [L, H, D] storage, of a wider buffer, or with
+    rows off the 16-byte boundary: the same columns and bits as contiguous
+    inputs, and an output laid out like q's storage."""
+    print(f"strided d={d} heads={heads} L={L} cut={cut} {layouts} big={big} given={given}", flush=True)
+    g = torch.Generator().manual_seed(L + d)
+    x = [torch.randn((1, heads, L, d), generator=g).to(torch.bfloat16).to(dev) for _ in range(3)]
+    if big:
+        x["qkv".index(big)][0, heads - 1, L - 1, 0] = 1.0e6
+    layout = ScoringLayout(L, L, 16)
+    pol = wan_policy(layout, 0.4)
+    row_ptr = torch.from_numpy(pol.row_ptr(heads)).to(dev)
+    perm = torch.randperm(L, generator=g).to(torch.int32).to(dev)
+    cu = None if cut is None else torch.tensor([0, cut, L], dtype=torch.int32, device=dev)
+    kw = dict(out_perm=perm, cu_seqlens_q=cu, cu_seqlens_k=cu)
+
+    def view(t, how):
+        if how == "token":
+            return t.transpose(1, 2).contiguous().transpose(1, 2)
+        if how == "head":
+            return t
+        pad = 8 if how == "slice" else 1  # a row pitch of D + 8 elements, or of D + 1 on odd bases
+        buf = torch.zeros((1, heads, L, d + pad), dtype=t.dtype, device=dev)
+        buf[..., pad:] = t
+        return buf[..., pad:]
+
+    ref = ops.Call(*x, perm, layout, pol, row_ptr, None, **kw)
+    ref.run()
+    got = ops.Call(*(view(t, how) for t, how in zip(x, layouts)), perm, layout, pol, row_ptr,
+                   ref.col_idx if given else None, **kw)
+    got.run()
+    assert torch.equal(got.col_idx, ref.col_idx) and torch.equal(got.out, ref.out)
+    token = layouts[0] == "token" and heads > 1
+    assert got.out.shape == ref.out.shape and got.out.transpose(1, 2).is_contiguous() == (token or heads == 1)
+
+
 def test_wrappers_reject_bad_index_operands(dev):
     """Index operands must be contiguous int32 on the operands' device, and
     CSR offsets must cover every (head, query block) row: checked on the host
