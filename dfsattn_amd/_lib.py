@@ -35,9 +35,9 @@ SIGNATURES = {
     "dfs_prepare_fixup": [_p, _p, _p, _p, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p],
     "dfs_bsa_fwd": [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i32, _i32, _f32, _p, _i32, _p, _p, _p, _p, _i64, _p,
                     _p, _p, _i32, _p],
-    "dfs_bsa_fwd_workspace_size": [_i64, _i64, _i64, _i64, _i64, _i64, _i64],
+    "dfs_bsa_fwd_workspace_size": [_i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64],
     "dfs_bsa_fwd_parts": [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i32, _i32, _f32, _p, _i32, _p, _p, _p, _p, _i64, _p,
-                          _p, _p, _i32, _i64, _i64, _i64, _i64, _i64, _i64, _p, _i64, _p],
+                          _p, _p, _i32, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _p, _i64, _p],
     "dfs_call_workspace_size": [_p],
     "dfs_call": [_p, _i32, _p],
     "dfs_mask_row_counts": [_p, _i64, _i64, _p, _p],
@@ -59,7 +59,7 @@ class CallArgs(ctypes.Structure):
     _fields_ = [(n, _i64) for n in (
         "heads", "seq_len", "head_dim", "video_len", "q_tile", "k_tile", "dtype", "operand_dtype", "out_dtype",
         "select", "q_blocks", "k_blocks", "scored_rows", "n_cand", "k_pick", "dense_col", "dense_row", "long_row",
-        "long_parts", "full_rows", "parts", "q_head_stride", "q_row_stride", "k_head_stride", "k_row_stride",
+        "long_parts", "full_rows", "parts", "chunks", "q_head_stride", "q_row_stride", "k_head_stride", "k_row_stride",
         "v_head_stride", "v_row_stride", "out_head_stride", "out_row_stride", "n_seq", "workspace_bytes")] + [
         ("scale", ctypes.c_double)] + [(n, _p) for n in (
             "q", "k", "v", "perm", "row_ptr", "col_idx", "out", "out_perm", "cu_seqlens_q", "cu_seqlens_k",

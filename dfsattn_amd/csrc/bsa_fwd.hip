@@ -71,6 +71,7 @@ struct BsaParams {
   // are started first, each by long_parts workgroups; of an XCD's other query
   // blocks the first full_rows are one workgroup each and the rest parts.
   int long_row, long_parts, full_rows, parts;
+  int chunks;  // contiguous ranges a head's ordinary query blocks are dealt to XCDs in (1, 2, 4 or 8)
   // Partial results of split query blocks: O [slot][128][D] and (m, l)
   // [slot][128][2], fp32, m in log2 units.
   float* part_o;
@@ -150,17 +151,21 @@ struct Work {
 // blocks / 8), when long_parts > 1), then the tails of the XCDs' lists.
 __host__ __device__ inline int long_per_head(const BsaParams& p) { return p.Qb - p.long_row; }
 __host__ __device__ inline int long_per_xcd(const BsaParams& p) { return (p.H * long_per_head(p) + 7) >> 3; }
-__host__ __device__ inline int blocks_per_xcd(const BsaParams& p) { return (p.long_row + 7) >> 3; }  // of one head
+__host__ __device__ inline int chunk_blocks(const BsaParams& p) { return (p.long_row + p.chunks - 1) / p.chunks; }
+__host__ __device__ inline int blocks_per_xcd(const BsaParams& p) {
+  return ((p.H * p.chunks + 7) >> 3) * chunk_blocks(p);
+}
 __host__ __device__ inline int split_long(const BsaParams& p) { return p.long_parts > 1 ? 8 * long_per_xcd(p) : 0; }
 __host__ __device__ inline int split_tail(const BsaParams& p) {
-  return p.parts > 1 ? 8 * (blocks_per_xcd(p) * p.H - p.full_rows) : 0;
+  return p.parts > 1 ? 8 * (blocks_per_xcd(p) - p.full_rows) : 0;
 }
 // Query block i of XCD x's list of ordinary blocks; false for a padding slot.
 __device__ __forceinline__ bool ordinary_block(const BsaParams& p, int x, int i, int& h, int& qb) {
-  const int S = blocks_per_xcd(p);
-  h = i / S;
-  qb = ((x + h) & 7) * S + (i - h * S);
-  return qb < p.long_row;
+  const int S = chunk_blocks(p), u = i / S;
+  const int g = u * 8 + x;  // this XCD's u-th (head, range)
+  h = g / p.chunks;
+  qb = ((g + h) & (p.chunks - 1)) * S + (i - u * S);
+  return h < p.H && qb < p.long_row;
 }
 __device__ __forceinline__ bool long_block(const BsaParams& p, int g, int& h, int& qb) {
   const int n = long_per_head(p);
@@ -171,11 +176,14 @@ __device__ __forceinline__ bool long_block(const BsaParams& p, int g, int& h, in
 
 // Work of this workgroup; false for a padding slot. Hardware deals workgroup
 // b to XCD b % 8 and each XCD runs its workgroups in increasing b.
-//  * Ordinary query blocks: the i-th of XCD x takes head h = i / S and query
-//    block ((x + h) % 8) * S + i % S (S = ceil(blocks / 8)), so all eight XCDs
-//    sweep the same head together: one head's K/V (38.7 MB at 75.6k tokens)
-//    stays resident in the shared last-level cache while each XCD's L2 serves
-//    neighbouring query blocks. The range an XCD takes rotates with the head.
+//  * Ordinary query blocks: a head's are dealt in `chunks` contiguous ranges,
+//    range g of all heads to XCD g % 8, so that an XCD's L2 serves neighbouring
+//    query blocks of 8 / chunks heads in flight. Fewer, longer ranges share
+//    more key blocks per L2 as long as the K/V of the heads in flight stays in
+//    the 256 MB last-level cache (head_chunks in the Python layout module):
+//    20,280 tokens x 40 heads 1,579 us with 8 ranges, 1,543 with 1; 4,680 x 40:
+//    170 and 150; 75,600 x 40 (38.7 MB a head): 32.4 ms with 8, 32.0 with 4,
+//    32.6 with 1. The ranges rotate with the head.
 //  * Long query blocks (HunyuanVideo's text rows keep every key block, three
 //    times the others at sparsity 0.3) go first: started in their place at the
 //    end of their head, the last head's ran on alone after everything else.
@@ -963,7 +971,7 @@ void launch_split_as(const BsaArgs& a, const BsaParams& p, hipStream_t s) {
   const size_t smem = static_cast<size_t>(p.Kb) * sizeof(int32_t) +
                       static_cast<size_t>(2 * ((2 * p.Kb + 31) / 32) + 1) * sizeof(uint32_t);
   if (!p.scale_all) {
-    const int per_xcd = long_per_xcd(p) * p.long_parts + p.full_rows + (blocks_per_xcd(p) * p.H - p.full_rows) * p.parts;
+    const int per_xcd = long_per_xcd(p) * p.long_parts + p.full_rows + (blocks_per_xcd(p) - p.full_rows) * p.parts;
     bsa_fwd_split_kernel<D, QK_F16, PV_F16, VARLEN, false><<<dim3(static_cast<unsigned>(8 * per_xcd)), 256, smem, s>>>(
         a.q, a.k, a.vt, a.row_ptr, a.col_idx, a.out, a.out_perm, a.lse, p);
     const int split = split_long(p) + split_tail(p);
@@ -1011,8 +1019,8 @@ int bsa_fwd_impl(const char* name, const void* q_perm, const void* k_perm, const
                            const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int64_t n_seq,
                            const int32_t* exps, const void* q_src, const int32_t* q_rows, int q_src_dtype,
                            int64_t out_head_stride, int64_t out_row_stride, int64_t long_row, int64_t long_parts,
-                           int64_t full_rows, int64_t parts, void* workspace, int64_t workspace_bytes,
-                           int32_t* q_marks, const int64_t* q_strides, dfs_stream_t stream) {
+                           int64_t full_rows, int64_t parts, int64_t chunks, void* workspace,
+                           int64_t workspace_bytes, int32_t* q_marks, const int64_t* q_strides, dfs_stream_t stream) {
   DFS_REQUIRE((q_perm || q_src) && k_perm && v_t && row_ptr && col_idx && out, "%s: NULL operand", name);
   DFS_REQUIRE(!q_src || q_rows, "%s: q_src needs q_rows", name);
   DFS_REQUIRE(!q_src || q_src_dtype == DFS_DTYPE_BF16 || q_src_dtype == DFS_DTYPE_F16,
@@ -1073,7 +1081,12 @@ int bsa_fwd_impl(const char* name, const void* q_perm, const void* k_perm, const
   p.o_sl = out_row_stride;
   DFS_REQUIRE(long_row >= 0 && long_row <= qb, "%s: long_row=%lld outside [0, %lld]", name, (long long)long_row,
               (long long)qb);
-  const int64_t per_xcd = heads * ((long_row + 7) / 8);
+  p.H = static_cast<int>(heads);
+  p.long_row = static_cast<int>(long_row);
+  DFS_REQUIRE(chunks == 1 || chunks == 2 || chunks == 4 || chunks == 8, "%s: chunks=%lld (supported: 1, 2, 4, 8)",
+              name, (long long)chunks);
+  p.chunks = static_cast<int>(chunks);
+  const int64_t per_xcd = blocks_per_xcd(p);
   DFS_REQUIRE(parts >= 1 && parts <= 64 && long_parts >= 1 && long_parts <= 64, "%s: parts=%lld, %lld outside [1, 64]",
               name, (long long)parts, (long long)long_parts);
   DFS_REQUIRE(full_rows >= 0 && full_rows <= per_xcd, "%s: full_rows=%lld outside [0, %lld]", name,
@@ -1139,11 +1152,13 @@ int bsa_fwd_impl(const char* name, const void* q_perm, const void* k_perm, const
 }  // namespace dfs
 
 extern "C" int64_t dfs_bsa_fwd_workspace_size(int64_t heads, int64_t seq_len, int64_t head_dim, int64_t long_row,
-                                              int64_t long_parts, int64_t full_rows, int64_t parts) {
+                                              int64_t long_parts, int64_t full_rows, int64_t parts,
+                                              int64_t chunks) {
   using namespace dfs;
   const int64_t qb = (seq_len + kBlock - 1) / kBlock;
   if (heads <= 0 || seq_len <= 0 || head_dim <= 0 || long_row < 0 || long_row > qb || long_parts < 1 || parts < 1 ||
-      full_rows < 0 || heads * qb >= (int64_t(1) << 31))
+      full_rows < 0 || heads * qb >= (int64_t(1) << 31) ||
+      (chunks != 1 && chunks != 2 && chunks != 4 && chunks != 8))
     return -1;
   BsaParams p{};
   p.H = static_cast<int>(heads);
@@ -1151,7 +1166,8 @@ extern "C" int64_t dfs_bsa_fwd_workspace_size(int64_t heads, int64_t seq_len, in
   p.long_row = static_cast<int>(long_row);
   p.long_parts = static_cast<int>(long_parts);
   p.parts = static_cast<int>(parts);
-  const int64_t per_xcd = static_cast<int64_t>(blocks_per_xcd(p)) * heads;
+  p.chunks = static_cast<int>(chunks);
+  const int64_t per_xcd = blocks_per_xcd(p);
   p.full_rows = static_cast<int>(full_rows < per_xcd ? full_rows : per_xcd);
   const int64_t slots = split_long(p) * long_parts + split_tail(p) * parts;
   return slots * 128 * (head_dim + 2) * static_cast<int64_t>(sizeof(float));
@@ -1167,7 +1183,7 @@ extern "C" int dfs_bsa_fwd(const void* q_perm, const void* k_perm, const void* v
   return dfs::bsa_fwd_impl("dfs_bsa_fwd", q_perm, k_perm, v_t, row_ptr, col_idx, heads, seq_len, head_dim, dtype,
                            pv_dtype, scale, out, out_dtype, out_perm, lse, cu_seqlens_q, cu_seqlens_k, n_seq, exps,
                            q_src, q_rows, q_src_dtype, seq_len * head_dim, head_dim,
-                           (seq_len + dfs::kBlock - 1) / dfs::kBlock, 1, 0, 1, nullptr, 0, nullptr, nullptr, stream);
+                           (seq_len + dfs::kBlock - 1) / dfs::kBlock, 1, 0, 1, 8, nullptr, 0, nullptr, nullptr, stream);
 }
 
 extern "C" int dfs_bsa_fwd_parts(const void* q_perm, const void* k_perm, const void* v_t, const int32_t* row_ptr,
@@ -1176,10 +1192,10 @@ extern "C" int dfs_bsa_fwd_parts(const void* q_perm, const void* k_perm, const v
                                  float* lse, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int64_t n_seq,
                                  const int32_t* exps, const void* q_src, const int32_t* q_rows, int q_src_dtype,
                                  int64_t out_head_stride, int64_t out_row_stride, int64_t long_row,
-                                 int64_t long_parts, int64_t full_rows, int64_t parts, void* workspace,
-                                 int64_t workspace_bytes, dfs_stream_t stream) {
+                                 int64_t long_parts, int64_t full_rows, int64_t parts, int64_t chunks,
+                                 void* workspace, int64_t workspace_bytes, dfs_stream_t stream) {
   return dfs::bsa_fwd_impl("dfs_bsa_fwd_parts", q_perm, k_perm, v_t, row_ptr, col_idx, heads, seq_len, head_dim, dtype,
                            pv_dtype, scale, out, out_dtype, out_perm, lse, cu_seqlens_q, cu_seqlens_k, n_seq, exps,
                            q_src, q_rows, q_src_dtype, out_head_stride, out_row_stride, long_row, long_parts,
-                           full_rows, parts, workspace, workspace_bytes, nullptr, nullptr, stream);
+                           full_rows, parts, chunks, workspace, workspace_bytes, nullptr, nullptr, stream);
 }

@@ -28,7 +28,7 @@ int bsa_fwd_impl(const char* name, const void* q_perm, const void* k_perm, const
                  const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int64_t n_seq, const int32_t* exps,
                  const void* q_src, const int32_t* q_rows, int q_src_dtype, int64_t out_head_stride,
                  int64_t out_row_stride, int64_t long_row, int64_t long_parts, int64_t full_rows, int64_t parts,
-                 void* workspace, int64_t workspace_bytes, int32_t* q_marks, const int64_t* q_strides,
+                 int64_t chunks, void* workspace, int64_t workspace_bytes, int32_t* q_marks, const int64_t* q_strides,
                  dfs_stream_t stream);
 
 namespace {
@@ -70,7 +70,7 @@ Regions regions(const dfs_call_args& a) {
     shared = r.score_bytes > 0 ? r.score_bytes : a.heads * a.scored_rows * a.k_blocks * 4;
   }
   r.part_bytes = std::max<int64_t>(0, dfs_bsa_fwd_workspace_size(a.heads, a.seq_len, a.head_dim, a.long_row,
-                                                                 a.long_parts, a.full_rows, a.parts));
+                                                                 a.long_parts, a.full_rows, a.parts, a.chunks));
   // The scoring is over when the attention writes its parts: one region.
   r.shared = take(std::max(shared, r.part_bytes));
   r.bytes = at;
@@ -156,7 +156,7 @@ extern "C" int dfs_call(const dfs_call_args* a, int phases, dfs_stream_t stream)
                         static_cast<int>(a->operand_dtype), static_cast<int>(a->operand_dtype),
                         static_cast<float>(a->scale), a->out, static_cast<int>(a->out_dtype), a->out_perm, nullptr,
                         a->cu_seqlens_q, a->cu_seqlens_k, a->n_seq, exps, a->q, a->perm, static_cast<int>(a->dtype),
-                        a->out_head_stride, a->out_row_stride, a->long_row, a->long_parts, a->full_rows, a->parts,
+                        a->out_head_stride, a->out_row_stride, a->long_row, a->long_parts, a->full_rows, a->parts, a->chunks,
                         r.part_bytes ? ws + r.shared : nullptr, r.part_bytes, skip_q ? exps : nullptr, strides, stream);
   return 0;
 }

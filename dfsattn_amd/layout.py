@@ -204,8 +204,23 @@ XCDS = 8
 XCD_SLOTS = 64  # attention workgroups an XCD holds: 32 CUs, two each
 
 
+CACHED_KV = 96 << 20  # bytes of K and V in flight that stay in the 256 MB last-level cache beside the rest
+
+
+def head_chunks(heads: int, rows: int, head_dim: int) -> int:
+    """Contiguous ranges a head's query blocks are dealt to the XCDs in: as
+    few as divide evenly (heads * ranges a multiple of 8) and keep the K/V of
+    the 8 / ranges heads then in flight in the last-level cache. The longer an
+    XCD's range, the more key blocks its query blocks share in its L2."""
+    chunks = XCDS // math.gcd(heads, XCDS)
+    while chunks < XCDS and XCDS // chunks * rows * head_dim * 4 > CACHED_KV:
+        chunks *= 2
+    return chunks
+
+
 @functools.lru_cache(maxsize=1024)
-def attention_plan(heads: int, q_blocks: int, long_row: int, kept: int, kept_long: int) -> Tuple[int, int, int]:
+def attention_plan(heads: int, q_blocks: int, long_row: int, kept: int, kept_long: int,
+                   chunks: int = XCDS) -> Tuple[int, int, int]:
     """(long_parts, full_rows, parts) of an attention call (see
     dfs_bsa_fwd_parts): how its query blocks are cut into workgroups along
     their column lists. ``kept`` / ``kept_long``: columns of a query block
@@ -227,7 +242,7 @@ def attention_plan(heads: int, q_blocks: int, long_row: int, kept: int, kept_lon
         tokens, 3 text blocks per head keeping 237 columns against 60: 515 ->
         248 us; with 44 rounds, as at 119,056 tokens and 24 heads, starting
         them first is enough)."""
-    per_xcd = heads * -(-long_row // XCDS)
+    per_xcd = -(-heads * chunks // XCDS) * -(-long_row // chunks)
     full_rows, parts = 0, 1
     if 0 < per_xcd <= 16:
         parts = max(1, min(XCD_SLOTS // 2 // per_xcd, kept // 4, 8))
@@ -241,10 +256,11 @@ def attention_plan(heads: int, q_blocks: int, long_row: int, kept: int, kept_lon
     return long_parts, full_rows if parts > 1 else 0, parts
 
 
-def query_plan(layout: ScoringLayout, heads: int, nnz: int) -> Tuple[int, int, int, int]:
-    """(long_row, long_parts, full_rows, parts) of a call whose mask keeps
-    ``nnz`` blocks: attention_plan with the text query blocks, which keep
-    every key block, as the long ones."""
+def query_plan(layout: ScoringLayout, heads: int, head_dim: int, nnz: int) -> Tuple[int, int, int, int, int]:
+    """(long_row, long_parts, full_rows, parts, chunks) of a call whose mask
+    keeps ``nnz`` blocks: attention_plan with the text query blocks, which
+    keep every key block, as the long ones."""
     long_row = layout.video_len // layout.block if layout.text_len > 0 else layout.q_blocks
     kept = max(0, nnz // heads - (layout.q_blocks - long_row) * layout.k_blocks) // max(long_row, 1)
-    return (long_row, *attention_plan(heads, layout.q_blocks, long_row, kept, layout.k_blocks))
+    chunks = head_chunks(heads, layout.rows, head_dim)
+    return (long_row, *attention_plan(heads, layout.q_blocks, long_row, kept, layout.k_blocks, chunks), chunks)

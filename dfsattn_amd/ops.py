@@ -336,18 +336,18 @@ def bsa_fwd(prep: Prepared, row_ptr: torch.Tensor, col_idx: torch.Tensor, scale:
         raise ValueError("out must be a contiguous [1, H, L, D] tensor of out_dtype")
     lse = torch.empty((prep.heads, L), dtype=torch.float32, device=out.device) if want_lse else None
     scale = 1.0 / math.sqrt(prep.head_dim) if scale is None else float(scale)
-    long_row, long_parts, full_rows, parts = query_plan(prep.layout, prep.heads, col_idx.numel())
+    long_row, long_parts, full_rows, parts, chunks = query_plan(prep.layout, prep.heads, prep.head_dim, col_idx.numel())
     ws_bytes = 0
     if long_parts > 1 or parts > 1:
         ws_bytes = int(_lib.lib().dfs_bsa_fwd_workspace_size(prep.heads, L, prep.head_dim, long_row, long_parts,
-                                                             full_rows, parts))
+                                                             full_rows, parts, chunks))
     ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=prep.device) if ws_bytes else None
     _lib.call("dfs_bsa_fwd_parts", _ptr(prep.q_perm), _ptr(prep.k_perm), _ptr(prep.v_t), _ptr(row_ptr),
               _ptr(col_idx), prep.heads, L, prep.head_dim, DTYPE_CODE[prep.operand_dtype],
               DTYPE_CODE[prep.operand_dtype], scale, _ptr(out), DTYPE_CODE[out_dtype], _ptr(out_perm),
               _ptr(lse), _ptr(cu_seqlens_q), _ptr(cu_seqlens_k), n_seq, _ptr(prep.exps), _ptr(prep.q_src),
               _ptr(prep.q_rows), DTYPE_CODE[prep.dtype], L * prep.head_dim, prep.head_dim, long_row, long_parts,
-              full_rows, parts, _ptr(ws), ws_bytes, _stream(prep.k_perm))
+              full_rows, parts, chunks, _ptr(ws), ws_bytes, _stream(prep.k_perm))
     return (out, lse) if want_lse else out
 
 
@@ -363,7 +363,7 @@ def _call_template(layout: ScoringLayout, policy: TopkPolicy, heads: int, dim: i
     a.dtype, a.operand_dtype, a.out_dtype = DTYPE_CODE[dtype], DTYPE_CODE[operand_dtype], DTYPE_CODE[dtype]
     a.select = int(select)
     (a.q_blocks, a.k_blocks, a.scored_rows, a.n_cand, a.k_pick, a.dense_col, a.dense_row) = _policy_args(policy)
-    a.long_row, a.long_parts, a.full_rows, a.parts = query_plan(layout, heads, nnz)
+    a.long_row, a.long_parts, a.full_rows, a.parts, a.chunks = query_plan(layout, heads, dim, nnz)
     a.n_seq, a.scale = 1, 1.0 / math.sqrt(dim)
     size = int(_lib.lib().dfs_call_workspace_size(ctypes.byref(a)))
     if size < 0:

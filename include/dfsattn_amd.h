@@ -292,15 +292,17 @@ int dfs_bsa_fwd(const void* q_perm, const void* k_perm, const void* v_t,
  * dfs_bsa_fwd with the output's strides, the order of its work and the split
  * of its query blocks over workgroups chosen by the caller (dfs_bsa_fwd is
  * this call with a contiguous [H][L][D] output, long_row = ceil(L / 128),
- * full_rows 0 and one part each):
+ * full_rows 0, one part each and 8 chunks):
  *   out_head_stride, out_row_stride  elements between heads and between rows
  *     of out (multiples of 4; [L][H][D] storage has strides D and H * D);
  *   long_row    query blocks long_row.. of every head keep more columns than
  *     the others (text rows): they are started first, each cut along its
  *     column list into long_parts workgroups;
- *   full_rows, parts  of the S * heads (S = ceil(long_row / 8)) other query
- *     blocks each XCD runs in order, those from full_rows on are cut into
- *     `parts` workgroups each;
+ *   chunks      contiguous ranges (1, 2, 4 or 8) a head's other query blocks
+ *     are dealt to the 8 XCDs in;
+ *   full_rows, parts  of the ceil(heads * chunks / 8) * ceil(long_row / chunks)
+ *     query blocks each XCD then runs in order, those from full_rows on are
+ *     cut into `parts` workgroups each;
  *   workspace   dfs_bsa_fwd_workspace_size bytes of device memory (16-byte
  *     aligned, may be NULL when nothing is cut): fp32 partial results, added
  *     up by a second kernel. Parts and long_parts lie in [1, 64].
@@ -310,7 +312,7 @@ int dfs_bsa_fwd(const void* q_perm, const void* k_perm, const void* v_t,
 int64_t dfs_bsa_fwd_workspace_size(int64_t heads, int64_t seq_len,
                                    int64_t head_dim, int64_t long_row,
                                    int64_t long_parts, int64_t full_rows,
-                                   int64_t parts);
+                                   int64_t parts, int64_t chunks);
 int dfs_bsa_fwd_parts(const void* q_perm, const void* k_perm, const void* v_t,
                       const int32_t* row_ptr, const int32_t* col_idx,
                       int64_t heads, int64_t seq_len, int64_t head_dim,
@@ -321,8 +323,8 @@ int dfs_bsa_fwd_parts(const void* q_perm, const void* k_perm, const void* v_t,
                       const int32_t* q_rows, int q_src_dtype,
                       int64_t out_head_stride, int64_t out_row_stride,
                       int64_t long_row, int64_t long_parts, int64_t full_rows,
-                      int64_t parts, void* workspace, int64_t workspace_bytes,
-                      dfs_stream_t stream);
+                      int64_t parts, int64_t chunks, void* workspace,
+                      int64_t workspace_bytes, dfs_stream_t stream);
 
 /*
  * One whole call: dfs_prepare_qkv (without a permuted Q) with its fixup,
@@ -343,7 +345,7 @@ typedef struct dfs_call_args {
   int64_t dtype, operand_dtype, out_dtype;
   int64_t select;
   int64_t q_blocks, k_blocks, scored_rows, n_cand, k_pick, dense_col, dense_row;
-  int64_t long_row, long_parts, full_rows, parts;
+  int64_t long_row, long_parts, full_rows, parts, chunks;
   int64_t q_head_stride, q_row_stride, k_head_stride, k_row_stride;
   int64_t v_head_stride, v_row_stride, out_head_stride, out_row_stride;
   int64_t n_seq, workspace_bytes;

@@ -587,15 +587,16 @@ def test_bsa_fwd_bf16_operands_moving_reference(dev, d, length, scale, v_size):
 
 
 @pytest.mark.parametrize("d,heads,video,text,cut,dtype,out_dtype,plan", [
-    (128, 3, 1300, 0, None, torch.bfloat16, torch.float32, (1, 0, 3)),   # every block in 3 parts, a ragged last one
-    (64, 2, 2000, 0, None, torch.float16, torch.bfloat16, (1, 3, 2)),    # the tail of each XCD's list
-    (128, 2, 1024, 200, None, torch.bfloat16, torch.bfloat16, (4, 0, 1)),  # long rows in parts, the rest whole
-    (128, 1, 1152, 150, 1200, torch.bfloat16, torch.float32, (8, 1, 5)),   # both, with a second sequence
-    (64, 3, 300, 0, None, torch.bfloat16, torch.float32, (1, 0, 64)),    # more parts than columns: empty parts
-    (128, 2, 1000, 0, 700, torch.bfloat16, torch.float16, (1, 0, 4)),    # whole query blocks past the first sequence
+    (128, 3, 1300, 0, None, torch.bfloat16, torch.float32, (1, 0, 3, 8)),   # every block in 3 parts, a ragged last one
+    (64, 2, 2000, 0, None, torch.float16, torch.bfloat16, (1, 3, 2, 4)),    # the tail of each XCD's list
+    (128, 2, 1024, 200, None, torch.bfloat16, torch.bfloat16, (4, 0, 1, 1)),  # long rows in parts, the rest whole
+    (128, 1, 1152, 150, 1200, torch.bfloat16, torch.float32, (8, 1, 5, 2)),   # both, with a second sequence
+    (64, 3, 300, 0, None, torch.bfloat16, torch.float32, (1, 0, 64, 1)),    # more parts than columns: empty parts
+    (128, 2, 1000, 0, 700, torch.bfloat16, torch.float16, (1, 0, 4, 4)),    # whole query blocks past the first sequence
 ])
 def test_bsa_fwd_parts_match_unsplit(dev, monkeypatch, d, heads, video, text, cut, dtype, out_dtype, plan):
-    """Query blocks cut into parts against the same call uncut: the sums run
+    """Query blocks cut into parts (long_parts, full_rows, parts) and dealt in
+    other ranges (chunks) against the same call uncut: the sums run
     in another order (and P is rounded against another reference), nothing
     else changes. Head 0 holds a value beyond f16, so its blocks run whole in
     the scaled instance beside the cut ones."""
@@ -617,7 +618,7 @@ def test_bsa_fwd_parts_match_unsplit(dev, monkeypatch, d, heads, video, text, cu
     row_ptr, col_idx = ops.mask_to_csr(mask.to(dev))
     cu = None if cut is None else torch.tensor([0, cut, L], dtype=torch.int32, device=dev)
     got = {}
-    for name, pl in (("whole", (1, 0, 1)), ("parts", plan)):
+    for name, pl in (("whole", (1, 0, 1, 8)), ("parts", plan)):
         monkeypatch.setattr(ops, "query_plan", lambda lay, *a: (lay.video_len // 128 if lay.text_len else lay.q_blocks, *pl))
         got[name] = ops.bsa_fwd(prep, row_ptr, col_idx, out_dtype=out_dtype, out_perm=perm.to(dev), want_lse=True,
                                 cu_seqlens_q=cu, cu_seqlens_k=cu)

@@ -251,25 +251,30 @@ def test_attention_plan_covers_every_block_once(heads, length, text, kept):
     restated here, visits every part of every query block exactly once under
     the plan, partial slots are distinct and lie inside the workspace, and
     the combining kernel's map finds the same blocks."""
-    from dfsattn_amd.layout import attention_plan
+    from dfsattn_amd.layout import attention_plan, head_chunks
     Qb = -(-length // 128)
+    c = head_chunks(heads, Qb * 128, 128)
+    assert c in (1, 2, 4, 8) and heads * c % 8 == 0
     long_row = (length - text) // 128 if text else Qb
-    lp, full, parts = attention_plan(heads, Qb, long_row, kept, Qb)
-    assert 1 <= lp <= 64 and 1 <= parts <= 64 and 0 <= full <= heads * -(-long_row // 8)
-    S, n_long = -(-long_row // 8), Qb - long_row
+    lp, full, parts = attention_plan(heads, Qb, long_row, kept, Qb, c)
+    assert 1 <= lp <= 64 and 1 <= parts <= 64 and 0 <= full <= -(-heads * c // 8) * -(-long_row // c)
+    S, n_long = -(-long_row // c), Qb - long_row
     long_x = -(-heads * n_long // 8)
-    full_k = full if parts > 1 else S * heads
+    in_order = -(-heads * c // 8) * S  # ordinary blocks per XCD
+    full_k = full if parts > 1 else in_order
     split_long = 8 * long_x if lp > 1 else 0
-    split_tail = 8 * (S * heads - full_k) if parts > 1 else 0
-    size = _lib.lib().dfs_bsa_fwd_workspace_size(heads, length, 128, long_row, lp, full, parts)
+    split_tail = 8 * (in_order - full_k) if parts > 1 else 0
+    size = _lib.lib().dfs_bsa_fwd_workspace_size(heads, length, 128, long_row, lp, full, parts, c)
     slots = split_long * lp + split_tail * parts
     assert size == slots * 128 * 130 * 4
-    per = long_x * lp + full_k + (S * heads - full_k) * parts
+    per = long_x * lp + full_k + (in_order - full_k) * parts
     seen, used = {}, {}
 
     def ordinary(x, i):
-        h, qb = i // S, ((x + i // S) & 7) * S + i % S
-        return (h, qb) if qb < long_row else None
+        g = (i // S) * 8 + x
+        h = g // c
+        qb = ((g + h) & (c - 1)) * S + i % S
+        return (h, qb) if h < heads and qb < long_row else None
 
     for b in range(8 * per):
         x, j = b & 7, b >> 3
