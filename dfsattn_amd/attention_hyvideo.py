@@ -199,10 +199,13 @@ def dfs_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, step_idx: i
                   flashinfer64_residual_min_top_k: int = 20, flashinfer64_residual_max_top_k: int = 32,
                   flashinfer64_route_cache: bool = False, flashinfer64_core_only: bool = False,
                   flashinfer64_direct_macro_csr: bool = True,
-                  flashinfer64_valid_sequence: Optional[int] = None) -> torch.Tensor:
+                  flashinfer64_valid_sequence: Optional[int] = None, *,
+                  token_major: bool = False) -> torch.Tensor:
     """DFS attention of one HunyuanVideo joint-attention call
     (attention_hyvideo.py:1743-1982). The flashinfer64_* arguments belong to a
-    research backend and are accepted for signature compatibility only."""
+    research backend and are accepted for signature compatibility only.
+    The output is contiguous or, with ``token_major``, a view of
+    [1, L, H, D] storage."""
     if sparse_execution == "flashinfer64":
         raise ValueError("sparse_execution='flashinfer64' is a research backend not provided by this build; "
                          "use 'native'")
@@ -213,6 +216,7 @@ def dfs_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, step_idx: i
             selector_mode, fine_top_p)
     attn = _dfs_attention_instances[layer_idx]
     attn.step_idx = step_idx
+    attn.token_major = token_major
     is_cache_step, current = _compute_cache_schedule(step_idx, skip_steps, cache_interval, sparsity, sparsity_dcrt)
     attn.sparse_ratio = current
     attn.cache_flag = cache_flag and is_cache_step

@@ -147,12 +147,13 @@ def dfs_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, step_idx: i
                   cu_seqlens_kv: Optional[torch.Tensor] = None, max_seqlen_q: Optional[int] = None,
                   max_seqlen_kv: Optional[int] = None, sparse_execution: str = "native", hybrid_threshold: int = 8,
                   flashinfer64_top_p: float = 0.25, flashinfer64_token_top_k: Optional[int] = None,
-                  flashinfer64_token_top_ratio: float = 0.10) -> torch.Tensor:
+                  flashinfer64_token_top_ratio: float = 0.10, *, token_major: bool = False) -> torch.Tensor:
     """DFS attention of one Wan self-attention call (attention_wan.py:673-825).
 
     q, k, v: [B=1, H, L, D] bf16/f16 on the GPU. ``step_idx`` counts CFG passes,
     so the schedule runs on 2*skip_steps and 2*cache_interval. Returns a new
-    [1, H, L, D] tensor in the input's dtype and token order."""
+    [1, H, L, D] tensor in the input's dtype and token order, contiguous or,
+    with ``token_major``, a view of [1, L, H, D] storage."""
     if sparse_execution == "flashinfer64":
         raise ValueError("sparse_execution='flashinfer64' is a research backend not provided by this build; "
                          "use 'native'")
@@ -162,6 +163,7 @@ def dfs_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, step_idx: i
                                                             hybrid_threshold)
     attn = _dfs_attention_instances[layer_idx]
     attn.step_idx = step_idx
+    attn.token_major = token_major
     is_cache_step, current = _compute_cache_schedule(step_idx, skip_steps * 2, cache_interval * 2, sparsity,
                                                      sparsity_dcrt)
     attn.sparse_ratio = current

@@ -72,6 +72,7 @@ class DfsCore:
     ``_policy`` and the class-level state dictionaries."""
 
     operand_dtype: Optional[torch.dtype] = None  # None -> operand_dtype_for default
+    token_major = False  # output as a view of [1, L, H, D] storage instead of contiguous
     # The fields a cache entry holds in the reference (attention_wan.py:466-470);
     # get_cache_info counts these per entry, as the reference does (:664-670).
     _entry_fields: Tuple[str, ...] = ("block_mask", "block_indices", "flex_block_mask")
@@ -202,7 +203,7 @@ class DfsCore:
             policy, row_ptr, col_idx = entry["policy"], entry["row_ptr"], entry["col_idx"]
         call = ops.Call(q, k, v, perm, layout, policy, row_ptr, col_idx,
                         operand_dtype=operand_dtype_for(q.dtype, self.operand_dtype), out_perm=perm,
-                        cu_seqlens_q=cu_q, cu_seqlens_k=cu_k)
+                        cu_seqlens_q=cu_q, cu_seqlens_k=cu_k, token_major=self.token_major)
         if recompute:
             entry = MaskEntry(row_ptr=row_ptr, col_idx=call.col_idx, policy=policy, heads=q.shape[1],
                               **{field: None for field in self._entry_fields})

@@ -54,7 +54,7 @@ def _identity(device: torch.device, length: int) -> torch.Tensor:
 
 def dense_attention_native(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                            cu_seqlens_q: Optional[torch.Tensor] = None, cu_seqlens_k: Optional[torch.Tensor] = None,
-                           operand_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
+                           operand_dtype: Optional[torch.dtype] = None, token_major: bool = False) -> torch.Tensor:
     """softmax(Q K^T / sqrt(D)) V of one [1, H, L, D] bf16/f16 row on the
     block-sparse kernel with a full mask (no permutation); device
     cu_seqlens (2 or 3 entries) split it into sequences as the varlen
@@ -63,7 +63,8 @@ def dense_attention_native(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     layout = scoring_layout(length, length, 16, 128, 16)
     row_ptr, col_idx = _dense_csr(q.device, heads, length)
     call = ops.Call(q, k, v, _identity(q.device, length), layout, dense_policy(layout), row_ptr, col_idx,
-                    operand_dtype=operand_dtype, cu_seqlens_q=cu_seqlens_q, cu_seqlens_k=cu_seqlens_k)
+                    operand_dtype=operand_dtype, cu_seqlens_q=cu_seqlens_q, cu_seqlens_k=cu_seqlens_k,
+                    token_major=token_major)
     call.run()
     return call.out
 
@@ -136,7 +137,8 @@ def _flash(q, k, v, cu_seqlens_q, cu_seqlens_kv, batch_size, operand_dtype=None)
         if cq is not None and cq.numel() != ck.numel():
             raise ValueError("cu_seqlens_q and cu_seqlens_kv describe different segment counts")
         if native and b == 1 and (q.is_contiguous() or q.transpose(1, 2).is_contiguous()):
-            return dense_attention_native(q, k, v, cq, ck, operand_dtype)
+            # the output in q's storage order, as empty_like below
+            return dense_attention_native(q, k, v, cq, ck, operand_dtype, token_major=not q.is_contiguous())
         if native:
             out = torch.empty_like(q)
             for bi in range(b):

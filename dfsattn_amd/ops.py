@@ -390,14 +390,16 @@ class Call:
     preparation, the mask selection (``col_idx`` None: a new mask, kept in
     ``self.col_idx``) and the attention, enqueued by ``run`` with every
     intermediate in one workspace. The same kernels as prepare_qkv,
-    block_score_topk and bsa_fwd, the output in the inputs' dtype."""
+    block_score_topk and bsa_fwd, the output in the inputs' dtype:
+    contiguous, or with ``token_major`` a view of [1, L, H, D] storage."""
 
     __slots__ = ("args", "out", "col_idx", "refs", "stream")
 
     def __init__(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, perm: torch.Tensor, layout: ScoringLayout,
                  policy: TopkPolicy, row_ptr: torch.Tensor, col_idx: Optional[torch.Tensor],
                  operand_dtype: Optional[torch.dtype] = None, out_perm: Optional[torch.Tensor] = None,
-                 cu_seqlens_q: Optional[torch.Tensor] = None, cu_seqlens_k: Optional[torch.Tensor] = None):
+                 cu_seqlens_q: Optional[torch.Tensor] = None, cu_seqlens_k: Optional[torch.Tensor] = None,
+                 token_major: bool = False):
         dev, dtype = q.device, q.dtype
         heads, length, dim = _heads_rows(q)
         if dtype not in (torch.bfloat16, torch.float16):
@@ -427,9 +429,7 @@ class Call:
         if col_idx is None:
             col_idx = torch.empty(nnz, dtype=torch.int32, device=dev)
         ws = torch.empty(size, dtype=torch.uint8, device=dev)
-        if a.q_head_stride == dim and a.q_row_stride == heads * dim and heads > 1:
-            # q is a view of [L, H, D] storage: so is the output, and its
-            # heads join into [L, H * D] without a copy
+        if token_major:  # heads join into [L, H * D] without a copy
             out = torch.empty((1, length, heads, dim), dtype=dtype, device=dev).permute(0, 2, 1, 3)
             a.out_head_stride, a.out_row_stride = dim, heads * dim
         else:

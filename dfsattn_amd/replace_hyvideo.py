@@ -272,7 +272,7 @@ class HunyuanVideo_DFSAttn_Processor2_0:
                 max_seqlen_kv=max_kv, sparse_execution=self.sparse_execution, hybrid_threshold=self.hybrid_threshold,
                 block_top_p=self.block_top_p, token_top_k=self.token_top_k,
                 residual_candidate_blocks=self.residual_candidate_blocks, selector_mode=self.selector_mode,
-                fine_top_p=self.fine_top_p, **self.flashinfer64)
+                fine_top_p=self.fine_top_p, token_major=True, **self.flashinfer64)
         else:
             full_mode = "flash" if mode == "dense" else mode
             start = DFS_Attention.timing_recorder.start(query.device)

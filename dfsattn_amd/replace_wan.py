@@ -224,7 +224,7 @@ class Wan_DFSAttn_Processor2_0:
                 cu_seqlens_q=cu_seqlens_q, cu_seqlens_kv=cu_seqlens_kv, max_seqlen_q=s_q, max_seqlen_kv=s_k_total,
                 sparse_execution=self.sparse_execution, hybrid_threshold=self.hybrid_threshold,
                 flashinfer64_top_p=self.flashinfer64_top_p, flashinfer64_token_top_k=self.flashinfer64_token_top_k,
-                flashinfer64_token_top_ratio=self.flashinfer64_token_top_ratio)
+                flashinfer64_token_top_ratio=self.flashinfer64_token_top_ratio, token_major=True)
         else:
             hidden_states = full_attention(
                 query, key, value, mode="flash", drop_rate=0.0, attn_mask=attention_mask, causal=False,

@@ -88,6 +88,30 @@ def test_wan_cfg0_shape_matches_oracle(dev):
     assert float((out.cpu().float() - ref_own).abs().max()) < 2e-2
 
 
+@pytest.mark.parametrize("dense", [False, True])
+def test_output_storage_order(dev, dense):
+    """Views of [L, H, D] projections give the bits of contiguous inputs; the
+    sparse call's output is contiguous unless token order is asked for, the
+    dense one keeps q's storage order."""
+    from dfsattn_amd.attention_wan import dfs_attention
+    from dfsattn_amd.fullattention import full_attention
+    from dfsattn_amd.utils.order import hilbert3d_perm
+    from dfsattn_amd.workloads import CONFIGS, synth_qkv
+
+    cfg = CONFIGS[0]
+    heads_first = [x.to(dev) for x in synth_qkv(cfg, dtype=torch.bfloat16)]
+    views = [x.transpose(1, 2).contiguous().transpose(1, 2) for x in heads_first]
+    if dense:
+        ref, out = full_attention(*heads_first, mode="flash"), full_attention(*views, mode="flash")
+        assert ref.is_contiguous() and out.transpose(1, 2).is_contiguous() and torch.equal(out, ref)
+        return
+    kw = dict(step_idx=24, layer_idx=3, sparsity=0.3, tile_size=16, video_perm=hilbert3d_perm(*cfg.grid))
+    ref, out = dfs_attention(*heads_first, **kw), dfs_attention(*views, **kw)
+    assert ref.is_contiguous() and out.is_contiguous() and torch.equal(out, ref)
+    out = dfs_attention(*views, token_major=True, **kw)
+    assert out.transpose(1, 2).is_contiguous() and torch.equal(out, ref)
+
+
 def test_wan_cache_reuses_mask_across_steps(dev):
     from dfsattn_amd.attention_wan import DFS_Attention, dfs_attention
     from dfsattn_amd.utils.order import hilbert3d_perm
