@@ -136,26 +136,32 @@ def topk_count(sparse_ratio: float, k_blocks: int) -> int:
     return max(1, int(sparse_ratio * k_blocks))
 
 
-@functools.lru_cache(maxsize=1024)
 def wan_policy(layout: ScoringLayout, sparse_ratio: float) -> TopkPolicy:
     """attention_wan.py:248-253: every row keeps its top-k columns."""
+    return _wan_policy(layout, topk_count(sparse_ratio, layout.k_blocks))
+
+
+@functools.lru_cache(maxsize=1024)
+def _wan_policy(layout: ScoringLayout, k: int) -> TopkPolicy:
     kb = layout.k_blocks
-    k = topk_count(sparse_ratio, kb)
     if k > kb:
         raise RuntimeError(f"selected index k out of range (k={k}, columns={kb})")
     return TopkPolicy(layout.q_blocks, kb, layout.q_blocks, kb, k, kb, layout.q_blocks)
 
 
-@functools.lru_cache(maxsize=1024)
 def hunyuan_policy(layout: ScoringLayout, sparse_ratio: float) -> TopkPolicy:
     """attention_hyvideo.py:424-501 (top-k selector): the columns from
     video_len // 128 on are kept in every video row, the video budget is
     k - text_blocks, and rows from video_len // 128 on are dense when text
     tokens exist."""
+    return _hunyuan_policy(layout, topk_count(sparse_ratio, layout.k_blocks))
+
+
+@functools.lru_cache(maxsize=1024)
+def _hunyuan_policy(layout: ScoringLayout, k: int) -> TopkPolicy:
     kb = layout.k_blocks
     dense_start = layout.video_len // layout.block
     text_blocks = max(0, kb - dense_start)
-    k = topk_count(sparse_ratio, kb)
     dense_row = dense_start if layout.text_len > 0 else layout.q_blocks
     if text_blocks > 0:
         budget = k - text_blocks
