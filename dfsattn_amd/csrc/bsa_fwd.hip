@@ -31,8 +31,8 @@
 #include <type_traits>
 
 #include "common.h"
+#include "head_range.h"
 #include "lds_copy.h"
-
 
 namespace dfs {
 namespace {
@@ -63,7 +63,8 @@ struct BsaParams {
   int q_src_f16;
   // Optional, = exps when nobody has looked at Q's range yet: the common
   // instance sets word h when a row of its Q leaves the f16 range, and the
-  // scaled instance, launched behind it, then does the whole head again.
+  // scaled instance, launched behind it, then does the whole head again. The
+  // common instance never reads these words (head_range.h).
   int32_t* q_marks;
   // Element strides of out between heads and between rows.
   int64_t o_sh, o_sl;
@@ -513,12 +514,6 @@ __device__ int distance_order_cols(int Kb, const int32_t* __restrict__ col_idx, 
       const int32_t *__restrict__ out_perm, float *__restrict__ lse, BsaParams p_in
 
 // Split schedule: two workgroups per CU, single K and V buffers.
-// Whether head h runs in the scaled instance: its operands carry exponents
-// (Q or K beyond the f16 range), or the scale lets an f16 q * c reach 2^15.
-__device__ __forceinline__ bool head_scaled(const BsaParams& p, int h) {
-  return p.scale_all || (p.exps && (p.exps[h] | p.exps[p.H + h]) != 0);
-}
-
 // One (head, 128-row query block) of the split schedule.
 // VARLEN: segment 0 of device cu_seqlens sets the rows and keys (a separate
 // instance, so the common one keeps the host lengths as kernel arguments).
@@ -673,7 +668,7 @@ __global__ void __launch_bounds__(256, 2) bsa_fwd_split_kernel(BSA_KERNEL_ARGS) 
     // Common instance: a query block of a head, or a part of one, XCD-aware.
     Work wk;
     if (!wg_work(p_in, wk)) return;
-    if (QK_F16 && head_scaled(p_in, wk.h)) return;  // the scaled instance's head
+    if (QK_F16 && common_skips(p_in, wk.h)) return;  // the scaled instance's head
     bsa_split_block<D, QK_F16, PV_F16, VARLEN, false>(q, k, vt, row_ptr, col_idx, out, out_perm, lse, p_in, wk, k_lds,
                                                       v_lds, cols);
   } else {

@@ -2,6 +2,8 @@
 import ctypes
 import os
 import re
+import shutil
+import subprocess
 
 import numpy as np
 import pytest
@@ -337,3 +339,42 @@ def test_call_checks_its_arguments_without_launching():
     with pytest.raises(_lib.DfsKernelError, match="NULL"):
         _lib.call("dfs_call", None, 7, None)
     assert _lib.lib().dfs_call_workspace_size(ref(args(head_dim=96))) == -1
+
+
+HEAD_RANGE_MODEL = r"""
+#include <cstdio>
+#include "head_range.h"
+struct P { const int32_t* exps; int32_t* q_marks; int H, scale_all; };
+int main() {
+  // exponent words of one head: Q's, K's; marked: another workgroup finds Q beyond the range
+  for (int marks = 0; marks < 2; ++marks)
+    for (int q = 0; q < 2 - marks; ++q)
+      for (int k = 0; k < 2; ++k)
+        for (int all = 0; all < 2; ++all) {
+          int32_t exps[3] = {q, k, 0};
+          const P p{exps, marks ? exps : nullptr, 1, all};
+          const bool first = dfs::common_skips(p, 0);   // the workgroup's first wave asks
+          if (marks) p.q_marks[0] = 1;                  // a workgroup of the same launch marks the head
+          const bool last = dfs::common_skips(p, 0);    // its last wave asks
+          printf("%d %d %d %d %d %d %d\n", marks, q, k, all, first, last, dfs::head_scaled(p, 0));
+        }
+}
+"""
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="no host compiler")
+def test_common_instance_exit_does_not_depend_on_marks_of_its_launch(tmp_path):
+    """The waves of a workgroup decide one by one whether the scaled instance
+    has their head, so the answer may not change while the common instance
+    runs and marks heads; the launches behind it see the mark. The rule of
+    csrc/head_range.h, compiled for the host."""
+    src, exe = tmp_path / "model.cpp", tmp_path / "model"
+    src.write_text(HEAD_RANGE_MODEL)
+    csrc = os.path.join(os.path.dirname(_lib.__file__), "csrc")
+    subprocess.run(["g++", "-std=c++17", "-I", csrc, str(src), "-o", str(exe)], check=True)
+    lines = subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split("\n")[:-1]
+    assert len(lines) == 12
+    for line in lines:
+        marks, q, k, scale_all, first, last, behind = map(int, line.split())
+        assert first == last == (scale_all or q or k), line
+        assert behind == (scale_all or q or k or marks), line
