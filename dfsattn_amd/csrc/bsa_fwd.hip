@@ -688,7 +688,10 @@ __global__ void __launch_bounds__(256, 2) bsa_fwd_split_kernel(BSA_KERNEL_ARGS) 
 // Adds up the parts of the split query blocks: O = sum_p 2^(m_p - M) O_p over
 // the same sum of l_p, M the largest m_p, then the scaling, rounding and
 // unpermute of store_out. One workgroup per 32 query rows, eight threads a
-// row. Reads each part once (64 KB of O per part and block at D = 128).
+// row. Reads each part once (64 KB of O per part and block at D = 128). Every
+// part enters both sums, so the NaN that a NaN or infinite operand leaves in a
+// part's l or O reaches the row as in an uncut block; the weight of a part
+// without keys (l = 0, O = 0) is 0.
 template <int D, bool VARLEN>
 __global__ void __launch_bounds__(256) bsa_combine_kernel(void* __restrict__ out, const int32_t* __restrict__ out_perm,
                                                           float* __restrict__ lse, int qk_f16, BsaParams p) {
@@ -716,13 +719,12 @@ __global__ void __launch_bounds__(256) bsa_combine_kernel(void* __restrict__ out
   float M = -INFINITY;
   for (int i = 0; i < parts; ++i) {
     const float2 ml = *reinterpret_cast<const float2*>(p.part_ml + (row0 + i * 128) * 2);
-    if (ml.y > 0.f) M = fmaxf(M, ml.x);
+    if (ml.y != 0.f) M = fmaxf(M, ml.x);
   }
   float acc[DPT] = {}, l = 0.f;
   for (int i = 0; i < parts; ++i) {
     const float2 ml = *reinterpret_cast<const float2*>(p.part_ml + (row0 + i * 128) * 2);
-    if (!(ml.y > 0.f)) continue;  // a part without keys
-    const float f = exp2_fast(ml.x - M);
+    const float f = ml.y != 0.f ? exp2_fast(ml.x - M) : 0.f;  // 0: a part without keys
     l += ml.y * f;
     const float4* src = reinterpret_cast<const float4*>(p.part_o + (row0 + i * 128) * D + d0);
 #pragma unroll

@@ -636,6 +636,41 @@ def test_bsa_fwd_parts_match_unsplit(dev, monkeypatch, d, heads, video, text, cu
     assert float((o0 - o1).abs().max()) <= 1e-2
 
 
+@pytest.mark.parametrize("value", [math.nan, math.inf, -math.inf])
+@pytest.mark.parametrize("where", ["q", "k", "v"])
+@pytest.mark.parametrize("d,heads,video,text,dtype,plan", [
+    (128, 2, 1300, 0, torch.bfloat16, (1, 0, 3, 4)),    # every block in 3 parts
+    (64, 1, 2000, 0, torch.float16, (1, 1, 2, 8)),      # the tail of each XCD's list
+    (128, 1, 1024, 200, torch.bfloat16, (4, 0, 1, 8)),  # long rows in parts, the rest whole
+])
+def test_bsa_fwd_parts_keep_nan(dev, monkeypatch, d, heads, video, text, dtype, plan, where, value):
+    """One NaN or infinity in Q, K or V shows in the same rows whether their
+    query blocks are cut or not."""
+    print(f"parts d={d} heads={heads} video={video} text={text} plan={plan} {where}={value}", flush=True)
+    L = video + text
+    g = torch.Generator().manual_seed(L)
+    x = {n: torch.randn((1, heads, L, d), generator=g).to(dtype) for n in "qkv"}
+    x[where][0, heads - 1, 1030, 3] = value
+    layout = ScoringLayout(L, video, 16)
+    mask = torch.rand((heads, layout.q_blocks, layout.k_blocks), generator=g) < 0.5
+    mask[:, video // 128:] = True
+    mask[:, 0] = False  # an empty row
+    prep = ops.prepare_qkv(*(x[n].to(dev) for n in "qkv"), torch.arange(L, dtype=torch.int32, device=dev), layout,
+                           pool=False, q_operand=False)
+    row_ptr, col_idx = ops.mask_to_csr(mask.to(dev))
+    got = []
+    for pl in ((1, 0, 1, 8), plan):
+        monkeypatch.setattr(ops, "query_plan", lambda lay, *a: (lay.video_len // 128 if lay.text_len else lay.q_blocks, *pl))
+        got.append([t.cpu() for t in ops.bsa_fwd(prep, row_ptr, col_idx, out_dtype=torch.float32, want_lse=True)])
+    (o0, l0), (o1, l1) = got
+    assert not torch.isfinite(o0).all()
+    if where == "v":  # infinite or NaN, as P of the key is above or rounds to 0 against either reference
+        assert torch.equal(torch.isfinite(o0), torch.isfinite(o1))
+    else:
+        assert torch.equal(torch.isnan(o0), torch.isnan(o1)) and not torch.isinf(o1).any()
+    assert torch.equal(torch.isfinite(l0), torch.isfinite(l1))
+
+
 @pytest.mark.parametrize("d,heads,video,text,tile,dtype,operand,big", [
     (128, 2, 1000, 0, 16, torch.bfloat16, None, ("k", 999)),   # one launch for q, k and v; flag in the last wave
     (64, 3, 1153, 0, 32, torch.bfloat16, None, ("v", 1152)),   # two V blocks per workgroup, an odd block count
