@@ -15,9 +15,10 @@
 // query rows walking the row's kept key blocks; two workgroups per CU, single
 // K and V buffers, the K copy of the next block overlapping softmax and PV,
 // the V copy overlapping the next QK^T; the other workgroup on the CU fills
-// the gaps. The row's reference maximum comes from its first block and later
-// blocks skip the maximum (a block is redone only if its P leaves its range);
-// the LDS operand reads run four MFMAs ahead, and the QK phase runs at raised
+// the gaps. With f16 operands the row's reference maximum comes from its first
+// block and later blocks skip the maximum (a block is redone only if its P
+// overflows); bf16 operands, whose P has 8 bits, keep the running maximum.
+// The LDS operand reads run four MFMAs ahead, and the QK phase runs at raised
 // wave priority. A row visits its key blocks in order of distance from its own
 // block, so neighbouring query blocks fetch shared key blocks together.
 //
@@ -288,26 +289,25 @@ __device__ __forceinline__ void scale_q(const uint4* raw, bool f16, const BsaPar
     for (int i = 0; i < 8; ++i) qf[s][i] = static_cast<_Float16>(x[s][i] * inv);
 }
 
-// Lazy online softmax on S' = S - m, where the running reference m enters
-// through the QK MFMA's C input (negm holds -m in every element, times qinv
-// = 2^-r for a row whose Q fragments carry 2^-r). S' and m are in units of
-// 1 / c in the log2 domain: c = 1 for f16 Q (prescaled), scale * log2(e) for
-// bf16 Q (whose bits are kept). On a row's first block m becomes the block
-// maximum; later, m moves only when some row of the wave sees a block maximum
-// above m + kLazyTau, and O and l are rescaled then. The result is the same
-// softmax: numerator and denominator share the reference. The kernel calls
-// this only for a row's first block and for a block whose P left its range.
+// Lazy online softmax on S' = S - m (f16 operands, log2 units), where the
+// running reference m enters through the QK MFMA's C input (negm holds -m in
+// every element, times qinv = 2^-r for a row whose Q fragments carry 2^-r). On
+// a row's first block m becomes the block maximum; later, m moves only when
+// some row of the wave sees a block maximum above m + kLazyTau, and O and l
+// are rescaled then. The result is the same softmax: numerator and denominator
+// share the reference. The kernel calls this only for a row's first block and
+// for a block whose P overflowed f16.
 constexpr float kLazyTau = 8.0f;
 template <int DCH>
-__device__ __forceinline__ void softmax_lazy(f32x16* s, float c, bool first, float& m, float& lsum, f32x16* o,
-                                             f32x16& negm, float qinv = 1.f) {
+__device__ __forceinline__ void softmax_lazy(f32x16* s, bool first, float& m, float& lsum, f32x16* o, f32x16& negm,
+                                             float qinv = 1.f) {
   float mx = -INFINITY;
 #pragma unroll
   for (int kc = 0; kc < 4; ++kc)
 #pragma unroll
     for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[kc][r]);
   const float bm = xhalf_max(mx);
-  if (first || __any(bm * c > kLazyTau)) {
+  if (first || __any(bm > kLazyTau)) {
     float shift = first ? bm : fmaxf(bm, 0.f);
     if (!(shift > -INFINITY)) shift = 0.f;  // a row with every key masked keeps m
 #pragma unroll
@@ -315,7 +315,7 @@ __device__ __forceinline__ void softmax_lazy(f32x16* s, float c, bool first, flo
 #pragma unroll
       for (int r = 0; r < 16; ++r) s[kc][r] -= shift;
     if (!first) {
-      const float alpha = exp2_fast(-shift * c);
+      const float alpha = exp2_fast(-shift);
       lsum *= alpha;
 #pragma unroll
       for (int i = 0; i < DCH; ++i)
@@ -377,12 +377,38 @@ __device__ __forceinline__ void qk_tile_ahead(const uint16_t* k_tile, const type
   pin_read_ahead_schedule<N>();
 }
 
-// P = exp2(c S') of a whole block as PV operands; lblk receives this lane's
-// share of the block's row sum (of the rounded values). LOG2: S' arrives in
-// log2 units (c = 1).
+// Running maximum of bf16 operands' scores (S = q.k, c = scale * log2(e); m
+// in log2 units), with O and l rescaled when some row's maximum moved. Taken
+// for every block: a row's largest weights are then 1 exactly or near it, and
+// with P rounded to 8 bits they carry most of the error. Against a reference
+// from the row's first block, as f16 operands use it, the error against 64
+// bits was 2.5 to 9% larger (1.558e-3 -> 1.627e-3 at 8,191 tokens) and O
+// overflowed fp32 for |V| a thousand times smaller; a call of 32,760 tokens x
+// 12 heads took 1.82 ms that way, 1.95 with the maximum.
+template <int DCH>
+__device__ __forceinline__ void softmax_max(const f32x16* s, float c, float& m, float& lsum, f32x16* o) {
+  float mx = -INFINITY;
+#pragma unroll
+  for (int kc = 0; kc < 4; ++kc)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[kc][r]);
+  const float mnew = fmaxf(m, xhalf_max(mx) * c);
+  if (__any(mnew > m)) {
+    const float alpha = exp2_fast(m - mnew);
+    lsum *= alpha;
+#pragma unroll
+    for (int i = 0; i < DCH; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[i][r] *= alpha;
+  }
+  m = mnew;
+}
+
+// P of a whole block as PV operands, added (the rounded values, this lane's
+// share of the row) to lsum. LOG2: S' arrives in log2 units relative to m;
+// otherwise P = exp2(S c - m).
 template <typename PvOp, bool LOG2>
-__device__ __forceinline__ void make_p(const f32x16* s, float c, typename PvOp::vec* pf, float& lblk) {
-  lblk = 0.f;
+__device__ __forceinline__ void make_p(const f32x16* s, float c, float m, typename PvOp::vec* pf, float& lsum) {
 #pragma unroll
   for (int ks = 0; ks < 8; ++ks) {
     const f32x16& src = s[ks >> 1];
@@ -391,8 +417,8 @@ __device__ __forceinline__ void make_p(const f32x16* s, float c, typename PvOp::
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const float x0 = src[r0 + 2 * j], x1 = src[r0 + 2 * j + 1];
-      pr[j] = PvOp::pack(exp2_fast(LOG2 ? x0 : x0 * c), exp2_fast(LOG2 ? x1 : x1 * c));
-      lblk = PvOp::sum2(pr[j], lblk);
+      pr[j] = PvOp::pack(exp2_fast(LOG2 ? x0 : fmaf(x0, c, -m)), exp2_fast(LOG2 ? x1 : fmaf(x1, c, -m)));
+      lsum = PvOp::sum2(pr[j], lsum);
     }
     pf[ks] = __builtin_bit_cast(typename PvOp::vec, pr);
   }
@@ -551,10 +577,9 @@ __device__ __forceinline__ void bsa_split_block(const uint16_t* __restrict__ q, 
   f32x16 o[DCH];
 #pragma unroll
   for (int i = 0; i < DCH; ++i) o[i] = f32x16{};
-  // Lazy softmax: S arrives relative to m, in log2 units with f16 Q/K (Q
-  // prescaled) and in units of q.k with bf16 Q/K (scaled in the exponent).
-  const float c = QK_F16 ? 1.f : p.scale_log2;
-  float m = 0.f, lsum = 0.f;
+  // f16 Q/K: S arrives in log2 units relative to m (lazy softmax); bf16 Q/K:
+  // S = q.k and m is the running maximum.
+  float m = QK_F16 ? 0.f : -INFINITY, lsum = 0.f;
 
   if (beg < end) {
     const uint32_t head_bytes = static_cast<uint32_t>(p.R) * D * 2;
@@ -627,21 +652,26 @@ __device__ __forceinline__ void bsa_split_block(const uint16_t* __restrict__ q, 
         asm volatile("" : "+s"(valid));  // compares stay in this (rare) branch
         mask_tail(s, valid, hl);
       }
-      // The row reference m is set from the first block's maximum. Later
-      // blocks skip the maximum: P = exp2(S - m) is formed directly and
-      // accepted unless it leaves its range (f16: some S - m >= 16 overflows,
-      // which turns the block's row sum inf; bf16: a sum above 2^16 moves the
-      // reference too, so that O keeps its fp32 range); only then is the
-      // block redone with a moved reference. P keeps its full precision.
-      if (t == t0) softmax_lazy<DCH>(s, c, true, m, lsum, o, negm, qinv);
       typename PvOp::vec pf[8];
-      float lblk;
-      make_p<PvOp, QK_F16>(s, c, pf, lblk);
-      if (t > t0 && __any(!(lblk < (PV_F16 ? INFINITY : 65536.f)))) {
-        softmax_lazy<DCH>(s, c, false, m, lsum, o, negm, qinv);
-        make_p<PvOp, QK_F16>(s, c, pf, lblk);
+      if constexpr (QK_F16) {
+        // The row reference m is set from the first block's maximum. Later
+        // blocks skip the maximum: P = exp2(S - m) is formed directly and
+        // accepted unless it overflows f16 (some S - m >= 16, which turns the
+        // block's row sum inf); only then is the block redone with a moved
+        // reference. P <= 2^16 keeps f16's 11-bit precision.
+        if (t == t0) softmax_lazy<DCH>(s, true, m, lsum, o, negm, qinv);
+        float lblk = 0.f;
+        make_p<PvOp, true>(s, 1.f, 0.f, pf, lblk);
+        if (t > t0 && __any(!(lblk < INFINITY))) {
+          softmax_lazy<DCH>(s, false, m, lsum, o, negm, qinv);
+          lblk = 0.f;
+          make_p<PvOp, true>(s, 1.f, 0.f, pf, lblk);
+        }
+        lsum += lblk;
+      } else {
+        softmax_max<DCH>(s, p.scale_log2, m, lsum, o);
+        make_p<PvOp, false>(s, p.scale_log2, m, pf, lsum);
       }
-      lsum += lblk;
       wait_vmcnt<K_LOADS>();  // V copies landed (the next K may be in flight)
       block_barrier();
       pv_tile_regs<D, PvOp>(v_lds, pf, o, l32, hl);
@@ -652,11 +682,11 @@ __device__ __forceinline__ void bsa_split_block(const uint16_t* __restrict__ q, 
     wait_vmcnt_0();  // the trailing copies have landed before the workgroup's LDS is released
   }
   if (!SCALED && wk.pieces > 1) {
-    store_part<D>(p, wk.slot, o, m * c, lsum, w, l32, hl);
+    store_part<D>(p, wk.slot, o, m, lsum, w, l32, hl);
     return;
   }
   store_out<D>(p, VARLEN ? min(max(p.cu_q[1], 0), p.L) : p.L, p.exps ? p.exps[2 * p.H + h] : 0, out, out_perm,
-               lse, o, m * c, lsum, h, qrow, hl);
+               lse, o, m, lsum, h, qrow, hl);
 }
 
 template <int D, bool QK_F16, bool PV_F16, bool VARLEN, bool SCALED>
