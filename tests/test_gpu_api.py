@@ -89,6 +89,24 @@ def test_wan_cfg0_shape_matches_oracle(dev):
 
 
 @pytest.mark.parametrize("dense", [False, True])
+@pytest.mark.parametrize("heads", [1, 2])
+def test_contiguous_inputs_off_16_bytes(dev, dense, heads):
+    """Contiguous q, k and v at an odd storage offset give the bits of aligned ones."""
+    from dfsattn_amd.attention_wan import dfs_attention
+    from dfsattn_amd.fullattention import full_attention
+    shape = (1, heads, 1000, 128)
+    g = torch.Generator().manual_seed(heads)
+    x = [torch.randn(shape, generator=g).to(dev, torch.bfloat16) for _ in range(3)]
+    odd = [torch.cat([t.new_zeros(1), t.flatten()])[1:].view(shape) for t in x]
+    assert all(t.is_contiguous() and t.data_ptr() % 16 for t in odd)
+    if dense:
+        assert torch.equal(full_attention(*odd), full_attention(*x))
+        return
+    kw = dict(step_idx=24, layer_idx=5, sparsity=0.5, tile_size=16)
+    assert torch.equal(dfs_attention(*odd, **kw), dfs_attention(*x, **kw))
+
+
+@pytest.mark.parametrize("dense", [False, True])
 def test_output_storage_order(dev, dense):
     """Views of [L, H, D] projections give the bits of contiguous inputs; the
     sparse call's output is contiguous unless token order is asked for, the

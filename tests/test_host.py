@@ -378,3 +378,29 @@ def test_common_instance_exit_does_not_depend_on_marks_of_its_launch(tmp_path):
         marks, q, k, scale_all, first, last, behind = map(int, line.split())
         assert first == last == (scale_all or q or k), line
         assert behind == (scale_all or q or k or marks), line
+
+
+@pytest.mark.parametrize("shape,how", [
+    ((1, 2, 40, 64), "contiguous"), ((3, 40, 64), "contiguous"),  # contiguous, off 16 bytes
+    ((1, 1, 40, 64), "one head"), ((1, 2, 1, 64), "one row"),     # any stride on an axis of one
+    ((1, 2, 40, 64), "rows"), ((1, 2, 40, 64), "token"), ((1, 2, 40, 64), "channels")])
+@pytest.mark.parametrize("offset", [0, 1, 8])
+def test_rows_in_place_gives_16_byte_rows(shape, how, offset):
+    """What the call passes to the kernels: the same rows, on 16-byte
+    boundaries and strides, whatever the caller's offset and strides."""
+    n = 1
+    for s in shape:
+        n *= s
+    buf = torch.arange(4 * n + offset + 64, dtype=torch.float32).to(torch.float16)[offset:]
+    h, l, d = shape[-3:]
+    strides = {"contiguous": (l * d, d, 1), "one head": (3, d, 1), "one row": (d, 5, 1), "rows": (l * (d + 3), d + 3, 1),
+               "token": (d, h * d, 1), "channels": (2 * l * d, 2 * d, 2)}[how]
+    x = buf.as_strided(shape, ((7,) if len(shape) == 4 else ()) + strides)
+    x.copy_(torch.randn(shape))
+    y, sh, sl = ops._rows_in_place(x)
+    assert y.data_ptr() % 16 == 0 and sh % 8 == 0 and sl % 8 == 0
+    room = y.untyped_storage().nbytes() // 2 - y.storage_offset()
+    assert (h - 1) * sh + (l - 1) * sl + d <= room
+    assert torch.equal(y.as_strided((h, l, d), (sh, sl, 1)), x.reshape(h, l, d))
+    if x.data_ptr() % 16 == 0 and how in ("contiguous", "token", "one head", "one row"):
+        assert y.data_ptr() == x.data_ptr()  # read where it is
