@@ -85,11 +85,13 @@ class DFS_Attention(DfsCore, nn.Module):
     def forward(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, attn_mask: Optional[torch.Tensor] = None,
                 causal: bool = False, drop_rate: float = 0.0, cu_seqlens_q: Optional[torch.Tensor] = None,
                 cu_seqlens_kv: Optional[torch.Tensor] = None, max_seqlen_q: Optional[int] = None,
-                max_seqlen_kv: Optional[int] = None, batch_size: int = 1) -> torch.Tensor:
+                max_seqlen_kv: Optional[int] = None, batch_size: int = 1, *,
+                token_major: bool = False) -> torch.Tensor:
         """q, k, v [1, H, L, D] with the text tokens after the video ->
         new [1, H, L, D] (attention_hyvideo.py:1090-1286)."""
         self._check_selector()
-        return self._dfs_forward(q, k, v, attn_mask, causal, drop_rate, cu_seqlens_q, cu_seqlens_kv, batch_size)
+        return self._dfs_forward(q, k, v, attn_mask, causal, drop_rate, cu_seqlens_q, cu_seqlens_kv, batch_size,
+                                 token_major)
 
     def _record_density(self, entry: MaskEntry, seq_len: int) -> None:
         """Interaction density of the block mask without padding tokens
@@ -216,7 +218,6 @@ def dfs_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, step_idx: i
             selector_mode, fine_top_p)
     attn = _dfs_attention_instances[layer_idx]
     attn.step_idx = step_idx
-    attn.token_major = token_major
     is_cache_step, current = _compute_cache_schedule(step_idx, skip_steps, cache_interval, sparsity, sparsity_dcrt)
     attn.sparse_ratio = current
     attn.cache_flag = cache_flag and is_cache_step
@@ -234,4 +235,4 @@ def dfs_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, step_idx: i
         DFS_Attention.set_record_density(True)
     return attn.forward(q=q, k=k, v=v, attn_mask=None, causal=False, drop_rate=0.0, cu_seqlens_q=cu_seqlens_q,
                         cu_seqlens_kv=cu_seqlens_kv, max_seqlen_q=max_seqlen_q, max_seqlen_kv=max_seqlen_kv,
-                        batch_size=q.shape[0])
+                        batch_size=q.shape[0], token_major=token_major)

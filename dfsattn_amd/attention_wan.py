@@ -88,9 +88,11 @@ class DFS_Attention(DfsCore, nn.Module):
     def forward(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, attn_mask: Optional[torch.Tensor] = None,
                 causal: bool = False, drop_rate: float = 0.0, cu_seqlens_q: Optional[torch.Tensor] = None,
                 cu_seqlens_kv: Optional[torch.Tensor] = None, max_seqlen_q: Optional[int] = None,
-                max_seqlen_kv: Optional[int] = None, batch_size: int = 1) -> torch.Tensor:
+                max_seqlen_kv: Optional[int] = None, batch_size: int = 1, *,
+                token_major: bool = False) -> torch.Tensor:
         """q, k, v [1, H, L, D] bf16/f16 -> new [1, H, L, D] (attention_wan.py:394-547)."""
-        return self._dfs_forward(q, k, v, attn_mask, causal, drop_rate, cu_seqlens_q, cu_seqlens_kv, batch_size)
+        return self._dfs_forward(q, k, v, attn_mask, causal, drop_rate, cu_seqlens_q, cu_seqlens_kv, batch_size,
+                                 token_major)
 
     def _record_density(self, entry: MaskEntry, seq_len: int) -> None:
         """Execution-tile records (attention_wan.py:514-532) from the policy's
@@ -163,7 +165,6 @@ def dfs_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, step_idx: i
                                                             hybrid_threshold)
     attn = _dfs_attention_instances[layer_idx]
     attn.step_idx = step_idx
-    attn.token_major = token_major
     is_cache_step, current = _compute_cache_schedule(step_idx, skip_steps * 2, cache_interval * 2, sparsity,
                                                      sparsity_dcrt)
     attn.sparse_ratio = current
@@ -174,4 +175,4 @@ def dfs_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, step_idx: i
         DFS_Attention.set_record_density(True)
     return attn.forward(q=q, k=k, v=v, attn_mask=None, causal=False, drop_rate=0.0, cu_seqlens_q=cu_seqlens_q,
                         cu_seqlens_kv=cu_seqlens_kv, max_seqlen_q=max_seqlen_q, max_seqlen_kv=max_seqlen_kv,
-                        batch_size=q.shape[0])
+                        batch_size=q.shape[0], token_major=token_major)

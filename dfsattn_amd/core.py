@@ -72,7 +72,6 @@ class DfsCore:
     ``_policy`` and the class-level state dictionaries."""
 
     operand_dtype: Optional[torch.dtype] = None  # None -> operand_dtype_for default
-    token_major = False  # output as a view of [1, L, H, D] storage instead of contiguous
     # The fields a cache entry holds in the reference (attention_wan.py:466-470);
     # get_cache_info counts these per entry, as the reference does (:664-670).
     _entry_fields: Tuple[str, ...] = ("block_mask", "block_indices", "flex_block_mask")
@@ -166,10 +165,12 @@ class DfsCore:
             return None  # a cached mask of another sequence length cannot be reused
         return entry
 
-    def _dfs_forward(self, q, k, v, attn_mask, causal, drop_rate, cu_seqlens_q, cu_seqlens_kv, batch_size):
+    def _dfs_forward(self, q, k, v, attn_mask, causal, drop_rate, cu_seqlens_q, cu_seqlens_kv, batch_size,
+                     token_major=False):
         """Common body of DFS_Attention.forward (attention_wan.py:394-547,
         attention_hyvideo.py:1090-1286): permute, refresh or reuse the mask,
-        execute, unpermute."""
+        execute, unpermute. ``token_major``: the output as a view of
+        [1, L, H, D] storage instead of contiguous."""
         cls = type(self)
         self._check_call(q, k, v, attn_mask, causal, drop_rate, batch_size)
         seq_len = q.shape[2]
@@ -203,7 +204,7 @@ class DfsCore:
             policy, row_ptr, col_idx = entry["policy"], entry["row_ptr"], entry["col_idx"]
         call = ops.Call(q, k, v, perm, layout, policy, row_ptr, col_idx,
                         operand_dtype=operand_dtype_for(q.dtype, self.operand_dtype), out_perm=perm,
-                        cu_seqlens_q=cu_q, cu_seqlens_k=cu_k, token_major=self.token_major)
+                        cu_seqlens_q=cu_q, cu_seqlens_k=cu_k, token_major=token_major)
         if recompute:
             entry = MaskEntry(row_ptr=row_ptr, col_idx=call.col_idx, policy=policy, heads=q.shape[1],
                               **{field: None for field in self._entry_fields})

@@ -130,6 +130,20 @@ def test_output_storage_order(dev, dense):
     assert out.transpose(1, 2).is_contiguous() and torch.equal(out, ref)
 
 
+@pytest.mark.parametrize("variant", ["wan", "hyvideo"])
+def test_token_order_is_asked_for_call_by_call(dev, variant):
+    """A call that asked for its output in token order leaves nothing behind
+    on the layer's object: its forward returns contiguous outputs."""
+    import importlib
+    mod = importlib.import_module(f"dfsattn_amd.attention_{variant}")
+    g = torch.Generator().manual_seed(1)
+    x = [torch.randn((1, 2, 1000, 128), generator=g).to(dev, torch.bfloat16) for _ in range(3)]
+    out = mod.dfs_attention(*x, step_idx=24, layer_idx=77, sparsity=0.5, tile_size=16, token_major=True)
+    assert out.transpose(1, 2).is_contiguous()
+    again = mod._dfs_attention_instances[77].forward(*x)
+    assert again.is_contiguous() and torch.equal(again, out)
+
+
 def test_wan_cache_reuses_mask_across_steps(dev):
     from dfsattn_amd.attention_wan import DFS_Attention, dfs_attention
     from dfsattn_amd.utils.order import hilbert3d_perm
