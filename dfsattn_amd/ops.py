@@ -409,10 +409,12 @@ class Call:
             raise RuntimeError("DFS native attention only supports fp16 and bf16 inputs")
         if k.shape != q.shape or v.shape != q.shape or k.dtype != dtype or v.dtype != dtype:
             raise ValueError("q, k and v must share shape and dtype")
-        _require_device(q, k, v, perm, row_ptr, col_idx, cu_seqlens_q, cu_seqlens_k)
+        _require_device(q, k, v, perm, row_ptr, col_idx, out_perm, cu_seqlens_q, cu_seqlens_k)
         _require_int32(perm=perm, row_ptr=row_ptr, col_idx=col_idx, out_perm=out_perm)
         if length != layout.seq_len or perm.numel() != length:
             raise ValueError(f"layout of {layout.seq_len} tokens and permutation of {perm.numel()} for {length} tokens")
+        if out_perm is not None and out_perm.numel() != length:
+            raise ValueError(f"out_perm has {out_perm.numel()} entries for {length} tokens")
         operand_dtype = operand_dtype or torch.float16
         if operand_dtype not in (torch.bfloat16, torch.float16):
             raise ValueError(f"operand_dtype must be bf16 or f16, got {operand_dtype}")
@@ -443,7 +445,7 @@ class Call:
         if out_perm is not None:
             a.out_perm = out_perm.data_ptr()
         self.args, self.out, self.col_idx, self.stream = a, out, col_idx, _stream(q)
-        self.refs = (q, k, v, perm, row_ptr, cu_seqlens_q, cu_seqlens_k, ws)
+        self.refs = (q, k, v, perm, row_ptr, out_perm, cu_seqlens_q, cu_seqlens_k, ws)
 
     def run(self, phases: int = PREPARE | SELECT | ATTEND) -> None:
         _lib.call("dfs_call", ctypes.byref(self.args), phases, self.stream)

@@ -856,6 +856,29 @@ def test_wrappers_reject_bad_index_operands(dev):
     assert bool(torch.isfinite(out.float()).all())
 
 
+def test_call_rejects_bad_output_permutations(dev):
+    """The call checks out_perm's place, type and length before it takes the
+    address, and holds it until its launches are enqueued."""
+    import gc
+    import weakref
+    length, heads = 300, 2
+    q = torch.randn(1, heads, length, 64).bfloat16().to(dev)
+    layout = ScoringLayout(length, length, 16)
+    pol = wan_policy(layout, 0.5)
+    row_ptr = torch.from_numpy(pol.row_ptr(heads)).to(dev)
+    ident = torch.arange(length, dtype=torch.int32, device=dev)
+    for bad, error in ((ident[:-1], ValueError), (ident.long(), ValueError), (ident.cpu(), RuntimeError)):
+        with pytest.raises(error):
+            ops.Call(q, q, q, ident, layout, pol, row_ptr, None, out_perm=bad)
+    own = ident.clone()
+    call, held = ops.Call(q, q, q, ident, layout, pol, row_ptr, None, out_perm=own), weakref.ref(own)
+    del own
+    gc.collect()
+    assert held() is not None
+    call.run()
+    assert bool(torch.isfinite(call.out.float()).all())
+
+
 @pytest.mark.parametrize("length,cu_q,cu_k", [
     (1300, [0, 1100, 1300], [0, 1100, 1300]),   # text padding: two sequences, blocks from each start
     (1300, [0, 1152, 1300], [0, 1152, 1300]),   # a split on a block boundary
