@@ -63,10 +63,12 @@ struct BsaParams {
   int64_t q_sh, q_sl;  // element strides of q_src between heads and between rows
   int q_src_f16;
   // Optional, = exps when nobody has looked at Q's range yet: the common
-  // instance sets word h when a row of its Q leaves the f16 range, and the
-  // scaled instance, launched behind it, then does the whole head again. The
-  // common instance never reads these words (head_range.h).
+  // instance sets word h, and the query block's word of q_block_marks [H][Qb],
+  // when a row of its Q leaves the f16 range, and leaves the block to the scaled
+  // instance, launched behind it. The common instance never reads these words
+  // (head_range.h).
   int32_t* q_marks;
+  int32_t* q_block_marks;
   // Element strides of out between heads and between rows.
   int64_t o_sh, o_sl;
   // Order and split of the work (see wg_work): query blocks from long_row on
@@ -238,6 +240,32 @@ __device__ __forceinline__ void mask_tail(f32x16* s, int valid, int hl) {
       if (kc * 32 + (r >> 2) * 8 + hl * 4 + (r & 3) >= valid) s[kc][r] = -INFINITY;
 }
 
+// Whether a finite bf16 value of this lane's share of a Q row reaches 2^15
+// times c (an infinity or NaN stays what it is in either instance). Looked at
+// here, a reused mask's call is spared the read of Q in the preparation (35 us
+// of 190 at 20,280 tokens x 40 heads).
+template <int D>
+__device__ __forceinline__ bool q_beyond_f16(const uint4* raw, float c) {
+  typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+  // Magnitudes order as their bits; the finite ones end at 0x7f7f.
+  auto largest = [&](auto&& keep) {
+    u16x2 mx = {0, 0};
+#pragma unroll
+    for (int s = 0; s < D / 16; ++s) {
+      const uint32_t w[4] = {raw[s].x, raw[s].y, raw[s].z, raw[s].w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        mx = __builtin_elementwise_max(mx, keep(__builtin_bit_cast(u16x2, w[i] & 0x7fff7fffu)));
+    }
+    return bf16_bits_to_f32(max(mx[0], mx[1])) * c;
+  };
+  if (largest([](u16x2 m) { return m; }) < 32768.f) return false;
+  return largest([](u16x2 m) {  // rare: infinities and NaN become 0
+    const u16x2 over = __builtin_elementwise_min(__builtin_elementwise_sub_sat(m, (u16x2)(0x7f7f)), (u16x2)(1));
+    return __builtin_elementwise_sub_sat(m, over << (u16x2)(15));
+  }) >= 32768.f;
+}
+
 // f16 Q fragments with c = scale * log2(e) folded in (q * c rounded to f16),
 // so that S^T = K (Q c)^T arrives in log2 units. In the SCALED instance the
 // per-head exponents of the f16 operands enter c exactly (q_perm holds
@@ -246,9 +274,8 @@ __device__ __forceinline__ void mask_tail(f32x16* s, int valid, int hl) {
 // power of two that fits): its S arrives as S 2^-r and the kernel multiplies
 // it by row_scale = 2^r. The common instance runs heads without exponents at
 // a scale where |q c| < 2^15 always holds (f16 q_perm values, or Q source
-// values of a head inside the f16 range, times c < 0.5); with q_marks it looks
-// for itself, which spares a reused mask's call the read of Q in the
-// preparation (35 us of 190 at 20,280 tokens x 40 heads).
+// values of a head inside the f16 range, times c < 0.5; q_beyond_f16 looks
+// where that is not known).
 template <int D, bool SCALED>
 __device__ __forceinline__ void scale_q(const uint4* raw, bool f16, const BsaParams& p, int h, f16x8* qf,
                                         float& row_scale) {
@@ -264,15 +291,6 @@ __device__ __forceinline__ void scale_q(const uint4* raw, bool f16, const BsaPar
       x[s][i] = (f16 ? f16_bits_to_f32(u16_at(raw[s], i)) : bf16_bits_to_f32(u16_at(raw[s], i))) * c;
       if (SCALED) mx = fmaxf(mx, fabsf(x[s][i]));
     }
-  }
-  if (!SCALED && p.q_marks) {
-    // The largest finite |q c|, where Q's range was not looked at before (an
-    // infinity or NaN stays what it is in either instance).
-#pragma unroll
-    for (int s = 0; s < D / 16; ++s)
-#pragma unroll
-      for (int i = 0; i < 8; ++i) mx = fmaxf(mx, fabsf(x[s][i]) < INFINITY ? fabsf(x[s][i]) : 0.f);
-    if (mx >= 32768.f) p.q_marks[h] = 1;  // every writer stores the same mark
   }
   float inv = 1.f;
   row_scale = 1.f;
@@ -483,15 +501,19 @@ __device__ __forceinline__ void store_part(const BsaParams& p, int slot, const f
 // the same key blocks at about the same time (2% fewer L2 misses than
 // ascending order with the partner row's shared columns first, 0.4-1.2%
 // faster). Columns live in a bitmap at bit 2|c - qb| + (c > qb), compacted in
-// bit order. Columns >= Kb (the keys' blocks) are dropped. bm: 2 W + 1 words of
-// LDS scratch, W = (2 Kb + 31) / 32. Every thread of the NT-thread workgroup
-// calls this; it returns the number of columns written to cols.
+// bit order. Columns >= Kb (the keys' blocks) are dropped, and all of them
+// where some thread asks to `skip`. bm: 2 W + 2 words of LDS scratch, W = (2 Kb
+// + 31) / 32. Every thread of the NT-thread workgroup calls this; it returns
+// the number of columns, the same to all of them, written to cols.
 template <int NT>
 __device__ int distance_order_cols(int Kb, const int32_t* __restrict__ col_idx, int qb, int beg, int n,
-                                   int32_t* cols, uint32_t* bm, int tid, int w, int lane) {
+                                   bool skip, int32_t* cols, uint32_t* bm, int tid, int w, int lane) {
   const int W = (2 * Kb + 31) >> 5;
   for (int i = tid; i < W; i += NT) bm[i] = 0u;
+  uint32_t* const skipped = bm + 2 * W + 1;
+  if (tid == 0) *skipped = 0u;
   block_barrier();
+  if (skip) *skipped = 1u;
   for (int i = tid; i < n; i += NT) {
     const int c = col_idx[beg + i];
     if (static_cast<unsigned>(c) < static_cast<unsigned>(Kb)) {
@@ -519,7 +541,7 @@ __device__ int distance_order_cols(int Kb, const int32_t* __restrict__ col_idx, 
       pre[w0 + j] = pos;
       pos += __popc(bm[w0 + j]);
     }
-    if (lane == 63) pre[W] = static_cast<uint32_t>(incl);  // this row's count
+    if (lane == 63) pre[W] = *skipped ? 0u : static_cast<uint32_t>(incl);  // this row's count
   }
   block_barrier();
   for (int i = tid; i < n; i += NT) {
@@ -596,9 +618,17 @@ __device__ __forceinline__ void bsa_split_block(const uint16_t* __restrict__ q, 
     uint4 q_raw[D / 16];
     load_q_raw<D>(q, p, h, qrow, hl, q_raw, q_f16);
     // Column list of this row into LDS (read back with uniform ds_reads).
+    // A block with a row of Q beyond the f16 range is left to the scaled
+    // instance, whole: its waves agree through the list's barriers.
+    bool skip = false;
+    if (QK_F16 && !SCALED && p.q_marks && q_beyond_f16<D>(q_raw, p.scale_log2)) {
+      p.q_marks[h] = 1;  // every writer stores the same marks
+      p.q_block_marks[static_cast<int64_t>(h) * p.Qb + qb] = 1;
+      skip = true;
+    }
     const int total = __builtin_amdgcn_readfirstlane(
-        distance_order_cols<256>(Kb, col_idx, qb, beg, end - beg, cols, reinterpret_cast<uint32_t*>(cols + p.Kb), tid,
-                                 w, lane));
+        distance_order_cols<256>(Kb, col_idx, qb, beg, end - beg, skip, cols, reinterpret_cast<uint32_t*>(cols + p.Kb),
+                                 tid, w, lane));
     // This workgroup's part of the list (all of it for an unsplit block).
     const int t0 = SCALED ? 0 : total * wk.piece / wk.pieces;
     const int n = SCALED ? total : total * (wk.piece + 1) / wk.pieces;
@@ -703,11 +733,13 @@ __global__ void __launch_bounds__(256, 2) bsa_fwd_split_kernel(BSA_KERNEL_ARGS) 
                                                       v_lds, cols);
   } else {
     // Scaled instance: a small grid (x: workgroups per head, y: head) whose
-    // workgroups walk the query blocks of the heads that carry exponents and
-    // exit at once for every other head.
+    // workgroups walk the query blocks of the heads that carry exponents
+    // (where only Q left the range, those blocks of them) and exit at once for
+    // every other head.
     const int h = blockIdx.y;
     if (!head_scaled(p_in, h)) return;
     for (int qb = blockIdx.x; qb < p_in.Qb; qb += gridDim.x) {
+      if (!scaled_block(p_in, h, qb)) continue;
       block_barrier();  // the previous block's LDS reads are done
       bsa_split_block<D, QK_F16, PV_F16, VARLEN, true>(q, k, vt, row_ptr, col_idx, out, out_perm, lse, p_in,
                                                        Work{h, qb, 0, 1, 0}, k_lds, v_lds, cols);
@@ -739,7 +771,10 @@ __global__ void __launch_bounds__(256) bsa_combine_kernel(void* __restrict__ out
     parts = p.parts;
     slot = n_long * p.long_parts + t * parts;
   }
-  if (qk_f16 && head_scaled(p, h)) return;  // written whole by the scaled instance
+  if (qk_f16 && head_scaled(p, h)) {  // written whole by the scaled instance
+    if (p.q_marks && threadIdx.x == 0) p.q_block_marks[static_cast<int64_t>(h) * p.Qb + qb] = 1;
+    return;
+  }
   const int Lq = VARLEN ? min(max(p.cu_q[1], 0), p.L) : p.L;
   const int in_block = (blockIdx.x & 3) * 32 + (threadIdx.x >> 3);
   const int qrow = qb * 128 + in_block;
@@ -996,7 +1031,7 @@ __global__ void __launch_bounds__(256) bsa_segment_kernel(const uint16_t* __rest
 template <int D, bool QK_F16, bool PV_F16, bool VARLEN>
 void launch_split_as(const BsaArgs& a, const BsaParams& p, hipStream_t s) {
   const size_t smem = static_cast<size_t>(p.Kb) * sizeof(int32_t) +
-                      static_cast<size_t>(2 * ((2 * p.Kb + 31) / 32) + 1) * sizeof(uint32_t);
+                      static_cast<size_t>(2 * ((2 * p.Kb + 31) / 32) + 2) * sizeof(uint32_t);
   if (!p.scale_all) {
     const int per_xcd = long_per_xcd(p) * p.long_parts + p.full_rows + (blocks_per_xcd(p) - p.full_rows) * p.parts;
     bsa_fwd_split_kernel<D, QK_F16, PV_F16, VARLEN, false><<<dim3(static_cast<unsigned>(8 * per_xcd)), 256, smem, s>>>(
@@ -1007,10 +1042,11 @@ void launch_split_as(const BsaArgs& a, const BsaParams& p, hipStream_t s) {
                                                                                           QK_F16 ? 1 : 0, p);
   }
   if constexpr (QK_F16) {
-    // Heads with exponents (only when some bf16 input exceeds the f16 range)
-    // or every head (large scales): a few workgroups per head.
+    // Heads with exponents (only when some bf16 input exceeds the f16 range):
+    // a workgroup per CU over all heads, but eight a head at least. Or every
+    // head (large scales).
     if (p.exps || p.scale_all) {
-      const unsigned per_head = p.scale_all ? static_cast<unsigned>(p.Qb) : 8u;
+      const unsigned per_head = static_cast<unsigned>(p.scale_all ? p.Qb : min(p.Qb, max(8, 256 / p.H)));
       bsa_fwd_split_kernel<D, QK_F16, PV_F16, VARLEN, true>
           <<<dim3(per_head, static_cast<unsigned>(p.H)), 256, smem, s>>>(a.q, a.k, a.vt, a.row_ptr, a.col_idx, a.out,
                                                                      a.out_perm, a.lse, p);
@@ -1047,7 +1083,8 @@ int bsa_fwd_impl(const char* name, const void* q_perm, const void* k_perm, const
                            const int32_t* exps, const void* q_src, const int32_t* q_rows, int q_src_dtype,
                            int64_t out_head_stride, int64_t out_row_stride, int64_t long_row, int64_t long_parts,
                            int64_t full_rows, int64_t parts, int64_t chunks, void* workspace,
-                           int64_t workspace_bytes, int32_t* q_marks, const int64_t* q_strides, dfs_stream_t stream) {
+                           int64_t workspace_bytes, int32_t* q_marks, int32_t* q_block_marks,
+                           const int64_t* q_strides, dfs_stream_t stream) {
   DFS_REQUIRE((q_perm || q_src) && k_perm && v_t && row_ptr && col_idx && out, "%s: NULL operand", name);
   DFS_REQUIRE(!q_src || q_rows, "%s: q_src needs q_rows", name);
   DFS_REQUIRE(!q_src || q_src_dtype == DFS_DTYPE_BF16 || q_src_dtype == DFS_DTYPE_F16,
@@ -1092,7 +1129,11 @@ int bsa_fwd_impl(const char* name, const void* q_perm, const void* k_perm, const
   p.cu_q = cu_seqlens_q;
   p.cu_k = cu_seqlens_k;
   p.exps = exps;
+  DFS_REQUIRE((q_marks == nullptr) == (q_block_marks == nullptr) &&
+                  (!q_marks || (q_marks == exps && q_src && q_src_dtype == DFS_DTYPE_BF16)),
+              "%s: Q's range is marked by head and block, for a bf16 Q source", name);
   p.q_marks = q_marks;
+  p.q_block_marks = q_block_marks;
   p.q_sh = q_strides ? q_strides[0] : seq_len * head_dim;
   p.q_sl = q_strides ? q_strides[1] : head_dim;
   DFS_REQUIRE(p.q_sh >= 0 && p.q_sl >= 0 && p.q_sh % 8 == 0 && p.q_sl % 8 == 0,
@@ -1210,7 +1251,7 @@ extern "C" int dfs_bsa_fwd(const void* q_perm, const void* k_perm, const void* v
   return dfs::bsa_fwd_impl("dfs_bsa_fwd", q_perm, k_perm, v_t, row_ptr, col_idx, heads, seq_len, head_dim, dtype,
                            pv_dtype, scale, out, out_dtype, out_perm, lse, cu_seqlens_q, cu_seqlens_k, n_seq, exps,
                            q_src, q_rows, q_src_dtype, seq_len * head_dim, head_dim,
-                           (seq_len + dfs::kBlock - 1) / dfs::kBlock, 1, 0, 1, 8, nullptr, 0, nullptr, nullptr, stream);
+                           (seq_len + dfs::kBlock - 1) / dfs::kBlock, 1, 0, 1, 8, nullptr, 0, nullptr, nullptr, nullptr, stream);
 }
 
 extern "C" int dfs_bsa_fwd_parts(const void* q_perm, const void* k_perm, const void* v_t, const int32_t* row_ptr,
@@ -1224,5 +1265,5 @@ extern "C" int dfs_bsa_fwd_parts(const void* q_perm, const void* k_perm, const v
   return dfs::bsa_fwd_impl("dfs_bsa_fwd_parts", q_perm, k_perm, v_t, row_ptr, col_idx, heads, seq_len, head_dim, dtype,
                            pv_dtype, scale, out, out_dtype, out_perm, lse, cu_seqlens_q, cu_seqlens_k, n_seq, exps,
                            q_src, q_rows, q_src_dtype, out_head_stride, out_row_stride, long_row, long_parts,
-                           full_rows, parts, chunks, workspace, workspace_bytes, nullptr, nullptr, stream);
+                           full_rows, parts, chunks, workspace, workspace_bytes, nullptr, nullptr, nullptr, stream);
 }

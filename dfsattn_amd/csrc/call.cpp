@@ -19,7 +19,7 @@ int64_t prepare_flag_words(int64_t heads, int64_t seq_len, int64_t head_dim, int
 int prepare_fixup_impl(const void* q, const void* k, const void* v, const int32_t* perm, int64_t heads,
                        int64_t seq_len, int64_t head_dim, void* q_perm, void* k_perm, void* v_t, int32_t* overflow,
                        int32_t* wave_flags, int64_t q_tile_size, int64_t k_tile_size, bool skip_q, int32_t* exps,
-                       const int64_t* strides, dfs_stream_t stream);
+                       int32_t* q_block_marks, const int64_t* strides, dfs_stream_t stream);
 
 // bsa_fwd.hip
 int bsa_fwd_impl(const char* name, const void* q_perm, const void* k_perm, const void* v_t, const int32_t* row_ptr,
@@ -28,14 +28,14 @@ int bsa_fwd_impl(const char* name, const void* q_perm, const void* k_perm, const
                  const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int64_t n_seq, const int32_t* exps,
                  const void* q_src, const int32_t* q_rows, int q_src_dtype, int64_t out_head_stride,
                  int64_t out_row_stride, int64_t long_row, int64_t long_parts, int64_t full_rows, int64_t parts,
-                 int64_t chunks, void* workspace, int64_t workspace_bytes, int32_t* q_marks, const int64_t* q_strides,
-                 dfs_stream_t stream);
+                 int64_t chunks, void* workspace, int64_t workspace_bytes, int32_t* q_marks, int32_t* q_block_marks,
+                 const int64_t* q_strides, dfs_stream_t stream);
 
 namespace {
 
 // Byte offsets of a call's intermediates in its workspace.
 struct Regions {
-  int64_t k_perm, v_t, exps, flags, q_hi, q_lo, k_hi, k_lo, shared, bytes;
+  int64_t k_perm, v_t, exps, flags, marks, q_hi, q_lo, k_hi, k_lo, shared, bytes;
   int64_t score_bytes;  // one-pass scoring workspace (0: the score matrix takes its place)
   int64_t part_bytes;   // partial results of the attention
 };
@@ -54,6 +54,7 @@ Regions regions(const dfs_call_args& a) {
   if (a.dtype == DFS_DTYPE_BF16 && a.operand_dtype == DFS_DTYPE_F16) {
     r.exps = take(3 * a.heads * 4);
     r.flags = take(prepare_flag_words(a.heads, a.seq_len, a.head_dim, a.q_tile, a.k_tile) * 4);
+    if (!a.select) r.marks = take(a.heads * (rows / kBlock) * 4);  // the attention's marks of Q's blocks
   }
   int64_t shared = 0;
   if (a.select) {
@@ -125,8 +126,10 @@ extern "C" int dfs_call(const dfs_call_args* a, int phases, dfs_stream_t stream)
     for (int i = 0; i < 4; ++i) pool[i] = reinterpret_cast<uint16_t*>(ws + at[i]);
   }
   // A call that reuses its mask reads Q in the attention kernel alone, which
-  // then also finds the heads whose Q leaves the f16 range.
+  // then also finds the heads and blocks whose Q leaves the f16 range.
   const bool skip_q = !a->select;
+  int32_t* const q_marks = skip_q ? exps : nullptr;
+  int32_t* const q_block_marks = q_marks ? reinterpret_cast<int32_t*>(ws + r.marks) : nullptr;
   const int64_t strides[6] = {a->q_head_stride, a->q_row_stride, a->k_head_stride,
                               a->k_row_stride,  a->v_head_stride, a->v_row_stride};
   if (phases & DFS_CALL_PREPARE) {
@@ -138,7 +141,8 @@ extern "C" int dfs_call(const dfs_call_args* a, int phases, dfs_stream_t stream)
       return rc;
     if (rounds)
       if (int rc = prepare_fixup_impl(a->q, a->k, a->v, a->perm, a->heads, a->seq_len, a->head_dim, nullptr, k_perm,
-                                      v_t, nullptr, flags, a->q_tile, a->k_tile, skip_q, exps, strides, stream))
+                                      v_t, nullptr, flags, a->q_tile, a->k_tile, skip_q, exps, q_block_marks, strides,
+                                      stream))
         return rc;
   }
   if ((phases & DFS_CALL_SELECT) && a->select) {
@@ -157,6 +161,6 @@ extern "C" int dfs_call(const dfs_call_args* a, int phases, dfs_stream_t stream)
                         static_cast<float>(a->scale), a->out, static_cast<int>(a->out_dtype), a->out_perm, nullptr,
                         a->cu_seqlens_q, a->cu_seqlens_k, a->n_seq, exps, a->q, a->perm, static_cast<int>(a->dtype),
                         a->out_head_stride, a->out_row_stride, a->long_row, a->long_parts, a->full_rows, a->parts, a->chunks,
-                        r.part_bytes ? ws + r.shared : nullptr, r.part_bytes, skip_q ? exps : nullptr, strides, stream);
+                        r.part_bytes ? ws + r.shared : nullptr, r.part_bytes, q_marks, q_block_marks, strides, stream);
   return 0;
 }

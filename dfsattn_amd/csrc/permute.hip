@@ -109,6 +109,7 @@ struct PrepParams {
   // [2][H][nqk], then V [H][nv]. prep_fixup_kernel joins them.
   int32_t* wave_flags;
   int nqk, nv;
+  int32_t* q_block_marks;  // optional [H][R/128], cleared by prep_fixup_kernel for the attention
   int L;         // tokens
   int Lv;        // video tokens (== L for Wan)
   int R;         // execution rows per head, ceil(L/128)*128
@@ -373,7 +374,10 @@ __global__ void __launch_bounds__(1024) prep_fixup_kernel(PrepParams p, int32_t*
   const int slot = t * H + h;
   int flagged;
   if (p.first && t == 0) {
-    flagged = 0;  // Q was not read: the attention kernel marks its head where a row leaves the range
+    flagged = 0;  // Q was not read: the attention kernel marks its head and block where a row leaves the range
+    const int nb = p.R / kBlock;
+    if (p.q_block_marks)
+      for (int i = threadIdx.x; i < nb; i += blockDim.x) p.q_block_marks[static_cast<int64_t>(h) * nb + i] = 0;
   } else if (p.wave_flags) {
     const int n = t < 2 ? p.nqk : p.nv;
     const int32_t* words = p.wave_flags + (t < 2 ? slot * static_cast<int64_t>(p.nqk)
@@ -575,7 +579,8 @@ int64_t prepare_flag_words(int64_t heads, int64_t seq_len, int64_t head_dim, int
 int prepare_fixup_impl(const void* q, const void* k, const void* v, const int32_t* perm, int64_t heads,
                       int64_t seq_len, int64_t head_dim, void* q_perm, void* k_perm, void* v_t,
                       int32_t* overflow, int32_t* wave_flags, int64_t q_tile_size, int64_t k_tile_size,
-                      bool skip_q, int32_t* exps, const int64_t* strides, dfs_stream_t stream) {
+                      bool skip_q, int32_t* exps, int32_t* q_block_marks, const int64_t* strides,
+                      dfs_stream_t stream) {
   DFS_REQUIRE(q && k && v && perm && k_perm && v_t && (overflow || wave_flags) && exps, "dfs_prepare_fixup: NULL operand");
   DFS_REQUIRE(head_dim == 64 || head_dim == 128, "dfs_prepare_fixup: head_dim=%lld (supported: 64, 128)",
               (long long)head_dim);
@@ -597,6 +602,7 @@ int prepare_fixup_impl(const void* q, const void* k, const void* v, const int32_
   p.R = static_cast<int>(kb * kBlock);
   p.wave_flags = wave_flags;
   p.first = skip_q ? 1 : 0;
+  p.q_block_marks = q_block_marks;
   if (wave_flags) wave_flag_counts(kb, head_dim, q_tile_size, k_tile_size, &p.nqk, &p.nv);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const dim3 grid(static_cast<unsigned>(heads), 3);
@@ -640,7 +646,7 @@ int dfs_prepare_fixup(const void* q, const void* k, const void* v, const int32_t
                       int64_t seq_len, int64_t head_dim, void* q_perm, void* k_perm, void* v_t,
                       int32_t* overflow, int32_t* exps, dfs_stream_t stream) {
   return dfs::prepare_fixup_impl(q, k, v, perm, heads, seq_len, head_dim, q_perm, k_perm, v_t, overflow, nullptr, 0, 0,
-                                 false, exps, nullptr, stream);
+                                 false, exps, nullptr, nullptr, stream);
 }
 
 }  // extern "C"

@@ -713,6 +713,55 @@ def test_whole_call_matches_single_entry_points(dev, d, heads, video, text, tile
         assert torch.equal(c.out, ref)
 
 
+@pytest.mark.parametrize("d,video,text,cut,plan", [
+    (128, 1300, 0, None, (1, 0, 1, 8)),    # uncut: the marked blocks alone are redone
+    (64, 1300, 0, None, (1, 0, 3, 4)),     # every block in parts
+    (128, 2000, 0, None, (1, 2, 2, 8)),    # the tail of each XCD's list in parts
+    (128, 1024, 200, None, (4, 0, 1, 8)),  # the text rows in parts
+    (128, 1024, 200, 1190, (4, 1, 2, 4)),  # both, with a second sequence
+])
+@pytest.mark.parametrize("rows", [(5,), (0, 700, 1023), "all", "inf"])
+def test_call_redoes_blocks_with_q_beyond_f16(dev, monkeypatch, d, video, text, cut, plan, rows):
+    """A given mask's call finds the rows of Q beyond f16 in the attention
+    itself and does their query blocks again in the scaled instance: the bits
+    of the separate calls, whose preparation finds the head and gives the
+    scaled instance all of it."""
+    L, heads = video + text, 2
+    print(f"q beyond f16 d={d} video={video} text={text} cut={cut} plan={plan} rows={rows}", flush=True)
+    g = torch.Generator().manual_seed(L)
+    q, k, v = (torch.randn((1, heads, L, d), generator=g).to(torch.bfloat16) for _ in range(3))
+    if rows == "inf":  # not beyond the range: it stays what it is in either instance
+        q[0, 1, 300, 3], q[0, 1, 301, 4] = math.inf, math.nan
+    else:
+        q[0, 1, slice(None) if rows == "all" else list(rows), 3] = 1.0e6
+    q, k, v = (t.to(dev) for t in (q, k, v))
+    layout = ScoringLayout(L, video, 16)
+    pol = hunyuan_policy(layout, 0.6) if text else wan_policy(layout, 0.4)
+    row_ptr = torch.from_numpy(pol.row_ptr(heads)).to(dev)
+    perm = torch.cat([torch.randperm(video, generator=g), torch.arange(video, L)]).to(torch.int32).to(dev)
+    cu = None if cut is None else torch.tensor([0, cut, L], dtype=torch.int32, device=dev)
+    prep = ops.prepare_qkv(q, k, v, perm, layout, q_operand=False)
+    cols, _, _ = ops.block_score_topk(prep, pol, row_ptr)
+    long_row = video // 128 if text else layout.q_blocks
+    monkeypatch.setattr(ops, "query_plan", lambda *a: (long_row, 1, 0, 1, 8))
+    ref = ops.bsa_fwd(prep, row_ptr, cols, out_perm=perm, cu_seqlens_q=cu, cu_seqlens_k=cu)
+    monkeypatch.setattr(ops, "query_plan", lambda *a: (long_row, *plan))
+    ops._call_template.cache_clear()
+    try:
+        call = ops.Call(q, k, v, perm, layout, pol, row_ptr, cols, out_perm=perm, cu_seqlens_q=cu, cu_seqlens_k=cu)
+        for _ in range(2):  # the marks of the first run are cleared
+            call.run()
+            got, want = call.out.nan_to_num(nan=7.0), ref.nan_to_num(nan=7.0)
+            if plan == (1, 0, 1, 8):
+                assert torch.equal(got, want)
+            elif rows == "inf":
+                assert torch.equal(call.out.isnan(), ref.isnan())
+            else:
+                assert torch.equal(got[0, 1], want[0, 1])
+    finally:
+        ops._call_template.cache_clear()
+
+
 @pytest.mark.parametrize("d,heads,L,cut,layouts,big", [
     (128, 3, 1000, None, ("token", "token", "token"), None),
     (64, 2, 700, None, ("head", "slice", "token"), None),

@@ -362,22 +362,56 @@ int main() {
 """
 
 
+def _run_on_host(tmp_path, source):
+    """Output lines, as integers, of a program over the kernels' host code."""
+    src, exe = tmp_path / "model.cpp", tmp_path / "model"
+    src.write_text(source)
+    csrc = os.path.join(os.path.dirname(_lib.__file__), "csrc")
+    subprocess.run(["g++", "-std=c++17", "-I", csrc, str(src), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout
+    return [[int(x) for x in line.split()] for line in out.splitlines()]
+
+
 @pytest.mark.skipif(shutil.which("g++") is None, reason="no host compiler")
 def test_common_instance_exit_does_not_depend_on_marks_of_its_launch(tmp_path):
     """The waves of a workgroup decide one by one whether the scaled instance
     has their head, so the answer may not change while the common instance
     runs and marks heads; the launches behind it see the mark. The rule of
     csrc/head_range.h, compiled for the host."""
-    src, exe = tmp_path / "model.cpp", tmp_path / "model"
-    src.write_text(HEAD_RANGE_MODEL)
-    csrc = os.path.join(os.path.dirname(_lib.__file__), "csrc")
-    subprocess.run(["g++", "-std=c++17", "-I", csrc, str(src), "-o", str(exe)], check=True)
-    lines = subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split("\n")[:-1]
+    lines = _run_on_host(tmp_path, HEAD_RANGE_MODEL)
     assert len(lines) == 12
-    for line in lines:
-        marks, q, k, scale_all, first, last, behind = map(int, line.split())
-        assert first == last == (scale_all or q or k), line
-        assert behind == (scale_all or q or k or marks), line
+    for marks, q, k, scale_all, first, last, behind in lines:
+        assert first == last == (scale_all or q or k)
+        assert behind == (scale_all or q or k or marks)
+
+
+SCALED_BLOCK_MODEL = r"""
+#include <cstdio>
+#include "head_range.h"
+struct P { const int32_t* exps; int32_t *q_marks, *q_block_marks; int H, Qb, scale_all; };
+int main() {
+  for (int marks = 0; marks < 2; ++marks)
+    for (int k = 0; k < 2; ++k)
+      for (int all = 0; all < 2; ++all) {
+        int32_t exps[6] = {0, 1, 0, k, 0, 0}, blocks[6] = {1, 0, 0, 0, 1, 0};  // of head 1, block 1 is marked
+        const P p{exps, marks ? exps : nullptr, marks ? blocks : nullptr, 2, 3, all};
+        printf("%d %d %d %d %d %d %d\n", marks, k, all, dfs::head_scaled(p, 1), dfs::scaled_block(p, 1, 0),
+               dfs::scaled_block(p, 1, 1), dfs::scaled_block(p, 1, 2));
+      }
+}
+"""
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="no host compiler")
+def test_scaled_instance_redoes_marked_blocks_only(tmp_path):
+    """Of a head whose Q alone left the range, found by the common instance,
+    the scaled instance does the marked query blocks; of any other head it has,
+    all."""
+    lines = _run_on_host(tmp_path, SCALED_BLOCK_MODEL)
+    assert len(lines) == 8
+    for marks, k, scale_all, takes, *blocks in lines:
+        assert takes
+        assert blocks == ([0, 1, 0] if marks and not k and not scale_all else [1, 1, 1])
 
 
 @pytest.mark.parametrize("shape,how", [
