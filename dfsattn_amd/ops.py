@@ -376,12 +376,13 @@ def _rows_in_place(x: torch.Tensor) -> Tuple[torch.Tensor, int, int]:
     """(x or a contiguous copy, head stride, row stride): the kernels read
     rows of D contiguous elements wherever they lie on 16-byte boundaries. An
     axis of one has no stride; a contiguous x may lie off the boundary too."""
-    heads, rows, dim = x.shape[-3:]
     sh, sl, sd = x.stride()[-3:]
-    sh, sl = (sh if heads > 1 else 0), (sl if rows > 1 else 0)
     if sd != 1 or sh % 8 or sl % 8 or x.data_ptr() % 16:
-        x = x.clone(memory_format=torch.contiguous_format)
-        sh, sl = rows * dim, dim
+        heads, rows, dim = x.shape[-3:]
+        sh, sl = (sh if heads > 1 else 0), (sl if rows > 1 else 0)
+        if sd != 1 or sh % 8 or sl % 8 or x.data_ptr() % 16:
+            x = x.clone(memory_format=torch.contiguous_format)
+            sh, sl = rows * dim, dim
     return x, sh, sl
 
 
