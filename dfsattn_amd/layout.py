@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import functools
 import math
+import operator
 from dataclasses import dataclass
 from typing import Optional, Tuple
 
@@ -124,9 +125,18 @@ class TopkPolicy:
         return (self.dense_row * kept + (self.q_blocks - self.dense_row) * self.k_blocks) * heads
 
 
+def scoring_layout(seq_len: int, video_len: int, tile: int, block: int, k_tile: Optional[int]) -> ScoringLayout:
+    """ScoringLayout of these sizes (checked once per set of sizes), in plain
+    integers whatever integer type they come in."""
+    if not type(seq_len) is type(video_len) is type(tile) is type(block) is type(k_tile) is int:
+        lay = ScoringLayout(seq_len, video_len, tile, block, k_tile=k_tile)
+        seq_len, video_len, tile, block, k_tile = map(
+            operator.index, (lay.seq_len, lay.video_len, lay.tile, lay.block, lay.k_tile))
+    return _scoring_layout(seq_len, video_len, tile, block, k_tile)
+
+
 @functools.lru_cache(maxsize=1024)
-def scoring_layout(seq_len: int, video_len: int, tile: int, block: int, k_tile: int) -> ScoringLayout:
-    """ScoringLayout of these sizes (checked once per set of sizes)."""
+def _scoring_layout(seq_len: int, video_len: int, tile: int, block: int, k_tile: int) -> ScoringLayout:
     return ScoringLayout(seq_len, video_len, tile, block, k_tile=k_tile)
 
 
@@ -154,25 +164,25 @@ def hunyuan_policy(layout: ScoringLayout, sparse_ratio: float) -> TopkPolicy:
     video_len // 128 on are kept in every video row, the video budget is
     k - text_blocks, and rows from video_len // 128 on are dense when text
     tokens exist."""
-    return _hunyuan_policy(layout, topk_count(sparse_ratio, layout.k_blocks))
-
-
-@functools.lru_cache(maxsize=1024)
-def _hunyuan_policy(layout: ScoringLayout, k: int) -> TopkPolicy:
     kb = layout.k_blocks
-    dense_start = layout.video_len // layout.block
+    return _hunyuan_policy(kb, layout.video_blocks, layout.video_len // layout.block, layout.text_len > 0,
+                           topk_count(sparse_ratio, kb))
+
+
+@functools.lru_cache(maxsize=1024, typed=True)  # a float video_len gives a policy of its own
+def _hunyuan_policy(kb: int, video_blocks: int, dense_start: int, text: bool, k: int) -> TopkPolicy:
     text_blocks = max(0, kb - dense_start)
-    dense_row = dense_start if layout.text_len > 0 else layout.q_blocks
+    dense_row = dense_start if text else kb
     if text_blocks > 0:
         budget = k - text_blocks
         if budget <= 0:
             raise AssertionError("num_video_blocks_to_select must be non-negative")
         if budget > dense_start:
             raise RuntimeError(f"selected index k out of range (k={budget}, columns={dense_start})")
-        return TopkPolicy(layout.q_blocks, kb, layout.video_blocks, dense_start, budget, dense_start, dense_row)
+        return TopkPolicy(kb, kb, video_blocks, dense_start, budget, dense_start, dense_row)
     if k > kb:
         raise RuntimeError(f"selected index k out of range (k={k}, columns={kb})")
-    return TopkPolicy(layout.q_blocks, kb, layout.video_blocks, kb, k, kb, dense_row)
+    return TopkPolicy(kb, kb, video_blocks, kb, k, kb, dense_row)
 
 
 @functools.lru_cache(maxsize=1024)

@@ -438,3 +438,27 @@ def test_rows_in_place_gives_16_byte_rows(shape, how, offset):
     assert torch.equal(y.as_strided((h, l, d), (sh, sl, 1)), x.reshape(h, l, d))
     if x.data_ptr() % 16 == 0 and how in ("contiguous", "token", "one head", "one row"):
         assert y.data_ptr() == x.data_ptr()  # read where it is
+
+
+def test_cached_layouts_and_policies_hold_plain_integers():
+    """Sizes that compare equal share a cache entry: one call's numpy, tensor
+    or refused float sizes leave nothing of their type to the next call."""
+    from dfsattn_amd.layout import scoring_layout
+    plain = (1511, 1401, 16, 128, 32)
+    for sizes in ((1511, np.int64(1401), 16, 128, 32), (1511, torch.tensor(1401), np.int32(16), 128, torch.tensor(32)),
+                  (1511, 1401, 16, 128, 32)):
+        lay = scoring_layout(*sizes)
+        assert lay == ScoringLayout(*plain[:4], k_tile=32)
+        assert all(type(x) is int for x in (lay.seq_len, lay.video_len, lay.tile, lay.block, lay.k_tile))
+    for i in range(1, 5):  # refused, as they always were further on, before and after the plain sizes are known
+        for base in ((1611, 1401, 16, 128, 32), plain):
+            sizes = [float(x) if j == i else x for j, x in enumerate(base)]
+            with pytest.raises(TypeError):
+                scoring_layout(*sizes)
+            assert type(scoring_layout(*base).video_len) is int
+    with pytest.raises(AssertionError, match="q_tile_size"):
+        scoring_layout(1511, 1401, 15.5, 128, 32)
+    assert scoring_layout(1511, 1401, 16, 128, None).k_tile == 16
+    hunyuan_policy(ScoringLayout(1521, 1401.0, 16), 0.5)
+    pol = hunyuan_policy(ScoringLayout(1521, 1401, 16), 0.5)
+    assert all(type(x) is int for x in (pol.n_cand, pol.k_pick, pol.dense_col, pol.dense_row))
