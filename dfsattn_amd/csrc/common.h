@@ -63,6 +63,18 @@ __device__ __forceinline__ void store_stream(uint4* p, const uint4& v) {
   const u32x4_t t = {v.x, v.y, v.z, v.w};
   __builtin_nontemporal_store(t, reinterpret_cast<u32x4_t*>(p));
 }
+template <bool STREAM>
+__device__ __forceinline__ uint4 load_chunk(const uint4* p) {
+  return STREAM ? load_stream(p) : *p;
+}
+template <bool STREAM>
+__device__ __forceinline__ void store_chunk(uint4* p, const uint4& v) {
+  if constexpr (STREAM)
+    store_stream(p, v);
+  else
+    *p = v;
+}
+constexpr int64_t kLastLevelCache = int64_t(256) << 20;  // bytes; all XCDs share it
 
 }  // namespace dfs
 

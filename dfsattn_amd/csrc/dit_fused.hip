@@ -170,16 +170,20 @@ void launch_adaln(const AdalnArgs& a, bool f16, hipStream_t s) {
 // out = float(x) + float(y) * gate[c], eight channels per thread. HBM-bound:
 // streaming accesses and one conversion per type reach 6.4 TB/s (158 us at
 // 32,760 x 5,120; 174 us with ordinary accesses and run-time types).
+// STREAM: for tensors beyond the last-level cache. Below it they take longer
+// than ordinary accesses where x and y were just written (8,000 x 5,120: 38.3
+// against 35.2 us; 4,000: 19.9, 18.0) and as long where they were not (40.3,
+// 39.1); above, 10,000 x 5,120: 48.1 against 52.1 and 49.8 against 51.2.
 // x and out may alias (each thread reads its eight elements before writing them).
-template <bool F16>
+template <bool F16, bool STREAM>
 __global__ void __launch_bounds__(256) gated_residual_kernel(const uint16_t* x, const uint16_t* __restrict__ y,
                                                              const float* __restrict__ gate, int64_t n8, int C,
                                                              uint16_t* out) {
   const int64_t i8 = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i8 >= n8) return;
   const int64_t e = i8 * 8;
-  const uint4 xv = load_stream(reinterpret_cast<const uint4*>(x + e));
-  const uint4 yv = load_stream(reinterpret_cast<const uint4*>(y + e));
+  const uint4 xv = load_chunk<STREAM>(reinterpret_cast<const uint4*>(x + e));
+  const uint4 yv = load_chunk<STREAM>(reinterpret_cast<const uint4*>(y + e));
   const int c = static_cast<int>(e % C);
   float g[8];
   load8(gate + c, g);
@@ -194,7 +198,7 @@ __global__ void __launch_bounds__(256) gated_residual_kernel(const uint16_t* x, 
     }
     packed[i / 2] = from_f32<F16>(r[0]) | (from_f32<F16>(r[1]) << 16);
   }
-  store_stream(reinterpret_cast<uint4*>(out + e), make_uint4(packed[0], packed[1], packed[2], packed[3]));
+  store_chunk<STREAM>(reinterpret_cast<uint4*>(out + e), make_uint4(packed[0], packed[1], packed[2], packed[3]));
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -255,9 +259,11 @@ extern "C" int dfs_gated_residual(const void* x, const void* y, const float* gat
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const uint16_t *xp = static_cast<const uint16_t*>(x), *yp = static_cast<const uint16_t*>(y);
   uint16_t* op = static_cast<uint16_t*>(out);
-  if (dtype == DFS_DTYPE_F16)
-    gated_residual_kernel<true><<<grid, block, 0, st>>>(xp, yp, gate, n8, static_cast<int>(channels), op);
+  const bool f16 = dtype == DFS_DTYPE_F16, stream_data = n8 * 16 * 3 > kLastLevelCache;
+  auto run = [&](auto kernel) { kernel<<<grid, block, 0, st>>>(xp, yp, gate, n8, static_cast<int>(channels), op); };
+  if (stream_data)
+    f16 ? run(gated_residual_kernel<true, true>) : run(gated_residual_kernel<false, true>);
   else
-    gated_residual_kernel<false><<<grid, block, 0, st>>>(xp, yp, gate, n8, static_cast<int>(channels), op);
+    f16 ? run(gated_residual_kernel<true, false>) : run(gated_residual_kernel<false, false>);
   return check_launch(name);
 }

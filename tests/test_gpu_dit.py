@@ -363,6 +363,19 @@ def test_gated_residual_bit_exact(dev):
     assert torch.equal(xd.cpu(), ref)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", [8738, 8739])  # x, y and out up to and beyond 256 MB: ordinary | streaming accesses
+@pytest.mark.parametrize("in_place", [False, True])
+def test_gated_residual_access_kinds(dev, dtype, rows, in_place):
+    from dfsattn_amd import ops
+    print(f"gated {dtype} rows={rows} in_place={in_place}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(rows)
+    x, y = (torch.randn(1, rows, 5120, generator=g, device=dev).to(dtype) for _ in range(2))
+    gate = torch.randn(5120, generator=g, device=dev)
+    ref = (x.float() + y.float() * gate).to(dtype)  # each product and sum rounded, as in the kernel
+    assert torch.equal(ops.gated_residual(x, y, gate, out=x if in_place else None), ref)
+
+
 @torch.no_grad()
 def test_dit_fused_elementwise_matches_torch_block(dev):
     """A dense step of the small DiT with the fused norm/modulation/residual
