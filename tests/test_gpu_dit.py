@@ -324,6 +324,22 @@ def test_adaln_modulate_matches_torch(dev, rows, C, mode):
     torch.testing.assert_close(got.float(), ref.float(), rtol=2.0 ** -7, atol=1e-5)
 
 
+@pytest.mark.parametrize("dtype,B,L,H,D", [
+    (torch.bfloat16, 1, 13107, 40, 128), (torch.bfloat16, 1, 13108, 40, 128),  # in and out up to | beyond 256 MB
+    (torch.float16, 2, 35, 3, 96), (torch.bfloat16, 1, 1, 1, 8), (torch.float16, 1, 9, 64, 128)])
+def test_head_split_alone(dev, dtype, B, L, H, D):
+    """The head split without norm and RoPE moves the bits, NaN and infinities
+    among them, with ordinary accesses inside the last-level cache and
+    streaming ones beyond."""
+    from dfsattn_amd import ops
+    print(f"split B={B} L={L} H={H} D={D} {dtype}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(L)
+    x = torch.randint(-2 ** 15, 2 ** 15, (B, L, H * D), generator=g, device=dev, dtype=torch.int16)
+    for out in (ops.norm_rope_heads(x.view(dtype), H), ops.head_norm_rope_heads(x.view(dtype), H) if D != 96 else None):
+        if out is not None:
+            assert torch.equal(out.view(torch.int16), x.unflatten(2, (H, D)).transpose(1, 2))
+
+
 @pytest.mark.parametrize("dtype,rows,C", [
     (torch.bfloat16, 8191, 520), (torch.bfloat16, 8192, 520), (torch.float16, 8193, 64),  # one | two rows per wave
     (torch.bfloat16, 8197, 5120),  # a lone last row in the widest two-row form
