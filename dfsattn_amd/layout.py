@@ -272,6 +272,7 @@ def attention_plan(heads: int, q_blocks: int, long_row: int, kept: int, kept_lon
     return long_parts, full_rows if parts > 1 else 0, parts
 
 
+@functools.lru_cache(maxsize=1024)
 def query_plan(layout: ScoringLayout, heads: int, head_dim: int, nnz: int) -> Tuple[int, int, int, int, int]:
     """(long_row, long_parts, full_rows, parts, chunks) of a call whose mask
     keeps ``nnz`` blocks: attention_plan with the text query blocks, which
