@@ -185,9 +185,10 @@ __device__ __forceinline__ bool long_block(const BsaParams& p, int g, int& h, in
 //    query blocks of 8 / chunks heads in flight. Fewer, longer ranges share
 //    more key blocks per L2 as long as the K/V of the heads in flight stays in
 //    the 256 MB last-level cache (head_chunks in the Python layout module):
-//    20,280 tokens x 40 heads 1,579 us with 8 ranges, 1,543 with 1; 4,680 x 40:
-//    170 and 150; 75,600 x 40 (38.7 MB a head): 32.4 ms with 8, 32.0 with 4,
-//    32.6 with 1. The ranges rotate with the head.
+//    whole calls in turn, 20,280 tokens x 40 heads 1,769 us with 8 ranges,
+//    1,738 with 4, 1,702 with 1; 4,680 x 40: 169 with 8, 155 with 1; 75,600 x 40
+//    (38.7 MB a head): 32.24 ms with 8, 31.90 with 4, 32.05 with 2, 32.41 with 1
+//    (a card drifts by about 1%). The ranges rotate with the head.
 //  * Long query blocks (HunyuanVideo's text rows keep every key block, three
 //    times the others at sparsity 0.3) go first: started in their place at the
 //    end of their head, the last head's ran on alone after everything else.

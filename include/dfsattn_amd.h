@@ -306,8 +306,10 @@ int dfs_bsa_fwd(const void* q_perm, const void* k_perm, const void* v_t,
  *   workspace   dfs_bsa_fwd_workspace_size bytes of device memory (16-byte
  *     aligned, may be NULL when nothing is cut): fp32 partial results, added
  *     up by a second kernel. Parts and long_parts lie in [1, 64].
- * The split changes the order of the fp32 sums only. Heads that need the
- * range exponents (exps) run uncut.
+ * Each part has its own softmax reference: the split changes the order of
+ * the fp32 sums and the 16-bit rounding of P (its error against exact results
+ * stays the same). NaN and infinities show in the same rows. Heads that need
+ * the range exponents (exps) run uncut.
  */
 int64_t dfs_bsa_fwd_workspace_size(int64_t heads, int64_t seq_len,
                                    int64_t head_dim, int64_t long_row,
