@@ -503,18 +503,18 @@ __device__ __forceinline__ void store_part(const BsaParams& p, int slot, const f
 // ascending order with the partner row's shared columns first, 0.4-1.2%
 // faster). Columns live in a bitmap at bit 2|c - qb| + (c > qb), compacted in
 // bit order. Columns >= Kb (the keys' blocks) are dropped, and all of them
-// where some thread asks to `skip`. bm: 2 W + 2 words of LDS scratch, W = (2 Kb
-// + 31) / 32. Every thread of the NT-thread workgroup calls this; it returns
-// the number of columns, the same to all of them, written to cols.
-template <int NT>
+// where skip() of some thread says so (asked last, when its operands have had
+// the list's time to arrive). bm: 2 W + 2 words of LDS scratch, W = (2 Kb +
+// 31) / 32. Every thread of the NT-thread workgroup calls this; it returns the
+// number of columns, the same to all of them, written to cols.
+template <int NT, typename Skip>
 __device__ int distance_order_cols(int Kb, const int32_t* __restrict__ col_idx, int qb, int beg, int n,
-                                   bool skip, int32_t* cols, uint32_t* bm, int tid, int w, int lane) {
+                                   int32_t* cols, uint32_t* bm, int tid, int w, int lane, Skip&& skip) {
   const int W = (2 * Kb + 31) >> 5;
   for (int i = tid; i < W; i += NT) bm[i] = 0u;
   uint32_t* const skipped = bm + 2 * W + 1;
   if (tid == 0) *skipped = 0u;
   block_barrier();
-  if (skip) *skipped = 1u;
   for (int i = tid; i < n; i += NT) {
     const int c = col_idx[beg + i];
     if (static_cast<unsigned>(c) < static_cast<unsigned>(Kb)) {
@@ -542,7 +542,7 @@ __device__ int distance_order_cols(int Kb, const int32_t* __restrict__ col_idx, 
       pre[w0 + j] = pos;
       pos += __popc(bm[w0 + j]);
     }
-    if (lane == 63) pre[W] = *skipped ? 0u : static_cast<uint32_t>(incl);  // this row's count
+    if (lane == 63) pre[W] = static_cast<uint32_t>(incl);  // this row's count
   }
   block_barrier();
   for (int i = tid; i < n; i += NT) {
@@ -552,9 +552,9 @@ __device__ int distance_order_cols(int Kb, const int32_t* __restrict__ col_idx, 
       cols[pre[b >> 5] + __popc(bm[b >> 5] & ((1u << (b & 31)) - 1u))] = c;
     }
   }
-  const int count = static_cast<int>(pre[W]);
+  if (skip()) *skipped = 1u;
   block_barrier();
-  return count;
+  return *skipped ? 0 : static_cast<int>(pre[W]);
 }
 
 #define BSA_KERNEL_ARGS                                                                                \
@@ -621,15 +621,15 @@ __device__ __forceinline__ void bsa_split_block(const uint16_t* __restrict__ q, 
     // Column list of this row into LDS (read back with uniform ds_reads).
     // A block with a row of Q beyond the f16 range is left to the scaled
     // instance, whole: its waves agree through the list's barriers.
-    bool skip = false;
-    if (QK_F16 && !SCALED && p.q_marks && q_beyond_f16<D>(q_raw, p.scale_log2)) {
+    auto left_to_scaled = [&] {
+      if (!QK_F16 || SCALED || !p.q_marks || !q_beyond_f16<D>(q_raw, p.scale_log2)) return false;
       p.q_marks[h] = 1;  // every writer stores the same marks
       p.q_block_marks[static_cast<int64_t>(h) * p.Qb + qb] = 1;
-      skip = true;
-    }
+      return true;
+    };
     const int total = __builtin_amdgcn_readfirstlane(
-        distance_order_cols<256>(Kb, col_idx, qb, beg, end - beg, skip, cols, reinterpret_cast<uint32_t*>(cols + p.Kb),
-                                 tid, w, lane));
+        distance_order_cols<256>(Kb, col_idx, qb, beg, end - beg, cols, reinterpret_cast<uint32_t*>(cols + p.Kb), tid,
+                                 w, lane, left_to_scaled));
     // This workgroup's part of the list (all of it for an unsplit block).
     const int t0 = SCALED ? 0 : total * wk.piece / wk.pieces;
     const int n = SCALED ? total : total * (wk.piece + 1) / wk.pieces;
